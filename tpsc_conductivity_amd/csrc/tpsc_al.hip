@@ -18,7 +18,6 @@
 
 namespace tpsc {
 
-#define AL_SLAB_THREADS 1024
 #define AL_PEN_THREADS 256
 #define AL_K_THREADS 512
 
@@ -35,39 +34,33 @@ __device__ __forceinline__ double al_dg0m(double x, double T, double nf)
 // Block j <= Nw: Grt[j*nk8 + w] = G0(r_w, -tau_j).  Block Nw+1: dGrt[w] = d/dtau G0(r,-tau) at
 // tau = 0 and dGrt[nk8 + w] = eps(r) - mu0 delta_r0 - dGrt[w] at tau = beta.
 template <int N>
-__global__ void __launch_bounds__(AL_SLAB_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_al_grt_slab(const double* __restrict__ ekw, const double* __restrict__ er, double mu0, double T, int Nw,
                   double* Grt, double* dGrt)
 {
-    constexpr int nk = N / 2 + 1;
-    constexpr long nk8 = (long)nk * (nk + 1) / 2;
+    constexpr long nk8 = (long)(N / 2 + 1) * (N / 2 + 2) / 2;
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int j = blockIdx.x;
-    const int tid = threadIdx.x, nt = blockDim.x;
     const double t = (double)j / (T * Nw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
+    each_wedge<N>([&](int l, int m, int i) {
         const double x = ekw[i] - mu0;
-        put_sym(slab, nk, l, m, (j <= Nw) ? al_g0m(x, t, T, nf) : al_dg0m(x, T, nf));
-    }
+        put_sym<N>(slab, l, m, (j <= Nw) ? al_g0m(x, t, T, nf) : al_dg0m(x, T, nf));
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        const double v = slab[m + l * nk];
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) {
+        const double v = slab[at<N>(l, m)];
         if (j <= Nw) {
             Grt[(long)j * nk8 + i] = v;
         } else {
             dGrt[i] = v;
             dGrt[nk8 + i] = ((i == 0) ? -mu0 : er[i]) - v;
         }
-    }
+    });
 }
 
 // Block j <= Nw: hGs[j*nq + q] = DST x DCT [h(r,tau_j) G0(r,-tau_j)] with h(r,tau) the
@@ -75,71 +68,54 @@ __global__ void __launch_bounds__(AL_SLAB_THREADS)
 // Blocks Nw+1+side: slope at tau = 0 / beta of the same product (:5159-5229),
 // dh(r) G0(r,-tau_b) + h(r,tau_b) dG0(r,-tau_b), back to q -> dhG[side*nq + q].
 template <int N>
-__global__ void __launch_bounds__(AL_SLAB_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_al_hg_slab(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ Grt,
                  const double* __restrict__ dGrt, double mu0, double T, int Nw, double* hGs, double* dhG)
 {
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    constexpr int PER = (int)((nq + AL_SLAB_THREADS - 1) / AL_SLAB_THREADS);
+    constexpr int PER = lambda_per_thread<N>();
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int b = blockIdx.x;
-    const int tid = threadIdx.x;
     const int jt = (b <= Nw) ? b : ((b == Nw + 1) ? 0 : Nw);
     const double t = (double)jt / (T * Nw);
-    for (long s = tid; s < nq; s += AL_SLAB_THREADS) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
-        slab[s] = hf0_val(0, ek[m + (l + 1) * nk], dek[s], mu0, T, t, nf);
-    }
+    each_lambda<N>([&](int l, int m, int s) {
+        slab[at<N>(l + 1, m)] = hf0_val(0, ek[m + (l + 1) * nk], dek[s], mu0, T, t, nf);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     if (b <= Nw) {
         const double* g = Grt + (long)b * nk8;
-        for (long s = tid; s < nq; s += AL_SLAB_THREADS) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
-            slab[s] *= g[fold_idx(l + 1, m, N)];
-        }
+        each_lambda<N>([&](int l, int m, int) { slab[at<N>(l + 1, m)] *= g[fold_idx(l + 1, m, N)]; });
         __syncthreads();
-        slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+        slab_r2r_2d<double, N, 1>(slab, tw);
         double* o = hGs + (long)b * nq;
-        for (long s = tid; s < nq; s += AL_SLAB_THREADS) o[s] = slab[s];
+        each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
         return;
     }
     const int side = b - Nw - 1;
     double st[PER];
-#pragma unroll
-    for (int c = 0; c < PER; c++) {
-        const long s = tid + (long)c * AL_SLAB_THREADS;
-        st[c] = 0.0;
-        if (s < nq) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
-            st[c] = slab[s] * dGrt[side * nk8 + fold_idx(l + 1, m, N)];
-        }
-    }
+    each_lambda_slot<N>([&](int l, int m, int, int c) {
+        st[c] = slab[at<N>(l + 1, m)] * dGrt[side * nk8 + fold_idx(l + 1, m, N)];
+    });
     __syncthreads();
-    for (long s = tid; s < nq; s += AL_SLAB_THREADS) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
-        slab[s] = h_slope_val(side, ek[m + (l + 1) * nk], dek[s], mu0, T, nf);
-    }
+    each_lambda<N>([&](int l, int m, int s) {
+        slab[at<N>(l + 1, m)] = h_slope_val(side, ek[m + (l + 1) * nk], dek[s], mu0, T, nf);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     const double* g = Grt + (long)jt * nk8;
-#pragma unroll
-    for (int c = 0; c < PER; c++) {
-        const long s = tid + (long)c * AL_SLAB_THREADS;
-        if (s < nq) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
-            slab[s] = slab[s] * g[fold_idx(l + 1, m, N)] + st[c];
-        }
-    }
+    each_lambda_slot<N>([&](int l, int m, int, int c) {
+        slab[at<N>(l + 1, m)] = slab[at<N>(l + 1, m)] * g[fold_idx(l + 1, m, N)] + st[c];
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-    for (long s = tid; s < nq; s += AL_SLAB_THREADS) dhG[side * nq + s] = slab[s];
+    slab_r2r_2d<double, N, 1>(slab, tw);
+    each_lambda<N>([&](int l, int m, int s) { dhG[side * nq + s] = slab[at<N>(l + 1, m)]; });
 }
 
 // Per Lambda point q: clamped spline of hG(q,tau_j), j = 0..L, slopes dhG; hw[q*H] = twice its
@@ -297,20 +273,19 @@ __global__ void __launch_bounds__(AL_PEN_THREADS)
 // dHG2(r,0) = -dHG(r,beta), dHG2(r,beta) = -dHG(r,0).
 // Planes: HGs, P1s, P2s [c][t][q]; dHq [c][side][q]; dP [which][side][c][q].
 template <int N>
-__global__ void __launch_bounds__(AL_SLAB_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_al_prod_slab(const double* __restrict__ HGs, const double* __restrict__ dHq, const double* __restrict__ Grt,
                    const double* __restrict__ dGrt, int L, double* P1s, double* P2s, double* dP)
 {
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    constexpr int PER = (int)((nq + AL_SLAB_THREADS - 1) / AL_SLAB_THREADS);
+    constexpr int PER = lambda_per_thread<N>();
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
-    const int tid = threadIdx.x;
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const long plane = (long)(L + 1) * nq;
     const int b = blockIdx.x;
     int tA, c, which = 0, side = 0;
@@ -326,60 +301,43 @@ __global__ void __launch_bounds__(AL_SLAB_THREADS)
         tA = which ? (side ? 0 : L) : (side ? L : 0);
     }
     const double* src = HGs + c * plane + (long)tA * nq;
-    for (long s = tid; s < nq; s += AL_SLAB_THREADS) slab[s] = nf * src[s];
+    each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = nf * src[s]; });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-    double st[PER];
-    int fo[PER];
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const long s = tid + (long)i * AL_SLAB_THREADS;
-        st[i] = 0.0;
-        fo[i] = 0;
-        if (s < nq) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
-            fo[i] = (int)fold_idx(l + 1, m, N);
-            st[i] = slab[s];
-        }
-    }
+    slab_r2r_2d<double, N, 1>(slab, tw);
+    double st[PER];  // HG(r,tau) of the thread's points
+    each_lambda_slot<N>([&](int l, int m, int, int i) { st[i] = slab[at<N>(l + 1, m)]; });
     __syncthreads();
     if (main_blk) {
 #pragma unroll 1
         for (int pass = 0; pass < 2; pass++) {
             const int tg = pass ? L - tA : tA;
             const double* g = Grt + (long)tg * nk8;
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                const long s = tid + (long)i * AL_SLAB_THREADS;
-                if (s < nq) slab[s] = st[i] * g[fo[i]];
-            }
+            each_lambda_slot<N>(
+                [&](int l, int m, int, int i) { slab[at<N>(l + 1, m)] = st[i] * g[fold_idx(l + 1, m, N)]; });
             __syncthreads();
-            slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+            slab_r2r_2d<double, N, 1>(slab, tw);
             double* o = (pass ? P2s : P1s) + c * plane + (long)tg * nq;
-            for (long s = tid; s < nq; s += AL_SLAB_THREADS) o[s] = slab[s];
+            each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
             __syncthreads();
         }
         return;
     }
     const double* dg = dGrt + side * nk8;
-#pragma unroll
-    for (int i = 0; i < PER; i++) st[i] *= dg[fo[i]];
+    each_lambda_slot<N>([&](int l, int m, int, int i) { st[i] *= dg[fold_idx(l + 1, m, N)]; });
     const int ds = which ? 1 - side : side;
     const double sgn = which ? -1.0 : 1.0;
     const double* dsrc = dHq + (long)(c * 2 + ds) * nq;
-    for (long s = tid; s < nq; s += AL_SLAB_THREADS) slab[s] = nf * dsrc[s];
+    each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = nf * dsrc[s]; });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     const double* g = Grt + (long)(side ? L : 0) * nk8;
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const long s = tid + (long)i * AL_SLAB_THREADS;
-        if (s < nq) slab[s] = sgn * slab[s] * g[fo[i]] + st[i];
-    }
+    each_lambda_slot<N>([&](int l, int m, int, int i) {
+        slab[at<N>(l + 1, m)] = sgn * slab[at<N>(l + 1, m)] * g[fold_idx(l + 1, m, N)] + st[i];
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     double* o = dP + (long)((which * 2 + side) * 2 + c) * nq;
-    for (long s = tid; s < nq; s += AL_SLAB_THREADS) o[s] = slab[s];
+    each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // Dyson G(k, i w_f) = 1/(i w_f + mu - e - Sigma(k,iw_f)), Sigma from the stored form for
@@ -493,13 +451,6 @@ __global__ void __launch_bounds__(NT)
 }
 
 // ================================================================== launchers
-static size_t al_slab_lds(int N, bool lambda)
-{
-    const int nk = N / 2 + 1;
-    const size_t n = lambda ? (size_t)nk * (nk - 2) : (size_t)nk * nk;
-    return ((n * sizeof(double) + 15) & ~(size_t)15) + 2 * sizeof(double) * (size_t)N;
-}
-
 #define AL_DISPATCH_N(N, ...)                                       \
     switch (N) {                                                    \
         case 4: { constexpr int NN = 4; __VA_ARGS__; } break;       \
@@ -549,12 +500,12 @@ static void al_set_lds(K kern, size_t bytes)
 hipError_t launch_al_setup(const Grid& g, const DevArrays& d, const ALArrays& a, double mu0, hipStream_t s)
 {
     AL_DISPATCH_N(g.N, {
-        const size_t lw = al_slab_lds(g.N, false), lq = al_slab_lds(g.N, true);
-        al_set_lds(k_al_grt_slab<NN>, lw);
-        hipLaunchKernelGGL(k_al_grt_slab<NN>, dim3(g.Nw + 2), dim3(AL_SLAB_THREADS), lw, s, d.ekw, d.er, mu0, g.T,
+        constexpr size_t lds = slab_bytes(NN, sizeof(double));
+        al_set_lds(k_al_grt_slab<NN>, lds);
+        hipLaunchKernelGGL(k_al_grt_slab<NN>, dim3(g.Nw + 2), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.er, mu0, g.T,
                            g.Nw, a.Grt, a.dGrt);
-        al_set_lds(k_al_hg_slab<NN>, lq);
-        hipLaunchKernelGGL(k_al_hg_slab<NN>, dim3(g.Nw + 3), dim3(AL_SLAB_THREADS), lq, s, d.ek, d.dek, a.Grt,
+        al_set_lds(k_al_hg_slab<NN>, lds);
+        hipLaunchKernelGGL(k_al_hg_slab<NN>, dim3(g.Nw + 3), dim3(SlabShape<NN>::NT), lds, s, d.ek, d.dek, a.Grt,
                            a.dGrt, mu0, g.T, g.Nw, a.P1s, a.dhG);
     });
     hipError_t e = launch_transpose_d(a.P1s, a.P1p, g.nq, g.Nw + 1, s);
@@ -580,9 +531,9 @@ hipError_t launch_al_freq(const Grid& g, const DevArrays& d, const ALArrays& a, 
         if ((e = launch_transpose_d(a.P1p + c * plane, a.HGs + c * plane, g.Nw + 1, (int)g.nq, s)) != hipSuccess)
             return e;
     AL_DISPATCH_N(g.N, {
-        const size_t lq = al_slab_lds(g.N, true);
-        al_set_lds(k_al_prod_slab<NN>, lq);
-        hipLaunchKernelGGL(k_al_prod_slab<NN>, dim3(2 * (g.Nw + 1) + 8), dim3(AL_SLAB_THREADS), lq, s, a.HGs, a.dHq,
+        constexpr size_t lds = slab_bytes(NN, sizeof(double));
+        al_set_lds(k_al_prod_slab<NN>, lds);
+        hipLaunchKernelGGL(k_al_prod_slab<NN>, dim3(2 * (g.Nw + 1) + 8), dim3(SlabShape<NN>::NT), lds, s, a.HGs, a.dHq,
                            a.Grt, a.dGrt, g.Nw, a.P1s, a.P2s, a.dP);
     });
     for (int c = 0; c < 2; c++) {

@@ -1497,7 +1497,6 @@ int tpsc_create(const tpsc_params* p, tpsc_ctx** out)
     rc |= dalloc(c, &d.df0V, 2 * std::max<long>(nq, 1));
     rc |= dalloc(c, &d.hVb, 2 * std::max<long>(nq, 1));
     rc |= dalloc(c, &d.f0Vb, 2 * std::max<long>(nq, 1));
-    rc |= dalloc(c, &d.bscr, 4 * std::max<long>(nq, 1));
     rc |= dalloc(c, &d.hT, (size_t)(Nw + 1) * std::max<long>(nq, 1), es);
     rc |= dalloc(c, &d.f0T, (size_t)(Nw + 1) * std::max<long>(nq, 1), es);
     rc |= dalloc(c, &d.poles, 64 * (size_t)std::max<long>(nq, 1));
@@ -1505,7 +1504,6 @@ int tpsc_create(const tpsc_params* p, tpsc_ctx** out)
     rc |= dalloc(c, &d.jjpart, (size_t)std::max<long>(nblk, 1) * 2 * nwb);
     rc |= dalloc(c, &d.jjscal, (size_t)std::max<long>(nblk, 1) * 4);
     rc |= dalloc(c, &d.kx0part, 2 * (size_t)nk);
-    rc |= dalloc(c, &d.tmp, 4 * (size_t)nk8);
     rc |= dalloc(c, &d.part, kPartCap);
     rc |= dalloc(c, &d.jjred, 2 * (size_t)nwb + 4);
     rc |= dalloc(c, &d.red, 16);

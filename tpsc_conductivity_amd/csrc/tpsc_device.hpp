@@ -2,9 +2,10 @@
 //
 //  * cd            : complex double; division by the plain formula with one reciprocal of
 //                    (c^2+d^2)
-//  * wave_r2r_*    : FFTW REDFT00 / RODFT00 of LDS-resident rows, two real rows packed
-//                    into one complex sequence, one length-N FFT per 64-lane wavefront
-//                    (R values per lane, cross-lane radix-2 stages with xor shuffles)
+//  * wave_r2r_lines: FFTW REDFT00 / RODFT00 of LDS-resident lines, two real lines packed into
+//                    one complex sequence of period N = A B: A-point and B-point DFTs in
+//                    registers, one exchange through the lines' own LDS, only the lanes that
+//                    the even (odd) symmetry leaves independent
 //  * block_fft     : workgroup Stockham radix-4/2 complex FFT of a tau-pencil in LDS
 //  * block_spline  : clamped cubic spline moments on a uniform grid, solved as a
 //                    causal + anti-causal first-order recursion (pole sqrt(3)-2) over
@@ -119,52 +120,8 @@ struct cplx_of<float> {
     using type = cf;
 };
 
-// v from lane (lane ^ M), M a power of two < 64.  M = 1, 2: DPP quad permutation; M = 4:
-// quad permutation 3-2-1-0 then the 8-lane mirror (i -> 7 - i = i ^ 7); M = 8: 8-lane mirror
-// then the 16-lane mirror (i ^ 7 ^ 15); these are VALU moves.  M = 16: ds_swizzle in
-// bitmask mode (xor within 32 lanes); M = 32: ds_bpermute.
-template <int M>
-__device__ __forceinline__ int xor_lane_i(int x)
-{
-    if constexpr (M == 1) return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, false);
-    else if constexpr (M == 2) return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, false);
-    else if constexpr (M == 4) {
-        const int t = __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xF, 0xF, false);
-        return __builtin_amdgcn_update_dpp(0, t, 0x141, 0xF, 0xF, false);
-    } else if constexpr (M == 8) {
-        const int t = __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, false);
-        return __builtin_amdgcn_update_dpp(0, t, 0x140, 0xF, 0xF, false);
-    } else if constexpr (M == 16)
-        return __builtin_amdgcn_ds_swizzle(x, 0x401F);
-    else
-        return __shfl_xor(x, M, 64);
-}
-template <int M>
-__device__ __forceinline__ float xor_lane(float v)
-{
-    return __int_as_float(xor_lane_i<M>(__float_as_int(v)));
-}
-template <int M>
-__device__ __forceinline__ double xor_lane(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = xor_lane_i<M>((int)(b & 0xffffffffLL));
-    const int hi = xor_lane_i<M>((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-template <int M>
-__device__ __forceinline__ cd shfl_xor_c(cd v)
-{
-    return cd{xor_lane<M>(v.x), xor_lane<M>(v.y)};
-}
-template <int M>
-__device__ __forceinline__ cf shfl_xor_c(cf v)
-{
-    return cf{xor_lane<M>(v.x), xor_lane<M>(v.y)};
-}
-
 // ---------------------------------------------------------------------------------
-// in-register DFT of length R (R = 1, 2, 3, 4, 8), forward sign, natural order output
+// in-register DFT of length R (R = 1, 2, 3, 4, 6, 8, 12, 16), forward sign, natural order output
 // ---------------------------------------------------------------------------------
 template <typename C>
 __device__ inline C mul_mi(C a) { return C{a.y, -a.x}; }  // a * (-i)
@@ -209,137 +166,284 @@ __device__ __forceinline__ void reg_dft(C* v)
             v[k] = e[k] + o[k];
             v[k + 4] = e[k] - o[k];
         }
-    }
-}
-
-// ---------------------------------------------------------------------------------
-// REDFT00 / RODFT00 of LDS rows by one length-L complex FFT per row pair.
-//   kind 0 (REDFT00): rows of n = L/2+1 values, even extension z_j = x_{min(j,L-j)}
-//   kind 1 (RODFT00): rows of n = L/2-1 values, odd extension z_0 = z_{L/2} = 0,
-//                     z_j = x_{j-1}, z_{L-j} = -x_{j-1}
-// Row r element e lives at base[r*rs + e*es].  The DFT of a real even (odd) sequence is
-// real (imaginary), so packing rows r and r+1 as real and imaginary parts yields both
-// transforms from one FFT.  L = R*G with G (lanes per FFT) the largest power of two that
-// divides L, at most 64, and R in {1, 2, 3, 4, 8} (L = 2^k or 3*2^k).  The arithmetic runs
-// in the precision of Real (FP64 or FP32).
-// Must be called by every thread of the block (uniform control flow); caller syncs.
-// tw: LDS table tw[t] = exp(-2 pi i t / L), t < L, in the precision of Real.
-// ---------------------------------------------------------------------------------
-// cross-lane DIF stages of span HH, HH/2, ..., 1 (lane p of a G-lane group).  The lower
-// lane of a pair keeps v + o, the upper one (o - v) w; both are fma(s, v, o) w' with
-// (s, w') = (1, 1) or (-1, w), so no lane evaluates both branches.  Exact: fma(+-1, v, o) rounds
-// as o +- v, and the product with 1 + 0i returns its operand.
-template <int HH, int R, int L, typename C>
-__device__ __forceinline__ void dif_stages(C* v, int p, const C* tw)
-{
-    if constexpr (HH >= 1) {
+    } else if constexpr (R == 6) {
+        // 2 x 3: two-point DFTs over n = n2 + 3 n1, w6^(n2 k1), three-point DFTs over n2
         using F = decltype(C{}.x);
-        const bool upper = (p & HH) != 0;
-        const C wt = tw[(p & (HH - 1)) * (L / (2 * HH))];
-        const C w = upper ? wt : C{(F)1, (F)0};
-        const F sg = upper ? (F)-1 : (F)1;
+        const F h = (F)0.86602540378443864676;
+        C e[3], o[3];
 #pragma unroll
-        for (int k1 = 0; k1 < R; k1++) {
-            const C o = shfl_xor_c<HH>(v[k1]);
-            v[k1] = C{fma(sg, v[k1].x, o.x), fma(sg, v[k1].y, o.y)} * w;
+        for (int i = 0; i < 3; i++) {
+            e[i] = v[i] + v[i + 3];
+            o[i] = v[i] - v[i + 3];
         }
-        dif_stages<HH / 2, R, L>(v, p, tw);
+        o[1] = o[1] * C{(F)0.5, -h};
+        o[2] = o[2] * C{(F)-0.5, -h};
+        reg_dft<3>(e);
+        reg_dft<3>(o);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            v[2 * i] = e[i];
+            v[2 * i + 1] = o[i];
+        }
+    } else if constexpr (R == 12) {
+        // 3 x 4: three-point DFTs over n = n2 + 4 n1, w12^(n2 k1), four-point DFTs over n2
+        using F = decltype(C{}.x);
+        const F h = (F)0.86602540378443864676, q = (F)0.5;
+        C a[3][4];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; n2++) {
+            C t[3] = {v[n2], v[n2 + 4], v[n2 + 8]};
+            reg_dft<3>(t);
+            a[0][n2] = t[0];
+            a[1][n2] = t[1];
+            a[2][n2] = t[2];
+        }
+        a[1][1] = a[1][1] * C{h, -q};
+        a[1][2] = a[1][2] * C{q, -h};
+        a[1][3] = mul_mi(a[1][3]);
+        a[2][1] = a[2][1] * C{q, -h};
+        a[2][2] = a[2][2] * C{-q, -h};
+        a[2][3] = C{-a[2][3].x, -a[2][3].y};
+#pragma unroll
+        for (int k1 = 0; k1 < 3; k1++) {
+            reg_dft<4>(a[k1]);
+#pragma unroll
+            for (int k2 = 0; k2 < 4; k2++) v[k1 + 3 * k2] = a[k1][k2];
+        }
+    } else if constexpr (R == 16) {
+        // 4 x 4: four-point DFTs over n = n2 + 4 n1, w16^(n2 k1), four-point DFTs over n2
+        using F = decltype(C{}.x);
+        const F h = (F)0.70710678118654752440, c1 = (F)0.92387953251128675613, s1 = (F)0.38268343236508977173;
+        C a[4][4];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; n2++) {
+            C t[4] = {v[n2], v[n2 + 4], v[n2 + 8], v[n2 + 12]};
+            reg_dft<4>(t);
+#pragma unroll
+            for (int k1 = 0; k1 < 4; k1++) a[k1][n2] = t[k1];
+        }
+        auto w2 = [&](C z) { return C{h * (z.x + z.y), h * (z.y - z.x)}; };   // z w16^2
+        auto w6 = [&](C z) { return C{h * (z.y - z.x), -h * (z.x + z.y)}; };  // z w16^6
+        a[1][1] = a[1][1] * C{c1, -s1};
+        a[1][2] = w2(a[1][2]);
+        a[1][3] = a[1][3] * C{s1, -c1};
+        a[2][1] = w2(a[2][1]);
+        a[2][2] = mul_mi(a[2][2]);
+        a[2][3] = w6(a[2][3]);
+        a[3][1] = a[3][1] * C{s1, -c1};
+        a[3][2] = w6(a[3][2]);
+        a[3][3] = a[3][3] * C{-c1, s1};
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++) {
+            reg_dft<4>(a[k1]);
+#pragma unroll
+            for (int k2 = 0; k2 < 4; k2++) v[k1 + 4 * k2] = a[k1][k2];
+        }
     }
 }
 
-template <typename Real, int R, int G, int KIND>
-__device__ __forceinline__ void wave_r2r_rows(Real* base, int nrows, int rs, int es,
-                                              const typename cplx_of<Real>::type* tw)
+// ---------------------------------------------------------------------------------
+// Slab transforms: REDFT00 (kind 0) and RODFT00 (kind 1) along both axes of an LDS slab.
+//
+// A slab holds element (i, j), 0 <= i, j < nk = N/2+1, at base[j + i * LD].  A kind-1 axis keeps the
+// natural index too: its elements are 1 .. nk-2, and lines 0 and nk-1 hold nothing.  The even
+// (odd) extension of a line has period N, and its DFT is real (imaginary), so lines f and f + P
+// (P = half the lines) packed as real and imaginary parts give both transforms from one complex
+// FFT of length N = A B:
+//   z[p + B k] -> A-point DFTs over k (lane p) -> w_N^(p k1) -> B-point DFTs over p (lane k1)
+//   -> Z[k1 + A k2].
+// The packed sequence is itself even (odd), so z[N - j] = +-z[j] fixes the DFTs of p > B/2 from
+// those of B - p, and the outputs of k1 > A/2 from those of A - k1: max(A, B)/2 + 1 lanes carry a
+// whole FFT (9 of 16 for N = 256) and 64 lanes hold SlabShape::F of them.  The intermediate values
+// are exchanged inside one wavefront through the LDS of the two lines themselves (real parts in line
+// f, imaginary parts in line f + P), so an axis takes one workgroup barrier.
+//
+// What bounds it: FP64 (FP32) VALU issue and LDS bandwidth, in about equal parts: at N = 256 a lane
+// issues two 16-point DFTs, 16 complex products and ~140 LDS accesses per line pair.  LD = lanes per
+// FFT (mod 16) spreads the lanes of a wavefront over the LDS banks in both axes; the exchange slots
+// are permuted by an exclusive or for the same reason.
+// Against cross-lane radix-2 stages (one FFT per wavefront, shuffles between lanes, a full-period FFT
+// for a line pair), kernel times at 256^2 x 2048 before -> after: FP64 chi0 1004 -> 461 us, vertex 298
+// -> 104, Sigma 1092 -> 362, h/f0 1636 -> 976, hV/f0V 1375 -> 844; FP32 384 -> 264, 115 -> 61, 440 ->
+// 222, 659 -> 628, 758 -> 399 (they overlap on three streams).
+// ---------------------------------------------------------------------------------
+constexpr int slab_A(int N)
 {
-    using C = typename cplx_of<Real>::type;
-    constexpr int L = R * G;
-    constexpr int P = 64 / G;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int nwaves = blockDim.x >> 6;
-    const int sub = lane / G, p = lane % G;
-    const int npairs = (nrows + 1) >> 1;
-    constexpr int half = L / 2;
-    const int rounds = (npairs + nwaves * P - 1) / (nwaves * P);
-    int br = 0;  // bit reversal of p over log2(G) bits
-#pragma unroll
-    for (int b = 1, q = G >> 1; b < G; b <<= 1, q >>= 1)
-        if (p & b) br |= q;
-    for (int rd = 0; rd < rounds; rd++) {
-        const int task = (rd * nwaves + wave) * P + sub;
-        const bool valid = task < npairs;
-        const int r1 = 2 * task, r2 = 2 * task + 1;
-        const bool has2 = valid && (r2 < nrows);
-        const long o1 = (long)r1 * rs, o2 = (long)r2 * rs;
-        C v[R];
-#pragma unroll
-        for (int k = 0; k < R; k++) {
-            const int j = p + G * k;
-            Real a = 0, b = 0;
-            if (KIND == 0) {
-                const int e = (j <= half) ? j : L - j;
-                if (valid) a = base[o1 + (long)e * es];
-                if (has2) b = base[o2 + (long)e * es];
-            } else if (j != 0 && j != half) {
-                const int e = (j < half) ? j - 1 : L - j - 1;
-                if (valid) a = base[o1 + (long)e * es];
-                if (has2) b = base[o2 + (long)e * es];
-                if (j > half) {
-                    a = -a;
-                    b = -b;
-                }
-            }
-            v[k] = C{a, b};
-        }
-        reg_dft<R>(v);
-        // twiddle by exp(-2 pi i p k1 / L)
-#pragma unroll
-        for (int k1 = 1; k1 < R; k1++) v[k1] = v[k1] * tw[(p * k1) % L];
-        // G-point DIF across lanes; lane p ends with output index bitrev(p)
-        dif_stages<G / 2, R, L>(v, p, tw);
-        if (valid) {
-#pragma unroll
-            for (int k1 = 0; k1 < R; k1++) {
-                const int k = k1 + R * br;
-                if (KIND == 0) {
-                    if (k <= half) {
-                        base[o1 + (long)k * es] = v[k1].x;
-                        if (has2) base[o2 + (long)k * es] = v[k1].y;
-                    }
-                } else if (k >= 1 && k <= half - 1) {
-                    base[o1 + (long)(k - 1) * es] = -v[k1].y;
-                    if (has2) base[o2 + (long)(k - 1) * es] = v[k1].x;
-                }
-            }
-        }
-    }
+    return N == 4 ? 2 : (N == 8 || N == 16) ? 4 : (N == 12 || N == 24 || N == 48) ? 6
+         : (N == 32 || N == 64 || N == 128) ? 8 : (N == 96 || N == 192) ? 12 : 16;
 }
-
-// fill tw[t] = exp(-2 pi i t / L) for t < L (block-cooperative; caller syncs); the angle
-// is evaluated in FP64 and rounded to the table precision
-template <typename C>
-__device__ __forceinline__ void fill_twiddles(C* tw, int L)
+struct SlabDims {
+    int nk, A, B, lanes, F, P, slots, LD, rows, waves, threads;
+    long elems;
+};
+constexpr SlabDims slab_dims(int N)
+{
+    SlabDims d{};
+    d.nk = N / 2 + 1;
+    d.A = slab_A(N);
+    d.B = N / d.A;
+    d.lanes = (d.A > d.B ? d.A : d.B) / 2 + 1;  // lanes per FFT
+    d.F = 64 / d.lanes;                         // FFTs per wavefront
+    d.P = (d.nk + 1) / 2;
+    d.slots = d.B * (d.A / 2 + 1) - (d.B - 1) / 2;  // exchanged values per FFT
+    const int least = d.slots > d.nk + 1 ? d.slots : d.nk + 1;
+    d.LD = least;
+    while (d.LD % 16 != d.lanes % 16) d.LD++;
+    d.rows = least;
+    d.waves = (d.P + d.F - 1) / d.F;
+    // one round of FFTs per axis, and at least four wavefronts for the pointwise phases
+    d.threads = 64 * (d.waves > 4 ? d.waves : 4);
+    d.elems = (long)d.rows * d.LD;
+    return d;
+}
+template <int N>
+struct SlabShape {
+    static constexpr SlabDims D = slab_dims(N);
+    static constexpr int A = D.A, B = D.B, F = D.F, LD = D.LD, NT = D.threads;
+};
+// LDS bytes of a slab and its twiddle table (N/4 + 1 entries)
+constexpr size_t slab_bytes(int N, size_t elem)
+{
+    return (((size_t)slab_dims(N).elems * elem + 15) & ~(size_t)15) + 2 * elem * (size_t)(N / 4 + 1);
+}
+// the twiddle table behind the slab, 16-byte aligned
+template <int N, typename Real>
+__device__ __forceinline__ typename cplx_of<Real>::type* slab_tw(Real* slab)
+{
+    constexpr size_t off = ((size_t)slab_dims(N).elems * sizeof(Real) + 15) & ~(size_t)15;
+    return (typename cplx_of<Real>::type*)((char*)slab + off);
+}
+// tw[t] = exp(-2 pi i t / N), t <= N/4 (block-cooperative; caller syncs); the angle is evaluated in
+// FP64 and rounded to the table precision
+template <int N, typename C>
+__device__ __forceinline__ void fill_twiddles(C* tw)
 {
     using F = decltype(C{}.x);
-    for (int t = threadIdx.x; t < L; t += blockDim.x) {
+    for (int t = threadIdx.x; t <= N / 4; t += blockDim.x) {
         double s, c;
-        sincospi(2.0 * (double)t / (double)L, &s, &c);
+        sincospi(2.0 * (double)t / (double)N, &s, &c);
         tw[t] = C{(F)c, (F)(-s)};
     }
 }
 
-// 2D transform of an n0 x n1 LDS slab (row-major, row stride ld): axis 1 then axis 0.
-// KIND0 along axis 0 (slow index), KIND1 along axis 1 (0: REDFT00, 1: RODFT00).  Both use
-// FFT length N.
-template <typename Real, int N, int KIND0, int KIND1>
-__device__ __forceinline__ void slab_r2r_2d(Real* slab, int n0, int n1, int ld, const typename cplx_of<Real>::type* tw)
+// LDS accesses of one wavefront complete in order; this keeps the compiler's order
+__device__ __forceinline__ void wave_lds_order()
 {
-    constexpr int G = ((N & -N) < 64) ? (N & -N) : 64;  // lanes: the power-of-two part of N, at most 64
-    constexpr int R = N / G;
-    static_assert(R == 1 || R == 2 || R == 3 || R == 4 || R == 8, "transform length 2^k or 3*2^k");
-    wave_r2r_rows<Real, R, G, KIND1>(slab, n0, ld, 1, tw);  // rows (axis 1)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// transforms of the lines base + i * LS, i < nlines; element e of a line at e * ES
+template <typename Real, int N, int KIND, int LS, int ES>
+__device__ __forceinline__ void wave_r2r_lines(Real* base, int nlines, const typename cplx_of<Real>::type* tw)
+{
+    using C = typename cplx_of<Real>::type;
+    constexpr SlabDims D = SlabShape<N>::D;
+    constexpr int A = D.A, B = D.B, F = D.F, MIR = (B - 1) / 2;
+    // the lane index through an empty asm: otherwise the compiler computes the lane's ~60 LDS offsets
+    // once for all the transforms of a kernel and keeps them in registers across them
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = SlabShape<N>::NT >> 6;
+    const int sub = lane / D.lanes, p = lane % D.lanes;
+    const int P = (nlines + 1) >> 1;
+    for (int t0 = wave * F; t0 < P; t0 += nwaves * F) {
+        const int f = t0 + sub;
+        const bool ok = sub < F && f < P;
+        const bool has2 = f + P < nlines;
+        Real* const la = base + f * LS;
+        Real* const lb = la + P * LS;
+        if (ok && p <= B / 2) {
+            // a lone last line is packed with itself; its partner's place only holds the exchange
+            const Real* const sb = has2 ? lb : la;
+            C v[A];
+#pragma unroll
+            for (int k = 0; k < A; k++) {
+                const int o = (k < A / 2) ? p * ES + B * k * ES : B * (A - k) * ES - p * ES;
+                Real a = la[o], b = sb[o];
+                if constexpr (KIND == 1) {
+                    if (k == 0 || k == A / 2) {
+                        a = (p == 0) ? (Real)0 : a;
+                        b = (p == 0) ? (Real)0 : b;
+                    }
+                    if (k >= A / 2) {
+                        a = -a;
+                        b = -b;
+                    }
+                }
+                v[k] = C{a, b};
+            }
+            reg_dft<A>(v);
+            la[p * ES] = v[0].x;
+            lb[p * ES] = v[0].y;
+            const bool mirror = p != 0 && 2 * p != B;
+#pragma unroll
+            for (int k1 = 1; k1 <= A / 2; k1++) {
+                const C w = tw[p * k1];
+                const C e = v[k1] * w;
+                const int o = (p ^ (k1 & (B - 1))) * ES + (B * k1 - MIR) * ES;
+                la[o] = e.x;
+                lb[o] = e.y;
+                if constexpr (B > 2) {
+                    if (mirror) {
+                        C m = v[A - k1] * C{w.x, -w.y};
+                        if constexpr (KIND == 1) m = C{-m.x, -m.y};
+                        const int om = ((B - p) ^ (k1 & (B - 1))) * ES + (B * k1 - MIR) * ES;
+                        la[om] = m.x;
+                        lb[om] = m.y;
+                    }
+                }
+            }
+        }
+        wave_lds_order();
+        if (ok && p <= A / 2) {
+            int q = p;
+            asm volatile("" : "+v"(q));
+            const int xr = q & (B - 1);
+            const int bq = (q == 0) ? 0 : B * q - MIR;
+            C v[B];
+#pragma unroll
+            for (int r = 0; r < B; r++) {
+                int o = bq + (r ^ xr);
+                if (r > B / 2) o = (q == 0) ? B - r : o;
+                Real a = la[o * ES], b = lb[o * ES];
+                if constexpr (KIND == 1) {
+                    if (r > B / 2) {
+                        a = (q == 0) ? -a : a;
+                        b = (q == 0) ? -b : b;
+                    }
+                }
+                v[r] = C{a, b};
+            }
+            reg_dft<B>(v);
+            wave_lds_order();
+            // Z[q + A k2]: the direct index up to N/2, the mirrored one beyond (equal up to the
+            // parity; lanes 0 and A/2 write some values twice)
+#pragma unroll
+            for (int k2 = 0; k2 < B; k2++) {
+                const bool direct = k2 < (B + 1) / 2;
+                const int o = direct ? q * ES + A * k2 * ES : A * (B - k2) * ES - q * ES;
+                if constexpr (KIND == 0) {
+                    la[o] = v[k2].x;
+                    if (has2) lb[o] = v[k2].y;
+                } else {
+                    la[o] = direct ? -v[k2].y : v[k2].y;
+                    if (has2) lb[o] = direct ? v[k2].x : -v[k2].x;
+                }
+            }
+        }
+    }
+}
+
+// 2D transform of a slab, axis 1 (the contiguous one) then axis 0: KIND0 along axis 0, KIND1 = 0
+// along axis 1
+template <typename Real, int N, int KIND0>
+__device__ __forceinline__ void slab_r2r_2d(Real* slab, const typename cplx_of<Real>::type* tw)
+{
+    constexpr int LD = SlabShape<N>::LD, nk = N / 2 + 1;
+    wave_r2r_lines<Real, N, 0, LD, 1>(slab + KIND0 * LD, nk - 2 * KIND0, tw);
     __syncthreads();
-    wave_r2r_rows<Real, R, G, KIND0>(slab, n1, 1, ld, tw);  // columns (axis 0)
+    wave_r2r_lines<Real, N, KIND0, 1, LD>(slab, nk, tw);
     __syncthreads();
 }
 
@@ -779,39 +883,90 @@ __device__ inline double block_sum(double v, double* scratch)
 // slab layout helpers, Sigma(k,iwn) storage forms and the Lambda-grid integrand h / f0
 // (shared by tpsc_kernels.hip and tpsc_al.hip)
 // ---------------------------------------------------------------------------------
-// wedge (l,m) of a packed index, m <= l
-// The first guess for l comes from the hardware FP32 square root (idx < 2^24 is exact in FP32,
-// the guess is within one of the row); the two loops make it exact.
-__device__ __forceinline__ void wedge_lm(long idx, int& l, int& m)
+// The t-th point (l, m), m <= l, of the wedge for the pointwise phases of a slab: rows r and
+// nk - 1 - r together hold nk + 1 points, so t runs over a rectangle of that width (nk is odd; the
+// middle row comes last) and no square root is needed.
+template <int N>
+__device__ __forceinline__ void wedge_pt(int t, int& l, int& m)
 {
-    const int id = (int)idx;
-    int L = (int)((__builtin_amdgcn_sqrtf(8.0f * (float)id + 1.0f) - 1.0f) * 0.5f);
-    while ((L + 1) * (L + 2) / 2 <= id) L++;
-    while (L * (L + 1) / 2 > id) L--;
-    l = L;
-    m = id - L * (L + 1) / 2;
+    constexpr int nk = N / 2 + 1;
+    static_assert(nk % 2 == 1, "the row pairing needs an odd nk");
+    const int r = t / (nk + 1), s = t - r * (nk + 1);
+    const bool low = s <= r;
+    l = low ? r : nk - 1 - r;
+    m = low ? s : s - r - 1;
 }
-
-// write a wedge value to both symmetric positions of an nk x nk LDS slab
-__device__ __forceinline__ void put_sym(double* slab, int nk, int l, int m, double v)
+// f(l, m, i) for every wedge point of the workgroup's share, i = its packed index
+template <int N, typename Fn>
+__device__ __forceinline__ void each_wedge(Fn&& f)
 {
-    slab[m + l * nk] = v;
-    slab[l + m * nk] = v;
+    constexpr int nk8 = (N / 2 + 1) * (N / 2 + 2) / 2;
+#pragma unroll 2
+    for (int t = threadIdx.x; t < nk8; t += SlabShape<N>::NT) {
+        int l, m;
+        wedge_pt<N>(t, l, m);
+        f(l, m, m + l * (l + 1) / 2);
+    }
 }
-
-// twiddle table placed after an n-element slab in LDS, 16-byte aligned
-template <typename Real>
-__device__ __forceinline__ typename cplx_of<Real>::type* slab_tw(Real* slab, long n)
+// the same with the slot c of the point among the thread's own, unrolled: f may index registers by c
+template <int N>
+constexpr int wedge_per_thread() { return ((N / 2 + 1) * (N / 2 + 2) / 2 + SlabShape<N>::NT - 1) / SlabShape<N>::NT; }
+template <int N, typename Fn>
+__device__ __forceinline__ void each_wedge_slot(Fn&& f)
 {
-    const long bytes = (n * (long)sizeof(Real) + 15) & ~15L;
-    return (typename cplx_of<Real>::type*)((char*)slab + bytes);
+    constexpr int nk8 = (N / 2 + 1) * (N / 2 + 2) / 2;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // the points' indices are recomputed in each phase, not kept
+#pragma unroll
+    for (int c = 0; c < wedge_per_thread<N>(); c++) {
+        const int t = tid + c * SlabShape<N>::NT;
+        if (t < nk8) {
+            int l, m;
+            wedge_pt<N>(t, l, m);
+            f(l, m, m + l * (l + 1) / 2, c);
+        }
+    }
 }
-
-template <typename Real>
-__device__ __forceinline__ void put_sym_t(Real* slab, int nk, int l, int m, Real v)
+// f(l, m, s) for every point of the Lambda grid: kx index l + 1 (slab line l + 1), s = m + l nk
+template <int N, typename Fn>
+__device__ __forceinline__ void each_lambda(Fn&& f)
 {
-    slab[m + l * nk] = v;
-    slab[l + m * nk] = v;
+    constexpr int nk = N / 2 + 1, nq = nk * (nk - 2);
+#pragma unroll 2
+    for (int s = threadIdx.x; s < nq; s += SlabShape<N>::NT) {
+        const int l = s / nk;
+        f(l, s - l * nk, s);
+    }
+}
+template <int N>
+constexpr int lambda_per_thread() { return ((N / 2 + 1) * (N / 2 - 1) + SlabShape<N>::NT - 1) / SlabShape<N>::NT; }
+template <int N, typename Fn>
+__device__ __forceinline__ void each_lambda_slot(Fn&& f)
+{
+    constexpr int nk = N / 2 + 1, nq = nk * (nk - 2);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+#pragma unroll
+    for (int c = 0; c < lambda_per_thread<N>(); c++) {
+        const int s = tid + c * SlabShape<N>::NT;
+        if (s < nq) {
+            const int l = s / nk;
+            f(l, s - l * nk, s, c);
+        }
+    }
+}
+// slab offset of element (l, m)
+template <int N>
+__device__ __forceinline__ int at(int l, int m)
+{
+    return m + l * SlabShape<N>::LD;
+}
+// write a wedge value to both symmetric positions of a slab
+template <int N, typename Real>
+__device__ __forceinline__ void put_sym(Real* slab, int l, int m, Real v)
+{
+    slab[at<N>(l, m)] = v;
+    slab[at<N>(m, l)] = v;
 }
 
 __device__ __forceinline__ cd sigma_mom(double Sinf, double s2, double s3, cd R, double wn)

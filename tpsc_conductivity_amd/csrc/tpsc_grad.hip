@@ -13,8 +13,6 @@
 
 namespace tpsc {
 
-#define GRAD_THREADS 1024
-
 // Fermi function f(x) = 1/(e^{x/T} + 1) and 1 - f, without overflow
 __device__ __forceinline__ void fermi2(double x, double T, double& f, double& g)
 {
@@ -37,7 +35,7 @@ __device__ __forceinline__ void fermi2(double x, double T, double& f, double& g)
 // Tangent outputs: tchi[0..nk8) = dchi0(q,0), tchirt[0..nk8) = dchi0(r,0), tchirt0,
 // tdchirt0, tdGrt0p, tdchiqt0.  scr: 5*nk8 doubles.
 template <int N>
-__global__ void __launch_bounds__(GRAD_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_chi0_tau0_tan(const double* __restrict__ ekw, const double* __restrict__ dekw, const double* __restrict__ er,
                     const double* __restrict__ der, double mu0, double dmu0, double T, double* tchi, double* tchirt,
                     double* tchirt0, double* tdchirt0, double* tdGrt0p, double* tdchiqt0, double* scr)
@@ -47,14 +45,12 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int tid = threadIdx.x, nt = blockDim.x;
     double *PdGp = scr, *TdGp = scr + nk8, *Pg = scr + 2 * nk8, *Tg = scr + 3 * nk8, *stg = scr + 4 * nk8;
     for (int pass = 0; pass < 4; pass++) {
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
+        each_wedge<N>([&](int l, int m, int i) {
             const double x = ekw[i] - mu0, dx = dekw[i] - dmu0;
             double f, g;
             fermi2(x, T, f, g);
@@ -63,16 +59,14 @@ __global__ void __launch_bounds__(GRAD_THREADS)
             else if (pass == 1) v = (g + x * f * g / T) * dx / nk02;
             else if (pass == 2) v = -g / nk02;
             else v = -f * g / T * dx / nk02;
-            put_sym(slab, nk, l, m, v);
-        }
+            put_sym<N>(slab, l, m, v);
+        });
         __syncthreads();
-        slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
+        slab_r2r_2d<double, N, 0>(slab, tw);
         double* o = (pass == 0) ? PdGp : (pass == 1) ? TdGp : (pass == 2) ? Pg : Tg;
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            o[i] = slab[m + l * nk];
-        }
+        each_wedge<N>([&](int l, int m, int i) {
+            o[i] = slab[at<N>(l, m)];
+        });
         __syncthreads();
     }
     // dchi0(r,0) and the tangent of d/dtau chi0(r,0)
@@ -91,19 +85,15 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     }
     __syncthreads();
     for (int pass = 0; pass < 2; pass++) {
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            put_sym(slab, nk, l, m, (pass == 0) ? tchirt[i] : stg[i]);
-        }
+        each_wedge<N>([&](int l, int m, int i) {
+            put_sym<N>(slab, l, m, (pass == 0) ? tchirt[i] : stg[i]);
+        });
         __syncthreads();
-        slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
+        slab_r2r_2d<double, N, 0>(slab, tw);
         double* o = (pass == 0) ? tchi : tdchiqt0;
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            o[i] = slab[m + l * nk];
-        }
+        each_wedge<N>([&](int l, int m, int i) {
+            o[i] = slab[at<N>(l, m)];
+        });
         __syncthreads();
     }
 }
@@ -126,7 +116,7 @@ __device__ __forceinline__ double g0m_val(double x, double t, double T, double n
 //   dchi0(r,tau) = -2 (dG(r,-tau) G(r,tau) + G(r,-tau) dG(r,tau)), tau = beta/2: 4 G dG
 // The block stages G(r,tau) in tchirt[j] and dG(r,tau) in tchi[j] before their final values.
 template <int N>
-__global__ void __launch_bounds__(GRAD_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_chi0_slab_tan(const double* __restrict__ ekw, const double* __restrict__ dekw, double mu0, double dmu0,
                     double T, int Nw, double* tchi, double* tchirt)
 {
@@ -135,8 +125,8 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int nwb = Nw / 2 + 1;
     const int j = blockIdx.x + 1;
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -146,9 +136,7 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     const double t = mid ? 1.0 / (2.0 * T) : j / (Nw * T);
     const int npass = mid ? 2 : 4;
     for (int pass = 0; pass < npass; pass++) {
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
+        each_wedge<N>([&](int l, int m, int i) {
             const double x = ekw[i] - mu0, dx = dekw[i] - dmu0;
             double f, g;
             fermi2(x, T, f, g);
@@ -160,36 +148,30 @@ __global__ void __launch_bounds__(GRAD_THREADS)
                 const double p = g0m_val(x, t, T, nk02);
                 v = (pass == 2) ? p : p * (t - g / T) * dx;
             }
-            put_sym(slab, nk, l, m, v);
-        }
+            put_sym<N>(slab, l, m, v);
+        });
         __syncthreads();
-        slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            const double v = slab[m + l * nk];
+        slab_r2r_2d<double, N, 0>(slab, tw);
+        each_wedge<N>([&](int l, int m, int i) {
+            const double v = slab[at<N>(l, m)];
             if (pass == 0) cr[i] = v;                        // G(r,tau)
             else if (pass == 1) cq[i] = mid ? 4.0 * cr[i] * v : v;  // dG(r,tau), or dchi0(r,beta/2)
             else if (pass == 2) cq[i] = -2.0 * v * cq[i];    // -2 G(r,-tau) dG(r,tau)
             else cr[i] = cq[i] - 2.0 * v * cr[i];            // - 2 dG(r,-tau) G(r,tau)
-        }
+        });
         __syncthreads();
     }
     if (mid)
         for (long i = tid; i < nk8; i += nt) cr[i] = cq[i];
     __syncthreads();
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        put_sym(slab, nk, l, m, cr[i]);
-    }
+    each_wedge<N>([&](int l, int m, int i) {
+        put_sym<N>(slab, l, m, cr[i]);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        cq[i] = slab[m + l * nk];
-    }
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) {
+        cq[i] = slab[at<N>(l, m)];
+    });
 }
 
 // Implicit derivatives of the sum rules (chi.cpp:738-843): per (q, n) partials of
@@ -237,7 +219,7 @@ __global__ void __launch_bounds__(256)
 //   normFact U/8 [3 Usp (chi_sp - chi0) + Uch (chi_ch - chi0)]
 //   d chi_sp = (dchi0 + dUsp chi0^2/2) r_sp^2,  d chi_ch = (dchi0 - dUch chi0^2/2) r_ch^2
 template <int N>
-__global__ void __launch_bounds__(GRAD_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_vertex_slab_tan(const double* __restrict__ chi, const double* __restrict__ tchi, double* tV, double normFact,
                       double U, double dU, double Usp, double dUsp, double Uch, double dUch)
 {
@@ -245,28 +227,24 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const long j = blockIdx.x;
     const int tid = threadIdx.x, nt = blockDim.x;
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
+    each_wedge<N>([&](int l, int m, int i) {
         const double c = chi[i + j * nk8], dc = tchi[i + j * nk8];
         const double rs = 1.0 / (1.0 - Usp * c / 2.0), rc = 1.0 / (1.0 + Uch * c / 2.0);
         const double csp = c * rs, cch = c * rc;
         const double dcsp = (dc + dUsp * c * c / 2.0) * rs * rs, dcch = (dc - dUch * c * c / 2.0) * rc * rc;
         const double P = 3.0 * Usp * (csp - c) + Uch * (cch - c);
         const double dP = 3.0 * dUsp * (csp - c) + 3.0 * Usp * (dcsp - dc) + dUch * (cch - c) + Uch * (dcch - dc);
-        put_sym(slab, nk, l, m, normFact * (dU * P + U * dP) / 8.0);
-    }
+        put_sym<N>(slab, l, m, normFact * (dU * P + U * dP) / 8.0);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        tV[i + j * nk8] = slab[m + l * nk];
-    }
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) {
+        tV[i + j * nk8] = slab[at<N>(l, m)];
+    });
 }
 
 // y[i] += a x[i]
@@ -283,7 +261,7 @@ __global__ void k_axpy(long n, double a, const double* __restrict__ x, double* y
 //   Sigma(r, 0 / beta) integrand: g V0
 // Outputs tdSig[side*nk8 + k], tSb[side*nk8 + k].  scr: 6*nk8 doubles.
 template <int N>
-__global__ void __launch_bounds__(GRAD_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_sigma_bnd_tan(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ er,
                     const double* __restrict__ der, const double* __restrict__ V0, const double* __restrict__ tV0,
                     const double* __restrict__ dchirt0, const double* __restrict__ tdchirt0,
@@ -295,35 +273,32 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int tid = threadIdx.x, nt = blockDim.x;
     const int side = blockIdx.x;
     double* Pg = scr + 3 * side * nk8;
     double* stg = Pg + nk8;  // 2*nk8
     for (int pass = 0; pass < 2; pass++) {
         for (int s = tid; s < nk * nk; s += nt) {
+            const int l = s / nk, m = s - l * nk;
             const double x = ek[s] - mu0, dx = dek[s] - dmu0;
             double f, g;
             fermi2(x, T, f, g);
             double v;
             if (pass == 0) v = (side == 0) ? -g / nk02 : -f / nk02;
             else v = (side == 0) ? -f * g / T * dx / nk02 : f * g / T * dx / nk02;
-            slab[s] = v;
+            slab[at<N>(l, m)] = v;
         }
         __syncthreads();
-        slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
+        slab_r2r_2d<double, N, 0>(slab, tw);
         if (pass == 0) {
-            for (long i = tid; i < nk8; i += nt) {
-                int l, m;
-                wedge_lm(i, l, m);
-                Pg[i] = slab[m + l * nk];
-            }
+            each_wedge<N>([&](int l, int m, int i) {
+                Pg[i] = slab[at<N>(l, m)];
+            });
         } else {
-            for (long i = tid; i < nk8; i += nt) {
-                int l, m;
-                wedge_lm(i, l, m);
-                const double g = Pg[i], dg = slab[m + l * nk];
+            each_wedge<N>([&](int l, int m, int i) {
+                const double g = Pg[i], dg = slab[at<N>(l, m)];
                 const double v = V0[i], dv = tV0[i];
                 const double c = dchirt0[i], dc = tdchirt0[i];
                 const double dfc = dfact * c * g + fact * dc * g + fact * c * dg;
@@ -334,24 +309,20 @@ __global__ void __launch_bounds__(GRAD_THREADS)
                     stg[i] = -dfc + dv * (-dGrt0p[i] + xi) + v * (-tdGrt0p[i] + dxi);
                 }
                 stg[nk8 + i] = dg * v + g * dv;
-            }
+            });
         }
         __syncthreads();
     }
     for (int pass = 0; pass < 2; pass++) {
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            put_sym(slab, nk, l, m, stg[pass * nk8 + i]);
-        }
+        each_wedge<N>([&](int l, int m, int i) {
+            put_sym<N>(slab, l, m, stg[pass * nk8 + i]);
+        });
         __syncthreads();
-        slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
+        slab_r2r_2d<double, N, 0>(slab, tw);
         double* o = (pass == 0) ? tdSig : tSb;
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            o[i + side * nk8] = slab[m + l * nk];
-        }
+        each_wedge<N>([&](int l, int m, int i) {
+            o[i + side * nk8] = slab[at<N>(l, m)];
+        });
         __syncthreads();
     }
 }
@@ -359,7 +330,7 @@ __global__ void __launch_bounds__(GRAD_THREADS)
 // tangent of Sigma(k,tau_j) = DCT[G0(r,tau_j) V(r,|tau_j|)] (green.cpp:1830-1892; forward
 // k_sigma_slab): DCT[dG0 V + G0 dV], G0 and dG0 recomputed; G0(r,tau) staged in tS[j].
 template <int N>
-__global__ void __launch_bounds__(GRAD_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_sigma_slab_tan(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ V,
                      const double* __restrict__ tV, double mu0, double dmu0, double T, int Nw, double* tS)
 {
@@ -368,8 +339,8 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int j = blockIdx.x;
     const int nwb = Nw / 2 + 1;
     const int jv = (j < nwb) ? j : Nw - j;
@@ -380,42 +351,35 @@ __global__ void __launch_bounds__(GRAD_THREADS)
     const double* tVj = tV + (long)jv * nk8;
     for (int pass = 0; pass < 2; pass++) {
         for (int s = tid; s < nk * nk; s += nt) {
+            const int l = s / nk, m = s - l * nk;
             const double x = ek[s] - mu0, dx = dek[s] - dmu0;
             double f, g;
             fermi2(x, T, f, g);
             const double p = (x > 0) ? -exp(-t * x) / (exp(-x / T) + 1.0) / nk02
                                      : -exp((1.0 / T - t) * x) / (exp(x / T) + 1.0) / nk02;
-            slab[s] = (pass == 0) ? p : p * (f / T - t) * dx;
+            slab[at<N>(l, m)] = (pass == 0) ? p : p * (f / T - t) * dx;
         }
         __syncthreads();
-        slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
+        slab_r2r_2d<double, N, 0>(slab, tw);
         if (pass == 0)
-            for (long i = tid; i < nk8; i += nt) {
-                int l, m;
-                wedge_lm(i, l, m);
-                o[i] = slab[m + l * nk];
-            }
+            each_wedge<N>([&](int l, int m, int i) {
+                o[i] = slab[at<N>(l, m)];
+            });
         __syncthreads();
     }
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        const double v = slab[m + l * nk] * Vj[i] + o[i] * tVj[i];
+    each_wedge<N>([&](int l, int m, int i) {
+        const double v = slab[at<N>(l, m)] * Vj[i] + o[i] * tVj[i];
         o[i] = v;
-    }
+    });
     __syncthreads();
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        put_sym(slab, nk, l, m, o[i]);
-    }
+    each_wedge<N>([&](int l, int m, int i) {
+        put_sym<N>(slab, l, m, o[i]);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        o[i] = slab[m + l * nk];
-    }
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) {
+        o[i] = slab[at<N>(l, m)];
+    });
 }
 
 // Sigma(k, i w0) = Sinf/z + C2/z^2 + C3/z^3 + R/z^4 at z = i w0 (green.cpp:3039):
@@ -438,12 +402,6 @@ __global__ void k_sigma_loss(const double* __restrict__ w, const double* __restr
 }
 
 // ================================================================== launchers
-static size_t grad_lds(int N)
-{
-    const int nk = N / 2 + 1;
-    return (((size_t)nk * nk * sizeof(double) + 15) & ~(size_t)15) + 2 * sizeof(double) * (size_t)N;
-}
-
 #define GRAD_DISPATCH_N(N, ...)                                     \
     switch (N) {                                                    \
         case 4: { constexpr int NN = 4; __VA_ARGS__; } break;       \
@@ -471,13 +429,13 @@ static void grad_set_lds(K kern, size_t bytes)
 hipError_t launch_chi0_tan(const Grid& g, const DevArrays& d, const TanArrays& t, double mu0, double dmu0,
                            hipStream_t s)
 {
-    const size_t lds = grad_lds(g.N);
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_DISPATCH_N(g.N, {
         grad_set_lds(k_chi0_tau0_tan<NN>, lds);
-        hipLaunchKernelGGL(k_chi0_tau0_tan<NN>, dim3(1), dim3(GRAD_THREADS), lds, s, d.ekw, t.dekw, d.er, t.der, mu0,
+        hipLaunchKernelGGL(k_chi0_tau0_tan<NN>, dim3(1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, t.dekw, d.er, t.der, mu0,
                            dmu0, g.T, t.chi, t.chirt, t.chirt0, t.dchirt0, t.dGrt0p, t.dchiqt0, t.scr);
         grad_set_lds(k_chi0_slab_tan<NN>, lds);
-        hipLaunchKernelGGL(k_chi0_slab_tan<NN>, dim3(g.nwb - 1), dim3(GRAD_THREADS), lds, s, d.ekw, t.dekw, mu0, dmu0,
+        hipLaunchKernelGGL(k_chi0_slab_tan<NN>, dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, t.dekw, mu0, dmu0,
                            g.T, g.Nw, t.chi, t.chirt);
     });
     return hipGetLastError();
@@ -497,10 +455,10 @@ hipError_t launch_vertex_slab_tan(const Grid& g, const DevArrays& d, const TanAr
                                   double Usp, double dUsp, double Uch, double dUch, hipStream_t s)
 {
     const double normFact = g.T / ((double)g.N * g.N);
-    const size_t lds = grad_lds(g.N);
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_DISPATCH_N(g.N, {
         grad_set_lds(k_vertex_slab_tan<NN>, lds);
-        hipLaunchKernelGGL(k_vertex_slab_tan<NN>, dim3(g.nwb), dim3(GRAD_THREADS), lds, s, d.chiw, t.chi, t.V,
+        hipLaunchKernelGGL(k_vertex_slab_tan<NN>, dim3(g.nwb), dim3(SlabShape<NN>::NT), lds, s, d.chiw, t.chi, t.V,
                            normFact, U, dU, Usp, dUsp, Uch, dUch);
     });
     return hipGetLastError();
@@ -515,14 +473,14 @@ hipError_t launch_axpy(long n, double a, const double* x, double* y, hipStream_t
 hipError_t launch_sigma_tan(const Grid& g, const DevArrays& d, const TanArrays& t, double mu0, double dmu0,
                             double fact, double dfact, hipStream_t s)
 {
-    const size_t lds = grad_lds(g.N);
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_DISPATCH_N(g.N, {
         grad_set_lds(k_sigma_bnd_tan<NN>, lds);
-        hipLaunchKernelGGL(k_sigma_bnd_tan<NN>, dim3(2), dim3(GRAD_THREADS), lds, s, d.ek, t.dek, d.er, t.der, d.V0,
+        hipLaunchKernelGGL(k_sigma_bnd_tan<NN>, dim3(2), dim3(SlabShape<NN>::NT), lds, s, d.ek, t.dek, d.er, t.der, d.V0,
                            t.V0, d.dchirt0, t.dchirt0, d.dGrt0p, t.dGrt0p, mu0, dmu0, g.T, fact, dfact, t.dSig, t.Sb,
                            t.scr);
         grad_set_lds(k_sigma_slab_tan<NN>, lds);
-        hipLaunchKernelGGL(k_sigma_slab_tan<NN>, dim3(g.Nw + 1), dim3(GRAD_THREADS), lds, s, d.ek, t.dek, d.V, t.V,
+        hipLaunchKernelGGL(k_sigma_slab_tan<NN>, dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.ek, t.dek, d.V, t.V,
                            mu0, dmu0, g.T, g.Nw, t.Stau);
     });
     return hipGetLastError();

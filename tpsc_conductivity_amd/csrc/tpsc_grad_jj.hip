@@ -18,8 +18,6 @@
 
 namespace tpsc {
 
-#define GRAD_JJ_THREADS 1024
-
 // ------------------------------------------------------------------ dual numbers
 struct dual {
     double v, d;  // value, tangent
@@ -174,7 +172,7 @@ __global__ void __launch_bounds__(256)
 // recomputed and parked in the block's own output plane (each thread reads back what it
 // wrote) while the tangent integrand is transformed; then 2 (dh V + h dV) is transformed.
 template <int N>
-__global__ void __launch_bounds__(GRAD_JJ_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_hVf0V_tan(const double* __restrict__ ek, const double* __restrict__ tek, const double* __restrict__ vel,
                 const double* __restrict__ tvel, const double* __restrict__ V, const double* __restrict__ tV,
                 double mu0, double dmu0, double T, int Nw, double* th, double* tf0)
@@ -185,38 +183,35 @@ __global__ void __launch_bounds__(GRAD_JJ_THREADS)
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int j = blockIdx.x, which = blockIdx.y;
     const double t = (double)j / (T * Nw);
     const int jv = (j > Nw / 2) ? Nw - j : j;
-    const int tid = threadIdx.x, nt = blockDim.x;
     double* const o = ((which == 0) ? th : tf0) + (long)j * nq;
     for (int pass = 0; pass < 2; pass++) {
-        for (long s = tid; s < nq; s += nt) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
+        each_lambda<N>([&](int l, int m, int s) {
             const long i = m + (long)(l + 1) * nk;
             dual hv, fv;
             hf0_dual(dual{ek[i] - mu0, tek[i] - dmu0}, dual{vel[s], tvel[s]}, T, t, nf, hv, fv);
             const dual a = (which == 0) ? hv : fv;
-            slab[s] = (pass == 0) ? a.v : a.d;
-        }
+            slab[at<N>(l + 1, m)] = (pass == 0) ? a.v : a.d;
+        });
         __syncthreads();
-        slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+        slab_r2r_2d<double, N, 1>(slab, tw);
         if (pass == 0)
-            for (long s = tid; s < nq; s += nt) o[s] = slab[s];
+            each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
         __syncthreads();
     }
     const double* Vj = V + (long)jv * nk8;
     const double* tVj = tV + (long)jv * nk8;
-    for (long s = tid; s < nq; s += nt) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
+    each_lambda<N>([&](int l, int m, int s) {
         const long r = fold_idx(l + 1, m, N);
-        slab[s] = 2.0 * (slab[s] * Vj[r] + o[s] * tVj[r]);
-    }
+        slab[at<N>(l + 1, m)] = 2.0 * (slab[at<N>(l + 1, m)] * Vj[r] + o[s] * tVj[r]);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-    for (long s = tid; s < nq; s += nt) o[s] = slab[s];
+    slab_r2r_2d<double, N, 1>(slab, tw);
+    each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // ------------------------------------------------------------------ boundary data
@@ -224,7 +219,7 @@ __global__ void __launch_bounds__(GRAD_JJ_THREADS)
 // 2697-2735, 2745-3114).  Block b: which = b/2 (0: h, 1: f0), side = b%2.  fact4 = U(3Usp+Uch)/4.
 // scr: 3*nq per block (primal h(r,tau_b), its tangent, the primal slope transform).
 template <int N>
-__global__ void __launch_bounds__(GRAD_JJ_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_hf0_bnd_tan(const double* __restrict__ ek, const double* __restrict__ tek, const double* __restrict__ vel,
                   const double* __restrict__ tvel, const double* __restrict__ V0, const double* __restrict__ tV0,
                   const double* __restrict__ dchirt0, const double* __restrict__ tdchirt0, double mu0, double dmu0,
@@ -236,18 +231,16 @@ __global__ void __launch_bounds__(GRAD_JJ_THREADS)
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int which = blockIdx.x >> 1, side = blockIdx.x & 1;
-    const int tid = threadIdx.x, nt = blockDim.x;
     double* const S0 = scr + (long)blockIdx.x * 3 * nq;  // h(r, tau_b)
     double* const S1 = S0 + nq;                           // its tangent
     double* const S2 = S1 + nq;                           // transformed slope integrand
     const double tb = (side == 0) ? 0.0 : (double)Nw / (T * Nw);
     // passes 0, 1: the integrand at tau_b and its tangent; 2, 3: the slope integrand and its tangent
     for (int pass = 0; pass < 4; pass++) {
-        for (long s = tid; s < nq; s += nt) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
+        each_lambda<N>([&](int l, int m, int s) {
             const long i = m + (long)(l + 1) * nk;
             const dual x{ek[i] - mu0, tek[i] - dmu0}, v{vel[s], tvel[s]};
             dual a;
@@ -258,40 +251,38 @@ __global__ void __launch_bounds__(GRAD_JJ_THREADS)
             } else {
                 a = slope_dual(which, side, x, v, T, nf);
             }
-            slab[s] = (pass & 1) ? a.d : a.v;
-        }
+            slab[at<N>(l + 1, m)] = (pass & 1) ? a.d : a.v;
+        });
         __syncthreads();
-        slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+        slab_r2r_2d<double, N, 1>(slab, tw);
         if (pass < 3) {
             double* o = (pass == 0) ? S0 : (pass == 1) ? S1 : S2;
-            for (long s = tid; s < nq; s += nt) o[s] = slab[s];
+            each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
             __syncthreads();
         }
     }
     // slope: DST x DCT[2 d V0 +- h fact4 dchi0(r,0)] (the sign of the tau = beta side is minus)
     const double sg = (side == 0) ? 1.0 : -1.0;
-    for (long s = tid; s < nq; s += nt) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
+    each_lambda<N>([&](int l, int m, int s) {
         const long r = fold_idx(l + 1, m, N);
         const double v0 = V0[r], dv0 = tV0[r], c0 = dchirt0[r], dc0 = tdchirt0[r];
-        slab[s] = 2.0 * (slab[s] * v0 + S2[s] * dv0) +
+        slab[at<N>(l + 1, m)] = 2.0 * (slab[at<N>(l + 1, m)] * v0 + S2[s] * dv0) +
                   sg * (S1[s] * fact4 * c0 + S0[s] * dfact4 * c0 + S0[s] * fact4 * dc0);
-    }
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     double* o = ((which == 0) ? tdhV : tdf0V) + side * nq;
-    for (long s = tid; s < nq; s += nt) o[s] = slab[s];
+    each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
     __syncthreads();
     // value: DST x DCT[2 h V0]
-    for (long s = tid; s < nq; s += nt) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
+    each_lambda<N>([&](int l, int m, int s) {
         const long r = fold_idx(l + 1, m, N);
-        slab[s] = 2.0 * (S1[s] * V0[r] + S0[s] * tV0[r]);
-    }
+        slab[at<N>(l + 1, m)] = 2.0 * (S1[s] * V0[r] + S0[s] * tV0[r]);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     double* ob = ((which == 0) ? thVb : tf0Vb) + side * nq;
-    for (long s = tid; s < nq; s += nt) ob[s] = slab[s];
+    each_lambda<N>([&](int l, int m, int s) { ob[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // ------------------------------------------------------------------ the Lambda pencil
@@ -614,13 +605,6 @@ __global__ void __launch_bounds__(NT)
 }
 
 // ================================================================== launchers
-static size_t grad_jj_lds(int N)
-{
-    const int nk = N / 2 + 1;
-    const size_t nq = (size_t)nk * (nk - 2);
-    return ((nq * sizeof(double) + 15) & ~(size_t)15) + 2 * sizeof(double) * (size_t)N;
-}
-
 #define GRAD_JJ_DISPATCH_N(N, ...)                                  \
     switch (N) {                                                    \
         case 8: { constexpr int NN = 8; __VA_ARGS__; } break;       \
@@ -666,10 +650,10 @@ hipError_t launch_trace_diffG_tan(const Grid& g, const DevArrays& d, const TanAr
 hipError_t launch_hVf0V_tan(const Grid& g, const DevArrays& d, const TanArrays& t, double mu0, double dmu0,
                             hipStream_t s)
 {
-    const size_t lds = grad_jj_lds(g.N);
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_JJ_DISPATCH_N(g.N, {
         grad_jj_set_lds(k_hVf0V_tan<NN>, lds);
-        hipLaunchKernelGGL(k_hVf0V_tan<NN>, dim3(g.Nw + 1, 2), dim3(GRAD_JJ_THREADS), lds, s, d.ek, t.dek, d.dek,
+        hipLaunchKernelGGL(k_hVf0V_tan<NN>, dim3(g.Nw + 1, 2), dim3(SlabShape<NN>::NT), lds, s, d.ek, t.dek, d.dek,
                            t.vel, d.V, t.V, mu0, dmu0, g.T, g.Nw, t.h, t.f0);
     });
     return hipGetLastError();
@@ -678,10 +662,10 @@ hipError_t launch_hVf0V_tan(const Grid& g, const DevArrays& d, const TanArrays& 
 hipError_t launch_hf0_bnd_tan(const Grid& g, const DevArrays& d, const TanArrays& t, double mu0, double dmu0,
                               double fact4, double dfact4, hipStream_t s)
 {
-    const size_t lds = grad_jj_lds(g.N);
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_JJ_DISPATCH_N(g.N, {
         grad_jj_set_lds(k_hf0_bnd_tan<NN>, lds);
-        hipLaunchKernelGGL(k_hf0_bnd_tan<NN>, dim3(4), dim3(GRAD_JJ_THREADS), lds, s, d.ek, t.dek, d.dek, t.vel, d.V0,
+        hipLaunchKernelGGL(k_hf0_bnd_tan<NN>, dim3(4), dim3(SlabShape<NN>::NT), lds, s, d.ek, t.dek, d.dek, t.vel, d.V0,
                            t.V0, d.dchirt0, t.dchirt0, mu0, dmu0, g.T, g.Nw, fact4, dfact4, t.dhV, t.df0V, t.hVb,
                            t.f0Vb, t.bscr);
     });

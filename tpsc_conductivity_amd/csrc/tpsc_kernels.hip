@@ -11,8 +11,8 @@
 //   k_hf0_slab, k_hf0_bnd,
 //   k_hVf0V_slab, k_jj_pencil,
 //   k_kx0_rows                   cond_opt.cpp:2584-4173 Lambda_jj bubble + Maki-Thompson + kx0
-// Slab kernels hold one (nk x nk) slab in LDS (133 KB at N=256 in FP64) and transform it with
-// wavefront FFTs; pencil kernels hold one tau-pencil per workgroup.
+// Slab kernels hold one (nk x nk) slab in LDS (151 KB at N=256 in FP64) and transform it with
+// register FFTs of line pairs; pencil kernels hold one tau-pencil per workgroup.
 // Precision: S is the storage and slab-arithmetic type of the tau arrays (chi0(q,tau),
 // chi0(r,tau), V, Sigma(k,tau), h, f0); chi0(q,iqn) is stored in FP64 in both paths.  S = double is the FP64 path.  S = float is the mixed path: the
 // slab transforms and pointwise products run in FP32, while the tau = 0 / beta boundary data,
@@ -26,17 +26,10 @@
 
 namespace tpsc {
 
-#define SLAB_THREADS 1024
-// waves per SIMD a slab kernel is compiled for: two FP32 workgroups (68 KB LDS each at N=256)
-// fit one CU when the kernel stays within 64 VGPRs; an FP64 slab (133 KB) runs alone
+// waves per SIMD a slab kernel is compiled for: two FP32 workgroups (76 KB of LDS and ten wavefronts
+// each at N = 256) share a CU within 96 VGPRs; an FP64 slab (151 KB) runs alone, within 168
 template <typename S>
-struct SlabOcc {
-    static constexpr int waves = 4;
-};
-template <>
-struct SlabOcc<float> {
-    static constexpr int waves = 8;
-};
+constexpr int slab_occ() { return sizeof(S) == sizeof(float) ? 5 : 1; }
 #define PEN_THREADS 256
 
 // ================================================================== small helpers
@@ -191,104 +184,65 @@ __device__ __forceinline__ double g0_minus(double x, double t, double T, double 
 }
 
 // tau = 0 slice plus the tau-derivative data (chi0.cpp:323-447); one block.
-// tmp[0:nk8] <- G(r,0), tmp[nk8:2nk8] <- dG(r,0-), tmp[2nk8:3nk8] <- staging
 // The boundary data are tail moments: this kernel runs in FP64 for both precisions and
 // only rounds the slice-0 values it stores into the S arrays.
 template <int N, typename S>
-__global__ void __launch_bounds__(SLAB_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_chi0_tau0(const double* __restrict__ ekw, const double* __restrict__ er, const double* __restrict__ mu0p,
-                double T, S* chi, S* chirt, double* dchirt0, double* dGrt0p, double* dchiqt0, double* chirt0,
-                double* tmp)
+                double T, S* chi, S* chirt, double* dchirt0, double* dGrt0p, double* dchiqt0, double* chirt0)
 {
     const double mu0 = *mu0p;
-    constexpr int nk = N / 2 + 1;
-    constexpr long nk8 = (long)nk * (nk + 1) / 2;
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
-    double* G0r = tmp;
-    double* dGm = tmp + nk8;
-    double* stg = tmp + 2 * nk8;
-    const int tid = threadIdx.x, nt = blockDim.x;
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     // d/dtau G(r,0+) = DCT[-ekmu Gkt / N^2]
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
+    each_wedge<N>([&](int l, int m, int i) {
         const double x = ekw[i] - mu0;
         const double Gkt = -1.0 / (exp(-x / T) + 1.0);
-        put_sym(slab, nk, l, m, -x * Gkt / nk02);
-    }
+        put_sym<N>(slab, l, m, -x * Gkt / nk02);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        const double v = slab[m + l * nk];
-        dGrt0p[i] = v;
-        dGm[i] = ((i == 0) ? -mu0 : er[i]) - v;
-    }
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) { dGrt0p[i] = slab[at<N>(l, m)]; });
     __syncthreads();
     // G(r,0)
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
+    each_wedge<N>([&](int l, int m, int i) {
         const double x = ekw[i] - mu0;
-        put_sym(slab, nk, l, m, (-1.0 / (exp(-x / T) + 1.0)) / nk02);
-    }
+        put_sym<N>(slab, l, m, (-1.0 / (exp(-x / T) + 1.0)) / nk02);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        const double g = slab[m + l * nk];
-        G0r[i] = g;
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    // chi0(r,0) and its transform (each thread replaces the points it read and keeps their G(r,0))
+    double G0r[wedge_per_thread<N>()];
+    each_wedge_slot<N>([&](int l, int m, int i, int k) {
+        const double g = slab[at<N>(l, m)];
+        G0r[k] = g;
         const double c = (i == 0) ? -2.0 * g * (g + 1.0) : -2.0 * g * g;
         chirt[i] = (S)c;
         chirt0[i] = c;
-        stg[i] = c;
-    }
+        put_sym<N>(slab, l, m, c);
+    });
     __syncthreads();
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        put_sym(slab, nk, l, m, stg[i]);
-    }
-    __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        chi[i] = (S)slab[m + l * nk];
-    }
-    __syncthreads();
+    slab_r2r_2d<double, N, 0>(slab, tw);
     // d/dtau chi0(r,0) and its transform
-    for (long i = tid; i < nk8; i += nt) {
-        const double g = G0r[i];
-        const double v = (i == 0) ? -2.0 * (dGrt0p[i] * (1.0 + g) + dGm[i] * g)
-                                  : -2.0 * (dGrt0p[i] * g + dGm[i] * g);
+    each_wedge_slot<N>([&](int l, int m, int i, int k) {
+        chi[i] = (S)slab[at<N>(l, m)];
+        const double g = G0r[k], dGp = dGrt0p[i];  // written above by this thread
+        const double dGm = ((i == 0) ? -mu0 : er[i]) - dGp;
+        const double v = (i == 0) ? -2.0 * (dGp * (1.0 + g) + dGm * g) : -2.0 * (dGp * g + dGm * g);
         dchirt0[i] = v;
-        stg[i] = v;
-    }
+        put_sym<N>(slab, l, m, v);
+    });
     __syncthreads();
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        put_sym(slab, nk, l, m, stg[i]);
-    }
-    __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        dchiqt0[i] = slab[m + l * nk];
-    }
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) { dchiqt0[i] = slab[at<N>(l, m)]; });
 }
 
 // slices j = 1 .. nwb-1 (chi0.cpp:454-559); block b handles j = b + 1
 template <int N, typename S>
-__global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
+__global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     k_chi0_slab(const double* __restrict__ ekw, const double* __restrict__ mu0p, double T, int Nw, S* chi, S* chirt)
 {
     const double mu0 = *mu0p;
@@ -297,71 +251,43 @@ __global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
-    auto* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    auto* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int nwb = Nw / 2 + 1;
     const int j = blockIdx.x + 1;
-    const int tid = threadIdx.x, nt = blockDim.x;
     S* cr = chirt + (long)j * nk8;
     S* cq = chi + (long)j * nk8;
     if (j < nwb - 1) {
         const double t = j / (Nw * T);
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            put_sym_t(slab, nk, l, m, (S)g0_plus(ekw[i] - mu0, t, T, nk02, 0));
-        }
+        each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, (S)g0_plus(ekw[i] - mu0, t, T, nk02, 0)); });
         __syncthreads();
-        slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
-        for (long i = tid; i < nk8; i += nt) {  // stage G(r,t) in chirt[j]
-            int l, m;
-            wedge_lm(i, l, m);
-            cr[i] = slab[m + l * nk];
-        }
+        slab_r2r_2d<S, N, 0>(slab, tw);
+        S g[wedge_per_thread<N>()];  // G(r,t) of the thread's points
+        each_wedge_slot<N>([&](int l, int m, int, int c) { g[c] = slab[at<N>(l, m)]; });
         __syncthreads();
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            put_sym_t(slab, nk, l, m, (S)g0_minus(ekw[i] - mu0, t, T, nk02));
-        }
+        each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, (S)g0_minus(ekw[i] - mu0, t, T, nk02)); });
         __syncthreads();
-        slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
-        for (long i = tid; i < nk8; i += nt) {  // chi0(r,t) = -2 G(r,-t) G(r,t)
-            int l, m;
-            wedge_lm(i, l, m);
-            cr[i] = (S)(-2) * slab[m + l * nk] * cr[i];
-        }
-        __syncthreads();
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            put_sym_t(slab, nk, l, m, cr[i]);
-        }
-        __syncthreads();
+        slab_r2r_2d<S, N, 0>(slab, tw);
+        // chi0(r,t) = -2 G(r,-t) G(r,t)
+        each_wedge_slot<N>([&](int l, int m, int i, int c) {
+            const S v = (S)(-2) * slab[at<N>(l, m)] * g[c];
+            cr[i] = v;
+            put_sym<N>(slab, l, m, v);
+        });
     } else {
         const double t = 1.0 / (2.0 * T);
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            put_sym_t(slab, nk, l, m, (S)g0_plus(ekw[i] - mu0, t, T, nk02, 1));
-        }
+        each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, (S)g0_plus(ekw[i] - mu0, t, T, nk02, 1)); });
         __syncthreads();
-        slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
-        for (int s = tid; s < nk * nk; s += nt) slab[s] = (S)2 * slab[s] * slab[s];
-        __syncthreads();
-        for (long i = tid; i < nk8; i += nt) {
-            int l, m;
-            wedge_lm(i, l, m);
-            cr[i] = slab[l + m * nk];
-        }
-        __syncthreads();
+        slab_r2r_2d<S, N, 0>(slab, tw);
+        each_wedge<N>([&](int l, int m, int i) {
+            const S v = slab[at<N>(l, m)], c = (S)2 * v * v;
+            cr[i] = c;
+            put_sym<N>(slab, l, m, c);
+        });
     }
-    slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        cq[i] = slab[m + l * nk];
-    }
+    __syncthreads();
+    slab_r2r_2d<S, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) { cq[i] = slab[at<N>(l, m)]; });
 }
 
 // ================================================================== chi0 pencils
@@ -765,7 +691,7 @@ __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ek
 // ================================================================== vertex V(r,tau)
 // chi.cpp:85-119, block j = iqn index
 template <int N, typename S>
-__global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
+__global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     k_vertex_slab(const double* __restrict__ chi, S* V, double normFact, double U, double Usp, double Uch,
                   const double* __restrict__ dsc)
 {
@@ -777,24 +703,17 @@ __global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
-    auto* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    auto* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const long j = blockIdx.x;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
+    each_wedge<N>([&](int l, int m, int i) {
         const double c = chi[i + j * nk8];
         const double csp = c / (1.0 - Usp * c / 2.0), cch = c / (1.0 + Uch * c / 2.0);
-        put_sym_t(slab, nk, l, m, (S)(normFact * U * (3.0 * Usp * (csp - c) + Uch * (cch - c)) / 8.0));
-    }
+        put_sym<N>(slab, l, m, (S)(normFact * U * (3.0 * Usp * (csp - c) + Uch * (cch - c)) / 8.0));
+    });
     __syncthreads();
-    slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        V[i + j * nk8] = slab[m + l * nk];
-    }
+    slab_r2r_2d<S, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) { V[i + j * nk8] = slab[at<N>(l, m)]; });
 }
 
 // chi.cpp:123-170: REDFT00 over n (length Nw/2+1) for two wedge points per block, as one
@@ -845,12 +764,11 @@ __device__ __forceinline__ void store_self(cf* Self, long o, cd R, double Sinf, 
 // V(r,beta) = V(r,0)).  Each block transforms G0(k,tau_b) to r itself (the two passes of a
 // side run side by side: two transforms in a row per block instead of three).
 // G0(k,0+) = -1/(e^{-x/T}+1) and G0(k,beta-) = -1/(e^{x/T}+1), both over N^2.
-// tmp: staging, nk8 per block.
 template <int N>
-__global__ void __launch_bounds__(SLAB_THREADS)
-    k_sigma_bnd(const double* __restrict__ ek, const double* __restrict__ er, const double* __restrict__ V0,
+__global__ void __launch_bounds__(SlabShape<N>::NT)
+    k_sigma_bnd(const double* __restrict__ ekw, const double* __restrict__ er, const double* __restrict__ V0,
                 const double* __restrict__ dchirt0, const double* __restrict__ dGrt0p, double mu0, double T,
-                double fact, double* dSig, double* Sb, double* tmp, const double* __restrict__ mu0p, double U,
+                double fact, double* dSig, double* Sb, const double* __restrict__ mu0p, double U,
                 const double* __restrict__ dsc)
 {
     if (mu0p) mu0 = *mu0p;
@@ -860,51 +778,40 @@ __global__ void __launch_bounds__(SLAB_THREADS)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
-    const int tid = threadIdx.x, nt = blockDim.x;
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int side = blockIdx.x & 1, pass = blockIdx.x >> 1;
-    double* stg = tmp + blockIdx.x * nk8;
-    for (int s = tid; s < nk * nk; s += nt) {
-        const double x = ek[s] - mu0;
-        slab[s] = (side == 0) ? -1.0 / (exp(-x / T) + 1.0) / nk02 : -1.0 / (exp(x / T) + 1.0) / nk02;
-    }
+    each_wedge<N>([&](int l, int m, int i) {
+        const double x = ekw[i] - mu0;
+        put_sym<N>(slab, l, m,
+                   (side == 0) ? -1.0 / (exp(-x / T) + 1.0) / nk02 : -1.0 / (exp(x / T) + 1.0) / nk02);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        const double g = slab[m + l * nk];
+    slab_r2r_2d<double, N, 0>(slab, tw);
+    each_wedge<N>([&](int l, int m, int i) {
+        const double g = slab[at<N>(l, m)];
         const double v = V0[i];
+        double r;
         if (pass == 1)
-            stg[i] = g * v;
+            r = g * v;
         else if (side == 0)
-            stg[i] = fact * dchirt0[i] * g + v * dGrt0p[i];
+            r = fact * dchirt0[i] * g + v * dGrt0p[i];
         else {
             const double xi = (i == 0) ? -mu0 : er[i];
-            stg[i] = -fact * dchirt0[i] * g + v * (-dGrt0p[i] + xi);
+            r = -fact * dchirt0[i] * g + v * (-dGrt0p[i] + xi);
         }
-    }
+        put_sym<N>(slab, l, m, r);
+    });
     __syncthreads();
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        put_sym(slab, nk, l, m, stg[i]);
-    }
-    __syncthreads();
-    slab_r2r_2d<double, N, 0, 0>(slab, nk, nk, nk, tw);
+    slab_r2r_2d<double, N, 0>(slab, tw);
     double* o = (pass == 0) ? dSig : Sb;
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        o[i + side * nk8] = slab[m + l * nk];
-    }
+    each_wedge<N>([&](int l, int m, int i) { o[i + side * nk8] = slab[at<N>(l, m)]; });
 }
 
 // Sigma(k,tau_j), j = 0..Nw (green.cpp:1822-1892): G0(k,tau) -> r, x V(r,|tau|), -> k
 template <int N, typename S>
-__global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
-    k_sigma_slab(const double* __restrict__ ek, const S* __restrict__ V, double mu0, double T, int Nw, S* Stau,
+__global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
+    k_sigma_slab(const double* __restrict__ ekw, const S* __restrict__ V, double mu0, double T, int Nw, S* Stau,
                  const double* __restrict__ mu0p)
 {
     if (mu0p) mu0 = *mu0p;
@@ -913,35 +820,26 @@ __global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
     const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
-    auto* tw = slab_tw(slab, (long)nk * nk);
-    fill_twiddles(tw, N);
+    auto* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int j = blockIdx.x;
     const int nwb = Nw / 2 + 1;
     const int jv = (j < nwb) ? j : Nw - j;
     const double t = j / (Nw * T);
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int s = tid; s < nk * nk; s += nt) {
-        const double x = ek[s] - mu0;
-        slab[s] = (S)((x > 0) ? -exp(-t * x) / (exp(-x / T) + 1.0) / nk02
-                              : -exp((1.0 / T - t) * x) / (exp(x / T) + 1.0) / nk02);
-    }
+    each_wedge<N>([&](int l, int m, int i) {
+        const double x = ekw[i] - mu0;
+        put_sym<N>(slab, l, m,
+                   (S)((x > 0) ? -exp(-t * x) / (exp(-x / T) + 1.0) / nk02
+                               : -exp((1.0 / T - t) * x) / (exp(x / T) + 1.0) / nk02));
+    });
     __syncthreads();
-    slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
+    slab_r2r_2d<S, N, 0>(slab, tw);
     const S* Vj = V + (long)jv * nk8;
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        const S v = slab[m + l * nk] * Vj[i];
-        put_sym_t(slab, nk, l, m, v);
-    }
+    each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, slab[at<N>(l, m)] * Vj[i]); });
     __syncthreads();
-    slab_r2r_2d<S, N, 0, 0>(slab, nk, nk, nk, tw);
+    slab_r2r_2d<S, N, 0>(slab, tw);
     S* o = Stau + (long)j * nk8;
-    for (long i = tid; i < nk8; i += nt) {
-        int l, m;
-        wedge_lm(i, l, m);
-        o[i] = slab[m + l * nk];
-    }
+    each_wedge<N>([&](int l, int m, int i) { o[i] = slab[at<N>(l, m)]; });
 }
 
 // green.cpp:1925-2018: per wedge k, spline of Sigma(k,tau_j) (j=0..Nw) with slopes dSig,
@@ -1249,7 +1147,7 @@ __global__ void k_model(int N, double t, double tp, double tpp, double t3, doubl
 // h(r,tau_j) and f0(r,tau_j), j = 0..Nw (cond_opt.cpp:2697-2735, 2795-2827):
 // RODFT00 along kx (index l+1), REDFT00 along ky.
 template <int N, typename S>
-__global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
+__global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     k_hf0_slab(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ mu0p,
                double T, int Nw, S* h, S* f0)
 {
@@ -1259,30 +1157,29 @@ __global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     S* slab = (S*)smem;
-    auto* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
+    auto* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int j = blockIdx.x;
     const double t = (double)j / (T * Nw);
-    const int tid = threadIdx.x, nt = blockDim.x;
     S* const oh = h + (long)j * nq;
     S* const of = f0 + (long)j * nq;
     // h and f0 together (hf0_pair); f0 waits in its output row, read back by the thread that
     // wrote it, while h is transformed
-    for (int s = tid; s < (int)nq; s += nt) {
-        const int l = s / nk, m = s % nk;
+    each_lambda<N>([&](int l, int m, int s) {
         double hv, fv;
         hf0_pair(ek[m + (l + 1) * nk], dek[s], mu0, T, t, nf, hv, fv);
-        slab[s] = (S)hv;
+        slab[at<N>(l + 1, m)] = (S)hv;
         of[s] = (S)fv;
-    }
+    });
     __syncthreads();
-    slab_r2r_2d<S, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-    for (int s = tid; s < (int)nq; s += nt) oh[s] = slab[s];
+    slab_r2r_2d<S, N, 1>(slab, tw);
+    each_lambda<N>([&](int l, int m, int s) {
+        oh[s] = slab[at<N>(l + 1, m)];
+        slab[at<N>(l + 1, m)] = of[s];
+    });
     __syncthreads();
-    for (int s = tid; s < (int)nq; s += nt) slab[s] = of[s];
-    __syncthreads();
-    slab_r2r_2d<S, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-    for (int s = tid; s < (int)nq; s += nt) of[s] = slab[s];
+    slab_r2r_2d<S, N, 1>(slab, tw);
+    each_lambda<N>([&](int l, int m, int s) { of[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // Boundary data of hV and f0V in FP64 (cond_opt.cpp:2697-2735, 2745-3114 at tau = 0, beta).
@@ -1292,13 +1189,12 @@ __global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
 //       slopes dhV / df0V (cond_opt.cpp:2745-3014)
 //   part 0: (3) 2 h(r,tau_b) V(r,0) -> k: hVb / f0Vb, the tau = 0, beta values of hV / f0V
 // Both parts of a (which, side) run (1) themselves and then side by side: three transforms in
-// a row per block instead of four.  Independent of the tau slabs.  bscr: staging, nq per
-// (which, side).
+// a row per block instead of four.  Independent of the tau slabs.
 template <int N>
-__global__ void __launch_bounds__(SLAB_THREADS)
+__global__ void __launch_bounds__(SlabShape<N>::NT)
     k_hf0_bnd(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ V0,
               const double* __restrict__ dchirt0, double mu0, double T, int Nw, double fact4, double* dhV,
-              double* df0V, double* hVb, double* f0Vb, double* bscr, const double* __restrict__ mu0p, double U,
+              double* df0V, double* hVb, double* f0Vb, const double* __restrict__ mu0p, double U,
               const double* __restrict__ dsc)
 {
     if (mu0p) mu0 = *mu0p;
@@ -1308,36 +1204,30 @@ __global__ void __launch_bounds__(SLAB_THREADS)
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
-    cd* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
+    cd* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     const int which = (blockIdx.x >> 1) & 1, side = blockIdx.x & 1, part = blockIdx.x >> 2;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    double* hr = bscr + (blockIdx.x & 3) * nq;
     const double tb = (side == 0) ? 0.0 : (double)Nw / (T * Nw);  // tau_j of k_hf0_slab at j = 0, Nw
     // (1)
-    for (long s = tid; s < nq; s += nt) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
-        slab[s] = hf0_val(which, ek[m + (l + 1) * nk], dek[s], mu0, T, tb, nf);
-    }
+    each_lambda<N>([&](int l, int m, int s) {
+        slab[at<N>(l + 1, m)] = hf0_val(which, ek[m + (l + 1) * nk], dek[s], mu0, T, tb, nf);
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     if (part == 0) {
         // (3), from h(r,tau_b) in place
-        for (long s = tid; s < nq; s += nt) {
-            const int l = (int)(s / nk), m = (int)(s % nk);
-            slab[s] = 2.0 * slab[s] * V0[fold_idx(l + 1, m, N)];
-        }
+        each_lambda<N>([&](int l, int m, int) { slab[at<N>(l + 1, m)] *= 2.0 * V0[fold_idx(l + 1, m, N)]; });
         __syncthreads();
-        slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+        slab_r2r_2d<double, N, 1>(slab, tw);
         double* ob = ((which == 0) ? hVb : f0Vb) + side * nq;
-        for (long s = tid; s < nq; s += nt) ob[s] = slab[s];
+        each_lambda<N>([&](int l, int m, int s) { ob[s] = slab[at<N>(l + 1, m)]; });
         return;
     }
-    for (long s = tid; s < nq; s += nt) hr[s] = slab[s];
+    double hr[lambda_per_thread<N>()];  // h(r,tau_b) of the thread's points
+    each_lambda_slot<N>([&](int l, int m, int, int c) { hr[c] = slab[at<N>(l + 1, m)]; });
     __syncthreads();
     // (2)
-    for (long s = tid; s < nq; s += nt) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
+    each_lambda<N>([&](int l, int m, int s) {
         const double e = ek[m + (l + 1) * nk], v = dek[s];
         double val;
         if (which == 0) {
@@ -1355,25 +1245,25 @@ __global__ void __launch_bounds__(SLAB_THREADS)
                           : nf * v * ((mu0 - e) * (1.0 / (T * (ex + 1.0)) - 1.0 / (T * (ex + 1.0) * (ex + 1.0))) + 1.0 / (ex + 1.0));
             }
         }
-        slab[s] = val;
-    }
+        slab[at<N>(l + 1, m)] = val;
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-    for (long s = tid; s < nq; s += nt) {
-        const int l = (int)(s / nk), m = (int)(s % nk);
+    slab_r2r_2d<double, N, 1>(slab, tw);
+    each_lambda_slot<N>([&](int l, int m, int, int c) {
         const long r = fold_idx(l + 1, m, N);
-        const double d = slab[s], v = V0[r], hs = hr[s];
-        slab[s] = (side == 0) ? 2.0 * d * v + hs * fact4 * dchirt0[r] : 2.0 * d * v - hs * fact4 * dchirt0[r];
-    }
+        const double d = slab[at<N>(l + 1, m)], v = V0[r], hs = hr[c];
+        slab[at<N>(l + 1, m)] =
+            (side == 0) ? 2.0 * d * v + hs * fact4 * dchirt0[r] : 2.0 * d * v - hs * fact4 * dchirt0[r];
+    });
     __syncthreads();
-    slab_r2r_2d<double, N, 1, 0>(slab, nk - 2, nk, nk, tw);
+    slab_r2r_2d<double, N, 1>(slab, tw);
     double* o = ((which == 0) ? dhV : df0V) + side * nq;
-    for (long s = tid; s < nq; s += nt) o[s] = slab[s];
+    each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // hV(k,tau) = DST x DCT [2 h(r,tau) V(r,|tau|)], same for f0, in place (cond_opt.cpp:3029-3114)
 template <int N, typename S>
-__global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
+__global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     k_hVf0V_slab(const S* __restrict__ V, int Nw, S* h, S* f0)
 {
     constexpr int nk = N / 2 + 1;
@@ -1381,22 +1271,20 @@ __global__ void __launch_bounds__(SLAB_THREADS, SlabOcc<S>::waves)
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
-    auto* tw = slab_tw(slab, nq);
-    fill_twiddles(tw, N);
-    const int tid = threadIdx.x, nt = blockDim.x;
+    auto* tw = slab_tw<N>(slab);
+    fill_twiddles<N>(tw);
     // slabs j = blockIdx.x, + gridDim.x, ...: the launch may hold fewer workgroups than slabs
     for (int j = blockIdx.x; j <= Nw; j += gridDim.x) {
         const int jv = (j > Nw / 2) ? Nw - j : j;
         const S* Vj = V + (long)jv * nk8;
         for (int which = 0; which < 2; which++) {
             S* a = ((which == 0) ? h : f0) + (long)j * nq;
-            for (long s = tid; s < nq; s += nt) {
-                const int l = (int)(s / nk), m = (int)(s % nk);
-                slab[s] = (S)2 * a[s] * Vj[fold_idx(l + 1, m, N)];
-            }
+            each_lambda<N>([&](int l, int m, int s) {
+                slab[at<N>(l + 1, m)] = (S)2 * a[s] * Vj[fold_idx(l + 1, m, N)];
+            });
             __syncthreads();
-            slab_r2r_2d<S, N, 1, 0>(slab, nk - 2, nk, nk, tw);
-            for (long s = tid; s < nq; s += nt) a[s] = slab[s];
+            slab_r2r_2d<S, N, 1>(slab, tw);
+            each_lambda<N>([&](int l, int m, int s) { a[s] = slab[at<N>(l + 1, m)]; });
             __syncthreads();
         }
     }
@@ -2006,15 +1894,6 @@ __global__ void __launch_bounds__(256)
 }
 
 // ================================================================== launchers
-// LDS bytes of a slab kernel: the slab (nk x nk, or (nk-2) x nk for Lambda_jj) of elem-byte
-// values, 16-byte aligned, then the N-point twiddle table of the same precision
-static size_t slab_lds(int N, bool lambda, size_t elem)
-{
-    const int nk = N / 2 + 1;
-    const size_t n = lambda ? (size_t)nk * (nk - 2) : (size_t)nk * nk;
-    return ((n * elem + 15) & ~(size_t)15) + 2 * elem * (size_t)N;
-}
-
 // lattice sizes with compiled slab transforms: 2^k (4..256) and 3*2^k (12..192)
 bool supported_N(int N)
 {
@@ -2115,11 +1994,11 @@ hipError_t launch_finalize(const double* part, int n, double* out, hipStream_t s
 
 hipError_t launch_chi0_tau0(const Grid& g, const DevArrays& d, hipStream_t s)
 {
-    const size_t lds = slab_lds(g.N, false, sizeof(double));
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
         set_lds(k_chi0_tau0<NN, SS>, lds);
-        hipLaunchKernelGGL((k_chi0_tau0<NN, SS>), dim3(1), dim3(SLAB_THREADS), lds, s, d.ekw, d.er, d.mu0v, g.T,
-                           (SS*)d.chi, (SS*)d.chirt, d.dchirt0, d.dGrt0p, d.dchiqt0, d.chirt0, d.tmp);
+        hipLaunchKernelGGL((k_chi0_tau0<NN, SS>), dim3(1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.er, d.mu0v, g.T,
+                           (SS*)d.chi, (SS*)d.chirt, d.dchirt0, d.dGrt0p, d.dchiqt0, d.chirt0);
     }));
     return hipGetLastError();
 }
@@ -2127,9 +2006,9 @@ hipError_t launch_chi0_tau0(const Grid& g, const DevArrays& d, hipStream_t s)
 hipError_t launch_chi0_slab(const Grid& g, const DevArrays& d, hipStream_t s)
 {
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
-        const size_t lds = slab_lds(g.N, false, sizeof(SS));
+        constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_chi0_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_chi0_slab<NN, SS>), dim3(g.nwb - 1), dim3(SLAB_THREADS), lds, s, d.ekw, d.mu0v, g.T, g.Nw,
+        hipLaunchKernelGGL((k_chi0_slab<NN, SS>), dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.mu0v, g.T, g.Nw,
                            (SS*)d.chi, (SS*)d.chirt);
     }));
     return hipGetLastError();
@@ -2250,9 +2129,9 @@ hipError_t launch_vertex_slab(const Grid& g, const DevArrays& d, double U, doubl
 {
     const double normFact = g.T / ((double)g.N * g.N);
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
-        const size_t lds = slab_lds(g.N, false, sizeof(SS));
+        constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_vertex_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_vertex_slab<NN, SS>), dim3(g.nwb), dim3(SLAB_THREADS), lds, s, d.chiw, (SS*)d.V,
+        hipLaunchKernelGGL((k_vertex_slab<NN, SS>), dim3(g.nwb), dim3(SlabShape<NN>::NT), lds, s, d.chiw, (SS*)d.V,
                            normFact, U, Usp, Uch, dsc);
     }));
     return hipGetLastError();
@@ -2272,11 +2151,11 @@ hipError_t launch_vertex_pencil(const Grid& g, const DevArrays& d, double U, dou
 hipError_t launch_sigma_bnd(const Grid& g, const DevArrays& d, double mu0, double fact, hipStream_t s,
                             const double* mu0p, double U, const double* dsc)
 {
-    const size_t lds = slab_lds(g.N, false, sizeof(double));
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     DISPATCH_N(g.N, {
         set_lds(k_sigma_bnd<NN>, lds);
-        hipLaunchKernelGGL(k_sigma_bnd<NN>, dim3(4), dim3(SLAB_THREADS), lds, s, d.ek, d.er, d.V0, d.dchirt0, d.dGrt0p,
-                           mu0, g.T, fact, d.dSig, d.Sb, d.tmp, mu0p, U, dsc);
+        hipLaunchKernelGGL(k_sigma_bnd<NN>, dim3(4), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.er, d.V0, d.dchirt0,
+                           d.dGrt0p, mu0, g.T, fact, d.dSig, d.Sb, mu0p, U, dsc);
     });
     return hipGetLastError();
 }
@@ -2284,9 +2163,9 @@ hipError_t launch_sigma_bnd(const Grid& g, const DevArrays& d, double mu0, doubl
 hipError_t launch_sigma_slab(const Grid& g, const DevArrays& d, double mu0, hipStream_t s, const double* mu0p)
 {
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
-        const size_t lds = slab_lds(g.N, false, sizeof(SS));
+        constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_sigma_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_sigma_slab<NN, SS>), dim3(g.Nw + 1), dim3(SLAB_THREADS), lds, s, d.ek, (const SS*)d.V,
+        hipLaunchKernelGGL((k_sigma_slab<NN, SS>), dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, (const SS*)d.V,
                            mu0, g.T, g.Nw, (SS*)d.Stau, mu0p);
     }));
     return hipGetLastError();
@@ -2343,9 +2222,9 @@ hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu0, dou
 hipError_t launch_hf0_slab(const Grid& g, const DevArrays& d, hipStream_t s)
 {
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
-        const size_t lds = slab_lds(g.N, true, sizeof(SS));
+        constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_hf0_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_hf0_slab<NN, SS>), dim3(g.Nw + 1), dim3(SLAB_THREADS), lds, s, d.ek, d.dek, d.mu0v, g.T,
+        hipLaunchKernelGGL((k_hf0_slab<NN, SS>), dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.ek, d.dek, d.mu0v, g.T,
                            g.Nw, (SS*)d.h, (SS*)d.f0);
     }));
     return hipGetLastError();
@@ -2354,11 +2233,11 @@ hipError_t launch_hf0_slab(const Grid& g, const DevArrays& d, hipStream_t s)
 hipError_t launch_hf0_bnd(const Grid& g, const DevArrays& d, double mu0, double fact4, hipStream_t s,
                           const double* mu0p, double U, const double* dsc)
 {
-    const size_t lds = slab_lds(g.N, true, sizeof(double));
+    const size_t lds = slab_bytes(g.N, sizeof(double));
     DISPATCH_N(g.N, {
         set_lds(k_hf0_bnd<NN>, lds);
-        hipLaunchKernelGGL(k_hf0_bnd<NN>, dim3(8), dim3(SLAB_THREADS), lds, s, d.ek, d.dek, d.V0, d.dchirt0, mu0, g.T,
-                           g.Nw, fact4, d.dhV, d.df0V, d.hVb, d.f0Vb, d.bscr, mu0p, U, dsc);
+        hipLaunchKernelGGL(k_hf0_bnd<NN>, dim3(8), dim3(SlabShape<NN>::NT), lds, s, d.ek, d.dek, d.V0, d.dchirt0, mu0, g.T,
+                           g.Nw, fact4, d.dhV, d.df0V, d.hVb, d.f0Vb, mu0p, U, dsc);
     });
     return hipGetLastError();
 }
@@ -2366,15 +2245,15 @@ hipError_t launch_hf0_bnd(const Grid& g, const DevArrays& d, double mu0, double 
 hipError_t launch_hVf0V_slab(const Grid& g, const DevArrays& d, hipStream_t s)
 {
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
-        const size_t lds = slab_lds(g.N, true, sizeof(SS));
+        constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_hVf0V_slab<NN, SS>, lds);
         // FP32: at most kHVBlocks workgroups, each looping over slabs.  This kernel runs beside
         // the latency-bound self-energy pencil and mu search; two of its workgroups fill a CU's
-        // waves, one leaves room for theirs.  An FP64 slab (133 KB of LDS) holds a CU alone
+        // waves, one leaves room for theirs.  An FP64 slab (151 KB of LDS) holds a CU alone
         // either way, and fewer of them only lengthen the kernel (measured at 256^2 x 2048:
         // -0.05 ms per solve in FP32, +0.2 ms in FP64).
         const unsigned nb = (unsigned)((sizeof(SS) == sizeof(float)) ? std::min(g.Nw + 1, kHVBlocks) : g.Nw + 1);
-        hipLaunchKernelGGL((k_hVf0V_slab<NN, SS>), dim3(nb), dim3(SLAB_THREADS), lds, s, (const SS*)d.V, g.Nw,
+        hipLaunchKernelGGL((k_hVf0V_slab<NN, SS>), dim3(nb), dim3(SlabShape<NN>::NT), lds, s, (const SS*)d.V, g.Nw,
                            (SS*)d.h, (SS*)d.f0);
     }));
     return hipGetLastError();

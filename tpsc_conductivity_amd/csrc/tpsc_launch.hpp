@@ -47,7 +47,6 @@ struct DevArrays {
     double* df0V = nullptr;      // 2*nq
     double* hVb = nullptr;       // 2*nq   hV(k, tau = 0), hV(k, tau = beta)
     double* f0Vb = nullptr;      // 2*nq   f0V(k, tau = 0), f0V(k, tau = beta)
-    double* bscr = nullptr;      // 4*nq   staging of the Lambda boundary kernel
     double* hT = nullptr;        // (Nw+1)*nq  hV in point-major layout [q][j]
     double* f0T = nullptr;       // (Nw+1)*nq  f0V in point-major layout
     double* poles = nullptr;     // nq * 64    two-pole data per Lambda point (k_jj_poles)
@@ -55,7 +54,6 @@ struct DevArrays {
     double* jjscal = nullptr;    // nblk * 4      per-workgroup k0, inf sums
     double* kx0part = nullptr;   // 2*nk
     double* jjred = nullptr;     // 2*nwb + 4 reduced Lambda rows and scalars
-    double* tmp = nullptr;       // scratch, >= 4*nk8
     double* part = nullptr;      // reduction partials
     double* red = nullptr;       // reduction result(s)
     HalleyState* root = nullptr;  // state of the device-driven root search
