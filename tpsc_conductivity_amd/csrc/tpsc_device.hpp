@@ -247,21 +247,23 @@ __device__ __forceinline__ void reg_dft(C* v)
 //
 // A slab holds element (i, j), 0 <= i, j < nk = N/2+1, at base[j + i * LD].  A kind-1 axis keeps the
 // natural index too: its elements are 1 .. nk-2, and lines 0 and nk-1 hold nothing.  The even
-// (odd) extension of a line has period N, and its DFT is real (imaginary), so lines f and f + P
-// (P = half the lines) packed as real and imaginary parts give both transforms from one complex
-// FFT of length N = A B:
+// (odd) extension of a line has period N, and its DFT is real (imaginary), so two lines packed as real
+// and imaginary parts give both transforms from one complex FFT of length N = A B:
 //   z[p + B k] -> A-point DFTs over k (lane p) -> w_N^(p k1) -> B-point DFTs over p (lane k1)
 //   -> Z[k1 + A k2].
 // The packed sequence is itself even (odd), so z[N - j] = +-z[j] fixes the DFTs of p > B/2 from
 // those of B - p, and the outputs of k1 > A/2 from those of A - k1: max(A, B)/2 + 1 lanes carry a
-// whole FFT (9 of 16 for N = 256) and 64 lanes hold SlabShape::F of them.  The intermediate values
-// are exchanged inside one wavefront through the LDS of the two lines themselves (real parts in line
-// f, imaginary parts in line f + P), so an axis takes one workgroup barrier.
+// whole FFT (9 of 16 for N = 256) and a wavefront takes 2F lines, line f with line f + F.  The
+// intermediate values are exchanged inside the wavefront through the LDS of the two lines themselves
+// (real parts in the first, imaginary parts in the second), so an axis takes one workgroup barrier.
 //
 // What bounds it: FP64 (FP32) VALU issue and LDS bandwidth, in about equal parts: at N = 256 a lane
 // issues two 16-point DFTs, 16 complex products and ~140 LDS accesses per line pair.  LD = lanes per
 // FFT (mod 16) spreads the lanes of a wavefront over the LDS banks in both axes; the exchange slots
-// are permuted by an exclusive or for the same reason.
+// are rotated within their blocks of B for the same reason, and every address is a lane register and
+// an immediate, with one select where the rotation wraps (1024 slabs of N = 256 alone on the chip:
+// 41.5 us per 2D transform in FP64, 25.2 in FP32; 48.5 and 27.1 with slots permuted by an exclusive or
+// and offsets computed per access).
 // Against cross-lane radix-2 stages (one FFT per wavefront, shuffles between lanes, a full-period FFT
 // for a line pair), kernel times at 256^2 x 2048 before -> after: FP64 chi0 1004 -> 461 us, vertex 298
 // -> 104, Sigma 1092 -> 362, h/f0 1636 -> 976, hV/f0V 1375 -> 844; FP32 384 -> 264, 115 -> 61, 440 ->
@@ -273,7 +275,7 @@ constexpr int slab_A(int N)
          : (N == 32 || N == 64 || N == 128) ? 8 : (N == 96 || N == 192) ? 12 : 16;
 }
 struct SlabDims {
-    int nk, A, B, lanes, F, P, slots, LD, rows, waves, threads;
+    int nk, A, B, lanes, F, slots, LD, rows, waves, threads;
     long elems;
 };
 constexpr SlabDims slab_dims(int N)
@@ -283,14 +285,20 @@ constexpr SlabDims slab_dims(int N)
     d.A = slab_A(N);
     d.B = N / d.A;
     d.lanes = (d.A > d.B ? d.A : d.B) / 2 + 1;  // lanes per FFT
-    d.F = 64 / d.lanes;                         // FFTs per wavefront
-    d.P = (d.nk + 1) / 2;
-    d.slots = d.B * (d.A / 2 + 1) - (d.B - 1) / 2;  // exchanged values per FFT
-    const int least = d.slots > d.nk + 1 ? d.slots : d.nk + 1;
+    const int most = 64 / d.lanes;
+    d.waves = (d.nk + 2 * most - 1) / (2 * most);
+    d.F = (d.nk + 2 * d.waves - 1) / (2 * d.waves);  // FFTs per wavefront
+    d.slots = d.B * (d.A / 2 + 1) - (d.B - 1) / 2;   // exchanged values per FFT
+    // the place of a lone line's partner lies beyond the lines: nk lines from 0, or nk - 2 from 1
+    int least = d.slots;
+    for (int kind = 0; kind < 2; kind++) {
+        const int n = d.nk - 2 * kind, w = (n + 2 * d.F - 1) / (2 * d.F), rest = n - 2 * d.F * (w - 1);
+        const int end = kind + 2 * d.F * (w - 1) + (rest < d.F ? rest : d.F) + d.F;
+        if (end > least) least = end;
+    }
     d.LD = least;
     while (d.LD % 16 != d.lanes % 16) d.LD++;
     d.rows = least;
-    d.waves = (d.P + d.F - 1) / d.F;
     // one round of FFTs per axis, and at least four wavefronts for the pointwise phases
     d.threads = 64 * (d.waves > 4 ? d.waves : 4);
     d.elems = (long)d.rows * d.LD;
@@ -301,10 +309,11 @@ struct SlabShape {
     static constexpr SlabDims D = slab_dims(N);
     static constexpr int A = D.A, B = D.B, F = D.F, LD = D.LD, NT = D.threads;
 };
-// LDS bytes of a slab and its twiddle table (N/4 + 1 entries)
+// LDS bytes of a slab and its twiddle table
 constexpr size_t slab_bytes(int N, size_t elem)
 {
-    return (((size_t)slab_dims(N).elems * elem + 15) & ~(size_t)15) + 2 * elem * (size_t)(N / 4 + 1);
+    return (((size_t)slab_dims(N).elems * elem + 15) & ~(size_t)15) +
+           2 * elem * (size_t)((slab_dims(N).B / 2 + 1) * (slab_dims(N).A / 2));
 }
 // the twiddle table behind the slab, 16-byte aligned
 template <int N, typename Real>
@@ -313,15 +322,17 @@ __device__ __forceinline__ typename cplx_of<Real>::type* slab_tw(Real* slab)
     constexpr size_t off = ((size_t)slab_dims(N).elems * sizeof(Real) + 15) & ~(size_t)15;
     return (typename cplx_of<Real>::type*)((char*)slab + off);
 }
-// tw[t] = exp(-2 pi i t / N), t <= N/4 (block-cooperative; caller syncs); the angle is evaluated in
-// FP64 and rounded to the table precision
+// tw[(k1 - 1)(B/2 + 1) + p] = exp(-2 pi i p k1 / N), 1 <= k1 <= A/2, p <= B/2: the lanes p of a product
+// read neighbours (block-cooperative; caller syncs); the angle is evaluated in FP64 and rounded to
+// the table precision
 template <int N, typename C>
 __device__ __forceinline__ void fill_twiddles(C* tw)
 {
     using F = decltype(C{}.x);
-    for (int t = threadIdx.x; t <= N / 4; t += blockDim.x) {
+    constexpr int W = SlabShape<N>::B / 2 + 1;
+    for (int t = threadIdx.x; t < W * (SlabShape<N>::A / 2); t += blockDim.x) {
         double s, c;
-        sincospi(2.0 * (double)t / (double)N, &s, &c);
+        sincospi(2.0 * (double)((t / W + 1) * (t % W)) / (double)N, &s, &c);
         tw[t] = C{(F)c, (F)(-s)};
     }
 }
@@ -333,6 +344,31 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_wave_barrier();
 }
 
+// A lane's LDS byte offset plus a compile-time constant c: the DS instructions add an immediate below
+// 64 KB, so a column (137 x 1096 bytes at N = 256 in FP64) takes up to three bases, kept apart from the
+// constants by an empty asm; a row takes one.
+template <int MAXC>
+struct LdsAddr {
+    static constexpr int H = 57344, NB = MAXC / H + 1;
+    int b[NB];
+    __device__ __forceinline__ explicit LdsAddr(int o)
+    {
+        b[0] = o;
+#pragma unroll
+        for (int i = 1; i < NB; i++) {
+            b[i] = o + i * H;
+            asm("" : "+v"(b[i]));
+        }
+    }
+    __device__ __forceinline__ int operator()(int c) const { return b[c / H] + c % H; }
+};
+template <int MAXC>
+__device__ __forceinline__ int lds_pick(bool t, const LdsAddr<MAXC>& x, const LdsAddr<MAXC>& y, int c)
+{
+    constexpr int H = LdsAddr<MAXC>::H;
+    return (t ? x.b[c / H] : y.b[c / H]) + c % H;
+}
+
 // transforms of the lines base + i * LS, i < nlines; element e of a line at e * ES
 template <typename Real, int N, int KIND, int LS, int ES>
 __device__ __forceinline__ void wave_r2r_lines(Real* base, int nlines, const typename cplx_of<Real>::type* tw)
@@ -340,73 +376,105 @@ __device__ __forceinline__ void wave_r2r_lines(Real* base, int nlines, const typ
     using C = typename cplx_of<Real>::type;
     constexpr SlabDims D = SlabShape<N>::D;
     constexpr int A = D.A, B = D.B, F = D.F, MIR = (B - 1) / 2;
-    // the lane index through an empty asm: otherwise the compiler computes the lane's ~60 LDS offsets
+    constexpr int E = ES * (int)sizeof(Real);          // bytes from one element to the next
+    constexpr int PAIR = F * LS * (int)sizeof(Real);   // bytes from a line to its partner
+    constexpr int MAXC = (N / 2 + B) * E;
+    // the lane index through an empty asm: otherwise the compiler computes the lane's LDS offsets
     // once for all the transforms of a kernel and keeps them in registers across them
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = SlabShape<N>::NT >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane / D.lanes, p = lane % D.lanes;
-    const int P = (nlines + 1) >> 1;
-    for (int t0 = wave * F; t0 < P; t0 += nwaves * F) {
-        const int f = t0 + sub;
-        const bool ok = sub < F && f < P;
-        const bool has2 = f + P < nlines;
-        Real* const la = base + f * LS;
-        Real* const lb = la + P * LS;
-        if (ok && p <= B / 2) {
-            // a lone last line is packed with itself; its partner's place only holds the exchange
-            const Real* const sb = has2 ? lb : la;
-            C v[A];
+    const int f = 2 * F * wave + sub;  // the first line
+    if (2 * F * wave >= nlines) return;
+    const bool ok = sub < F && f < nlines;
+    const bool has2 = f + F < nlines;
+    // element at byte offset o of the first (a) or the second (b) line
+    const int lb0 = f * LS * (int)sizeof(Real);
+    auto la = [&](int o) -> Real& { return *(Real*)((char*)base + o); };
+    auto lb = [&](int o) -> Real& { return *(Real*)((char*)base + o + PAIR); };
+    if (ok && p <= B / 2) {
+        const LdsAddr<MAXC> up(lb0 + p * E), down(lb0 - p * E), upw(lb0 + p * E - B * E);
+        // a lone last line is packed with itself; its partner's place only holds the exchange
+        const int pair = has2 ? PAIR : 0;
+        C v[A];
 #pragma unroll
-            for (int k = 0; k < A; k++) {
-                const int o = (k < A / 2) ? p * ES + B * k * ES : B * (A - k) * ES - p * ES;
-                Real a = la[o], b = sb[o];
-                if constexpr (KIND == 1) {
-                    if (k == 0 || k == A / 2) {
-                        a = (p == 0) ? (Real)0 : a;
-                        b = (p == 0) ? (Real)0 : b;
-                    }
-                    if (k >= A / 2) {
-                        a = -a;
-                        b = -b;
-                    }
+        for (int k = 0; k < A; k++) {
+            const int o = (k < A / 2) ? up(B * k * E) : down(B * (A - k) * E);
+            Real a = la(o), b = *(Real*)((char*)base + o + pair);
+            if constexpr (KIND == 1) {
+                if (k == 0 || k == A / 2) {
+                    a = (p == 0) ? (Real)0 : a;
+                    b = (p == 0) ? (Real)0 : b;
                 }
-                v[k] = C{a, b};
+                if (k >= A / 2) {
+                    a = -a;
+                    b = -b;
+                }
             }
-            reg_dft<A>(v);
-            la[p * ES] = v[0].x;
-            lb[p * ES] = v[0].y;
-            const bool mirror = p != 0 && 2 * p != B;
+            v[k] = C{a, b};
+        }
+        reg_dft<A>(v);
+        la(up(0)) = v[0].x;
+        lb(up(0)) = v[0].y;
+        // slot of (p, k1 > 0): B k1 - MIR + (p + k1 + MIR) mod B, of (p, 0): p
+        const bool mirror = p != 0 && 2 * p != B;
 #pragma unroll
-            for (int k1 = 1; k1 <= A / 2; k1++) {
-                const C w = tw[p * k1];
-                const C e = v[k1] * w;
-                const int o = (p ^ (k1 & (B - 1))) * ES + (B * k1 - MIR) * ES;
-                la[o] = e.x;
-                lb[o] = e.y;
-                if constexpr (B > 2) {
-                    if (mirror) {
-                        C m = v[A - k1] * C{w.x, -w.y};
-                        if constexpr (KIND == 1) m = C{-m.x, -m.y};
-                        const int om = ((B - p) ^ (k1 & (B - 1))) * ES + (B * k1 - MIR) * ES;
-                        la[om] = m.x;
-                        lb[om] = m.y;
-                    }
+        for (int k1 = 1; k1 <= A / 2; k1++) {
+            constexpr int W = B / 2 + 1;
+            const int kk = (k1 + MIR) % B;
+            const C w = tw[(k1 - 1) * W + p];
+            const C e = v[k1] * w;
+            const int o = lds_pick(p >= B - kk, upw, up, (B * k1 - MIR + kk) * E);
+            la(o) = e.x;
+            lb(o) = e.y;
+            if constexpr (B > 2) {
+                if (mirror) {
+                    C m = v[A - k1] * C{w.x, -w.y};
+                    if constexpr (KIND == 1) m = C{-m.x, -m.y};
+                    const int om = down((B * k1 - MIR + kk) * E) + ((kk >= MIR || p <= kk) ? 0 : B * E);
+                    la(om) = m.x;
+                    lb(om) = m.y;
                 }
             }
         }
-        wave_lds_order();
-        if (ok && p <= A / 2) {
-            int q = p;
-            asm volatile("" : "+v"(q));
-            const int xr = q & (B - 1);
-            const int bq = (q == 0) ? 0 : B * q - MIR;
-            C v[B];
+    }
+    wave_lds_order();
+    if (ok && p <= A / 2) {
+        int q = p;
+        asm volatile("" : "+v"(q));
+        C v[B];
+        if constexpr (B == 16) {
+            // q > 0: (r + q + 7) mod 16 wraps at r + q >= 9, always for r > 8; q = 0 reads r, and the
+            // value of 16 - r for r > 8
+            const int at0 = lb0 + 17 * q * E, atw = at0 - B * E;
+            const unsigned q17 = 17u * q * E;
 #pragma unroll
             for (int r = 0; r < B; r++) {
-                int o = bq + (r ^ xr);
-                if (r > B / 2) o = (q == 0) ? B - r : o;
-                Real a = la[o * ES], b = lb[o * ES];
+                int o;
+                if (r <= 8) {
+                    o = ((q >= 9 - r) ? atw : at0) + r * E;
+                } else {
+                    const unsigned c = (16 - r) * E;
+                    o = (int)((q17 > c ? q17 : c) - (q17 < c ? q17 : c)) + lb0;
+                }
+                Real a = la(o), b = lb(o);
+                if constexpr (KIND == 1) {
+                    if (r > 8) {
+                        a = (q == 0) ? -a : a;
+                        b = (q == 0) ? -b : b;
+                    }
+                }
+                v[r] = C{a, b};
+            }
+        } else {
+            const int qm = (q == 0) ? 0 : (q + MIR) & (B - 1);
+            const int at0 = lb0 + ((q == 0) ? 0 : B * q - MIR + qm) * E, atw = at0 - B * E;
+#pragma unroll
+            for (int r = 0; r < B; r++) {
+                int o = ((qm >= B - r) ? atw : at0) + r * E;
+                if (r > B / 2) o = (q == 0) ? lb0 + (B - r) * E : o;
+                Real a = la(o), b = lb(o);
                 if constexpr (KIND == 1) {
                     if (r > B / 2) {
                         a = (q == 0) ? -a : a;
@@ -415,21 +483,22 @@ __device__ __forceinline__ void wave_r2r_lines(Real* base, int nlines, const typ
                 }
                 v[r] = C{a, b};
             }
-            reg_dft<B>(v);
-            wave_lds_order();
-            // Z[q + A k2]: the direct index up to N/2, the mirrored one beyond (equal up to the
-            // parity; lanes 0 and A/2 write some values twice)
+        }
+        reg_dft<B>(v);
+        wave_lds_order();
+        // Z[q + A k2]: the direct index up to N/2, the mirrored one beyond (equal up to the
+        // parity; lanes 0 and A/2 write some values twice)
+        const LdsAddr<MAXC> up(lb0 + q * E), down(lb0 - q * E);
 #pragma unroll
-            for (int k2 = 0; k2 < B; k2++) {
-                const bool direct = k2 < (B + 1) / 2;
-                const int o = direct ? q * ES + A * k2 * ES : A * (B - k2) * ES - q * ES;
-                if constexpr (KIND == 0) {
-                    la[o] = v[k2].x;
-                    if (has2) lb[o] = v[k2].y;
-                } else {
-                    la[o] = direct ? -v[k2].y : v[k2].y;
-                    if (has2) lb[o] = direct ? v[k2].x : -v[k2].x;
-                }
+        for (int k2 = 0; k2 < B; k2++) {
+            const bool direct = k2 < (B + 1) / 2;
+            const int o = direct ? up(A * k2 * E) : down(A * (B - k2) * E);
+            if constexpr (KIND == 0) {
+                la(o) = v[k2].x;
+                if (has2) lb(o) = v[k2].y;
+            } else {
+                la(o) = direct ? -v[k2].y : v[k2].y;
+                if (has2) lb(o) = direct ? v[k2].x : -v[k2].x;
             }
         }
     }
