@@ -21,39 +21,30 @@ namespace tpsc {
 #define AL_PEN_THREADS 256
 #define AL_K_THREADS 512
 
-// G0(k,-tau)/N^2 (cond_opt.cpp:4396-4400) and its tau = 0 slope (:4417-4421)
-__device__ __forceinline__ double al_g0m(double x, double t, double T, double nf)
-{
-    return (x < 0) ? nf * exp(x * t) / (exp(x / T) + 1.0) : nf * exp(x * (t - 1.0 / T)) / (exp(-x / T) + 1.0);
-}
-__device__ __forceinline__ double al_dg0m(double x, double T, double nf)
-{
-    return (x < 0) ? nf * x / (exp(x / T) + 1.0) : nf * x * exp(-x / T) / (exp(-x / T) + 1.0);
-}
-
-// Block j <= Nw: Grt[j*nk8 + w] = G0(r_w, -tau_j).  Block Nw+1: dGrt[w] = d/dtau G0(r,-tau) at
-// tau = 0 and dGrt[nk8 + w] = eps(r) - mu0 delta_r0 - dGrt[w] at tau = beta.
+// Block j <= Nw: Grt[j*nk8 + w] = G0(r_w, -tau_j) (cond_opt.cpp:4396-4400).  Block Nw+1: dGrt[w] = d/dtau
+// G0(r,-tau) at tau = 0 (x G0(k,0-), :4417-4421) and dGrt[nk8 + w] = eps(r) - mu0 delta_r0 - dGrt[w] at
+// tau = beta.
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_al_grt_slab(const double* __restrict__ ekw, const double* __restrict__ er, double mu0, double T, int Nw,
-                  double* Grt, double* dGrt)
+    k_al_grt_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+                  const double* __restrict__ er, double mu0, double T, int Nw, double* Grt, double* dGrt)
 {
     constexpr long nk8 = (long)(N / 2 + 1) * (N / 2 + 2) / 2;
-    const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const int j = blockIdx.x;
-    const double t = (double)j / (T * Nw);
-    each_wedge<N>([&](int l, int m, int i) {
+    const double t = (j <= Nw) ? (double)j / (T * Nw) : 0.0, bt = 1.0 / T - t;
+    each_wedge<N>(wt, [&](int a, int b, int i) {
         const double x = ekw[i] - mu0;
-        put_sym<N>(slab, l, m, (j <= Nw) ? al_g0m(x, t, T, nf) : al_dg0m(x, T, nf));
+        const double g = g0_exp(x, bt, t) * fw[i];
+        slab[a] = slab[b] = (j <= Nw) ? g : x * g;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) {
-        const double v = slab[at<N>(l, m)];
+    each_wedge<N>(wt, [&](int a, int, int i) {
+        const double v = slab[a];
         if (j <= Nw) {
             Grt[(long)j * nk8 + i] = v;
         } else {
@@ -66,52 +57,62 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
 // Block j <= Nw: hGs[j*nq + q] = DST x DCT [h(r,tau_j) G0(r,-tau_j)] with h(r,tau) the
 // DST x DCT of the k-space integrand (cond_opt.cpp:4302-4330, 5231-5261).
 // Blocks Nw+1+side: slope at tau = 0 / beta of the same product (:5159-5229),
-// dh(r) G0(r,-tau_b) + h(r,tau_b) dG0(r,-tau_b), back to q -> dhG[side*nq + q].
+// dh(r) G0(r,-tau_b) + h(r,tau_b) dG0(r,-tau_b), dh(k) = -x h(k), back to q -> dhG[side*nq + q].
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_al_hg_slab(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ Grt,
-                 const double* __restrict__ dGrt, double mu0, double T, int Nw, double* hGs, double* dhG)
+    k_al_hg_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+                 const double* __restrict__ vw, const double* __restrict__ Grt, const double* __restrict__ dGrt,
+                 double mu0, double T, int Nw, double* hGs, double* dhG)
 {
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
-    constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    constexpr int PER = lambda_per_thread<N>();
-    const double nf = 1.0 / ((double)N * N);
+    constexpr int nk8 = nk * (nk + 1) / 2, PER = wedge_per_thread<N>();
     extern __shared__ double smem[];
     double* slab = smem;
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const int b = blockIdx.x;
     const int jt = (b <= Nw) ? b : ((b == Nw + 1) ? 0 : Nw);
-    const double t = (double)jt / (T * Nw);
-    each_lambda<N>([&](int l, int m, int s) {
-        slab[at<N>(l + 1, m)] = hf0_val(0, ek[m + (l + 1) * nk], dek[s], mu0, T, t, nf);
+    const double t = (double)jt / (T * Nw), bt = 1.0 / T - t;
+    each_wedge<N>(wt, [&](int o, int p, int i) {
+        const double g = g0_exp(ekw[i] - mu0, t, bt) * fw[i];
+        slab[o] = g * vw[i];
+        slab[p] = g * vw[nk8 + i];
     });
+    const double* g = Grt + (long)jt * nk8;
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
     if (b <= Nw) {
-        const double* g = Grt + (long)b * nk8;
-        each_lambda<N>([&](int l, int m, int) { slab[at<N>(l + 1, m)] *= g[fold_idx(l + 1, m, N)]; });
+        each_wedge<N>(wt, [&](int o, int p, int i) {
+            const double v = g[i], ra = slab[o] * v, rb = slab[p] * v;
+            slab[o] = ra;
+            slab[p] = rb;
+        });
         __syncthreads();
         slab_r2r_2d<double, N, 1>(slab, tw);
-        double* o = hGs + (long)b * nq;
-        each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
+        double* out = hGs + (long)b * nq;
+        each_lambda<N>([&](int l, int m, int s) { out[s] = slab[at<N>(l + 1, m)]; });
         return;
     }
     const int side = b - Nw - 1;
-    double st[PER];
-    each_lambda_slot<N>([&](int l, int m, int, int c) {
-        st[c] = slab[at<N>(l + 1, m)] * dGrt[side * nk8 + fold_idx(l + 1, m, N)];
+    double sa[PER], sb[PER];
+    each_wedge_slot<N>(wt, [&](int o, int p, int i, int c) {
+        const double v = dGrt[side * nk8 + i];
+        sa[c] = slab[o] * v;
+        sb[c] = slab[p] * v;
     });
     __syncthreads();
-    each_lambda<N>([&](int l, int m, int s) {
-        slab[at<N>(l + 1, m)] = h_slope_val(side, ek[m + (l + 1) * nk], dek[s], mu0, T, nf);
+    each_wedge<N>(wt, [&](int o, int p, int i) {
+        const double x = ekw[i] - mu0, v = -x * g0_exp(x, t, bt) * fw[i];
+        slab[o] = v * vw[i];
+        slab[p] = v * vw[nk8 + i];
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
-    const double* g = Grt + (long)jt * nk8;
-    each_lambda_slot<N>([&](int l, int m, int, int c) {
-        slab[at<N>(l + 1, m)] = slab[at<N>(l + 1, m)] * g[fold_idx(l + 1, m, N)] + st[c];
+    each_wedge_slot<N>(wt, [&](int o, int p, int i, int c) {
+        const double ra = slab[o] * g[i] + sa[c], rb = slab[p] * g[i] + sb[c];
+        slab[o] = ra;
+        slab[p] = rb;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
@@ -274,13 +275,14 @@ __global__ void __launch_bounds__(AL_PEN_THREADS)
 // Planes: HGs, P1s, P2s [c][t][q]; dHq [c][side][q]; dP [which][side][c][q].
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_al_prod_slab(const double* __restrict__ HGs, const double* __restrict__ dHq, const double* __restrict__ Grt,
-                   const double* __restrict__ dGrt, int L, double* P1s, double* P2s, double* dP)
+    k_al_prod_slab(const unsigned* __restrict__ wt, const double* __restrict__ HGs, const double* __restrict__ dHq,
+                   const double* __restrict__ Grt, const double* __restrict__ dGrt, int L, double* P1s, double* P2s,
+                   double* dP)
 {
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    constexpr int PER = lambda_per_thread<N>();
+    constexpr int PER = wedge_per_thread<N>();
     const double nf = 1.0 / ((double)N * N);
     extern __shared__ double smem[];
     double* slab = smem;
@@ -304,26 +306,30 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = nf * src[s]; });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
-    double st[PER];  // HG(r,tau) of the thread's points
-    each_lambda_slot<N>([&](int l, int m, int, int i) { st[i] = slab[at<N>(l + 1, m)]; });
+    double sa[PER], sb[PER];  // HG(r,tau) at (l, m) and (m, l) of the thread's points
+    each_wedge_slot<N>(wt, [&](int o, int p, int, int i) {
+        sa[i] = slab[o];
+        sb[i] = slab[p];
+    });
     __syncthreads();
     if (main_blk) {
 #pragma unroll 1
         for (int pass = 0; pass < 2; pass++) {
             const int tg = pass ? L - tA : tA;
             const double* g = Grt + (long)tg * nk8;
-            each_lambda_slot<N>(
-                [&](int l, int m, int, int i) { slab[at<N>(l + 1, m)] = st[i] * g[fold_idx(l + 1, m, N)]; });
+            each_wedge_slot<N>(wt, [&](int o, int p, int w, int i) {
+                slab[o] = sa[i] * g[w];
+                slab[p] = sb[i] * g[w];
+            });
             __syncthreads();
             slab_r2r_2d<double, N, 1>(slab, tw);
-            double* o = (pass ? P2s : P1s) + c * plane + (long)tg * nq;
-            each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
+            double* out = (pass ? P2s : P1s) + c * plane + (long)tg * nq;
+            each_lambda<N>([&](int l, int m, int s) { out[s] = slab[at<N>(l + 1, m)]; });
             __syncthreads();
         }
         return;
     }
     const double* dg = dGrt + side * nk8;
-    each_lambda_slot<N>([&](int l, int m, int, int i) { st[i] *= dg[fold_idx(l + 1, m, N)]; });
     const int ds = which ? 1 - side : side;
     const double sgn = which ? -1.0 : 1.0;
     const double* dsrc = dHq + (long)(c * 2 + ds) * nq;
@@ -331,13 +337,15 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
     const double* g = Grt + (long)(side ? L : 0) * nk8;
-    each_lambda_slot<N>([&](int l, int m, int, int i) {
-        slab[at<N>(l + 1, m)] = sgn * slab[at<N>(l + 1, m)] * g[fold_idx(l + 1, m, N)] + st[i];
+    each_wedge_slot<N>(wt, [&](int o, int p, int w, int i) {
+        const double ra = sgn * slab[o] * g[w] + sa[i] * dg[w], rb = sgn * slab[p] * g[w] + sb[i] * dg[w];
+        slab[o] = ra;
+        slab[p] = rb;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
-    double* o = dP + (long)((which * 2 + side) * 2 + c) * nq;
-    each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
+    double* out = dP + (long)((which * 2 + side) * 2 + c) * nq;
+    each_lambda<N>([&](int l, int m, int s) { out[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // Dyson G(k, i w_f) = 1/(i w_f + mu - e - Sigma(k,iw_f)), Sigma from the stored form for
@@ -502,11 +510,11 @@ hipError_t launch_al_setup(const Grid& g, const DevArrays& d, const ALArrays& a,
     AL_DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(double));
         al_set_lds(k_al_grt_slab<NN>, lds);
-        hipLaunchKernelGGL(k_al_grt_slab<NN>, dim3(g.Nw + 2), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.er, mu0, g.T,
-                           g.Nw, a.Grt, a.dGrt);
+        hipLaunchKernelGGL(k_al_grt_slab<NN>, dim3(g.Nw + 2), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw, d.er,
+                           mu0, g.T, g.Nw, a.Grt, a.dGrt);
         al_set_lds(k_al_hg_slab<NN>, lds);
-        hipLaunchKernelGGL(k_al_hg_slab<NN>, dim3(g.Nw + 3), dim3(SlabShape<NN>::NT), lds, s, d.ek, d.dek, a.Grt,
-                           a.dGrt, mu0, g.T, g.Nw, a.P1s, a.dhG);
+        hipLaunchKernelGGL(k_al_hg_slab<NN>, dim3(g.Nw + 3), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw, d.vw,
+                           a.Grt, a.dGrt, mu0, g.T, g.Nw, a.P1s, a.dhG);
     });
     hipError_t e = launch_transpose_d(a.P1s, a.P1p, g.nq, g.Nw + 1, s);
     if (e != hipSuccess) return e;
@@ -533,7 +541,7 @@ hipError_t launch_al_freq(const Grid& g, const DevArrays& d, const ALArrays& a, 
     AL_DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(double));
         al_set_lds(k_al_prod_slab<NN>, lds);
-        hipLaunchKernelGGL(k_al_prod_slab<NN>, dim3(2 * (g.Nw + 1) + 8), dim3(SlabShape<NN>::NT), lds, s, a.HGs, a.dHq,
+        hipLaunchKernelGGL(k_al_prod_slab<NN>, dim3(2 * (g.Nw + 1) + 8), dim3(SlabShape<NN>::NT), lds, s, d.wt, a.HGs, a.dHq,
                            a.Grt, a.dGrt, g.Nw, a.P1s, a.P2s, a.dP);
     });
     for (int c = 0; c < 2; c++) {

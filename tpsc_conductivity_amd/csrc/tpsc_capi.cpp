@@ -96,8 +96,6 @@ struct tpsc_ctx {
     hipStream_t stream = nullptr;
     hipStream_t side = nullptr;  // boundary kernels, overlapped with the slab kernels
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    hipEvent_t ev_tau0 = nullptr, ev_hf0 = nullptr;
-    bool hf0_pending = false;  // h(r,tau), f0(r,tau) queued on the prep stream at the chi0 stage
     // third stream: the Lambda stage's hV/f0V slabs, transposes and boundary data, queued at the
     // end of the vertex stage and overlapped with the self-energy and mu stages
     hipStream_t prep = nullptr;
@@ -416,9 +414,8 @@ int mu0_ready(tpsc_ctx* c)
 // The device arrays are kept.
 int invalidate_stages(tpsc_ctx* c)
 {
-    if (c->hv_pending || c->hf0_pending) {
+    if (c->hv_pending) {
         HIPCHK(c, hipStreamSynchronize(c->prep));
-        c->hf0_pending = false;
         c->hv_pending = false;
     }
     c->have_chi0 = c->have_U = c->have_V = c->have_sigma = c->have_jj = false;
@@ -478,10 +475,6 @@ int stage_chi0(tpsc_ctx* c, int nq0, int nw0, bool defer = false)
     int rc = settle_prep(c, false);
     if (rc) return rc;
     hipStream_t s = c->stream;
-    if (c->hf0_pending) {  // h, f0 of an earlier chain, still read on the prep stream, use eps(k)
-        HIPCHK(c, hipStreamWaitEvent(s, c->ev_hf0, 0));
-        c->hf0_pending = false;
-    }
     rc = set_grid(c, nq0, nw0);
     if (rc) return rc;
     // the arrays and precision this stage computes in: FP64 throughout for a promoted full grid
@@ -506,19 +499,7 @@ int stage_chi0(tpsc_ctx* c, int nq0, int nw0, bool defer = false)
     prof_begin(c, "chi0_tau0");
     HIPCHK(c, launch_chi0_tau0(gx, dx, s));
     prof_end(c);
-    HIPCHK(c, hipEventRecord(c->ev_tau0, s));
     if ((rc = join_side(c))) return rc;
-    // h(r,tau) and f0(r,tau) of the Lambda stage need only mu0 and eps(k): on the full grid
-    // they are queued now on the prep stream, behind the tau = 0 slice, and run beside the chi0
-    // slab and pencils and the sum-rule passes; the Lambda stage waits for ev_hf0
-    if (full_grid(c)) {
-        HIPCHK(c, hipStreamWaitEvent(c->prep, c->ev_tau0, 0));
-        prof_begin(c, "jj_hf0_slab", c->prep);
-        HIPCHK(c, launch_hf0_slab(c->g, c->d, c->prep));
-        prof_end(c);
-        HIPCHK(c, hipEventRecord(c->ev_hf0, c->prep));
-        c->hf0_pending = true;
-    }
     if (c->keep_chi_tau && c->chi_tau) {
         HIPCHK(c, hipMemcpyAsync(c->chi_tau, dx.chi, (f64 ? sizeof(double) : elem_bytes(c)) * c->g.nwb * c->g.nk8,
                                  hipMemcpyDeviceToDevice, s));
@@ -691,24 +672,31 @@ int stage_vertex(tpsc_ctx* c)
     HIPCHK(c, hipEventRecord(c->ev_v, c->stream));  // V and V(r,0) are complete here
     prof_flush(c);
     c->have_V = true;
-    // The Lambda stage's boundary data, hV and f0V slabs (h, f0 times V) and their point-major
-    // transposes need V, mu0, Usp, Uch and the h, f0 slabs of the chi0 stage only.  They run on
-    // the prep stream: the boundary kernel (four workgroups) from here, the slabs once the
-    // self-energy slab is done (queued by stage_sigma), beside the latency-bound self-energy
-    // pencil, traces and mu search.
-    if (c->hf0_pending) {
-        const double fact4 = c->p.U * (3.0 * c->Usp + c->Uch) / 4;
-        HIPCHK(c, hipStreamWaitEvent(c->prep, c->ev_hf0, 0));
-        HIPCHK(c, hipStreamWaitEvent(c->prep, c->ev_v, 0));
-        c->hf0_pending = false;
-        prof_begin(c, "jj_hf0_bnd", c->prep);
-        HIPCHK(c, launch_hf0_bnd(c->g, c->d, c->mu0, fact4, c->prep));
-        HIPCHK(c, hipEventRecord(c->ev_bnd, c->prep));
+    // The Lambda stage's boundary data, hV and f0V slabs and their point-major transposes need V,
+    // mu0, Usp and Uch only.  They run on the prep stream: the boundary kernel (eight workgroups) from
+    // here, the slabs once the self-energy slab is done (queued by stage_sigma), beside the
+    // latency-bound self-energy pencil, traces and mu search.
+    const double fact4 = c->p.U * (3.0 * c->Usp + c->Uch) / 4;
+    HIPCHK(c, hipStreamWaitEvent(c->prep, c->ev_v, 0));
+    prof_begin(c, "jj_hf0_bnd", c->prep);
+    HIPCHK(c, launch_hf0_bnd(c->g, c->d, c->mu0, fact4, c->prep));
+    HIPCHK(c, hipEventRecord(c->ev_bnd, c->prep));
+    prof_end(c);
+    c->hv_slabs_due = true;
+    c->hv_dropped = false;
+    HIPCHK(c, hipEventRecord(c->ev_hv, c->prep));
+    c->hv_pending = true;
+    return 0;
+}
+
+// the hV and f0V slabs on stream st (profile regions: "jj_hf0_slab" the h, hV slices, "jj_hVf0V_slab" the
+// f0, f0V slices)
+int launch_lambda_slabs(tpsc_ctx* c, hipStream_t st)
+{
+    for (int which = 0; which < 2; which++) {
+        prof_begin(c, which == 0 ? "jj_hf0_slab" : "jj_hVf0V_slab", st);
+        HIPCHK(c, launch_hV_slab(c->g, c->d, which, st));
         prof_end(c);
-        c->hv_slabs_due = true;
-        c->hv_dropped = false;
-        HIPCHK(c, hipEventRecord(c->ev_hv, c->prep));
-        c->hv_pending = true;
     }
     return 0;
 }
@@ -721,9 +709,7 @@ int queue_hv_slabs(tpsc_ctx* c)
     c->hv_slabs_due = false;
     HIPCHK(c, hipEventRecord(c->ev_sig, c->stream));
     HIPCHK(c, hipStreamWaitEvent(c->prep, c->ev_sig, 0));
-    prof_begin(c, "jj_hVf0V_slab", c->prep);
-    HIPCHK(c, launch_hVf0V_slab(c->g, c->d, c->prep));
-    prof_end(c);
+    if (int rc = launch_lambda_slabs(c, c->prep)) return rc;
     prof_begin(c, "jj_transpose", c->prep);
     HIPCHK(c, launch_jj_transpose(c->g, c->d, c->prep));
     prof_end(c);
@@ -933,17 +919,7 @@ int stage_chijj(tpsc_ctx* c, int ntheta)
         prof_end(c);
     }
     if (!prepared) {
-        if (c->hf0_pending) {
-            HIPCHK(c, hipStreamWaitEvent(s, c->ev_hf0, 0));
-            c->hf0_pending = false;
-        } else {
-            prof_begin(c, "jj_hf0_slab");
-            HIPCHK(c, launch_hf0_slab(g, c->d, s));
-            prof_end(c);
-        }
-        prof_begin(c, "jj_hVf0V_slab");
-        HIPCHK(c, launch_hVf0V_slab(g, c->d, s));
-        prof_end(c);
+        if ((rc = launch_lambda_slabs(c, s))) return rc;
         prof_begin(c, "jj_transpose");
         HIPCHK(c, launch_jj_transpose(g, c->d, s));
         prof_end(c);
@@ -1448,9 +1424,7 @@ int tpsc_create(const tpsc_params* p, tpsc_ctx** out)
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_sig, hipEventDisableTiming));
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
-    HIPCHK(c, hipEventCreateWithFlags(&c->ev_tau0, hipEventDisableTiming));
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_bnd, hipEventDisableTiming));
-    HIPCHK(c, hipEventCreateWithFlags(&c->ev_hf0, hipEventDisableTiming));
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_mu0, hipEventDisableTiming));
     HIPCHK(c, hipHostMalloc((void**)&c->host_scalar, kHostScalars * sizeof(double), hipHostMallocMapped));
     HIPCHK(c, hipHostGetDevicePointer((void**)&c->dev_scalar, c->host_scalar, 0));
@@ -1465,6 +1439,9 @@ int tpsc_create(const tpsc_params* p, tpsc_ctx** out)
     rc |= dalloc(c, &d.ekw, nk8);
     rc |= dalloc(c, &d.wq, nk8);
     rc |= dalloc(c, &d.er, std::max<long>(nk8, 5));
+    rc |= dalloc(c, &d.wt, nk8);
+    rc |= dalloc(c, &d.fw, 2 * nk8);
+    rc |= dalloc(c, &d.vw, 2 * nk8);
     rc |= dalloc(c, &d.chi, (size_t)nwb * nk8, es);
     if (p->precision)
         rc |= dalloc(c, &d.chiw, (size_t)nwb * nk8);
@@ -1545,9 +1522,7 @@ void tpsc_destroy(tpsc_ctx* c)
     if (c->host_scalar) (void)hipHostFree(c->host_scalar);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-    if (c->ev_tau0) (void)hipEventDestroy(c->ev_tau0);
     if (c->ev_bnd) (void)hipEventDestroy(c->ev_bnd);
-    if (c->ev_hf0) (void)hipEventDestroy(c->ev_hf0);
     if (c->ev_mu0) (void)hipEventDestroy(c->ev_mu0);
     for (auto& rg : c->root_graphs)
         if (rg.exec) (void)hipGraphExecDestroy(rg.exec);
@@ -2225,9 +2200,8 @@ int tpsc_queue_solve(tpsc_ctx* c, const tpsc_params* p, double* slot_dev, bool c
     HIPCHK(c, launch_halley_init(d.root, s0, nullptr, psc + kPscMu, s, d.mu0v));
     for (int k = 0; k < nmu; k++) HIPCHK(c, launch_trace_diffG3_pass(g, d, psc + kPscMu, s));
     // Lambda_jj bubble + Maki-Thompson and the diamagnetic rows (stage_chijj, N_theta_k = 1)
-    HIPCHK(c, launch_hf0_slab(g, d, s));
     HIPCHK(c, launch_hf0_bnd(g, d, 0.0, 0.0, s, d.mu0v, U, psc));
-    HIPCHK(c, launch_hVf0V_slab(g, d, s));
+    for (int which = 0; which < 2; which++) HIPCHK(c, launch_hV_slab(g, d, which, s));
     HIPCHK(c, launch_jj_transpose(g, d, s));
     double* const slot_rows = slot_dev + kPscDoubles;  // reduced Lambda rows, scalar sums, kx0 rows
     HIPCHK(c, launch_kx0_rows(g, d, 0.0, s, psc, slot_rows + 2 * g.nwb + 4));

@@ -949,51 +949,57 @@ __device__ inline double block_sum(double v, double* scratch)
 
 
 // ---------------------------------------------------------------------------------
-// slab layout helpers, Sigma(k,iwn) storage forms and the Lambda-grid integrand h / f0
-// (shared by tpsc_kernels.hip and tpsc_al.hip)
+// pointwise loops over a slab, the tau dependence of G0 and the Sigma(k,iwn) storage forms (shared by
+// the slab and pencil kernels of all files)
 // ---------------------------------------------------------------------------------
-// The t-th point (l, m), m <= l, of the wedge for the pointwise phases of a slab: rows r and
-// nk - 1 - r together hold nk + 1 points, so t runs over a rectangle of that width (nk is odd; the
-// middle row comes last) and no square root is needed.
-template <int N>
-__device__ __forceinline__ void wedge_pt(int t, int& l, int& m)
-{
-    constexpr int nk = N / 2 + 1;
-    static_assert(nk % 2 == 1, "the row pairing needs an odd nk");
-    const int r = t / (nk + 1), s = t - r * (nk + 1);
-    const bool low = s <= r;
-    l = low ? r : nk - 1 - r;
-    m = low ? s : s - r - 1;
-}
-// f(l, m, i) for every wedge point of the workgroup's share, i = its packed index
-template <int N, typename Fn>
-__device__ __forceinline__ void each_wedge(Fn&& f)
-{
-    constexpr int nk8 = (N / 2 + 1) * (N / 2 + 2) / 2;
-#pragma unroll 2
-    for (int t = threadIdx.x; t < nk8; t += SlabShape<N>::NT) {
-        int l, m;
-        wedge_pt<N>(t, l, m);
-        f(l, m, m + l * (l + 1) / 2);
-    }
-}
-// the same with the slot c of the point among the thread's own, unrolled: f may index registers by c
+// f(a, b, i) for every wedge point i (packed index) of the workgroup's share, a and b the slab offsets
+// of (l, m) and (m, l), from the table wt (k_model): a pointwise phase then reads its wedge arrays in
+// order and does no index arithmetic.  The loop is unrolled in at most two batches, so that the loads of
+// a batch are in flight together.
 template <int N>
 constexpr int wedge_per_thread() { return ((N / 2 + 1) * (N / 2 + 2) / 2 + SlabShape<N>::NT - 1) / SlabShape<N>::NT; }
 template <int N, typename Fn>
-__device__ __forceinline__ void each_wedge_slot(Fn&& f)
+__device__ __forceinline__ void each_wedge(const unsigned* __restrict__ wt, Fn&& f)
+{
+    constexpr int nk8 = (N / 2 + 1) * (N / 2 + 2) / 2;
+    constexpr int PER = wedge_per_thread<N>(), U = (PER <= 8) ? PER : (PER + 1) / 2;
+#pragma unroll 1
+    for (int c0 = 0; c0 < PER; c0 += U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = threadIdx.x + (c0 + u) * SlabShape<N>::NT;
+            if (i < nk8) {
+                const unsigned w = wt[i];
+                f((int)(w & 0xffffu), (int)(w >> 16), i);
+            }
+        }
+    }
+}
+// the same with the slot c of the point among the thread's own, fully unrolled: f may index registers by c
+template <int N, typename Fn>
+__device__ __forceinline__ void each_wedge_slot(const unsigned* __restrict__ wt, Fn&& f)
 {
     constexpr int nk8 = (N / 2 + 1) * (N / 2 + 2) / 2;
     int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));  // the points' indices are recomputed in each phase, not kept
+    asm volatile("" : "+v"(tid));  // indices and offsets are read again in each phase, not kept
 #pragma unroll
     for (int c = 0; c < wedge_per_thread<N>(); c++) {
-        const int t = tid + c * SlabShape<N>::NT;
-        if (t < nk8) {
-            int l, m;
-            wedge_pt<N>(t, l, m);
-            f(l, m, m + l * (l + 1) / 2, c);
+        const int i = tid + c * SlabShape<N>::NT;
+        if (i < nk8) {
+            const unsigned w = wt[i];
+            f((int)(w & 0xffffu), (int)(w >> 16), i, c);
         }
+    }
+}
+// the thread's wedge values of a global array, ahead of a transform that hides their latency
+template <int N, typename S>
+__device__ __forceinline__ void load_wedge(const S* __restrict__ a, S* v)
+{
+    constexpr int nk8 = (N / 2 + 1) * (N / 2 + 2) / 2;
+#pragma unroll
+    for (int c = 0; c < wedge_per_thread<N>(); c++) {
+        const int i = threadIdx.x + c * SlabShape<N>::NT;
+        v[c] = (i < nk8) ? a[i] : (S)0;
     }
 }
 // f(l, m, s) for every point of the Lambda grid: kx index l + 1 (slab line l + 1), s = m + l nk
@@ -1007,36 +1013,16 @@ __device__ __forceinline__ void each_lambda(Fn&& f)
         f(l, s - l * nk, s);
     }
 }
-template <int N>
-constexpr int lambda_per_thread() { return ((N / 2 + 1) * (N / 2 - 1) + SlabShape<N>::NT - 1) / SlabShape<N>::NT; }
-template <int N, typename Fn>
-__device__ __forceinline__ void each_lambda_slot(Fn&& f)
-{
-    constexpr int nk = N / 2 + 1, nq = nk * (nk - 2);
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-#pragma unroll
-    for (int c = 0; c < lambda_per_thread<N>(); c++) {
-        const int s = tid + c * SlabShape<N>::NT;
-        if (s < nq) {
-            const int l = s / nk;
-            f(l, s - l * nk, s, c);
-        }
-    }
-}
 // slab offset of element (l, m)
 template <int N>
 __device__ __forceinline__ int at(int l, int m)
 {
     return m + l * SlabShape<N>::LD;
 }
-// write a wedge value to both symmetric positions of a slab
-template <int N, typename Real>
-__device__ __forceinline__ void put_sym(Real* slab, int l, int m, Real v)
-{
-    slab[at<N>(l, m)] = v;
-    slab[at<N>(m, l)] = v;
-}
+// G0(k,tau) without its weight, e^{-x t} (x = eps - mu0 >= 0) or e^{x (beta - t)}: times
+// fw = f / N^2, f = 1/(e^{-|x|/T} + 1) (k_mu0_root), it is -G0(k,t)/N^2 and, with t -> beta - t,
+// G0(k,-t)/N^2 (chi0.cpp:468-471, 486-489)
+__device__ __forceinline__ double g0_exp(double x, double t, double bt) { return exp(x >= 0.0 ? -t * x : bt * x); }
 
 __device__ __forceinline__ cd sigma_mom(double Sinf, double s2, double s3, cd R, double wn)
 {
@@ -1056,53 +1042,6 @@ __device__ __forceinline__ cd sigma_kw(const cf* __restrict__ Self, long o, doub
 {
     const cf v = Self[o];
     return cd{(double)v.x, (double)v.y};
-}
-// k-space integrand of h (which = 0) or f0 (which = 1) at tau = t (cond_opt.cpp:2697-2735,
-// 2795-2827); nf = 1/N^2, v = v_x(k)
-__device__ __forceinline__ double hf0_val(int which, double e, double v, double mu0, double T, double t, double nf)
-{
-    if (which == 0) {
-        const double x = e - mu0;
-        return (x > 0) ? nf * v * exp(-x * t) / (exp(-x / T) + 1.0)
-                       : nf * v * exp(x * (1.0 / T - t)) / (exp(x / T) + 1.0);
-    }
-    if (e > mu0) {
-        const double ex = exp((mu0 - e) / T);
-        return nf * v * exp((mu0 - e) * t) * (t / (ex + 1.0) - ex / (T * (ex + 1.0) * (ex + 1.0)));
-    }
-    const double ex = exp((e - mu0) / T);
-    return nf * v * exp((e - mu0) * (1.0 / T - t)) * (t / (ex + 1.0) - 1.0 / (T * (ex + 1.0) * (ex + 1.0)));
-}
-
-// h and f0 of the same point at once: they share both exponentials, exp(-x t) (x = e - mu0 > 0)
-// or exp(x (1/T - t)), and exp(-|x|/T), whose arguments are the same numbers (mu0 - e = -x
-// exactly), so hv, fv equal hf0_val(0, ...), hf0_val(1, ...) bit for bit.
-__device__ __forceinline__ void hf0_pair(double e, double v, double mu0, double T, double t, double nf, double& hv,
-                                         double& fv)
-{
-    const double x = e - mu0;
-    if (x > 0) {
-        const double E = exp(-x * t), ex = exp(-x / T);
-        hv = nf * v * E / (ex + 1.0);
-        fv = nf * v * E * (t / (ex + 1.0) - ex / (T * (ex + 1.0) * (ex + 1.0)));
-    } else {
-        const double E = exp(x * (1.0 / T - t)), ex = exp(x / T);
-        hv = nf * v * E / (ex + 1.0);
-        fv = nf * v * E * (t / (ex + 1.0) - 1.0 / (T * (ex + 1.0) * (ex + 1.0)));
-    }
-}
-
-
-// tau-derivative of the h integrand at tau = 0+ (side 0) or beta- (side 1)
-// (cond_opt.cpp:2745-2781)
-__device__ __forceinline__ double h_slope_val(int side, double e, double v, double mu0, double T, double nf)
-{
-    if (e > mu0) {
-        const double ex = exp((mu0 - e) / T);
-        return (side == 0) ? -nf * v * (e - mu0) / (ex + 1.0) : -nf * v * (e - mu0) * ex / (ex + 1.0);
-    }
-    const double ex = exp((e - mu0) / T);
-    return (side == 0) ? -nf * v * (e - mu0) * ex / (ex + 1.0) : -nf * v * (e - mu0) / (ex + 1.0);
 }
 
 }  // namespace tpsc

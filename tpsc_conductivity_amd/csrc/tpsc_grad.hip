@@ -36,7 +36,7 @@ __device__ __forceinline__ void fermi2(double x, double T, double& f, double& g)
 // tdchirt0, tdGrt0p, tdchiqt0.  scr: 5*nk8 doubles.
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_chi0_tau0_tan(const double* __restrict__ ekw, const double* __restrict__ dekw, const double* __restrict__ er,
+    k_chi0_tau0_tan(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ dekw, const double* __restrict__ er,
                     const double* __restrict__ der, double mu0, double dmu0, double T, double* tchi, double* tchirt,
                     double* tchirt0, double* tdchirt0, double* tdGrt0p, double* tdchiqt0, double* scr)
 {
@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     const int tid = threadIdx.x, nt = blockDim.x;
     double *PdGp = scr, *TdGp = scr + nk8, *Pg = scr + 2 * nk8, *Tg = scr + 3 * nk8, *stg = scr + 4 * nk8;
     for (int pass = 0; pass < 4; pass++) {
-        each_wedge<N>([&](int l, int m, int i) {
+        each_wedge<N>(wt, [&](int a, int b, int i) {
             const double x = ekw[i] - mu0, dx = dekw[i] - dmu0;
             double f, g;
             fermi2(x, T, f, g);
@@ -59,13 +59,13 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
             else if (pass == 1) v = (g + x * f * g / T) * dx / nk02;
             else if (pass == 2) v = -g / nk02;
             else v = -f * g / T * dx / nk02;
-            put_sym<N>(slab, l, m, v);
+            slab[a] = slab[b] = v;
         });
         __syncthreads();
         slab_r2r_2d<double, N, 0>(slab, tw);
         double* o = (pass == 0) ? PdGp : (pass == 1) ? TdGp : (pass == 2) ? Pg : Tg;
-        each_wedge<N>([&](int l, int m, int i) {
-            o[i] = slab[at<N>(l, m)];
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            o[i] = slab[a];
         });
         __syncthreads();
     }
@@ -85,14 +85,14 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     }
     __syncthreads();
     for (int pass = 0; pass < 2; pass++) {
-        each_wedge<N>([&](int l, int m, int i) {
-            put_sym<N>(slab, l, m, (pass == 0) ? tchirt[i] : stg[i]);
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            slab[a] = slab[b] = (pass == 0) ? tchirt[i] : stg[i];
         });
         __syncthreads();
         slab_r2r_2d<double, N, 0>(slab, tw);
         double* o = (pass == 0) ? tchi : tdchiqt0;
-        each_wedge<N>([&](int l, int m, int i) {
-            o[i] = slab[at<N>(l, m)];
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            o[i] = slab[a];
         });
         __syncthreads();
     }
@@ -117,7 +117,7 @@ __device__ __forceinline__ double g0m_val(double x, double t, double T, double n
 // The block stages G(r,tau) in tchirt[j] and dG(r,tau) in tchi[j] before their final values.
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_chi0_slab_tan(const double* __restrict__ ekw, const double* __restrict__ dekw, double mu0, double dmu0,
+    k_chi0_slab_tan(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ dekw, double mu0, double dmu0,
                     double T, int Nw, double* tchi, double* tchirt)
 {
     constexpr int nk = N / 2 + 1;
@@ -136,7 +136,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     const double t = mid ? 1.0 / (2.0 * T) : j / (Nw * T);
     const int npass = mid ? 2 : 4;
     for (int pass = 0; pass < npass; pass++) {
-        each_wedge<N>([&](int l, int m, int i) {
+        each_wedge<N>(wt, [&](int a, int b, int i) {
             const double x = ekw[i] - mu0, dx = dekw[i] - dmu0;
             double f, g;
             fermi2(x, T, f, g);
@@ -148,12 +148,12 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
                 const double p = g0m_val(x, t, T, nk02);
                 v = (pass == 2) ? p : p * (t - g / T) * dx;
             }
-            put_sym<N>(slab, l, m, v);
+            slab[a] = slab[b] = v;
         });
         __syncthreads();
         slab_r2r_2d<double, N, 0>(slab, tw);
-        each_wedge<N>([&](int l, int m, int i) {
-            const double v = slab[at<N>(l, m)];
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            const double v = slab[a];
             if (pass == 0) cr[i] = v;                        // G(r,tau)
             else if (pass == 1) cq[i] = mid ? 4.0 * cr[i] * v : v;  // dG(r,tau), or dchi0(r,beta/2)
             else if (pass == 2) cq[i] = -2.0 * v * cq[i];    // -2 G(r,-tau) dG(r,tau)
@@ -164,13 +164,13 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     if (mid)
         for (long i = tid; i < nk8; i += nt) cr[i] = cq[i];
     __syncthreads();
-    each_wedge<N>([&](int l, int m, int i) {
-        put_sym<N>(slab, l, m, cr[i]);
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        slab[a] = slab[b] = cr[i];
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) {
-        cq[i] = slab[at<N>(l, m)];
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        cq[i] = slab[a];
     });
 }
 
@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(256)
 //   d chi_sp = (dchi0 + dUsp chi0^2/2) r_sp^2,  d chi_ch = (dchi0 - dUch chi0^2/2) r_ch^2
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_vertex_slab_tan(const double* __restrict__ chi, const double* __restrict__ tchi, double* tV, double normFact,
+    k_vertex_slab_tan(const unsigned* __restrict__ wt, const double* __restrict__ chi, const double* __restrict__ tchi, double* tV, double normFact,
                       double U, double dU, double Usp, double dUsp, double Uch, double dUch)
 {
     constexpr int nk = N / 2 + 1;
@@ -230,20 +230,19 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const long j = blockIdx.x;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    each_wedge<N>([&](int l, int m, int i) {
+    each_wedge<N>(wt, [&](int a, int b, int i) {
         const double c = chi[i + j * nk8], dc = tchi[i + j * nk8];
         const double rs = 1.0 / (1.0 - Usp * c / 2.0), rc = 1.0 / (1.0 + Uch * c / 2.0);
         const double csp = c * rs, cch = c * rc;
         const double dcsp = (dc + dUsp * c * c / 2.0) * rs * rs, dcch = (dc - dUch * c * c / 2.0) * rc * rc;
         const double P = 3.0 * Usp * (csp - c) + Uch * (cch - c);
         const double dP = 3.0 * dUsp * (csp - c) + 3.0 * Usp * (dcsp - dc) + dUch * (cch - c) + Uch * (dcch - dc);
-        put_sym<N>(slab, l, m, normFact * (dU * P + U * dP) / 8.0);
+        slab[a] = slab[b] = normFact * (dU * P + U * dP) / 8.0;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) {
-        tV[i + j * nk8] = slab[at<N>(l, m)];
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        tV[i + j * nk8] = slab[a];
     });
 }
 
@@ -262,7 +261,7 @@ __global__ void k_axpy(long n, double a, const double* __restrict__ x, double* y
 // Outputs tdSig[side*nk8 + k], tSb[side*nk8 + k].  scr: 6*nk8 doubles.
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_sigma_bnd_tan(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ er,
+    k_sigma_bnd_tan(const unsigned* __restrict__ wt, const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ er,
                     const double* __restrict__ der, const double* __restrict__ V0, const double* __restrict__ tV0,
                     const double* __restrict__ dchirt0, const double* __restrict__ tdchirt0,
                     const double* __restrict__ dGrt0p, const double* __restrict__ tdGrt0p, double mu0, double dmu0,
@@ -293,12 +292,12 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
         __syncthreads();
         slab_r2r_2d<double, N, 0>(slab, tw);
         if (pass == 0) {
-            each_wedge<N>([&](int l, int m, int i) {
-                Pg[i] = slab[at<N>(l, m)];
+            each_wedge<N>(wt, [&](int a, int b, int i) {
+                Pg[i] = slab[a];
             });
         } else {
-            each_wedge<N>([&](int l, int m, int i) {
-                const double g = Pg[i], dg = slab[at<N>(l, m)];
+            each_wedge<N>(wt, [&](int a, int b, int i) {
+                const double g = Pg[i], dg = slab[a];
                 const double v = V0[i], dv = tV0[i];
                 const double c = dchirt0[i], dc = tdchirt0[i];
                 const double dfc = dfact * c * g + fact * dc * g + fact * c * dg;
@@ -314,14 +313,14 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
         __syncthreads();
     }
     for (int pass = 0; pass < 2; pass++) {
-        each_wedge<N>([&](int l, int m, int i) {
-            put_sym<N>(slab, l, m, stg[pass * nk8 + i]);
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            slab[a] = slab[b] = stg[pass * nk8 + i];
         });
         __syncthreads();
         slab_r2r_2d<double, N, 0>(slab, tw);
         double* o = (pass == 0) ? tdSig : tSb;
-        each_wedge<N>([&](int l, int m, int i) {
-            o[i + side * nk8] = slab[at<N>(l, m)];
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            o[i + side * nk8] = slab[a];
         });
         __syncthreads();
     }
@@ -331,7 +330,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
 // k_sigma_slab): DCT[dG0 V + G0 dV], G0 and dG0 recomputed; G0(r,tau) staged in tS[j].
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_sigma_slab_tan(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ V,
+    k_sigma_slab_tan(const unsigned* __restrict__ wt, const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ V,
                      const double* __restrict__ tV, double mu0, double dmu0, double T, int Nw, double* tS)
 {
     constexpr int nk = N / 2 + 1;
@@ -362,23 +361,23 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
         __syncthreads();
         slab_r2r_2d<double, N, 0>(slab, tw);
         if (pass == 0)
-            each_wedge<N>([&](int l, int m, int i) {
-                o[i] = slab[at<N>(l, m)];
+            each_wedge<N>(wt, [&](int a, int b, int i) {
+                o[i] = slab[a];
             });
         __syncthreads();
     }
-    each_wedge<N>([&](int l, int m, int i) {
-        const double v = slab[at<N>(l, m)] * Vj[i] + o[i] * tVj[i];
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        const double v = slab[a] * Vj[i] + o[i] * tVj[i];
         o[i] = v;
     });
     __syncthreads();
-    each_wedge<N>([&](int l, int m, int i) {
-        put_sym<N>(slab, l, m, o[i]);
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        slab[a] = slab[b] = o[i];
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) {
-        o[i] = slab[at<N>(l, m)];
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        o[i] = slab[a];
     });
 }
 
@@ -432,10 +431,10 @@ hipError_t launch_chi0_tan(const Grid& g, const DevArrays& d, const TanArrays& t
     const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_DISPATCH_N(g.N, {
         grad_set_lds(k_chi0_tau0_tan<NN>, lds);
-        hipLaunchKernelGGL(k_chi0_tau0_tan<NN>, dim3(1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, t.dekw, d.er, t.der, mu0,
+        hipLaunchKernelGGL(k_chi0_tau0_tan<NN>, dim3(1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, t.dekw, d.er, t.der, mu0,
                            dmu0, g.T, t.chi, t.chirt, t.chirt0, t.dchirt0, t.dGrt0p, t.dchiqt0, t.scr);
         grad_set_lds(k_chi0_slab_tan<NN>, lds);
-        hipLaunchKernelGGL(k_chi0_slab_tan<NN>, dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, t.dekw, mu0, dmu0,
+        hipLaunchKernelGGL(k_chi0_slab_tan<NN>, dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, t.dekw, mu0, dmu0,
                            g.T, g.Nw, t.chi, t.chirt);
     });
     return hipGetLastError();
@@ -458,7 +457,7 @@ hipError_t launch_vertex_slab_tan(const Grid& g, const DevArrays& d, const TanAr
     const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_DISPATCH_N(g.N, {
         grad_set_lds(k_vertex_slab_tan<NN>, lds);
-        hipLaunchKernelGGL(k_vertex_slab_tan<NN>, dim3(g.nwb), dim3(SlabShape<NN>::NT), lds, s, d.chiw, t.chi, t.V,
+        hipLaunchKernelGGL(k_vertex_slab_tan<NN>, dim3(g.nwb), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.chiw, t.chi, t.V,
                            normFact, U, dU, Usp, dUsp, Uch, dUch);
     });
     return hipGetLastError();
@@ -476,11 +475,11 @@ hipError_t launch_sigma_tan(const Grid& g, const DevArrays& d, const TanArrays& 
     const size_t lds = slab_bytes(g.N, sizeof(double));
     GRAD_DISPATCH_N(g.N, {
         grad_set_lds(k_sigma_bnd_tan<NN>, lds);
-        hipLaunchKernelGGL(k_sigma_bnd_tan<NN>, dim3(2), dim3(SlabShape<NN>::NT), lds, s, d.ek, t.dek, d.er, t.der, d.V0,
+        hipLaunchKernelGGL(k_sigma_bnd_tan<NN>, dim3(2), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ek, t.dek, d.er, t.der, d.V0,
                            t.V0, d.dchirt0, t.dchirt0, d.dGrt0p, t.dGrt0p, mu0, dmu0, g.T, fact, dfact, t.dSig, t.Sb,
                            t.scr);
         grad_set_lds(k_sigma_slab_tan<NN>, lds);
-        hipLaunchKernelGGL(k_sigma_slab_tan<NN>, dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.ek, t.dek, d.V, t.V,
+        hipLaunchKernelGGL(k_sigma_slab_tan<NN>, dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ek, t.dek, d.V, t.V,
                            mu0, dmu0, g.T, g.Nw, t.Stau);
     });
     return hipGetLastError();

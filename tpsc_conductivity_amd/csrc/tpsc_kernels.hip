@@ -8,9 +8,8 @@
 //   k_vertex_slab/_pencil        chi.cpp:85-170     V(r,tau)
 //   k_sigma_bnd/_slab/_pencil    green.cpp:1743-2018 Sigma(k,iwn) moments + remainder
 //   k_trace_diffG, k_trace_selfG green.cpp:2929-3182 traces for mu and consistency checks
-//   k_hf0_slab, k_hf0_bnd,
-//   k_hVf0V_slab, k_jj_pencil,
-//   k_kx0_rows                   cond_opt.cpp:2584-4173 Lambda_jj bubble + Maki-Thompson + kx0
+//   k_hf0_bnd, k_hV_slab,
+//   k_jj_pencil, k_kx0_rows      cond_opt.cpp:2584-4173 Lambda_jj bubble + Maki-Thompson + kx0
 // Slab kernels hold one (nk x nk) slab in LDS (151 KB at N=256 in FP64) and transform it with
 // register FFTs of line pairs; pencil kernels hold one tau-pencil per workgroup.
 // Precision: S is the storage and slab-arithmetic type of the tau arrays (chi0(q,tau),
@@ -169,125 +168,103 @@ __global__ void __launch_bounds__(256) k_halley_step(const double* part, int n, 
 }
 
 // ================================================================== chi0 slabs
-// G(k,t)/N^2, chi0.cpp:468-471 (form==0) and :535-538 (form==1, tau = beta/2)
-__device__ __forceinline__ double g0_plus(double x, double t, double T, double nk02, int form)
-{
-    if (x >= 0.0) return exp(-t * x) * (-1.0 / (exp(-x / T) + 1.0)) / nk02;
-    if (form == 0) return -exp((1.0 / T - t) * x) / (exp(x / T) + 1.0) / nk02;
-    return -exp((1.0 / T - t) * x) / ((exp(x / T) + 1.0) * nk02);
-}
-// G(k,-t)/N^2, chi0.cpp:486-489
-__device__ __forceinline__ double g0_minus(double x, double t, double T, double nk02)
-{
-    if (x >= 0.0) return -exp((t - 1.0 / T) * x) * (-1.0 / (exp(-x / T) + 1.0)) / nk02;
-    return exp(t * x) / ((exp(x / T) + 1.0) * nk02);
-}
-
 // tau = 0 slice plus the tau-derivative data (chi0.cpp:323-447); one block.
 // The boundary data are tail moments: this kernel runs in FP64 for both precisions and
 // only rounds the slice-0 values it stores into the S arrays.
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_chi0_tau0(const double* __restrict__ ekw, const double* __restrict__ er, const double* __restrict__ mu0p,
-                double T, S* chi, S* chirt, double* dchirt0, double* dGrt0p, double* dchiqt0, double* chirt0)
+    k_chi0_tau0(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+                const double* __restrict__ er, const double* __restrict__ mu0p, double T, S* chi, S* chirt,
+                double* dchirt0, double* dGrt0p, double* dchiqt0, double* chirt0)
 {
-    const double mu0 = *mu0p;
-    const double nk02 = (double)N * N;
+    const double mu0 = *mu0p, beta = 1.0 / T;
     extern __shared__ double smem[];
     double* slab = smem;
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
-    // d/dtau G(r,0+) = DCT[-ekmu Gkt / N^2]
-    each_wedge<N>([&](int l, int m, int i) {
+    // d/dtau G(r,0+) = DCT[-x G0(k,0) / N^2]
+    each_wedge<N>(wt, [&](int a, int b, int i) {
         const double x = ekw[i] - mu0;
-        const double Gkt = -1.0 / (exp(-x / T) + 1.0);
-        put_sym<N>(slab, l, m, -x * Gkt / nk02);
+        slab[a] = slab[b] = x * g0_exp(x, 0.0, beta) * fw[i];
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) { dGrt0p[i] = slab[at<N>(l, m)]; });
+    each_wedge<N>(wt, [&](int a, int, int i) { dGrt0p[i] = slab[a]; });
     __syncthreads();
     // G(r,0)
-    each_wedge<N>([&](int l, int m, int i) {
-        const double x = ekw[i] - mu0;
-        put_sym<N>(slab, l, m, (-1.0 / (exp(-x / T) + 1.0)) / nk02);
-    });
+    each_wedge<N>(wt, [&](int a, int b, int i) { slab[a] = slab[b] = -g0_exp(ekw[i] - mu0, 0.0, beta) * fw[i]; });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
     // chi0(r,0) and its transform (each thread replaces the points it read and keeps their G(r,0))
     double G0r[wedge_per_thread<N>()];
-    each_wedge_slot<N>([&](int l, int m, int i, int k) {
-        const double g = slab[at<N>(l, m)];
+    each_wedge_slot<N>(wt, [&](int a, int b, int i, int k) {
+        const double g = slab[a];
         G0r[k] = g;
         const double c = (i == 0) ? -2.0 * g * (g + 1.0) : -2.0 * g * g;
         chirt[i] = (S)c;
         chirt0[i] = c;
-        put_sym<N>(slab, l, m, c);
+        slab[a] = slab[b] = c;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
     // d/dtau chi0(r,0) and its transform
-    each_wedge_slot<N>([&](int l, int m, int i, int k) {
-        chi[i] = (S)slab[at<N>(l, m)];
+    each_wedge_slot<N>(wt, [&](int a, int b, int i, int k) {
+        chi[i] = (S)slab[a];
         const double g = G0r[k], dGp = dGrt0p[i];  // written above by this thread
         const double dGm = ((i == 0) ? -mu0 : er[i]) - dGp;
         const double v = (i == 0) ? -2.0 * (dGp * (1.0 + g) + dGm * g) : -2.0 * (dGp * g + dGm * g);
         dchirt0[i] = v;
-        put_sym<N>(slab, l, m, v);
+        slab[a] = slab[b] = v;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) { dchiqt0[i] = slab[at<N>(l, m)]; });
+    each_wedge<N>(wt, [&](int a, int, int i) { dchiqt0[i] = slab[a]; });
 }
 
 // slices j = 1 .. nwb-1 (chi0.cpp:454-559); block b handles j = b + 1
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
-    k_chi0_slab(const double* __restrict__ ekw, const double* __restrict__ mu0p, double T, int Nw, S* chi, S* chirt)
+    k_chi0_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+                const double* __restrict__ mu0p, double T, int Nw, S* chi, S* chirt)
 {
     const double mu0 = *mu0p;
     constexpr int nk = N / 2 + 1;
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
     auto* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const int nwb = Nw / 2 + 1;
     const int j = blockIdx.x + 1;
+    const double t = (j < nwb - 1) ? j / (Nw * T) : 1.0 / (2.0 * T), bt = 1.0 / T - t;
     S* cr = chirt + (long)j * nk8;
     S* cq = chi + (long)j * nk8;
+    each_wedge<N>(wt, [&](int a, int b, int i) { slab[a] = slab[b] = (S)(-g0_exp(ekw[i] - mu0, t, bt) * fw[i]); });
+    __syncthreads();
+    slab_r2r_2d<S, N, 0>(slab, tw);
     if (j < nwb - 1) {
-        const double t = j / (Nw * T);
-        each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, (S)g0_plus(ekw[i] - mu0, t, T, nk02, 0)); });
-        __syncthreads();
-        slab_r2r_2d<S, N, 0>(slab, tw);
         S g[wedge_per_thread<N>()];  // G(r,t) of the thread's points
-        each_wedge_slot<N>([&](int l, int m, int, int c) { g[c] = slab[at<N>(l, m)]; });
+        each_wedge_slot<N>(wt, [&](int a, int, int, int c) { g[c] = slab[a]; });
         __syncthreads();
-        each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, (S)g0_minus(ekw[i] - mu0, t, T, nk02)); });
+        each_wedge<N>(wt, [&](int a, int b, int i) { slab[a] = slab[b] = (S)(g0_exp(ekw[i] - mu0, bt, t) * fw[i]); });
         __syncthreads();
         slab_r2r_2d<S, N, 0>(slab, tw);
         // chi0(r,t) = -2 G(r,-t) G(r,t)
-        each_wedge_slot<N>([&](int l, int m, int i, int c) {
-            const S v = (S)(-2) * slab[at<N>(l, m)] * g[c];
+        each_wedge_slot<N>(wt, [&](int a, int b, int i, int c) {
+            const S v = (S)(-2) * slab[a] * g[c];
             cr[i] = v;
-            put_sym<N>(slab, l, m, v);
+            slab[a] = slab[b] = v;
         });
-    } else {
-        const double t = 1.0 / (2.0 * T);
-        each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, (S)g0_plus(ekw[i] - mu0, t, T, nk02, 1)); });
-        __syncthreads();
-        slab_r2r_2d<S, N, 0>(slab, tw);
-        each_wedge<N>([&](int l, int m, int i) {
-            const S v = slab[at<N>(l, m)], c = (S)2 * v * v;
+    } else {  // tau = beta/2: G(r,-t) = -G(r,t)
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            const S v = slab[a], c = (S)2 * v * v;
             cr[i] = c;
-            put_sym<N>(slab, l, m, c);
+            slab[a] = slab[b] = c;
         });
     }
     __syncthreads();
     slab_r2r_2d<S, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) { cq[i] = slab[at<N>(l, m)]; });
+    each_wedge<N>(wt, [&](int a, int, int i) { cq[i] = slab[a]; });
 }
 
 // ================================================================== chi0 pencils
@@ -625,20 +602,12 @@ constexpr int kMu0K = 9;
 // that blockDim.x * kMu0K >= nk8.
 // The root goes to out (mapped host memory) and to the device slot mu0v, which the chi0 and
 // h/f0 kernels read, so that the host need not wait for it; a failed search leaves mu0v as it
-// was (the previous mu0).  A preset value (not NaN) is stored without a search.
+// was (the previous mu0).  A preset value (not NaN) is stored without a search.  fw (2 nk8): the
+// Fermi factors of the slabs at that mu0.
 __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ekw, const double* __restrict__ wq,
                                                    long nk8, double Nk2, double T, double dens, double preset,
-                                                   double* out, double* mu0v)
+                                                   double* out, double* mu0v, double* fw)
 {
-    if (!isnan(preset)) {
-        if (threadIdx.x == 0) {
-            out[0] = 1.0;
-            out[1] = preset;
-            out[2] = 0.0;
-            *mu0v = preset;
-        }
-        return;
-    }
     __shared__ double sc[3 * 16];
     double e[kMu0K], w[kMu0K];
 #pragma unroll
@@ -648,6 +617,29 @@ __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ek
         w[k] = (i < nk8) ? 2.0 * wq[i] / Nk2 : 0.0;
     }
     const double iT = 1.0 / T;
+    // f = 1/(e^{-|x|/T} + 1) / N^2 (x = eps - mu0) and f2 = (e^{-x/T} or 1) f^2 / (T N^2): the parts of
+    // G0, h and f0 that do not depend on tau, once per mu0 for all the slabs
+    auto weights = [&](double mu) {
+#pragma unroll
+        for (int k = 0; k < kMu0K; k++) {
+            const long i = threadIdx.x + (long)k * blockDim.x;
+            if (i < nk8) {
+                const double x = e[k] - mu, ex = exp(-fabs(x) / T), f = 1.0 / (ex + 1.0);
+                fw[i] = f / Nk2;
+                fw[nk8 + i] = (x > 0 ? ex : 1.0) * f * f / (T * Nk2);
+            }
+        }
+    };
+    if (!isnan(preset)) {
+        if (threadIdx.x == 0) {
+            out[0] = 1.0;
+            out[1] = preset;
+            out[2] = 0.0;
+            *mu0v = preset;
+        }
+        weights(preset);
+        return;
+    }
     // v = {n(mu) - dens, n'(mu), n''(mu)}
     auto density3 = [&](double mup, double* v) {
         v[0] = v[1] = v[2] = 0.0;
@@ -680,6 +672,7 @@ __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ek
         ok = bracket_root(density, 0.0, -8.0, 8.0, nullptr, 1.0e-16, &root, &nb);
         ne += nb;
     }
+    weights(ok ? root : *mu0v);
     if (threadIdx.x == 0) {
         out[0] = ok ? 1.0 : 0.0;
         out[1] = root;
@@ -692,7 +685,7 @@ __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ek
 // chi.cpp:85-119, block j = iqn index
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
-    k_vertex_slab(const double* __restrict__ chi, S* V, double normFact, double U, double Usp, double Uch,
+    k_vertex_slab(const unsigned* __restrict__ wt, const double* __restrict__ chi, S* V, double normFact, double U, double Usp, double Uch,
                   const double* __restrict__ dsc)
 {
     if (dsc) {
@@ -706,14 +699,14 @@ __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     auto* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const long j = blockIdx.x;
-    each_wedge<N>([&](int l, int m, int i) {
+    each_wedge<N>(wt, [&](int a, int b, int i) {
         const double c = chi[i + j * nk8];
         const double csp = c / (1.0 - Usp * c / 2.0), cch = c / (1.0 + Uch * c / 2.0);
-        put_sym<N>(slab, l, m, (S)(normFact * U * (3.0 * Usp * (csp - c) + Uch * (cch - c)) / 8.0));
+        slab[a] = slab[b] = (S)(normFact * U * (3.0 * Usp * (csp - c) + Uch * (cch - c)) / 8.0);
     });
     __syncthreads();
     slab_r2r_2d<S, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) { V[i + j * nk8] = slab[at<N>(l, m)]; });
+    each_wedge<N>(wt, [&](int a, int, int i) { V[i + j * nk8] = slab[a]; });
 }
 
 // chi.cpp:123-170: REDFT00 over n (length Nw/2+1) for two wedge points per block, as one
@@ -766,30 +759,26 @@ __device__ __forceinline__ void store_self(cf* Self, long o, cd R, double Sinf, 
 // G0(k,0+) = -1/(e^{-x/T}+1) and G0(k,beta-) = -1/(e^{x/T}+1), both over N^2.
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_sigma_bnd(const double* __restrict__ ekw, const double* __restrict__ er, const double* __restrict__ V0,
-                const double* __restrict__ dchirt0, const double* __restrict__ dGrt0p, double mu0, double T,
-                double fact, double* dSig, double* Sb, const double* __restrict__ mu0p, double U,
-                const double* __restrict__ dsc)
+    k_sigma_bnd(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+                const double* __restrict__ er, const double* __restrict__ V0, const double* __restrict__ dchirt0,
+                const double* __restrict__ dGrt0p, double mu0, double T, double fact, double* dSig, double* Sb,
+                const double* __restrict__ mu0p, double U, const double* __restrict__ dsc)
 {
     if (mu0p) mu0 = *mu0p;
     if (dsc) fact = vfact(U, dsc[kPscUsp + 1], dsc[kPscUch + 1], 8.0);
     constexpr int nk = N / 2 + 1;
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     double* slab = smem;
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const int side = blockIdx.x & 1, pass = blockIdx.x >> 1;
-    each_wedge<N>([&](int l, int m, int i) {
-        const double x = ekw[i] - mu0;
-        put_sym<N>(slab, l, m,
-                   (side == 0) ? -1.0 / (exp(-x / T) + 1.0) / nk02 : -1.0 / (exp(x / T) + 1.0) / nk02);
-    });
+    const double t = side ? 1.0 / T : 0.0, bt = side ? 0.0 : 1.0 / T;
+    each_wedge<N>(wt, [&](int a, int b, int i) { slab[a] = slab[b] = -g0_exp(ekw[i] - mu0, t, bt) * fw[i]; });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
-    each_wedge<N>([&](int l, int m, int i) {
-        const double g = slab[at<N>(l, m)];
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        const double g = slab[a];
         const double v = V0[i];
         double r;
         if (pass == 1)
@@ -800,24 +789,23 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
             const double xi = (i == 0) ? -mu0 : er[i];
             r = -fact * dchirt0[i] * g + v * (-dGrt0p[i] + xi);
         }
-        put_sym<N>(slab, l, m, r);
+        slab[a] = slab[b] = r;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 0>(slab, tw);
     double* o = (pass == 0) ? dSig : Sb;
-    each_wedge<N>([&](int l, int m, int i) { o[i + side * nk8] = slab[at<N>(l, m)]; });
+    each_wedge<N>(wt, [&](int a, int, int i) { o[i + side * nk8] = slab[a]; });
 }
 
 // Sigma(k,tau_j), j = 0..Nw (green.cpp:1822-1892): G0(k,tau) -> r, x V(r,|tau|), -> k
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
-    k_sigma_slab(const double* __restrict__ ekw, const S* __restrict__ V, double mu0, double T, int Nw, S* Stau,
-                 const double* __restrict__ mu0p)
+    k_sigma_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+                 const S* __restrict__ V, double mu0, double T, int Nw, S* Stau, const double* __restrict__ mu0p)
 {
     if (mu0p) mu0 = *mu0p;
     constexpr int nk = N / 2 + 1;
     constexpr long nk8 = (long)nk * (nk + 1) / 2;
-    const double nk02 = (double)N * N;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
     auto* tw = slab_tw<N>(slab);
@@ -825,21 +813,17 @@ __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     const int j = blockIdx.x;
     const int nwb = Nw / 2 + 1;
     const int jv = (j < nwb) ? j : Nw - j;
-    const double t = j / (Nw * T);
-    each_wedge<N>([&](int l, int m, int i) {
-        const double x = ekw[i] - mu0;
-        put_sym<N>(slab, l, m,
-                   (S)((x > 0) ? -exp(-t * x) / (exp(-x / T) + 1.0) / nk02
-                               : -exp((1.0 / T - t) * x) / (exp(x / T) + 1.0) / nk02));
-    });
+    const double t = j / (Nw * T), bt = 1.0 / T - t;
+    each_wedge<N>(wt, [&](int a, int b, int i) { slab[a] = slab[b] = (S)(-g0_exp(ekw[i] - mu0, t, bt) * fw[i]); });
+    S v[wedge_per_thread<N>()];  // V(r,|tau|) of the thread's points, in flight during the transform
+    load_wedge<N>(V + (long)jv * nk8, v);
     __syncthreads();
     slab_r2r_2d<S, N, 0>(slab, tw);
-    const S* Vj = V + (long)jv * nk8;
-    each_wedge<N>([&](int l, int m, int i) { put_sym<N>(slab, l, m, slab[at<N>(l, m)] * Vj[i]); });
+    each_wedge_slot<N>(wt, [&](int a, int b, int, int c) { slab[a] = slab[b] = slab[a] * v[c]; });
     __syncthreads();
     slab_r2r_2d<S, N, 0>(slab, tw);
     S* o = Stau + (long)j * nk8;
-    each_wedge<N>([&](int l, int m, int i) { o[i] = slab[at<N>(l, m)]; });
+    each_wedge<N>(wt, [&](int a, int, int i) { o[i] = slab[a]; });
 }
 
 // green.cpp:1925-2018: per wedge k, spline of Sigma(k,tau_j) (j=0..Nw) with slopes dSig,
@@ -1113,14 +1097,21 @@ __global__ void __launch_bounds__(1024) k_reduce_cols2(const double* __restrict_
         for (int i = threadIdx.x; i < ncopy; i += blockDim.x) cdst[i] = csrc[i];
 }
 
-// dispersion tables on the device (hamiltonien.cpp:49-68,125-155; green0 wedge weights)
-__global__ void k_model(int N, double t, double tp, double tpp, double t3, double* ek, double* ekw, double* wq,
-                        double* er, double* d2ek, double* dek)
+// dispersion tables on the device (hamiltonien.cpp:49-68,125-155; green0 wedge weights).  wt[w]: the slab
+// offsets of wedge point (l, m) (low half) and of (m, l) (high half), line stride LD.  vw, vw + nk8:
+// v_x at (kx, ky) = (l, m) and (m, l), 0 at kx = 0 and pi, for the Lambda slabs.
+__global__ void k_model(int N, int LD, double t, double tp, double tpp, double t3, double* ek, double* ekw, double* wq,
+                        double* er, double* d2ek, double* dek, unsigned* wt, double* vw)
 {
     const int nk = N / 2 + 1;
     const long nk8 = (long)nk * (nk + 1) / 2, nq = (long)nk * (nk - 2);
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
     const double dk = kPi / (nk - 1);
+    auto vx = [&](int l, int m) {
+        const double kx = l * dk, ky = m * dk;
+        return 2.0 * t * sin(kx) + 4.0 * tp * sin(kx) * cos(ky) + 4.0 * tpp * sin(2 * kx) +
+               4 * t3 * (2.0 * sin(2 * kx) * cos(ky) + cos(2 * ky) * sin(kx));
+    };
     if (i < (long)nk * nk) {
         const int l = (int)(i / nk), m = (int)(i % nk);
         const double kx = l * dk, ky = m * dk;
@@ -1132,128 +1123,92 @@ __global__ void k_model(int N, double t, double tp, double tpp, double t3, doubl
             ekw[w] = ek[i];
             wq[w] = wedge_weight(l, m, nk);
             er[w] = (w == 1) ? -t : (w == 2) ? -tp : (w == 3) ? -tpp : (w == 4) ? -t3 : 0.0;
+            wt[w] = (unsigned)(m + l * LD) | ((unsigned)(l + m * LD) << 16);
+            vw[w] = (l >= 1 && l <= nk - 2) ? vx(l, m) : 0.0;
+            vw[nk8 + w] = (m >= 1 && m <= nk - 2) ? vx(m, l) : 0.0;
         }
     }
-    if (i < nq) {
-        const int l = (int)(i / nk), m = (int)(i % nk);
-        const double kx = (l + 1) * dk, ky = m * dk;
-        dek[i] = 2.0 * t * sin(kx) + 4.0 * tp * sin(kx) * cos(ky) + 4.0 * tpp * sin(2 * kx) +
-                 4 * t3 * (2.0 * sin(2 * kx) * cos(ky) + cos(2 * ky) * sin(kx));
-    }
-    (void)nk8;
+    if (i < nq) dek[i] = vx((int)(i / nk) + 1, (int)(i % nk));
 }
 
 // ================================================================== Lambda_jj slabs
-// h(r,tau_j) and f0(r,tau_j), j = 0..Nw (cond_opt.cpp:2697-2735, 2795-2827):
-// RODFT00 along kx (index l+1), REDFT00 along ky.
-template <int N, typename S>
-__global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
-    k_hf0_slab(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ mu0p,
-               double T, int Nw, S* h, S* f0)
+// The Lambda integrands h (which = 0) and f0 (1) of cond_opt.cpp:2697-2735, 2795-2827 at one tau without
+// the velocity: with E = g0_exp(x, t, beta - t), fw = f/N^2 and fw2 = (e^{-x/T} or 1) f^2/(T N^2)
+// (k_mu0_root), h = v E fw and f0 = v E (t fw - fw2).
+__device__ __forceinline__ double lam_val(int which, double E, double t, double fw, double fw2)
 {
-    const double mu0 = *mu0p;
-    constexpr int nk = N / 2 + 1;
-    constexpr long nq = (long)nk * (nk - 2);
-    const double nf = 1.0 / ((double)N * N);
-    extern __shared__ double smem[];
-    S* slab = (S*)smem;
-    auto* tw = slab_tw<N>(slab);
-    fill_twiddles<N>(tw);
-    const int j = blockIdx.x;
-    const double t = (double)j / (T * Nw);
-    S* const oh = h + (long)j * nq;
-    S* const of = f0 + (long)j * nq;
-    // h and f0 together (hf0_pair); f0 waits in its output row, read back by the thread that
-    // wrote it, while h is transformed
-    each_lambda<N>([&](int l, int m, int s) {
-        double hv, fv;
-        hf0_pair(ek[m + (l + 1) * nk], dek[s], mu0, T, t, nf, hv, fv);
-        slab[at<N>(l + 1, m)] = (S)hv;
-        of[s] = (S)fv;
-    });
-    __syncthreads();
-    slab_r2r_2d<S, N, 1>(slab, tw);
-    each_lambda<N>([&](int l, int m, int s) {
-        oh[s] = slab[at<N>(l + 1, m)];
-        slab[at<N>(l + 1, m)] = of[s];
-    });
-    __syncthreads();
-    slab_r2r_2d<S, N, 1>(slab, tw);
-    each_lambda<N>([&](int l, int m, int s) { of[s] = slab[at<N>(l + 1, m)]; });
+    return E * (which == 0 ? fw : t * fw - fw2);
 }
 
 // Boundary data of hV and f0V in FP64 (cond_opt.cpp:2697-2735, 2745-3114 at tau = 0, beta).
 // Block b: which = (b/2)%2 (0: h, 1: f0), side = b%2 (0: tau = 0, 1: tau = beta), part = b/4:
 //   (1) h(r,tau_b) (or f0) by DST x DCT of the k-space integrand at t = 0 or beta
 //   part 1: (2) the tau-derivative integrand -> r, combined with V(r,0), dchi0(r,0) -> k:
-//       slopes dhV / df0V (cond_opt.cpp:2745-3014)
+//       slopes dhV / df0V (cond_opt.cpp:2745-3014); dh/dtau = -x h, df0/dtau = -x f0 + h
 //   part 0: (3) 2 h(r,tau_b) V(r,0) -> k: hVb / f0Vb, the tau = 0, beta values of hV / f0V
 // Both parts of a (which, side) run (1) themselves and then side by side: three transforms in
 // a row per block instead of four.  Independent of the tau slabs.
 template <int N>
 __global__ void __launch_bounds__(SlabShape<N>::NT)
-    k_hf0_bnd(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ V0,
-              const double* __restrict__ dchirt0, double mu0, double T, int Nw, double fact4, double* dhV,
-              double* df0V, double* hVb, double* f0Vb, const double* __restrict__ mu0p, double U,
-              const double* __restrict__ dsc)
+    k_hf0_bnd(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+              const double* __restrict__ vw, const double* __restrict__ V0, const double* __restrict__ dchirt0,
+              double mu0, double T, double fact4, double* dhV, double* df0V, double* hVb, double* f0Vb,
+              const double* __restrict__ mu0p, double U, const double* __restrict__ dsc)
 {
     if (mu0p) mu0 = *mu0p;
     if (dsc) fact4 = vfact(U, dsc[kPscUsp + 1], dsc[kPscUch + 1], 4.0);
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
-    const double nf = 1.0 / ((double)N * N);
+    constexpr int nk8 = nk * (nk + 1) / 2;
     extern __shared__ double smem[];
     double* slab = smem;
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
     const int which = (blockIdx.x >> 1) & 1, side = blockIdx.x & 1, part = blockIdx.x >> 2;
-    const double tb = (side == 0) ? 0.0 : (double)Nw / (T * Nw);  // tau_j of k_hf0_slab at j = 0, Nw
+    const double t = side ? 1.0 / T : 0.0, bt = side ? 0.0 : 1.0 / T;
     // (1)
-    each_lambda<N>([&](int l, int m, int s) {
-        slab[at<N>(l + 1, m)] = hf0_val(which, ek[m + (l + 1) * nk], dek[s], mu0, T, tb, nf);
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        const double g = lam_val(which, g0_exp(ekw[i] - mu0, t, bt), t, fw[i], fw[nk8 + i]);
+        slab[a] = g * vw[i];
+        slab[b] = g * vw[nk8 + i];
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
     if (part == 0) {
         // (3), from h(r,tau_b) in place
-        each_lambda<N>([&](int l, int m, int) { slab[at<N>(l + 1, m)] *= 2.0 * V0[fold_idx(l + 1, m, N)]; });
+        each_wedge<N>(wt, [&](int a, int b, int i) {
+            const double v = 2.0 * V0[i], ha = slab[a] * v, hb = slab[b] * v;
+            slab[a] = ha;
+            slab[b] = hb;
+        });
         __syncthreads();
         slab_r2r_2d<double, N, 1>(slab, tw);
         double* ob = ((which == 0) ? hVb : f0Vb) + side * nq;
         each_lambda<N>([&](int l, int m, int s) { ob[s] = slab[at<N>(l + 1, m)]; });
         return;
     }
-    double hr[lambda_per_thread<N>()];  // h(r,tau_b) of the thread's points
-    each_lambda_slot<N>([&](int l, int m, int, int c) { hr[c] = slab[at<N>(l + 1, m)]; });
+    double ha[wedge_per_thread<N>()], hb[wedge_per_thread<N>()];  // h(r,tau_b) of the thread's points
+    each_wedge_slot<N>(wt, [&](int a, int b, int, int c) {
+        ha[c] = slab[a];
+        hb[c] = slab[b];
+    });
     __syncthreads();
     // (2)
-    each_lambda<N>([&](int l, int m, int s) {
-        const double e = ek[m + (l + 1) * nk], v = dek[s];
-        double val;
-        if (which == 0) {
-            val = h_slope_val(side, e, v, mu0, T, nf);
-        } else {
-            if (e > mu0) {
-                const double ex = exp((mu0 - e) / T);
-                val = (side == 0)
-                          ? nf * v * ((e - mu0) * ex / (T * (ex + 1.0) * (ex + 1.0)) + 1.0 / (ex + 1.0))
-                          : nf * v * ex * ((mu0 - e) * (1.0 / (T * (ex + 1.0)) - ex / (T * (ex + 1.0) * (ex + 1.0))) + 1.0 / (ex + 1.0));
-            } else {
-                const double ex = exp((e - mu0) / T);
-                val = (side == 0)
-                          ? nf * v * ex * ((e - mu0) / (T * (ex + 1.0) * (ex + 1.0)) + 1.0 / (ex + 1.0))
-                          : nf * v * ((mu0 - e) * (1.0 / (T * (ex + 1.0)) - 1.0 / (T * (ex + 1.0) * (ex + 1.0))) + 1.0 / (ex + 1.0));
-            }
-        }
-        slab[at<N>(l + 1, m)] = val;
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        const double x = ekw[i] - mu0, E = g0_exp(x, t, bt);
+        double g = -x * lam_val(which, E, t, fw[i], fw[nk8 + i]);
+        if (which == 1) g += E * fw[i];
+        slab[a] = g * vw[i];
+        slab[b] = g * vw[nk8 + i];
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
-    each_lambda_slot<N>([&](int l, int m, int, int c) {
-        const long r = fold_idx(l + 1, m, N);
-        const double d = slab[at<N>(l + 1, m)], v = V0[r], hs = hr[c];
-        slab[at<N>(l + 1, m)] =
-            (side == 0) ? 2.0 * d * v + hs * fact4 * dchirt0[r] : 2.0 * d * v - hs * fact4 * dchirt0[r];
+    const double sf = (side == 0) ? fact4 : -fact4;
+    each_wedge_slot<N>(wt, [&](int a, int b, int i, int c) {
+        const double v = 2.0 * V0[i], f = sf * dchirt0[i];
+        const double ra = slab[a] * v + ha[c] * f, rb = slab[b] * v + hb[c] * f;
+        slab[a] = ra;
+        slab[b] = rb;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
@@ -1261,36 +1216,49 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
 }
 
-// hV(k,tau) = DST x DCT [2 h(r,tau) V(r,|tau|)], same for f0, in place (cond_opt.cpp:3029-3114)
+// hV(k,tau_j) = DST x DCT [2 h(r,tau_j) V(r,|tau_j|)] with h(r,tau_j) = DST x DCT [h(k,tau_j)]
+// (RODFT00 along kx, REDFT00 along ky; cond_opt.cpp:2697-2735, 2795-2827, 3029-3114), or f0V for
+// which = 1, j = 1 .. Nw-1 (the end slices come from k_hf0_bnd).  h and f0 stay in LDS.  The pointwise
+// phases run over the wedge: one exponential serves (kx, ky) and (ky, kx), and V(r) is read in order.
+// Bound by the two transforms (VALU and LDS).  At 256^2 x 2048 the h and f0 slices took 976 + 844 us (FP64)
+// and 628 + 399 us (FP32) as two kernels with h, f0 in global memory between them, two exponentials and
+// two divisions per point and index; now 2 x 513 and 2 x 374 us beside the self-energy pencil.
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
-    k_hVf0V_slab(const S* __restrict__ V, int Nw, S* h, S* f0)
+    k_hV_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
+              const double* __restrict__ vw, const double* __restrict__ mu0p, double T, int Nw,
+              const S* __restrict__ V, int which, S* out)
 {
+    const double mu0 = *mu0p;
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
-    constexpr long nk8 = (long)nk * (nk + 1) / 2;
+    constexpr int nk8 = nk * (nk + 1) / 2;
     extern __shared__ double smem[];
     S* slab = (S*)smem;
     auto* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
-    // slabs j = blockIdx.x, + gridDim.x, ...: the launch may hold fewer workgroups than slabs
-    for (int j = blockIdx.x; j <= Nw; j += gridDim.x) {
-        const int jv = (j > Nw / 2) ? Nw - j : j;
-        const S* Vj = V + (long)jv * nk8;
-        for (int which = 0; which < 2; which++) {
-            S* a = ((which == 0) ? h : f0) + (long)j * nq;
-            each_lambda<N>([&](int l, int m, int s) {
-                slab[at<N>(l + 1, m)] = (S)2 * a[s] * Vj[fold_idx(l + 1, m, N)];
-            });
-            __syncthreads();
-            slab_r2r_2d<S, N, 1>(slab, tw);
-            each_lambda<N>([&](int l, int m, int s) { a[s] = slab[at<N>(l + 1, m)]; });
-            __syncthreads();
-        }
-    }
+    const int j = blockIdx.x + 1;
+    const int jv = (j > Nw / 2) ? Nw - j : j;
+    const double t = (double)j / (T * Nw), bt = 1.0 / T - t;
+    each_wedge<N>(wt, [&](int a, int b, int i) {
+        const double g = lam_val(which, g0_exp(ekw[i] - mu0, t, bt), t, fw[i], fw[nk8 + i]);
+        slab[a] = (S)(g * vw[i]);
+        slab[b] = (S)(g * vw[nk8 + i]);
+    });
+    S v[wedge_per_thread<N>()];  // V(r,|tau|) of the thread's points, in flight during the transform
+    load_wedge<N>(V + (long)jv * nk8, v);
+    __syncthreads();
+    slab_r2r_2d<S, N, 1>(slab, tw);
+    each_wedge_slot<N>(wt, [&](int a, int b, int, int c) {
+        const S va = (S)2 * slab[a] * v[c], vb = (S)2 * slab[b] * v[c];
+        slab[a] = va;
+        slab[b] = vb;
+    });
+    __syncthreads();
+    slab_r2r_2d<S, N, 1>(slab, tw);
+    S* o = out + (long)j * nq;
+    each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
 }
-
-constexpr int kHVBlocks = 256;  // workgroups of the FP32 hV/f0V slab kernel
 
 // ================================================================== Lambda_jj pencils
 struct Poles {
@@ -1997,8 +1965,8 @@ hipError_t launch_chi0_tau0(const Grid& g, const DevArrays& d, hipStream_t s)
     const size_t lds = slab_bytes(g.N, sizeof(double));
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
         set_lds(k_chi0_tau0<NN, SS>, lds);
-        hipLaunchKernelGGL((k_chi0_tau0<NN, SS>), dim3(1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.er, d.mu0v, g.T,
-                           (SS*)d.chi, (SS*)d.chirt, d.dchirt0, d.dGrt0p, d.dchiqt0, d.chirt0);
+        hipLaunchKernelGGL((k_chi0_tau0<NN, SS>), dim3(1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw,
+                           d.er, d.mu0v, g.T, (SS*)d.chi, (SS*)d.chirt, d.dchirt0, d.dGrt0p, d.dchiqt0, d.chirt0);
     }));
     return hipGetLastError();
 }
@@ -2008,8 +1976,8 @@ hipError_t launch_chi0_slab(const Grid& g, const DevArrays& d, hipStream_t s)
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_chi0_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_chi0_slab<NN, SS>), dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.mu0v, g.T, g.Nw,
-                           (SS*)d.chi, (SS*)d.chirt);
+        hipLaunchKernelGGL((k_chi0_slab<NN, SS>), dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw,
+                           d.mu0v, g.T, g.Nw, (SS*)d.chi, (SS*)d.chirt);
     }));
     return hipGetLastError();
 }
@@ -2093,8 +2061,8 @@ hipError_t launch_model(const Grid& g, const DevArrays& d, double t, double tp, 
                         hipStream_t s)
 {
     const long n = std::max<long>((long)g.nk * g.nk, g.nq);
-    hipLaunchKernelGGL(k_model, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g.N, t, tp, tpp, t3, d.ek, d.ekw,
-                       d.wq, d.er, d.d2ek, d.dek);
+    hipLaunchKernelGGL(k_model, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g.N, slab_dims(g.N).LD, t, tp,
+                       tpp, t3, d.ek, d.ekw, d.wq, d.er, d.d2ek, d.dek, d.wt, d.vw);
     return hipGetLastError();
 }
 
@@ -2120,7 +2088,7 @@ hipError_t launch_mu0_root(const Grid& g, const DevArrays& d, double n, double p
     const long waves = (g.nk8 + 64L * kMu0K - 1) / (64L * kMu0K);
     if (waves > 16) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_mu0_root, dim3(1), dim3((unsigned)(64 * waves)), 0, s, d.ekw, d.wq, g.nk8, Nk2, g.T, n,
-                       preset, out, d.mu0v);
+                       preset, out, d.mu0v, d.fw);
     return hipGetLastError();
 }
 
@@ -2131,7 +2099,7 @@ hipError_t launch_vertex_slab(const Grid& g, const DevArrays& d, double U, doubl
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_vertex_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_vertex_slab<NN, SS>), dim3(g.nwb), dim3(SlabShape<NN>::NT), lds, s, d.chiw, (SS*)d.V,
+        hipLaunchKernelGGL((k_vertex_slab<NN, SS>), dim3(g.nwb), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.chiw, (SS*)d.V,
                            normFact, U, Usp, Uch, dsc);
     }));
     return hipGetLastError();
@@ -2154,8 +2122,8 @@ hipError_t launch_sigma_bnd(const Grid& g, const DevArrays& d, double mu0, doubl
     const size_t lds = slab_bytes(g.N, sizeof(double));
     DISPATCH_N(g.N, {
         set_lds(k_sigma_bnd<NN>, lds);
-        hipLaunchKernelGGL(k_sigma_bnd<NN>, dim3(4), dim3(SlabShape<NN>::NT), lds, s, d.ekw, d.er, d.V0, d.dchirt0,
-                           d.dGrt0p, mu0, g.T, fact, d.dSig, d.Sb, mu0p, U, dsc);
+        hipLaunchKernelGGL(k_sigma_bnd<NN>, dim3(4), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw, d.er, d.V0,
+                           d.dchirt0, d.dGrt0p, mu0, g.T, fact, d.dSig, d.Sb, mu0p, U, dsc);
     });
     return hipGetLastError();
 }
@@ -2165,8 +2133,8 @@ hipError_t launch_sigma_slab(const Grid& g, const DevArrays& d, double mu0, hipS
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(SS));
         set_lds(k_sigma_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_sigma_slab<NN, SS>), dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.ekw, (const SS*)d.V,
-                           mu0, g.T, g.Nw, (SS*)d.Stau, mu0p);
+        hipLaunchKernelGGL((k_sigma_slab<NN, SS>), dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw,
+                           (const SS*)d.V, mu0, g.T, g.Nw, (SS*)d.Stau, mu0p);
     }));
     return hipGetLastError();
 }
@@ -2219,42 +2187,25 @@ hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu0, dou
     return hipGetLastError();
 }
 
-hipError_t launch_hf0_slab(const Grid& g, const DevArrays& d, hipStream_t s)
-{
-    DISPATCH_S(g.prec, DISPATCH_N(g.N, {
-        constexpr size_t lds = slab_bytes(NN, sizeof(SS));
-        set_lds(k_hf0_slab<NN, SS>, lds);
-        hipLaunchKernelGGL((k_hf0_slab<NN, SS>), dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.ek, d.dek, d.mu0v, g.T,
-                           g.Nw, (SS*)d.h, (SS*)d.f0);
-    }));
-    return hipGetLastError();
-}
-
 hipError_t launch_hf0_bnd(const Grid& g, const DevArrays& d, double mu0, double fact4, hipStream_t s,
                           const double* mu0p, double U, const double* dsc)
 {
     const size_t lds = slab_bytes(g.N, sizeof(double));
     DISPATCH_N(g.N, {
         set_lds(k_hf0_bnd<NN>, lds);
-        hipLaunchKernelGGL(k_hf0_bnd<NN>, dim3(8), dim3(SlabShape<NN>::NT), lds, s, d.ek, d.dek, d.V0, d.dchirt0, mu0, g.T,
-                           g.Nw, fact4, d.dhV, d.df0V, d.hVb, d.f0Vb, mu0p, U, dsc);
+        hipLaunchKernelGGL(k_hf0_bnd<NN>, dim3(8), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw, d.vw, d.V0,
+                           d.dchirt0, mu0, g.T, fact4, d.dhV, d.df0V, d.hVb, d.f0Vb, mu0p, U, dsc);
     });
     return hipGetLastError();
 }
 
-hipError_t launch_hVf0V_slab(const Grid& g, const DevArrays& d, hipStream_t s)
+hipError_t launch_hV_slab(const Grid& g, const DevArrays& d, int which, hipStream_t s)
 {
     DISPATCH_S(g.prec, DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(SS));
-        set_lds(k_hVf0V_slab<NN, SS>, lds);
-        // FP32: at most kHVBlocks workgroups, each looping over slabs.  This kernel runs beside
-        // the latency-bound self-energy pencil and mu search; two of its workgroups fill a CU's
-        // waves, one leaves room for theirs.  An FP64 slab (151 KB of LDS) holds a CU alone
-        // either way, and fewer of them only lengthen the kernel (measured at 256^2 x 2048:
-        // -0.05 ms per solve in FP32, +0.2 ms in FP64).
-        const unsigned nb = (unsigned)((sizeof(SS) == sizeof(float)) ? std::min(g.Nw + 1, kHVBlocks) : g.Nw + 1);
-        hipLaunchKernelGGL((k_hVf0V_slab<NN, SS>), dim3(nb), dim3(SlabShape<NN>::NT), lds, s, (const SS*)d.V, g.Nw,
-                           (SS*)d.h, (SS*)d.f0);
+        set_lds(k_hV_slab<NN, SS>, lds);
+        hipLaunchKernelGGL((k_hV_slab<NN, SS>), dim3(g.Nw - 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw,
+                           d.vw, d.mu0v, g.T, g.Nw, (const SS*)d.V, which, (SS*)(which == 0 ? d.h : d.f0));
     }));
     return hipGetLastError();
 }

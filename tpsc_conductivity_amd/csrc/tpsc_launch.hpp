@@ -18,6 +18,9 @@ struct DevArrays {
     double* ekw = nullptr;       // nk8  wedge-packed eps(k)
     double* wq = nullptr;        // nk8  wedge weight 8/2^(edges+diag)
     double* er = nullptr;        // nk8
+    unsigned* wt = nullptr;      // nk8  slab offsets of a wedge point's two places (k_model)
+    double* fw = nullptr;        // 2*nk8  Fermi factors f/N^2 and (e^{-x/T} or 1) f^2/(T N^2) at mu0 (k_mu0_root)
+    double* vw = nullptr;        // 2*nk8  v_x at (l, m) and (m, l) of a wedge point, 0 at kx = 0, pi
     double* chi = nullptr;       // nwb*nk8 : chi0(q,tau)
     double* chiw = nullptr;      // nwb*nk8 : chi0(q,iqn), FP64 (== chi in the FP64 path)
     double* chirt = nullptr;     // nwb*nk8 : chi0(r,tau)
@@ -41,8 +44,8 @@ struct DevArrays {
     double* Sinf = nullptr;      // 1
     double* dek = nullptr;       // nq   (v_x on the Lambda grid)
     double* d2ek = nullptr;      // nk*nk
-    double* h = nullptr;         // (Nw+1)*nq
-    double* f0 = nullptr;        // (Nw+1)*nq
+    double* h = nullptr;         // (Nw+1)*nq  hV(k,tau_j), 0 < j < Nw
+    double* f0 = nullptr;        // (Nw+1)*nq  f0V(k,tau_j), 0 < j < Nw
     double* dhV = nullptr;       // 2*nq
     double* df0V = nullptr;      // 2*nq
     double* hVb = nullptr;       // 2*nq   hV(k, tau = 0), hV(k, tau = beta)
@@ -220,10 +223,10 @@ hipError_t launch_trace_diffG(const Grid& g, const DevArrays& d, double pmu, dou
                               hipStream_t s);
 hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu0, double mu, int which, double* out,
                               hipStream_t s);
-hipError_t launch_hf0_slab(const Grid& g, const DevArrays& d, hipStream_t s);
 hipError_t launch_hf0_bnd(const Grid& g, const DevArrays& d, double mu0, double fact4, hipStream_t s,
                           const double* mu0p = nullptr, double U = 0.0, const double* dsc = nullptr);
-hipError_t launch_hVf0V_slab(const Grid& g, const DevArrays& d, hipStream_t s);
+// hV (which 0, into d.h) or f0V (1, into d.f0) for tau_j, 0 < j < Nw
+hipError_t launch_hV_slab(const Grid& g, const DevArrays& d, int which, hipStream_t s);
 hipError_t launch_jj_poles(const Grid& g, const DevArrays& d, double mu, hipStream_t s, const double* dsc = nullptr);
 hipError_t launch_jj_transpose(const Grid& g, const DevArrays& d, hipStream_t s);
 // partial rows to part (nblk x ntheta x 2*nwb); bins: the angle bin of each Lambda point, or null

@@ -44,10 +44,10 @@ def kernel_bytes(N, Nw, precision="fp64"):
         "sigma_slab": 2 * nt * nk8 * s,
         # read Sigma(k,tau), write Sigma(k,iwn) and three moment arrays
         "sigma_pencil": nt * nk8 * s + (Nw // 2) * nk8 * sc + 3 * nk8 * d,
-        # write h(r,tau), f0(r,tau)
-        "jj_hf0_slab": 2 * nt * nq * s,
-        # read and write h, f0; read V(r,|tau|)
-        "jj_hVf0V_slab": 4 * nt * nq * s + nt * nk8 * s,
+        # the h slices: read V(r,|tau|), write hV (h(r,tau) stays in LDS)
+        "jj_hf0_slab": nt * nq * s + nt * nk8 * s,
+        # the f0 slices: read V(r,|tau|), write f0V
+        "jj_hVf0V_slab": nt * nq * s + nt * nk8 * s,
         # read hV, f0V and (once) Sigma(k,iwn); partial rows out
         "jj_pencil": 2 * nt * nq * s + (Nw // 2) * nk8 * sc + 2 * ((nq + 15) // 16) * 2 * nwb * d,
         # one sum-rule evaluation: read chi0(q,iqn)
