@@ -1024,11 +1024,15 @@ __device__ __forceinline__ int at(int l, int m)
 // G0(k,-t)/N^2 (chi0.cpp:468-471, 486-489)
 __device__ __forceinline__ double g0_exp(double x, double t, double bt) { return exp(x >= 0.0 ? -t * x : bt * x); }
 
+// Sinf/z + s2/z^2 + s3/z^3 + R/z^4, z = i wn (green.cpp:3039), iw = 1/wn
+__device__ __forceinline__ cd sigma_mom_i(double Sinf, double s2, double s3, cd R, double iw)
+{
+    const double iw2 = iw * iw;
+    return cd{(-s2 + R.x * iw2) * iw2, (-Sinf + (s3 + R.y * iw) * iw2) * iw};
+}
 __device__ __forceinline__ cd sigma_mom(double Sinf, double s2, double s3, cd R, double wn)
 {
-    // Sinf/z + s2/z^2 + s3/z^3 + R/z^4, z = i wn (green.cpp:3039), with one reciprocal of wn
-    const double iw = 1.0 / wn, iw2 = iw * iw;
-    return cd{(-s2 + R.x * iw2) * iw2, (-Sinf + (s3 + R.y * iw) * iw2) * iw};
+    return sigma_mom_i(Sinf, s2, s3, R, rcp_nr(wn));
 }
 
 // Sigma(k, i w_n), w_n > 0, at offset o of the stored form: the remainder R (FP64 path,

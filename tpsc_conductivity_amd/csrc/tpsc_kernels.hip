@@ -1,6 +1,6 @@
 // tpsc_kernels.hip -- HIP kernels of the TPSC hot path for gfx950.
 //
-// Stage map (reference = dbergeron1/TPSC_conductivity):
+// Stage map (tpsc_jj.hip holds the Lambda pencils; reference = dbergeron1/TPSC_conductivity):
 //   k_chi0_tau0, k_chi0_slab     chi0.cpp:310-559   G0(k,+-tau) -> G(r,+-tau) -> chi0(r,tau) -> chi0(q,tau)
 //   k_chi0_pencil                chi0.cpp:566-698   clamped spline in tau + DFT -> chi0(q,iqn), tails
 //   k_sum_rule                   chi.cpp:738-830    sum-rule traces (one candidate U per launch)
@@ -8,8 +8,7 @@
 //   k_vertex_slab/_pencil        chi.cpp:85-170     V(r,tau)
 //   k_sigma_bnd/_slab/_pencil    green.cpp:1743-2018 Sigma(k,iwn) moments + remainder
 //   k_trace_diffG, k_trace_selfG green.cpp:2929-3182 traces for mu and consistency checks
-//   k_hf0_bnd, k_hV_slab,
-//   k_jj_pencil, k_kx0_rows      cond_opt.cpp:2584-4173 Lambda_jj bubble + Maki-Thompson + kx0
+//   k_hf0_bnd, k_hV_slab         cond_opt.cpp:2584-3180 Lambda_jj: hV, f0V
 // Slab kernels hold one (nk x nk) slab in LDS (151 KB at N=256 in FP64) and transform it with
 // register FFTs of line pairs; pencil kernels hold one tau-pencil per workgroup.
 // Precision: S is the storage and slab-arithmetic type of the tau arrays (chi0(q,tau),
@@ -22,6 +21,7 @@
 #include <unordered_map>
 
 #include "tpsc_launch.hpp"
+#include "tpsc_pencil.hpp"
 
 namespace tpsc {
 
@@ -1260,176 +1260,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     each_lambda<N>([&](int l, int m, int s) { o[s] = slab[at<N>(l + 1, m)]; });
 }
 
-// ================================================================== Lambda_jj pencils
-struct Poles {
-    cd r1, r2, a1, a2, b1, b2, den1, den2;
-};
-
-// roots of z^2 + (mu - e) z - Sigma_inf with Newton polish (generique.cpp:1666-1726)
-__device__ __forceinline__ void roots2(cd A, cd B, cd Cc, cd* roots)
-{
-    if (!(cabs2(A) > 1.0e-15)) return;
-    const cd Rr = csqrtd(B * B - 4.0 * A * Cc);
-    roots[0] = (-B - Rr) / (2.0 * A);
-    roots[1] = (-B + Rr) / (2.0 * A);
-    for (int j = 0; j < 2; j++) {
-        cd x = roots[j];
-        cd yv = A * x * x + B * x + Cc;
-        cd p = 2.0 * A * x + B;
-        const cd y0 = yv;
-        int it = 0;
-        while (cabs2(p) != 0.0 && it < 10 && cabs2(yv) > 1.0e-16) {
-            const cd x2 = x, y2 = yv;
-            const cd cc = yv - p * x;
-            x = (-cc) / p;
-            yv = A * x * x + B * x + Cc;
-            p = 2.0 * A * x + B;
-            if (cabs2(y2) < cabs2(yv)) {
-                x = 0.5 * (x + x2);
-                yv = A * x * x + B * x + Cc;
-                p = 2.0 * A * x + B;
-            }
-            it++;
-        }
-        if (cabs2(yv) < cabs2(y0)) roots[j] = x;
-    }
-}
-
-__device__ __forceinline__ Poles make_poles(double e, double mu, double Sinf, double CJ1, double T)
-{
-    Poles P;
-    cd roots[2] = {cd{0, 0}, cd{0, 0}};
-    roots2(cd{1.0, 0.0}, cd{-e + mu, 0.0}, cd{-Sinf, 0.0}, roots);
-    P.r1 = roots[0];
-    P.r2 = roots[1];
-    P.a1 = P.r1 / (P.r1 - P.r2);
-    P.a2 = P.r2 / (P.r2 - P.r1);
-    P.b1 = CJ1 / (P.r1 - P.r2);
-    P.b2 = -P.b1;
-    P.den1 = (P.r1.x > 0 ? cexpd(-(P.r1 / T)) : cexpd(P.r1 / T)) + cd{1.0, 0.0};
-    P.den2 = (P.r2.x > 0 ? cexpd(-(P.r2 / T)) : cexpd(P.r2 / T)) + cd{1.0, 0.0};
-    return P;
-}
-
-// Dyson G at Matsubara slot s (n = s - Nw/2), with the conjugate Sigma for n < 0
-// (cond_opt.cpp:3354-3407).  dyson_n: the stored frequency index of slot s.
-__device__ __forceinline__ int dyson_n(int s, int H) { return (s < H) ? H - s - 1 : s - H; }
-// from the stored value raw = Self[ki * H + dyson_n(s, H)]
-template <typename SelfT>
-__device__ __forceinline__ cd dyson_G_raw(SelfT raw, int s, int H, double C2, double C3, double Sinf, double e,
-                                          double mu, double T, double& kn)
-{
-    kn = (2.0 * (s - H) + 1) * kPi * T;
-    cd sg = sigma_kw(&raw, 0, Sinf, C2, C3, fabs(kn));
-    if (s < H) sg = conjg(sg);
-    const cd den = cd{0.0 - e, kn} + cd{mu, 0.0} - sg;
-    return sdiv_rcp(T, den);
-}
-template <typename SelfT>
-__device__ __forceinline__ cd dyson_G(const SelfT* __restrict__ Self, long ki, long nk8, int s, int H, double C2,
-                                      double C3, double Sinf, double e, double mu, double T, double& kn)
-{
-    return dyson_G_raw(Self[ki * H + dyson_n(s, H)], s, H, C2, C3, Sinf, e, mu, T, kn);
-}
-
-// Two-pole asymptote data of every Lambda-grid point (cond_opt.cpp:3409-3467): the roots of
-// z^2 + (mu - e) z - Sigma_inf, the residues, and the tau = 0+ / beta- pole sums used for the
-// boundary slopes.  One thread per point.
-struct JJPoles {
-    Poles P;
-    cd f1p, f1m, fj1, fj1b, f2p, f2m, fj2, fj2b;
-    // e1(t) ej1(t) = C1 for all t (C1 = e^{-beta r1} if Re r1 > 0, else e^{beta r1}); used when
-    // beta |Re r1| < 600, so that 1/e1 stays finite.  Same for the second pole.
-    cd C1, C2;
-    int rec1, rec2;
-    cd a1d, a2d, b1d, b2d;  // a1/den1, a2/den2, b1/den1, b2/den2
-    // the pencil's per-step factors exp(-dt r), exp(dt r) of each pole (dt = NT/(L T), its
-    // threads' stride in tau), and the two-pole part of J at tau = beta
-    cd s1, sj1, s2, sj2;
-    double Jinf_beta;
-};
-static_assert(sizeof(JJPoles) <= 64 * sizeof(double), "DevArrays::poles holds 64 doubles per point");
-
-// The two factors of pole r in the tau = t asymptote (cond_opt.cpp:3409-3467), both of modulus
-// <= 1 on [0, beta]: e(t) = exp(-t r) (Re r > 0) or exp((beta - t) r), and its partner
-// ej(t) = exp(r (t - beta)) or exp(r t), taken as C / e(t) when rec is set (e ej = C).
-__device__ __forceinline__ cd pole_e(cd r, double t, double T)
-{
-    return (r.x > 0) ? cexpd(-t * r) : cexpd((1.0 / T - t) * r);
-}
-__device__ __forceinline__ cd pole_ej(cd r, double t, double T, int rec, cd C, cd e)
-{
-    if (rec) return C / e;
-    return (r.x > 0) ? cexpd(r * (t - 1.0 / T)) : cexpd(r * t);
-}
-__device__ __forceinline__ bool pole_off(cd v)
-{
-    const double a = fabs(v.x) + fabs(v.y);
-    return !(a >= 1.0e-280 && a <= 2.0);
-}
-
-__global__ void k_jj_poles(const double* __restrict__ ek, const double* __restrict__ hVb,
-                           const double* __restrict__ Sinfp, int N, double T, double mu, double dt, JJPoles* out,
-                           const double* __restrict__ dsc)
-{
-    if (dsc) mu = dsc[kPscMu + 1];
-    const int nk = N / 2 + 1;
-    const long nq = (long)nk * (nk - 2);
-    const long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (q >= nq) return;
-    const int l = (int)(q / nk), m = (int)(q % nk);
-    const double e = ek[m + (l + 1) * nk];
-    const double CJ1 = -hVb[q] - hVb[nq + q];
-    JJPoles o;
-    const Poles P = make_poles(e, mu, Sinfp[0], CJ1, T);
-    o.P = P;
-    const double beta = 1.0 / T;
-    o.C1 = (P.r1.x > 0) ? cexpd(-(beta * P.r1)) : cexpd(beta * P.r1);
-    o.C2 = (P.r2.x > 0) ? cexpd(-(beta * P.r2)) : cexpd(beta * P.r2);
-    o.rec1 = fabs(P.r1.x) * beta < 600.0;
-    o.rec2 = fabs(P.r2.x) * beta < 600.0;
-    o.a1d = P.a1 / P.den1;
-    o.a2d = P.a2 / P.den2;
-    o.b1d = P.b1 / P.den1;
-    o.b2d = P.b2 / P.den2;
-    o.s1 = cexpd(-dt * P.r1);
-    o.sj1 = cexpd(dt * P.r1);
-    o.s2 = cexpd(-dt * P.r2);
-    o.sj2 = cexpd(dt * P.r2);
-    {
-        const cd ej1 = (P.r1.x > 0) ? cd{1.0, 0.0} : cexpd(P.r1 * beta);
-        const cd ej2 = (P.r2.x > 0) ? cd{1.0, 0.0} : cexpd(P.r2 * beta);
-        o.Jinf_beta = (P.b1 * ej1 / P.den1 + P.b2 * ej2 / P.den2).x;
-    }
-    if (P.r1.x > 0) {
-        const cd ex = cexpd(-(P.r1 / T));
-        o.f1p = P.a1 / P.den1;
-        o.f1m = P.a1 * ex / P.den1;
-        o.fj1 = P.r1 * P.b1 * ex / P.den1;
-        o.fj1b = P.r1 * P.b1 / P.den1;
-    } else {
-        const cd ex = cexpd(P.r1 / T);
-        o.f1p = P.a1 * ex / P.den1;
-        o.f1m = P.a1 / P.den1;
-        o.fj1 = P.r1 * P.b1 / P.den1;
-        o.fj1b = P.r1 * P.b1 * ex / P.den1;
-    }
-    if (P.r2.x > 0) {
-        const cd ex = cexpd(-(P.r2 / T));
-        o.f2p = P.a2 / P.den2;
-        o.f2m = P.a2 * ex / P.den2;
-        o.fj2 = P.r2 * P.b2 * ex / P.den2;
-        o.fj2b = P.r2 * P.b2 / P.den2;
-    } else {
-        const cd ex = cexpd(P.r2 / T);
-        o.f2p = P.a2 * ex / P.den2;
-        o.f2m = P.a2 / P.den2;
-        o.fj2 = P.r2 * P.b2 / P.den2;
-        o.fj2b = P.r2 * P.b2 * ex / P.den2;
-    }
-    out[q] = o;
-}
-
+// ================================================================== transposes
 // [j][q] (j < nj, q < nq) -> [q][j]: kTT x kTT tiles through LDS, both sides coalesced (a
 // wave moves 64 consecutive elements of one row per access; 16 accesses per thread in flight).
 // Rows of odd length (nq = nk (nk - 2), nj = Nw + 1) rule out vector accesses.  The Lambda
@@ -1463,373 +1294,6 @@ __global__ void __launch_bounds__(256) k_transpose(const S* __restrict__ in0, S*
     for (int r = 0; r < kTT; r += 4) {
         const long q = q0 + ty + r;
         if (j < nj && q < nq) out[q * nj + j] = t[tx][ty + r];
-    }
-}
-
-// Per-k Lambda_jj contributions (cond_opt.cpp:3179-3822).  One workgroup of NT threads per
-// Lambda-grid point at a time; workgroup blk handles the points q = blk + kk*nblk,
-// kk < jj_points(L), and accumulates into its own partial rows, one pair per angle bin b of the
-// point (bins[q], cond_opt.cpp:3792-3793; bin 0 when bins is null):
-// part[(blk*ntheta + b)*2*nwb + n] (bubble) and part[(blk*ntheta + b)*2*nwb + nwb + n]
-// (Maki-Thompson).
-//
-// The six length-L transforms of the reference run as three complex FFTs of pairs of
-// sequences whose transforms have a known symmetry:
-//   (1) the f0V and hV spline moments 6a_j (real) with the phase exp(i pi j/L): for real a,
-//       A(n) = sum_j a_j e^{2 pi i j (n + 1/2)/L} obeys A(L-1-n) = conj A(n), so the FFT F of
-//       (a + i b) e^{i pi j/L} splits into A(n) = (F_n + conj F_{L-1-n})/2 and
-//       B(n) = (F_n - conj F_{L-1-n})/(2i);
-//   (2) G(ikn) - G2 and conj(J(ikn)) (both Hermitian in n -> -n-1): ph_j * FFT_-(.)_j is real
-//       for each, so ph_j * FFT_-(Gn + i conj Jn)_j = G(tau_j) + i J(tau_j) before the two-pole
-//       terms (FFT_+(Jn)_j / ph_j = conj(ph_j FFT_-(conj Jn)_j));
-//   (3) the Maki-Thompson and bubble moments (real): A_n = (F_n + conj F_{L-n})/2,
-//       B_n = (F_n - conj F_{L-n})/(2i).
-// Imaginary parts of G(tau), J(tau) are zero in exact arithmetic and are not formed.
-// LDS: the spline samples / moments (Y1, Y2, in place), which also hold the packed slot
-// values W of step (2), and one transform buffer X.  hT, f0T are the hV, f0V pencils in
-// point-major layout [q][j] (k_transpose); the pole data come from k_jj_poles.
-
-#ifndef JJ_WAVES_PER_SIMD
-#define JJ_WAVES_PER_SIMD 2  // two 256-thread workgroups per CU (74 KB LDS each), no register cap
-#endif
-// L = 4096 takes 139 KB of LDS: one workgroup per CU
-template <int L, int NT, typename S, typename SelfT>
-__global__ void __launch_bounds__(NT, (L > 2048 ? 1 : JJ_WAVES_PER_SIMD))
-    k_jj_pencil(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ d2ek,
-                const S* __restrict__ hT, const S* __restrict__ f0T, const double* __restrict__ dhV,
-                const double* __restrict__ df0V, const double* __restrict__ hVb, const double* __restrict__ f0Vb,
-                const JJPoles* __restrict__ poles, const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
-                const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, double T, double mu,
-                const cd* __restrict__ tw,
-                const cd* __restrict__ twX, const cd* __restrict__ twS, const cd* __restrict__ twM,
-                const cd* __restrict__ phT, double* part, double* scal, const int* __restrict__ bins, int ntheta,
-                const double* __restrict__ dsc)
-{
-    if (dsc) mu = dsc[kPscMu + 1];
-    constexpr int H = L / 2;
-    constexpr int NWB = H + 1;
-    constexpr int CS = (L + 1 + NT - 1) / NT;  // spline chunk
-    __shared__ __align__(16) double Yb[2 * (L + 1)];
-    __shared__ cd X[L];
-    __shared__ double sc[8 * (NT / 64)];
-    __shared__ double ES[2 * (2 * NT + 8)];
-    __shared__ double Jbeta_s;
-    double* Y1 = Yb;
-    double* Y2 = Yb + (L + 1);
-    cd* W = (cd*)Yb;  // L complex values, used while Y1, Y2 are free
-    const int nk = N / 2 + 1;
-    const long nq = (long)nk * (nk - 2);
-    const double nf = 1.0 / ((double)N * N);
-    const double Sinf = Sinfp[0];
-    const double hstep = 1.0 / (L * T), ihstep = L * T, iT = 1.0 / T;
-    const int tid = threadIdx.x;
-    const int blk = xcd_remap(blockIdx.x, gridDim.x);
-    const long nblk = gridDim.x;
-    double* const rows = part + (long)blk * 2 * NWB * ntheta;
-    for (int n = tid; n < 2 * NWB * ntheta; n += NT) rows[n] = 0.0;  // the barrier below orders it
-    double k0acc = 0.0, inf1 = 0.0, inf2 = 0.0, inf4 = 0.0;
-    // The interior samples j = 1..L-1 of the f0V and hV pencils of the next point go from HBM
-    // straight into LDS (global_load_lds, no registers) while the current point's last
-    // accumulation runs: they are issued once Yb is free (after the last transform, which
-    // uses it as its second buffer).  FP64 rows land in Y1 + 1 and Y2 + 1 themselves;
-    // FP32 rows land in the upper half of Yb (stage0, stage1) and are widened at the top of
-    // the next point.  Each wave copies 256-byte chunks c = wave, wave + NT/64, ... of a row,
-    // one dword per lane.
-    constexpr bool kWide = sizeof(S) == sizeof(double);
-    char* const stage0 = kWide ? (char*)(Y1 + 1) : (char*)Y2;
-    char* const stage1 = kWide ? (char*)(Y2 + 1) : (char*)Y2 + 4 * L;
-    auto dma_rows = [&](long qq) {
-        constexpr int NDW = (L - 1) * (int)sizeof(S) / 4;  // dwords per row
-        // the LDS destination (M0) must be wave-uniform: the wave index is made provably so
-        const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const char* src0 = (const char*)(f0T + qq * (L + 1) + 1);
-        const char* src1 = (const char*)(hT + qq * (L + 1) + 1);
-        for (int c = wv; c * 64 < NDW; c += NT / 64) {
-            const int i = c * 64 + lane;
-            if (i < NDW) {
-                __builtin_amdgcn_global_load_lds((const void*)(src0 + 4 * i), (void*)(stage0 + 256 * c), 4, 0, 0);
-                __builtin_amdgcn_global_load_lds((const void*)(src1 + 4 * i), (void*)(stage1 + 256 * c), 4, 0, 0);
-            }
-        }
-    };
-    if (blk < nq) dma_rows(blk);
-    __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS DMA has landed (the barrier below covers the others)
-    __syncthreads();
-    // point kk of workgroup blk is q = blk + kk * nblk: the workgroups resident on one XCD
-    // (consecutive blk) work on consecutive q at the same time and share the cache lines of
-    // the tau-major hV / f0V rows and of Sigma
-    constexpr int KP = jj_points(L);
-    for (int kk = 0; kk < KP; kk++) {
-        const long q = (long)blk + kk * nblk;
-        if (q >= nq) break;
-        const int l = (int)(q / nk), m = (int)(q % nk);
-        const long ki = fold_idx(l + 1, m, N);
-        const double e = ek[m + (l + 1) * nk];
-        const double v = dek[q];
-        const double wt = (m == 0 || m == nk - 1) ? 2.0 : 4.0;
-        double* const c1 = rows + (long)(bins ? bins[q] : 0) * 2 * NWB;
-        double* const c2 = c1 + NWB;
-        // (1) f0V and hV pencils (interior samples already in LDS), their splines, one packed FFT
-        if constexpr (kWide) {
-            if (tid == 0) {
-                Y1[0] = f0Vb[q];
-                Y1[L] = f0Vb[nq + q];
-                Y2[0] = hVb[q];
-                Y2[L] = hVb[nq + q];
-            }
-        } else {
-            const float* sf = (const float*)stage0;
-            const float* sh = (const float*)stage1;
-            float fa[CS], ha[CS];
-#pragma unroll
-            for (int c = 0; c < CS; c++) {
-                const int j = tid + c * NT;
-                fa[c] = (j > 0 && j < L) ? sf[j - 1] : 0.0f;
-                ha[c] = (j > 0 && j < L) ? sh[j - 1] : 0.0f;
-            }
-            __syncthreads();  // the staged rows overlap Y2
-#pragma unroll
-            for (int c = 0; c < CS; c++) {
-                const int j = tid + c * NT;
-                if (j <= L) {
-                    Y1[j] = (j == 0) ? f0Vb[q] : (j == L) ? f0Vb[nq + q] : (double)fa[c];
-                    Y2[j] = (j == 0) ? hVb[q] : (j == L) ? hVb[nq + q] : (double)ha[c];
-                }
-            }
-        }
-        const double CJ1 = -hVb[q] - hVb[nq + q];
-        __syncthreads();
-        {
-            double* const ys[2] = {Y1, Y2};
-            const double d0s[2] = {df0V[q], dhV[q]}, dNs[2] = {df0V[q + nq], dhV[q + nq]};
-            block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, nullptr);
-        }
-        for (int j = tid; j < L; j += NT) {
-            const double a = (Y1[j + 1] - Y1[j]) * ihstep, b = (Y2[j + 1] - Y2[j]) * ihstep;
-            X[j] = twX[j] * cd{a, b};
-        }
-        const double cj03 = -(Y1[0] + Y1[L]), cj3 = -(Y2[0] + Y2[L]);
-        __syncthreads();
-        block_fft_pp<L, NT>(X, W, +1, tw);  // Y1, Y2 (W) are free: their last reads are above
-        // (2) per Matsubara slot s (n = s - L/2): Dyson G, J0 (f0V), J (hV) -> W
-        double r6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // qn0 (re, im), sum Gn (re, im), dGp, dJ0
-        {
-            const double C2 = Sinf2[ki], C3 = Sinf3[ki];
-            const double cj01 = -f0Vb[q] - f0Vb[nq + q], cj02 = df0V[q] + df0V[q + nq];
-            const double cj2 = dhV[q] + dhV[q + nq];
-            // the global reads of slot s + NT (Sigma, twS) are issued before the work of slot s
-            const SelfT* Sk = Self + ki * H;
-            auto slot_jx = [&](int s) { return (s >= H) ? s - H : s + H; };  // transform index of slot s
-            SelfT sv_next = Sk[dyson_n(tid, H)];
-            cd ts_next = twS[slot_jx(tid)];
-#pragma unroll 1
-            for (int s = tid; s < L; s += NT) {
-                const SelfT sv = sv_next;
-                const cd ts = ts_next;
-                if (s + NT < L) {
-                    sv_next = Sk[dyson_n(s + NT, H)];
-                    ts_next = twS[slot_jx(s + NT)];
-                }
-                const int jx = slot_jx(s);
-                const cd Fj = X[jx], Fc = conjg(X[L - 1 - jx]);
-                const cd Af = cd{0.5 * (Fj.x + Fc.x), 0.5 * (Fj.y + Fc.y)};
-                const cd Bh = cd{0.5 * (Fj.y - Fc.y), -0.5 * (Fj.x - Fc.x)};
-                const double knj = (jx < H) ? (2 * jx + 1) * kPi * T : (2 * (jx - L) + 1) * kPi * T;
-                // -i c1/k - c2/k^2 + i c3/k^3 + a/k^4 with one reciprocal of k (cond_opt.cpp:3302-3311)
-                const double ik = rcp_nr(knj), ik2 = ik * ik;
-                const cd af = ts * Af, ah = ts * Bh;
-                const cd J0 = cd{(-cj02 + af.x * ik2) * ik2, (-cj01 + (cj03 + af.y * ik) * ik2) * ik};
-                const cd Jv = cd{(-cj2 + ah.x * ik2) * ik2, (-CJ1 + (cj3 + ah.y * ik) * ik2) * ik};
-                double kn;
-                const cd Gv = dyson_G_raw(sv, s, H, C2, C3, Sinf, e, mu, T, kn);
-                const cd t = (Gv * Gv * J0) * iT;
-                r6[0] += t.x;
-                r6[1] += t.y;
-                const double ikn = rcp_nr(kn);
-                const cd G2 = sdiv_rcp(T, cd{-e + mu, kn + Sinf * ikn});
-                const cd Jn = Gv * Jv - G2 * cd{0.0, -CJ1 * ikn};
-                const cd Gn = Gv - G2;
-                r6[2] += Gn.x;
-                r6[3] += Gn.y;
-                r6[4] += kn * Gn.y;
-                r6[5] -= kn * Jn.y;
-                W[s] = cd{Gn.x + Jn.y, Gn.y + Jn.x};  // Gn + i conj(Jn)
-            }
-        }
-        // the six sums: wave sums parked in sc[k * nw + wave], added in the order of block_sum_k
-        // where they are used (after the transform: fewer registers live across it)
-        constexpr int nw = NT / 64;
-        {
-            const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-            for (int k = 0; k < 6; k++) r6[k] = wave_sum(r6[k]);
-            if (lane == 0)
-#pragma unroll
-                for (int k = 0; k < 6; k++) sc[k * nw + wave] = r6[k];
-        }
-        __syncthreads();  // the W writes and the parked sums; X's last reads (step 2) are above
-        auto sum6 = [&](int k) {
-            double t = 0.0;
-            for (int i = 0; i < nw; i++) t += sc[k * nw + i];
-            return t;
-        };
-        // (3) two-pole asymptote: pole data from k_jj_poles
-        const JJPoles& pp = poles[q];
-        const Poles& P = pp.P;
-        // (4) to imaginary time: X_j <- (G(tau_j), J(tau_j))
-        block_fft_pp<L, NT>(W, X, -1, tw);
-        if (tid == 0) Jbeta_s = (cd{W[0].y, 0.0} / phT[L]).x + pp.Jinf_beta;  // W[0].y = FFT_+(Jn)_0 (ph_0 = 1)
-        {
-            // the pole factors are geometric in j: from tau_j to tau_{j+NT} e_p gains
-            // exp(-dt r_p) and ej_p exp(+dt r_p), dt = NT/(L T) (the step factors come with the
-            // pole data); a factor that leaves [1e-280, 2] on the way (underflow of a factor
-            // that grows again, overflow of a step) is evaluated directly again
-            double t = tid / (L * T);
-            cd e1 = pole_e(P.r1, t, T), e2 = pole_e(P.r2, t, T);
-            cd ej1 = pole_ej(P.r1, t, T, pp.rec1, pp.C1, e1), ej2 = pole_ej(P.r2, t, T, pp.rec2, pp.C2, e2);
-            const cd s1 = pp.s1, sj1 = pp.sj1, s2 = pp.s2, sj2 = pp.sj2;
-            cd ph_next = phT[tid];
-#pragma unroll 1
-            for (int j = tid; j < L; j += NT) {
-                const cd ph = ph_next;
-                if (j + NT < L) ph_next = phT[j + NT];
-                const double G0t = (-(pp.a1d * e1) - pp.a2d * e2).x;
-                const double Jinf = (pp.b1d * ej1 + pp.b2d * ej2).x;
-                const cd R = ph * W[j];
-                X[j] = cd{R.x + G0t, R.y + Jinf};
-                if (j + NT < L) {
-                    t = (j + NT) / (L * T);
-                    e1 = e1 * s1;
-                    e2 = e2 * s2;
-                    ej1 = ej1 * sj1;
-                    ej2 = ej2 * sj2;
-                    if (pole_off(e1)) e1 = pole_e(P.r1, t, T);
-                    if (pole_off(e2)) e2 = pole_e(P.r2, t, T);
-                    if (pole_off(ej1)) ej1 = pole_ej(P.r1, t, T, pp.rec1, pp.C1, e1);
-                    if (pole_off(ej2)) ej2 = pole_ej(P.r2, t, T, pp.rec2, pp.C2, e2);
-                }
-            }
-        }
-        __syncthreads();
-        const double G0 = X[0].x, J0t = X[0].y, Jbeta = Jbeta_s;
-        // sums of this point with the pole parts
-        const double k0r = sum6(2) + (pp.f1m + pp.f2m).x;
-        const double s4 = sum6(4), s5 = sum6(5);
-        const double dGp = s4 + (P.r1 * pp.f1p + P.r2 * pp.f2p).x;
-        const double dGm = -s4 + (P.r1 * pp.f1m + P.r2 * pp.f2m).x;
-        const double dJ0 = s5 + (pp.fj1 + pp.fj2).x;
-        const double dJb = -s5 + (pp.fj1b + pp.fj2b).x;
-        // (5) Maki-Thompson samples G(tau) J(-tau) -> Y1; bubble samples -G(tau) G(-tau) -> Y2 over
-        // the whole of [0, beta].  They are symmetric about beta/2 (the product is the same in
-        // both orders), so the clamped spline over [0, beta] with end slopes (dchi, -dchi) is, on
-        // [0, beta/2], the reference's spline with slopes (dchi, 0), and its integral is twice
-        // that of the half: the two splines run in one call.
-        for (int j = tid; j < L; j += NT) {
-            const cd gj = X[j];
-            Y1[j] = gj.x * gj.y;
-            Y2[j] = (j == 0) ? G0 * (G0 + 1.0) : -(gj.x * X[L - j].x);
-        }
-        if (tid == 0) {
-            Y1[L] = (-G0 - 1.0) * Jbeta;
-            Y2[L] = G0 * (G0 + 1.0);
-        }
-        __syncthreads();
-        const double gd0 = dGp * J0t + G0 * dJ0;
-        const double gdN = dGm * Jbeta - (G0 + 1.0) * dJb;
-        const double MJ1 = Y1[0] - Y1[L];
-        const double dchi = dGp * (G0 + 1.0) + G0 * dGm;
-        double integ[2] = {0.0, 0.0};
-        {
-            double* const ys[2] = {Y1, Y2};
-            const double d0s[2] = {gd0, dchi}, dNs[2] = {gdN, -dchi};
-            block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, integ);
-        }
-        // the bubble over [0, beta] is used by thread 0 only (n = 0): each wave parks its sum in
-        // sc[6 nw + wave], which thread 0 adds in the accumulation below (after two barriers)
-        {
-            const double ws = wave_sum(integ[1]);
-            if ((tid & 63) == 0) sc[6 * (NT / 64) + (tid >> 6)] = ws;
-        }
-        const double MJ3 = Y1[0] - Y1[L];
-        // (6) packed transform of the two moment sequences
-        for (int j = tid; j < L; j += NT) {
-            const double a = (Y1[j + 1] - Y1[j]) * ihstep;
-            const double b = (j < H) ? (Y2[j + 1] - Y2[j]) * ihstep : -(Y2[L - j] - Y2[L - 1 - j]) * ihstep;
-            X[j] = cd{a, b};
-        }
-        __syncthreads();  // Y1, Y2 read for the last time; the bubble's wave sums are in sc
-        block_fft_pp<L, NT>(X, W, -1, tw);
-        if (kk + 1 < KP && q + nblk < nq) dma_rows(q + nblk);  // W is free again
-        const double wv = nf * wt * v;
-#pragma unroll 1
-        for (int n = tid; n <= H; n += NT) {
-            const cd Fn = X[n], Fc = conjg(X[(L - n) & (L - 1)]);
-            double bub;
-            if (n == 0) {
-                bub = sum6(6);  // the bubble's wave sums
-                c2[0] -= wv * sum6(0);
-            } else {
-                const double iw = 1.0 / (2 * n * kPi * T), iw2 = iw * iw;
-                const cd tm = twM[n];
-                const cd a = tm * cd{0.5 * (Fn.x + Fc.x), 0.5 * (Fn.y + Fc.y)};
-                // -2 MJ1/wn + 2 MJ3/wn^3 + 2 a/wn^4, then / wn
-                const double imJ = (-2.0 * MJ1 + (2.0 * MJ3 + 2.0 * a.y * iw) * iw2) * iw;
-                c2[n] -= wv * imJ * iw;
-                const cd b = tm * cd{0.5 * (Fn.y - Fc.y), -0.5 * (Fn.x - Fc.x)};
-                bub = (-2.0 * dchi + b.x * iw2) * iw2;
-            }
-            c1[n] -= 2.0 * wv * v * bub;
-        }
-        k0acc -= 2.0 * wt * nf * d2ek[m + (l + 1) * nk] * k0r;
-        inf1 += 4.0 * dchi * wv * v;
-        inf2 += wv * 2.0 * MJ1;
-        inf4 -= wv * 2.0 * MJ3;
-        __builtin_amdgcn_s_waitcnt(0);  // the next point's rows have landed in LDS
-        __syncthreads();
-    }
-    if (tid == 0) {
-        scal[blk * 4 + 0] = k0acc;
-        scal[blk * 4 + 1] = inf1;
-        scal[blk * 4 + 2] = inf2;
-        scal[blk * 4 + 3] = inf4;
-    }
-}
-
-// kx = 0 and kx = pi rows of the diamagnetic term (cond_opt.cpp:3993-4173); block b:
-// row l = (b < nk ? 0 : nk-1), m = b % nk
-template <typename SelfT>
-__global__ void k_kx0_rows(const double* __restrict__ ek, const double* __restrict__ d2ek, const SelfT* __restrict__ Self,
-                           const double* __restrict__ Sinf2, const double* __restrict__ Sinf3,
-                           const double* __restrict__ Sinfp, int N, int L, double T, double mu, double* out,
-                           const double* __restrict__ dsc)
-{
-    if (dsc) mu = dsc[kPscMu + 1];
-    __shared__ double sc[16];
-    const int nk = N / 2 + 1;
-    const long nk8 = (long)nk * (nk + 1) / 2;
-    const int l = (blockIdx.x < nk) ? 0 : nk - 1, m = blockIdx.x % nk;
-    const long ki = fold_idx(l, m, N);
-    const double C2 = Sinf2[ki], C3 = Sinf3[ki], Sinf = Sinfp[0];
-    const double e = ek[m + l * nk];
-    const int H = L / 2;
-    cd k0 = cd{0, 0};
-    for (int s = threadIdx.x; s < L; s += blockDim.x) {
-        double kn;
-        const cd Gv = dyson_G(Self, ki, nk8, s, H, C2, C3, Sinf, e, mu, T, kn);
-        const cd G0v = T / cd{-e + mu, kn + Sinf / kn};
-        k0 = k0 + (Gv - G0v);
-    }
-    double kv[2] = {k0.x, k0.y};
-    block_sum_k<2>(kv, sc);
-    k0 = cd{kv[0], kv[1]};
-    if (threadIdx.x == 0) {
-        const Poles P = make_poles(e, mu, Sinf, 0.0, T);
-        const cd f1m = (P.r1.x > 0) ? P.a1 * cexpd(-(P.r1 / T)) / P.den1 : P.a1 / P.den1;
-        const cd f2m = (P.r2.x > 0) ? P.a2 * cexpd(-(P.r2 / T)) / P.den2 : P.a2 / P.den2;
-        const double k0r = k0.x + (f1m + f2m).x;
-        double wt = 2;
-        if (m == 0 || m == nk - 1) wt = wt / 2;
-        out[blockIdx.x] = -2.0 * wt / ((double)N * N) * d2ek[m + l * nk] * k0r;
     }
 }
 
@@ -1894,46 +1358,6 @@ bool supported_Nw(int Nw)
         case 256: { constexpr int NN = 256; __VA_ARGS__; } break; \
         default: return hipErrorInvalidValue;       \
     }
-#define DISPATCH_L(Lv, ...)                           \
-    switch (Lv) {                                     \
-        case 16: { constexpr int LL = 16; __VA_ARGS__; } break;     \
-        case 32: { constexpr int LL = 32; __VA_ARGS__; } break;     \
-        case 64: { constexpr int LL = 64; __VA_ARGS__; } break;     \
-        case 128: { constexpr int LL = 128; __VA_ARGS__; } break;   \
-        case 256: { constexpr int LL = 256; __VA_ARGS__; } break;   \
-        case 512: { constexpr int LL = 512; __VA_ARGS__; } break;   \
-        case 1024: { constexpr int LL = 1024; __VA_ARGS__; } break; \
-        case 2048: { constexpr int LL = 2048; __VA_ARGS__; } break; \
-        case 4096: { constexpr int LL = 4096; __VA_ARGS__; } break; \
-        default: return hipErrorInvalidValue;         \
-    }
-
-#define DISPATCH_LJJ(Lv, ...)                         \
-    switch (Lv) {                                     \
-        case 16: { constexpr int LL = 16; __VA_ARGS__; } break;     \
-        case 32: { constexpr int LL = 32; __VA_ARGS__; } break;     \
-        case 64: { constexpr int LL = 64; __VA_ARGS__; } break;     \
-        case 128: { constexpr int LL = 128; __VA_ARGS__; } break;   \
-        case 256: { constexpr int LL = 256; __VA_ARGS__; } break;   \
-        case 512: { constexpr int LL = 512; __VA_ARGS__; } break;   \
-        case 1024: { constexpr int LL = 1024; __VA_ARGS__; } break; \
-        case 2048: { constexpr int LL = 2048; __VA_ARGS__; } break; \
-        case 4096: { constexpr int LL = 4096; __VA_ARGS__; } break; \
-        default: return hipErrorInvalidValue;         \
-    }
-
-// SS: storage / slab type of the tau and iqn arrays; ST: stored form of Sigma(k,iwn)
-#define DISPATCH_S(prec, ...)     \
-    if (prec) {                   \
-        using SS = float;         \
-        using ST = cf;            \
-        __VA_ARGS__;              \
-    } else {                      \
-        using SS = double;        \
-        using ST = cd;            \
-        __VA_ARGS__;              \
-    }
-
 // the dynamic-LDS limit of a kernel, raised once to the largest size asked for (the attribute
 // holds for the process; each host thread keeps its own record of what it has set)
 template <typename K>
@@ -2210,14 +1634,6 @@ hipError_t launch_hV_slab(const Grid& g, const DevArrays& d, int which, hipStrea
     return hipGetLastError();
 }
 
-hipError_t launch_jj_poles(const Grid& g, const DevArrays& d, double mu, hipStream_t s, const double* dsc)
-{
-    const double dt = jj_threads(g.Nw) / (g.Nw * g.T);  // = NT / (L T) of k_jj_pencil
-    hipLaunchKernelGGL(k_jj_poles, dim3((unsigned)((g.nq + 127) / 128)), dim3(128), 0, s, d.ek, d.hVb, d.Sinf, g.N,
-                       g.T, mu, dt, (JJPoles*)d.poles, dsc);
-    return hipGetLastError();
-}
-
 hipError_t launch_jj_transpose(const Grid& g, const DevArrays& d, hipStream_t s)
 {
     const dim3 gr((unsigned)((g.nq + kTT - 1) / kTT), (unsigned)((g.Nw + 1 + kTT - 1) / kTT), 2);
@@ -2225,20 +1641,6 @@ hipError_t launch_jj_transpose(const Grid& g, const DevArrays& d, hipStream_t s)
         hipLaunchKernelGGL(k_transpose<SS>, gr, dim3(256), 0, s, (const SS*)d.h, (SS*)d.hT, (const SS*)d.f0,
                            (SS*)d.f0T, g.nq, g.Nw + 1);
     });
-    return hipGetLastError();
-}
-
-hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double* part, const int* bins, int ntheta,
-                            hipStream_t s, const double* dsc)
-{
-    const unsigned nblk = (unsigned)((g.nq + jj_points(g.Nw) - 1) / jj_points(g.Nw));
-    DISPATCH_S(g.prec, DISPATCH_LJJ(g.Nw, {
-        constexpr int NTJ = jj_threads(LL);
-        hipLaunchKernelGGL((k_jj_pencil<LL, NTJ, SS, ST>), dim3(nblk), dim3(NTJ), 0, s, d.ek, d.dek,
-                           d.d2ek, (const SS*)d.hT, (const SS*)d.f0T, d.dhV, d.df0V, d.hVb, d.f0Vb,
-                           (const JJPoles*)d.poles, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, g.T, mu, d.twN,
-                           d.twX, d.twS, d.twM, d.ph, part, d.jjscal, bins, ntheta, dsc);
-    }));
     return hipGetLastError();
 }
 
@@ -2302,16 +1704,6 @@ hipError_t launch_sum_rows(const double* part, int nrows, int n, double* out, hi
 {
     if (nrows <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_finalize_k, dim3(nrows), dim3(256), 0, s, part, n, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_kx0_rows(const Grid& g, const DevArrays& d, double mu, hipStream_t s, const double* dsc,
-                           double* out)
-{
-    DISPATCH_S(g.prec, {
-        hipLaunchKernelGGL(k_kx0_rows<ST>, dim3(2 * g.nk), dim3(256), 0, s, d.ek, d.d2ek, (const ST*)d.Self, d.Sinf2,
-                           d.Sinf3, d.Sinf, g.N, g.Nw, g.T, mu, out ? out : d.kx0part, dsc);
-    });
     return hipGetLastError();
 }
 

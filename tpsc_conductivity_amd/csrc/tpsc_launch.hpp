@@ -164,12 +164,16 @@ constexpr int kSRM = kSRK + 2;
 // ... used on grids of at least this many chi0(q,iqn) values (16 MB in FP64): on smaller ones a
 // pass is launch-bound, and the two moment kernels would cost more than the rows they save
 constexpr long kSRMinElems = 2L << 20;
-constexpr int kJJK = 16;  // k-points per Lambda workgroup for Nw > 256
-// Lambda pencil shape: up to Nw = 256 one wavefront per workgroup (its barriers are then free)
-// and 4 points per workgroup, so that small grids still spread over the CUs; beyond, 256
-// threads and kJJK points
-constexpr int jj_points(int Nw) { return Nw <= 256 ? 4 : kJJK; }
-constexpr int jj_threads(int Nw) { return Nw <= 256 ? 64 : 256; }
+// Lambda points per workgroup, and samples of a pencil per thread (512 .. 4096: eight, one wavefront up to 256).
+// About 1024 workgroups: fewer leave CUs idle, more give the column reduction that follows more rows (pencil +
+// reduction at 512, 1024, 2048, 4096 workgroups: 64 batched grids up to 32^2 x 128 together 4.9, 3.9, 3.7, 4.7 ms;
+// 96^2 x 512 -, 48, 54, 73 us; 128^2 x 1024 -, 109, 117, 164 us; 256^2 x 2048 -, 448, 456, 529 us).
+constexpr int jj_points(long nq)
+{
+    const long kp = (nq + 1023) / 1024;
+    return kp > 16 ? 16 : kp < 1 ? 1 : (int)kp;
+}
+constexpr int jj_samples(int Nw) { return Nw > 256 ? 8 : Nw > 64 ? Nw / 64 : 1; }
 
 // ---- launchers; each returns hipGetLastError() of its launch
 hipError_t launch_fill_tw(const DevArrays& d, int L, hipStream_t s);

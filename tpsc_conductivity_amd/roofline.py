@@ -31,6 +31,8 @@ def kernel_bytes(N, Nw, precision="fp64"):
     nk8, nwb, nt, nq = z["nk8"], z["nwb"], z["nt"], z["nq"]
     s, sc = elem_sizes(precision)
     d = 8
+    kp = min(16, max(1, (nq + 1023) // 1024))  # Lambda points per workgroup
+    nblk = (nq + kp - 1) // kp
     return {
         # write chi0(q,tau) and chi0(r,tau) for slices 1..nwb-1
         "chi0_slab": 2 * (nwb - 1) * nk8 * s,
@@ -49,7 +51,7 @@ def kernel_bytes(N, Nw, precision="fp64"):
         # the f0 slices: read V(r,|tau|), write f0V
         "jj_hVf0V_slab": nt * nq * s + nt * nk8 * s,
         # read hV, f0V and (once) Sigma(k,iwn); partial rows out
-        "jj_pencil": 2 * nt * nq * s + (Nw // 2) * nk8 * sc + 2 * ((nq + 15) // 16) * 2 * nwb * d,
+        "jj_pencil": 2 * nt * nq * s + (Nw // 2) * nk8 * sc + nblk * 2 * nwb * d,
         # one sum-rule evaluation: read chi0(q,iqn)
         "sum_rule_eval": nwb * nk8 * d,
         # one Tr(G-G0) evaluation: read Sigma(k,iwn)
