@@ -31,3 +31,26 @@ def test_lambda(N, Nw, oracle_mod):
         bins = g.get(f + "_k").reshape(Nw // 2 + 1, 3)
         assert relerr(bins.sum(axis=1), total[f]) < 1e-13, f
     g.close()
+
+
+@pytest.mark.parametrize("N,Nw", [(4, 256), (8, 512), (12, 512), (4, 1024), (12, 1024), (16, 2048), (8, 4096)])
+def test_tau_pencils(N, Nw, oracle_mod):
+    """chi0, V and what Sigma gives (mu, Tr Sigma G), pencils in pairs: odd and even counts of wedge points"""
+    from tpsc_conductivity_amd.tpsc import CondOpt
+
+    print(f"[pencils] N = {N} Nw = {Nw}", flush=True)
+    o = oracle_mod.Oracle(N, Nw, P["n"], P["T"], P["U"], tp=P["tp"], coarse_pass=False)
+    assert o.solve()
+    g = CondOpt(N, Nw, P["n"], P["T"], params=(P["tp"], 0.0, 0.0, P["U"]), coarse_pass=False)
+    g.solve()
+    assert relerr(g.get("chi0"), o.get("chiqw")) < 1e-10
+    assert relerr(g.get("V"), o.get("V")) < 1e-10
+    s = o.scalars()
+    for k in ("mu", "kx0", "Usp", "Uch"):
+        assert abs(g.scalar(k) - s[k]) < 1e-10 * max(1.0, abs(s[k])), k
+    m = CondOpt(N, Nw, P["n"], P["T"], params=(P["tp"], 0.0, 0.0, P["U"]), coarse_pass=False, precision="mixed")
+    m.solve()
+    for f in ("chi0", "V", "Sigma_kw"):
+        assert relerr(m.get(f), g.get(f)) < 1e-6, f
+    g.close()
+    m.close()

@@ -224,7 +224,8 @@ int dalloc(tpsc_ctx* c, T** ptr, size_t count, size_t elem = 0)
 {
     void* p = nullptr;
     const size_t bytes = (elem ? elem : sizeof(T)) * (count ? count : 1);
-    hipError_t e = hipMalloc(&p, bytes);
+    // one element past the end may be read: the tau pencil kernels load rows in pairs
+    hipError_t e = hipMalloc(&p, bytes + 64);
     if (e != hipSuccess) return fail(c, TPSC_E_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
     c->allocs.push_back(p);
     c->dev_bytes += bytes;
@@ -1489,6 +1490,7 @@ int tpsc_create(const tpsc_params* p, tpsc_ctx** out)
     rc |= dalloc(c, &d.twX, (size_t)Nw);
     rc |= dalloc(c, &d.twS, (size_t)Nw);
     rc |= dalloc(c, &d.twM, (size_t)Nw);
+    rc |= dalloc(c, &d.tw4, (size_t)Nw / 2);
     rc |= dalloc(c, &d.ph, (size_t)Nw + 1);
     rc |= dalloc(c, &d.imax, 4);
     rc |= dalloc(c, &d.mu0v, 1);

@@ -752,7 +752,8 @@ __device__ __forceinline__ void block_spline_fixed(double* const* yM, double h, 
 #pragma unroll
         for (int c = 0; c < C; c++) {
             const int j = j0 + c;
-            const double r = 6.0 * ih * ih * (yv[c + 2] - 2.0 * yv[c + 1] + yv[c]);
+            // from first differences, exact for neighbouring samples: 6/h^2 multiplies their rounding
+            const double r = 6.0 * ih * ih * ((yv[c + 2] - yv[c + 1]) - (yv[c + 1] - yv[c]));
             ri[k][c] = (j >= 1 && j <= N - 1) ? r : 0.0;
             if (trap && j < N) tr[k] += h * (yv[c + 1] + yv[c + 2]) * 0.5;
         }
@@ -1046,6 +1047,21 @@ __device__ __forceinline__ cd sigma_kw(const cf* __restrict__ Self, long o, doub
 {
     const cf v = Self[o];
     return cd{(double)v.x, (double)v.y};
+}
+
+// Point scalars formed on the device by the queued solve (tpsc_capi.cpp) where the host passes
+// them by value otherwise, with the host's rounding (no contraction into fused multiply-adds):
+// U (3 Usp + Uch) / div, and the charge sum rule's constant part
+// A0 - (nsr + Usp nsr^2 / (2U) - nsr^2), A0 = n - n^2/2 (chi.cpp:830-843).
+__device__ __forceinline__ double vfact(double U, double Usp, double Uch, double div)
+{
+#pragma clang fp contract(off)
+    return U * (3.0 * Usp + Uch) / div;
+}
+__device__ __forceinline__ double uch_a0(double A0, double nsr, double U, double Usp)
+{
+#pragma clang fp contract(off)
+    return A0 - (nsr + Usp * nsr * nsr / (2.0 * U) - nsr * nsr);
 }
 
 }  // namespace tpsc

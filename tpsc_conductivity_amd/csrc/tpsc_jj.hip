@@ -144,8 +144,10 @@ __global__ void k_jj_poles(const double* __restrict__ ek, const double* __restri
 //       Gn + i conj Jn at tau_j is real for each, G(tau_j) + i J(tau_j) before the two-pole terms.
 // Everything after the products -G(tau) G(-tau) and G(tau) J(-tau) is linear in them: the spline
 // over [0, beta], its integral and the third transform.  The weighted products and end slopes
-// are therefore summed over the points of a bin (thread j's own samples, in registers), and the
-// spline and the transform follow once per bin and workgroup instead of once per point.
+// are therefore summed over the points of a bin, and the spline and the transform follow once per
+// bin and workgroup instead of once per point.  The sums of up to 16 points carry their
+// rounding along (add_lo), since the spline divides second differences by h^2; up to L = 256 that
+// factor is small and plain sums do.
 // The bubble samples are symmetric about beta/2 (the product is the same in both orders), so
 // the clamped spline over [0, beta] with end slopes (dchi, -dchi) is, on [0, beta/2], the
 // reference's spline with slopes (dchi, 0), and its integral is twice that of the half.
@@ -257,16 +259,28 @@ __device__ __forceinline__ void jj_poles_add(cd* v, const JJPoles& pp, double t0
     for (int m = 0; m < M; m++) v[m] = cell[m * stride];
 }
 
-// Lambda rows at i w_n, n >= 1, from the packed transform of the two moment sequences (Fn at n, Fq at L - n)
-__device__ __forceinline__ void jj_rows(double* c1, double* c2, int n, cd Fn, cd Fq, cd tm, double MJ1, double MJ3,
-                                        double dchi, double w1)
+// Lambda rows at i w_n, n >= 1, from the packed transform of the two splines' moments (Fn at n, Fq at L - n).  Summed by
+// parts, with phi = 2 pi n/L and C'_n the transform with half weights at both ends,
+//   (1 - e^{-i phi}) sum_j 6a_j e^{-i phi j} = -(4 sin^2(phi/2)/h) C'_n + i (sin phi/h) (M_L - M_0),
+// whose explicit small factor keeps the rounding of the transform out of the low frequencies.  x = exp(i phi/2), w1 =
+// 2 pi T, ih = 1/h.
+__device__ __forceinline__ void jj_rows(double* c1, double* c2, int n, cd Fn, cd Fq, cd x, double MJ1, double MJ3,
+                                        double dchi, double w1, double ih)
 {
     const double iw = rcp_nr(n * w1), iw2 = iw * iw;
-    const cd a = tm * cd{0.5 * (Fn.x + Fq.x), 0.5 * (Fn.y - Fq.y)};
-    const cd b = tm * cd{0.5 * (Fn.y + Fq.y), -0.5 * (Fn.x - Fq.x)};
+    const double s2 = 2.0 * x.y * ih, u = s2 * x.y;  // 4 sin^2(phi/2)/(2h): the halves of the split of F
+    const double ay = -u * (Fn.y - Fq.y) - s2 * x.x * MJ3, bx = -u * (Fn.y + Fq.y);
     // -2 MJ1/wn + 2 MJ3/wn^3 + 2 a/wn^4, then / wn
-    c2[n] = -((-2.0 * MJ1 + (2.0 * MJ3 + 2.0 * a.y * iw) * iw2) * iw) * iw;
-    c1[n] = -((-2.0 * dchi + b.x * iw2) * iw2);
+    c2[n] = -((-2.0 * MJ1 + (2.0 * MJ3 + 2.0 * ay * iw) * iw2) * iw) * iw;
+    c1[n] = -((-2.0 * dchi + bx * iw2) * iw2);
+}
+
+// hi += p, the rounding of the sum added to lo
+__device__ __forceinline__ void add_lo(double& hi, float& lo, double p)
+{
+    const double s = hi + p, b = s - hi;
+    lo += (float)((hi - (s - b)) + (p - b));
+    hi = s;
 }
 
 #ifndef JJ_OCC
@@ -279,8 +293,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
                 const double* __restrict__ df0V, const double* __restrict__ hVb, const double* __restrict__ f0Vb,
                 const JJPoles* __restrict__ poles, const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
                 const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, PenStep g, JJScale u, double mu,
-                const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS,
-                const cd* __restrict__ twM, double* part, double* scal, const int* __restrict__ bins, int ntheta,
+                const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS, double* part, double* scal, const int* __restrict__ bins, int ntheta,
                 int kp, const double* __restrict__ dsc)
 {
     if (dsc) mu = dsc[kPscMu + 1];
@@ -288,7 +301,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
     constexpr int NT = P8::NT, W = P8::W, PS = P8::PS, H = L / 2, NWB = H + 1;
     __shared__ __align__(16) cd Z[P8::ZD / 2];
     __shared__ double aM[L];
-    __shared__ double sx[4 * W];   // spline carries
+    __shared__ double sx[6 * W];   // spline carries
     __shared__ double ends[4];     // end moments of the two splines
     __shared__ double sc[4 * W];   // wavefront sums
     __shared__ double tot[4];      // thread 0's sums over the points: end slopes and sample L of the Maki-Thompson
@@ -308,10 +321,17 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
         // sums of the products at j = beta + NT m: bubble (j <= L/2) in registers, Maki-Thompson in the thread's
         // own LDS cells
         double aB[4], aH = 0.0, aq = 0.0;
+        float lM[8], lB[4];
 #pragma unroll
-        for (int m = 0; m < 8; m++) aM[m * NT + tid] = 0.0;
+        for (int m = 0; m < 8; m++) {
+            aM[m * NT + tid] = 0.0;
+            lM[m] = 0.0f;
+        }
 #pragma unroll
-        for (int m = 0; m < 4; m++) aB[m] = 0.0;
+        for (int m = 0; m < 4; m++) {
+            aB[m] = 0.0;
+            lB[m] = 0.0f;
+        }
         if (tid == 0) tot[0] = tot[1] = tot[2] = tot[3] = 0.0;
         bool any = false;
         // the workgroups resident on one XCD (consecutive blk) work on consecutive q at the same time and
@@ -453,7 +473,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
             for (int m = 4; m < 8; m++) gz[2 * PS * pen_row<L>(t) + pen_o<L>(t) + (NT / 8) * m] = v[m].x;
             __syncthreads();
 #pragma unroll
-            for (int m = 0; m < 8; m++) aM[m * NT + t] += wv * (v[m].x * v[m].y);
+            for (int m = 0; m < 8; m++) add_lo(aM[m * NT + t], lM[m], wv * (v[m].x * v[m].y));
             const int rb = NT - beta;  // L - j = rb + NT (7 - m); for beta = 0 the next row up
             const double* const gr = gz + 2 * PS * (rb & 7) + (rb >> 3);
 #pragma unroll
@@ -462,7 +482,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
                 const double gm = z0 ? 0.0 : gr[(NT / 8) * (7 - m)];
                 // at tau = 0: G(0-) = G(0+) + 1
                 const double x = z0 ? -(v[m].x + 1.0) : gm;
-                aB[m] -= wb * (v[m].x * x);
+                add_lo(aB[m], lB[m], -wb * (v[m].x * x));
             }
             if (t == 0) {
                 aH -= wb * (v[4].x * v[4].x);
@@ -496,18 +516,28 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
         double* const Y1 = (double*)Z;
         double* const Y2 = Y1 + P8::YS;
         __syncthreads();
+        float* const l1 = (float*)aM;  // the low-order parts, once the sums are read
+        float* const l2 = l1 + L;
+        double am[8];
+#pragma unroll
+        for (int m = 0; m < 8; m++) am[m] = aM[m * NT + t];
+        __syncthreads();
 #pragma unroll
         for (int m = 0; m < 8; m++) {
             const int j = beta + NT * m;
-            Y1[j + (j >> 3)] = aM[m * NT + t];
+            Y1[j + (j >> 3)] = am[m];
+            l1[j] = lM[m];
             if (m < 4) {
                 Y2[j + (j >> 3)] = aB[m];
                 Y2[(L - j) + ((L - j) >> 3)] = aB[m];
+                l2[j] = lB[m];
+                if (j > 0) l2[L - j] = lB[m];
             }
         }
         if (t == 0) {
             Y1[9 * NT] = tot[2];
             Y2[H + H / 8] = aH;
+            l2[H] = 0.0f;
         }
         __syncthreads();
         const double MJ1 = Y1[0] - Y1[9 * NT], dchi = tot[3];
@@ -515,22 +545,28 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
         double bsum;
         {
             double y[2][10], M[2][9], integ[2];
+            float yl[2][10];
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 const double* const Y = (k == 0 ? Y1 : Y2) + 9 * t;
+                const float* const l = (k == 0 ? l1 : l2) + 8 * t;
+                yl[k][0] = (t > 0) ? l[-1] : 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; i++) yl[k][1 + i] = l[i];
+                yl[k][9] = (t < NT - 1) ? l[8] : (k == 0) ? 0.0f : l2[0];
                 y[k][0] = (t > 0) ? Y[-2] : 0.0;
 #pragma unroll
                 for (int i = 0; i < 8; i++) y[k][1 + i] = Y[i];
                 y[k][9] = Y[9];
             }
             const double d0[2] = {tot[0], dchi}, dN[2] = {tot[1], -dchi};
-            pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, integ, t);
+            pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, integ, t, yl);
             bsum = integ[1];
             if (t == 0) ends[0] = M[0][0];
             if (t == NT - 1) ends[1] = M[0][8];
 #pragma unroll
             for (int i = 0; i < 8; i++)
-                v[i] = cd{(M[0][i + 1] - M[0][i]) * g.ih, (M[1][i + 1] - M[1][i]) * g.ih};
+                v[i] = cd{M[0][i], M[1][i]};
         }
         bsum = wave_total63(bsum);
         aq = wave_total63(aq);
@@ -544,7 +580,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
         for (int m = 0; m < 4; m++) Z[m * PS + t] = v[4 + m];
         __syncthreads();
         const double MJ3 = ends[0] - ends[1];
-        auto row_n = [&](int n, cd Fn, cd Fq) { jj_rows(c1, c2, n, Fn, Fq, twM[n], MJ1, MJ3, dchi, 2.0 * u.piT); };
+        auto row_n = [&](int n, cd Fn, cd Fq) { jj_rows(c1, c2, n, Fn, Fq, twX[n], MJ1, MJ3, dchi, 2.0 * u.piT, g.ih); };
         // L - n = NT - t + NT (7 - m); for t = 0 the next row's first column
         const cd* const zq = Z + NT - t + (t == 0 ? 1 : 0);
 #pragma unroll
@@ -591,7 +627,7 @@ __global__ void __launch_bounds__(64)
                       const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
                       const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, double T, double mu,
                       const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS,
-                      const cd* __restrict__ twM, const cd* __restrict__ phT, double* part, double* scal,
+                      const cd* __restrict__ phT, double* part, double* scal,
                       const int* __restrict__ bins, int ntheta, int kp, const double* __restrict__ dsc)
 {
     if (dsc) mu = dsc[kPscMu + 1];
@@ -737,7 +773,7 @@ __global__ void __launch_bounds__(64)
         }
         const double MJ3 = Y1[0] - Y1[L];
         const double bub0 = wave_sum(integ[1]), q0 = 2.0 * iT * wave_sum(aq);
-        for (int j = tid; j < L; j += NT) X[j] = cd{(Y1[j + 1] - Y1[j]) * ihstep, (Y2[j + 1] - Y2[j]) * ihstep};
+        for (int j = tid; j < L; j += NT) X[j] = cd{Y1[j], Y2[j]};
         __syncthreads();
         block_fft_pp<L, NT>(X, Wk, -1, tw);
         for (int n = tid; n <= H; n += NT) {
@@ -745,7 +781,7 @@ __global__ void __launch_bounds__(64)
                 c1[0] = -bub0;
                 c2[0] = -q0;
             } else {
-                jj_rows(c1, c2, n, X[n], X[L - n], twM[n], MJ1, MJ3, dchi, 2.0 * kPi * T);
+                jj_rows(c1, c2, n, X[n], X[L - n], twX[n], MJ1, MJ3, dchi, 2.0 * kPi * T, ihstep);
             }
         }
         inf1 += 2.0 * dchi;
@@ -821,12 +857,12 @@ hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double
             DISPATCH_L_SHORT(g.Nw, hipLaunchKernelGGL((k_jj_pencil_short<LL, SS, ST>), dim3(nblk), dim3(64), 0, s,
                              d.ek, d.dek, d.d2ek, (const SS*)d.hT, (const SS*)d.f0T, d.dhV, d.df0V, d.hVb, d.f0Vb,
                              (const JJPoles*)d.poles, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, g.T, mu,
-                             d.twN, d.twX, d.twS, d.twM, d.ph, part, d.jjscal, bins, ntheta, kp, dsc));
+                             d.twN, d.twX, d.twS, d.ph, part, d.jjscal, bins, ntheta, kp, dsc));
         } else {
             DISPATCH_L_LONG(g.Nw, hipLaunchKernelGGL((k_jj_pencil<LL, SS, ST>), dim3(nblk), dim3(Pen<LL>::NT), 0, s,
                             d.ek, d.dek, d.d2ek, (const SS*)d.hT, (const SS*)d.f0T, d.dhV, d.df0V, d.hVb, d.f0Vb,
                             (const JJPoles*)d.poles, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, step, sc, mu,
-                            d.twN, d.twX, d.twS, d.twM, part, d.jjscal, bins, ntheta, kp, dsc));
+                            d.twN, d.twX, d.twS, part, d.jjscal, bins, ntheta, kp, dsc));
         }
     });
     return hipGetLastError();

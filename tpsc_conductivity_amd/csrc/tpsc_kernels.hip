@@ -2,7 +2,7 @@
 //
 // Stage map (tpsc_jj.hip holds the Lambda pencils; reference = dbergeron1/TPSC_conductivity):
 //   k_chi0_tau0, k_chi0_slab     chi0.cpp:310-559   G0(k,+-tau) -> G(r,+-tau) -> chi0(r,tau) -> chi0(q,tau)
-//   k_chi0_pencil                chi0.cpp:566-698   clamped spline in tau + DFT -> chi0(q,iqn), tails
+
 //   k_sum_rule                   chi.cpp:738-830    sum-rule traces (one candidate U per launch)
 //   k_mu0_root                   green0.cpp:182-203, 240-262 finite-lattice density and the mu0 root
 //   k_vertex_slab/_pencil        chi.cpp:85-170     V(r,tau)
@@ -29,7 +29,6 @@ namespace tpsc {
 // each at N = 256) share a CU within 96 VGPRs; an FP64 slab (151 KB) runs alone, within 168
 template <typename S>
 constexpr int slab_occ() { return sizeof(S) == sizeof(float) ? 5 : 1; }
-#define PEN_THREADS 256
 
 // ================================================================== small helpers
 __global__ void k_fill_tw(cd* tw, int L)
@@ -70,21 +69,6 @@ __global__ void k_finalize_k(const double* __restrict__ part, int n, double* out
 // chi0max != nullptr (the Usp search): the bracket is (0, 2/chi0max - 2 eps) from the device
 // maximum of chi0, with the start s0.x kept when it lies inside and the midpoint otherwise, so
 // that the host need not wait for chi0max before the first pass
-// Point scalars formed on the device by the queued solve (tpsc_capi.cpp) where the host passes
-// them by value otherwise, with the host's rounding (no contraction into fused multiply-adds):
-// U (3 Usp + Uch) / div, and the charge sum rule's constant part
-// A0 - (nsr + Usp nsr^2 / (2U) - nsr^2), A0 = n - n^2/2 (chi.cpp:830-843).
-__device__ __forceinline__ double vfact(double U, double Usp, double Uch, double div)
-{
-#pragma clang fp contract(off)
-    return U * (3.0 * Usp + Uch) / div;
-}
-__device__ __forceinline__ double uch_a0(double A0, double nsr, double U, double Usp)
-{
-#pragma clang fp contract(off)
-    return A0 - (nsr + Usp * nsr * nsr / (2.0 * U) - nsr * nsr);
-}
-
 // a0src (device Usp, may be null): a0 = uch_a0(a0A, nsr, U, *a0src); mu0p (may be null): the
 // state's mu0 from the device
 __global__ void k_halley_init(HalleyState* st, HalleyState s0, const double* chi0max, double* mirror,
@@ -267,78 +251,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     each_wedge<N>(wt, [&](int a, int, int i) { cq[i] = slab[a]; });
 }
 
-// ================================================================== chi0 pencils
-// chi0.cpp:586-698: per wedge q, clamped spline of chi0(q,tau_j), j=0..Nw/2, slopes
-// (dchiqt0[q], 0); F = BACKWARD DFT_Nw of the antisymmetrised 6a_j; tails.
-// Reads chi0(q,tau) from chit, writes chi0(q,iqn) to chiw in FP64 (chiw may alias chit in
-// the FP64 path: each block reads its column completely before writing it).
-template <int L, typename S>
-__global__ void __launch_bounds__(PEN_THREADS)
-    k_chi0_pencil(const S* chit, double* chiw, const double* __restrict__ dchiqt0, double* chi0inf,
-                  double* chi0inf2, long nk8, double T, const cd* __restrict__ tw)
-{
-    constexpr int NS = L / 2;  // intervals
-    constexpr int PJ = (NS + PEN_THREADS - 1) / PEN_THREADS;  // intervals per thread
-    // The spline samples, then in place their moments (NS + 1 doubles), live in the FFT buffer
-    // until the transform input is formed: 36 KB of LDS per workgroup, four per CU.
-    static_assert(NS + 1 <= 2 * L, "the spline array fits in the transform buffer");
-    __shared__ cd X[L];
-    __shared__ double ES[2 * PEN_THREADS + 8];
-    __shared__ double sc[16];
-    const long q = xcd_remap(blockIdx.x, gridDim.x);
-    if (q >= nk8) return;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    double* y = (double*)X;
-    for (int j = tid; j <= NS; j += nt) y[j] = (double)chit[q + (long)j * nk8];
-    const double d0 = dchiqt0[q], dN = 0.0;
-    const double h = 1.0 / (L * T);
-    __syncthreads();
-    // y -> moments M in place; integ: this thread's part of the spline's integral
-    double integ = 0.0, a6v[PJ];
-    {
-        double* const ys[1] = {y};
-        block_spline_fixed<NS, PEN_THREADS, 1>(ys, h, &d0, &dN, ES, &integ);
-    }
-    const double* M = y;
-#pragma unroll
-    for (int c = 0; c < PJ; c++) {
-        const int j = tid + c * nt;
-        a6v[c] = (j < NS) ? (M[j + 1] - M[j]) / h : 0.0;
-    }
-    __syncthreads();  // every read of y and M is done: X may be written
-#pragma unroll
-    for (int c = 0; c < PJ; c++) {
-        const int j = tid + c * nt;
-        if (j < NS) {
-            X[j] = cd{a6v[c], 0.0};
-            X[L - 1 - j] = cd{-a6v[c], 0.0};
-        }
-    }
-    integ = block_sum(integ, sc);
-    block_fft<L, PEN_THREADS>(X, +1, tw);
-    if (tid == 0) chiw[q] = 2 * integ;
-    if (q != 0) {
-        const double inf = -2.0 * d0;
-        for (int j = 1 + tid; j <= NS; j += nt) {
-            const double wn = 2 * j * kPi * T;
-            // cos, sin of 2 pi j / L from the twiddle table tw[j] = exp(-2 pi i j / L)
-            const cd e = tw[j];
-            chiw[q + (long)j * nk8] =
-                inf / (wn * wn) + ((1.0 - e.x) * X[j].x - e.y * X[j].y) / (wn * wn * wn * wn);
-        }
-        if (tid == 0) {
-            chi0inf[q] = inf;
-            chi0inf2[q] = 2.0 * X[NS].x;
-        }
-    } else {
-        for (int j = 1 + tid; j <= NS; j += nt) chiw[(long)j * nk8] = 0.0;
-        if (tid == 0) {
-            chi0inf[0] = 0.0;
-            chi0inf2[0] = 0.0;
-        }
-    }
-}
-
+// ================================================================== chi0 maximum
 // chi0max and its wedge position (chi0.cpp:703-717): largest value, ties to the
 // larger packed index (the reference scans l, m downwards with a strict >).
 // out2 (may be null): a second copy of the maximum
@@ -709,47 +622,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     each_wedge<N>(wt, [&](int a, int, int i) { V[i + j * nk8] = slab[a]; });
 }
 
-// chi.cpp:123-170: REDFT00 over n (length Nw/2+1) for two wedge points per block, as one
-// complex FFT of length Nw of the even extensions; then V += fact * chi0(r,tau)
-template <int L, typename S>
-__global__ void __launch_bounds__(PEN_THREADS)
-    k_vertex_pencil(S* V, const S* __restrict__ chirt, const double* __restrict__ chirt0, double* V0, long nk8,
-                    double fact, const cd* __restrict__ tw, double U, const double* __restrict__ dsc)
-{
-    if (dsc) fact = vfact(U, dsc[kPscUsp + 1], dsc[kPscUch + 1], 8.0);
-    constexpr int H = L / 2;
-    __shared__ cd X[L];
-    const long q = 2 * (long)xcd_remap(blockIdx.x, gridDim.x);
-    if (q >= nk8) return;
-    const bool two = (q + 1) < nk8;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int j = tid; j <= H; j += nt) {
-        const double a = (double)V[q + (long)j * nk8];
-        const double b = two ? (double)V[q + 1 + (long)j * nk8] : 0.0;
-        X[j] = cd{a, b};
-        if (j > 0 && j < H) X[L - j] = cd{a, b};
-    }
-    __syncthreads();
-    block_fft<L, PEN_THREADS>(X, -1, tw);
-    for (int j = tid; j <= H; j += nt) {
-        const long o = q + (long)j * nk8;
-        V[o] = (S)(X[j].x + fact * (double)chirt[o]);
-        if (two) V[o + 1] = (S)(X[j].y + fact * (double)chirt[o + 1]);
-    }
-    if (tid == 0) {  // tau = 0 in FP64 for the boundary kernels
-        V0[q] = X[0].x + fact * chirt0[q];
-        if (two) V0[q + 1] = X[0].y + fact * chirt0[q + 1];
-    }
-}
-
 // ================================================================== self-energy
-__device__ __forceinline__ void store_self(cd* Self, long o, cd R, double, double, double, double) { Self[o] = R; }
-__device__ __forceinline__ void store_self(cf* Self, long o, cd R, double Sinf, double s2, double s3, double wn)
-{
-    const cd v = sigma_mom(Sinf, s2, s3, R, wn);
-    Self[o] = cf{(float)v.x, (float)v.y};
-}
-
 // Sigma_inf = -(Sigma(k=0,0) + Sigma(k=0,beta)) (green.cpp:1996); one thread
 // Boundary data of Sigma(k,tau) in FP64, block b: side = b % 2 (0: tau = 0, 1: tau = beta),
 // pass = b / 2: the slope dSigma/dtau (pass 0, green.cpp:1743-1817) or the value
@@ -826,62 +699,13 @@ __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     each_wedge<N>(wt, [&](int a, int, int i) { o[i] = slab[a]; });
 }
 
-// green.cpp:1925-2018: per wedge k, spline of Sigma(k,tau_j) (j=0..Nw) with slopes dSig,
-// F = BACKWARD DFT[exp(i pi j/Nw) 6a_j], R(k,n) = (1 - exp(i pi (2n+1)/Nw)) F_n
-// threads of the self-energy pencil: 512 for the long transforms of the mixed path, which
-// stores the assembled FP32 Sigma(k,iwn) (at Nw = 2048: 0.59 against 0.63 ms at 256); 256 in
-// FP64, which stores the remainder (0.48 against 0.57 ms at 512)
-template <typename SelfT>
-constexpr int sigma_pen_threads(int L) { return (L >= 1024 && sizeof(SelfT) == sizeof(cf)) ? 512 : PEN_THREADS; }
-template <int L, typename S, typename SelfT, int NT = sigma_pen_threads<SelfT>(L)>
-__global__ void __launch_bounds__(NT)
-    k_sigma_pencil(const S* __restrict__ Stau, const double* __restrict__ Sb, const double* __restrict__ dSig,
-                   long nk8, double T, SelfT* Self,
-                   double* Sinf2, double* Sinf3, double* Sinf4, double* Sinfp,
-                   const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS)
-{
-    __shared__ double y[L + 1];  // the samples, then in place their spline moments
-    __shared__ cd X[L];
-    __shared__ double ES[2 * NT + 8];
-    const long k = xcd_remap(blockIdx.x, gridDim.x);
-    if (k >= nk8) return;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int j = tid; j <= L; j += nt)
-        y[j] = (j == 0) ? Sb[k] : (j == L) ? Sb[nk8 + k] : (double)Stau[k + (long)j * nk8];
-    const double d0 = dSig[k], dN = dSig[k + nk8];
-    const double h = 1.0 / (L * T);
-    __syncthreads();
-    {
-        double* const ys[1] = {y};
-        block_spline_fixed<L, NT, 1>(ys, h, &d0, &dN, ES, nullptr);
-    }
-    const double* M = y;
-    for (int j = tid; j < L; j += nt) {
-        const double a6 = (M[j + 1] - M[j]) / h;
-        X[j] = twX[j] * a6;
-    }
-    __syncthreads();
-    block_fft<L, NT>(X, +1, tw);
-    // Sigma_inf = -(Sigma(k=0, 0+) + Sigma(k=0, beta-)) from the boundary values; stored by k = 0
-    const double s2 = d0 + dN, s3 = -(M[0] + M[L]), Si = -(Sb[0] + Sb[nk8]);
-    if (k == 0 && tid == 0) Sinfp[0] = Si;
-    for (int n = tid; n < L / 2; n += nt) {
-        const cd R = twS[n] * X[n];
-        store_self(Self, k * (L / 2) + n, R, Si, s2, s3, (2 * n + 1) * kPi * T);
-        if (n == L / 2 - 1) Sinf4[k] = R.x;
-    }
-    if (tid == 0) {
-        Sinf2[k] = s2;
-        Sinf3[k] = s3;
-    }
-}
-
 // phase tables of the pencil transforms, evaluated from the same double arguments as the
 // reference: twX[j] = exp(i j pi/L) (green.cpp:1957, cond_opt.cpp:3290); twS[j] = 1 -
 // exp(i a_j pi/L) with a_j = 2j+1 (j < L/2) or 2(j-L)+1 (green.cpp:2006,
 // cond_opt.cpp:3305-3310); twM[n] = 1 - exp(-2 n i pi/L) (cond_opt.cpp:3731,3805);
-// ph[j] = exp(i (j pi (L-1))/L) (cond_opt.cpp:3635), ph[L] = exp(i pi (L-1)) (:3693)
-__global__ void k_fill_tables(int L, cd* twX, cd* twS, cd* twM, cd* ph)
+// ph[j] = exp(i (j pi (L-1))/L) (cond_opt.cpp:3635), ph[L] = exp(i pi (L-1)) (:3693);
+// tw4[n] = 4 sin^2((2n+1) pi/(2L)), n < L/2
+__global__ void k_fill_tables(int L, cd* twX, cd* twS, cd* twM, double* tw4, cd* ph)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < L) {
@@ -892,6 +716,10 @@ __global__ void k_fill_tables(int L, cd* twX, cd* twS, cd* twM, cd* ph)
         const cd em = cis(-2 * j * kPi / L);
         twM[j] = cd{1.0 - em.x, -em.y};
         ph[j] = cis((j * kPi * (L - 1)) / L);
+        if (j < L / 2) {
+            const double sh = 2.0 * sin((2 * j + 1) * kPi / (2 * L));
+            tw4[j] = sh * sh;
+        }
     }
     if (j == L) ph[L] = cis(kPi * (L - 1));
 }
@@ -1374,7 +1202,7 @@ static void set_lds(K kern, size_t bytes)
 hipError_t launch_fill_tw(const DevArrays& d, int L, hipStream_t s)
 {
     hipLaunchKernelGGL(k_fill_tw, dim3((L + 255) / 256), dim3(256), 0, s, d.twN, L);
-    hipLaunchKernelGGL(k_fill_tables, dim3((L + 256) / 256), dim3(256), 0, s, L, d.twX, d.twS, d.twM, d.ph);
+    hipLaunchKernelGGL(k_fill_tables, dim3((L + 256) / 256), dim3(256), 0, s, L, d.twX, d.twS, d.twM, d.tw4, d.ph);
     return hipGetLastError();
 }
 
@@ -1402,15 +1230,6 @@ hipError_t launch_chi0_slab(const Grid& g, const DevArrays& d, hipStream_t s)
         set_lds(k_chi0_slab<NN, SS>, lds);
         hipLaunchKernelGGL((k_chi0_slab<NN, SS>), dim3(g.nwb - 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw,
                            d.mu0v, g.T, g.Nw, (SS*)d.chi, (SS*)d.chirt);
-    }));
-    return hipGetLastError();
-}
-
-hipError_t launch_chi0_pencil(const Grid& g, const DevArrays& d, hipStream_t s)
-{
-    DISPATCH_S(g.prec, DISPATCH_L(g.Nw, {
-        hipLaunchKernelGGL((k_chi0_pencil<LL, SS>), dim3((unsigned)g.nk8), dim3(PEN_THREADS), 0, s,
-                           (const SS*)d.chi, d.chiw, d.dchiqt0, d.chi0inf, d.chi0inf2, g.nk8, g.T, d.twN);
     }));
     return hipGetLastError();
 }
@@ -1529,17 +1348,6 @@ hipError_t launch_vertex_slab(const Grid& g, const DevArrays& d, double U, doubl
     return hipGetLastError();
 }
 
-hipError_t launch_vertex_pencil(const Grid& g, const DevArrays& d, double U, double Usp, double Uch, hipStream_t s,
-                                const double* dsc)
-{
-    const double fact = U * (3.0 * Usp + Uch) / 8.0;
-    DISPATCH_S(g.prec, DISPATCH_L(g.Nw, {
-        hipLaunchKernelGGL((k_vertex_pencil<LL, SS>), dim3((unsigned)((g.nk8 + 1) / 2)), dim3(PEN_THREADS), 0, s,
-                           (SS*)d.V, (const SS*)d.chirt, d.chirt0, d.V0, g.nk8, fact, d.twN, U, dsc);
-    }));
-    return hipGetLastError();
-}
-
 hipError_t launch_sigma_bnd(const Grid& g, const DevArrays& d, double mu0, double fact, hipStream_t s,
                             const double* mu0p, double U, const double* dsc)
 {
@@ -1559,16 +1367,6 @@ hipError_t launch_sigma_slab(const Grid& g, const DevArrays& d, double mu0, hipS
         set_lds(k_sigma_slab<NN, SS>, lds);
         hipLaunchKernelGGL((k_sigma_slab<NN, SS>), dim3(g.Nw + 1), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw,
                            (const SS*)d.V, mu0, g.T, g.Nw, (SS*)d.Stau, mu0p);
-    }));
-    return hipGetLastError();
-}
-
-hipError_t launch_sigma_pencil(const Grid& g, const DevArrays& d, hipStream_t s)
-{
-    DISPATCH_S(g.prec, DISPATCH_L(g.Nw, {
-        hipLaunchKernelGGL((k_sigma_pencil<LL, SS, ST>), dim3((unsigned)g.nk8), dim3(sigma_pen_threads<ST>(LL)), 0, s,
-                           (const SS*)d.Stau, d.Sb, d.dSig, g.nk8, g.T, (ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf4, d.Sinf,
-                           d.twN, d.twX, d.twS);
     }));
     return hipGetLastError();
 }

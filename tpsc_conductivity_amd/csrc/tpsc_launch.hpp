@@ -64,6 +64,7 @@ struct DevArrays {
     cd* twX = nullptr;           // Nw   phase tables of the pencil transforms (k_fill_tables)
     cd* twS = nullptr;
     cd* twM = nullptr;
+    double* tw4 = nullptr;       // Nw/2
     cd* ph = nullptr;            // Nw+1
     int* imax = nullptr;         // argmax result
     double* mu0v = nullptr;      // 1  mu0 of the current grid (k_mu0_root), read by the chi0 and h/f0 kernels

@@ -11,29 +11,20 @@
 #pragma once
 #include "tpsc_device.hpp"
 
-#define DISPATCH_L_SHORT(Lv, ...)                     \
-    switch (Lv) {                                     \
-        case 16: { constexpr int LL = 16; __VA_ARGS__; } break;     \
-        case 32: { constexpr int LL = 32; __VA_ARGS__; } break;     \
-        case 64: { constexpr int LL = 64; __VA_ARGS__; } break;     \
-        case 128: { constexpr int LL = 128; __VA_ARGS__; } break;   \
-        case 256: { constexpr int LL = 256; __VA_ARGS__; } break;   \
-        default: return hipErrorInvalidValue;         \
-    }
-#define DISPATCH_L_LONG(Lv, ...)                      \
-    switch (Lv) {                                     \
-        case 512: { constexpr int LL = 512; __VA_ARGS__; } break;   \
-        case 1024: { constexpr int LL = 1024; __VA_ARGS__; } break; \
-        case 2048: { constexpr int LL = 2048; __VA_ARGS__; } break; \
-        case 4096: { constexpr int LL = 4096; __VA_ARGS__; } break; \
-        default: return hipErrorInvalidValue;         \
-    }
-#define DISPATCH_L(Lv, ...)                                              \
-    if ((Lv) <= 256) {                                                   \
-        DISPATCH_L_SHORT(Lv, __VA_ARGS__)                                \
-    } else {                                                             \
-        DISPATCH_L_LONG(Lv, __VA_ARGS__)                                 \
-    }
+#define TPSC_CASE_L(X, ...) case X: { constexpr int LL = X; __VA_ARGS__; } break;
+#define TPSC_LS_256(...)                                                                               \
+    TPSC_CASE_L(16, __VA_ARGS__) TPSC_CASE_L(32, __VA_ARGS__) TPSC_CASE_L(64, __VA_ARGS__)             \
+    TPSC_CASE_L(128, __VA_ARGS__) TPSC_CASE_L(256, __VA_ARGS__)
+#define TPSC_LS_1024(...)                                                                              \
+    TPSC_CASE_L(1024, __VA_ARGS__) TPSC_CASE_L(2048, __VA_ARGS__) TPSC_CASE_L(4096, __VA_ARGS__)
+#define DISPATCH_L_SHORT(Lv, ...) \
+    switch (Lv) { TPSC_LS_256(__VA_ARGS__) default: return hipErrorInvalidValue; }
+#define DISPATCH_L_TO512(Lv, ...) \
+    switch (Lv) { TPSC_LS_256(__VA_ARGS__) TPSC_CASE_L(512, __VA_ARGS__) default: return hipErrorInvalidValue; }
+#define DISPATCH_L_LONG(Lv, ...) \
+    switch (Lv) { TPSC_CASE_L(512, __VA_ARGS__) TPSC_LS_1024(__VA_ARGS__) default: return hipErrorInvalidValue; }
+#define DISPATCH_L_FROM1024(Lv, ...) \
+    switch (Lv) { TPSC_LS_1024(__VA_ARGS__) default: return hipErrorInvalidValue; }
 
 // SS: storage / slab type of the tau and iqn arrays; ST: stored form of Sigma(k,iwn)
 #define DISPATCH_S(prec, ...)     \
@@ -96,15 +87,15 @@ __device__ __forceinline__ int pen_beta(int t)
 
 // Forward DFTs of length NT of the rows of Z, in place of registers: on exit v[m] is output
 // pen_o + (NT/8) m of the thread's row.  The rows must be complete (barrier); every exchange stays in the
-// wavefront's own rows.  tw[t] = exp(-2 pi i t / L).  Stage B: eight points over r of row[l + G1 r];
+// wavefront's own rows.  tw[TS t] = exp(-2 pi i t / L).  Stage B: eight points over r of row[l + G1 r];
 // stage C: eight over r of l = lam + W r; stage D: W over lam.
-template <int L>
+template <int L, int TS = 1>
 __device__ __forceinline__ void pen_rows(cd* v, cd* Z, const cd* __restrict__ tw, int t)
 {
     constexpr int W = Pen<L>::W, G1 = Pen<L>::G1, PS = Pen<L>::PS, M = 8 / W - 1;
     const int lane = t & 63;
     const int l = lane % G1, lam = lane % W, k2 = (lane / W) % 8, xm = k2 & M;
-    const cd b1 = tw[8 * l], b2 = tw[16 * l], b4 = tw[32 * l];
+    const cd b1 = tw[8 * TS * l], b2 = tw[16 * TS * l], b4 = tw[32 * TS * l];
     cd* const row = Z + pen_row<L>(t) * PS;
 #pragma unroll
     for (int r = 0; r < 8; r++) v[r] = row[l + G1 * r];
@@ -119,7 +110,7 @@ __device__ __forceinline__ void pen_rows(cd* v, cd* Z, const cd* __restrict__ tw
     for (int r = 0; r < 8; r++) v[r] = rc[lam + W * (r ^ xm)];
     reg_dft<8>(v);
     if constexpr (W > 1) {
-        twiddle8(v, tw[64 * lam], tw[128 * lam], tw[256 * lam]);
+        twiddle8(v, tw[64 * TS * lam], tw[128 * TS * lam], tw[256 * TS * lam]);
         wave_lds_order();
 #pragma unroll
         for (int k = 0; k < 8; k++) rc[((lam + k) & (W - 1)) + W * (k ^ xm)] = v[k];
@@ -153,18 +144,16 @@ __device__ __forceinline__ void pen_fft_dif(cd* v, cd* Z, const cd* __restrict__
     pen_rows<L>(v, Z, tw, t);
 }
 
-// Forward DFT, v[c] = x[8 t + c] on entry, v[m] = X[t + NT m] on exit, t = the thread.  w1, w2, w4: the
-// factors exp(-2 pi i (t + s)/L) and its powers (s = 0; s = 1/2 for frequencies shifted by one half, the
-// caller then also multiplies x[8 t + c] by exp(-8 pi i t/L)).  Z must be free on entry; its last reads are
-// of columns Z[k PS + .] of the thread's own wavefront.
-template <int L>
-__device__ __forceinline__ void pen_fft_dit(cd* v, cd* Z, const cd* __restrict__ tw, cd w1, cd w2, cd w4, int t)
+// Forward DFT of x, whose element 8 p + c lies at Z[c PS + p] (written before, no barrier yet); on exit v[m] = X[t +
+// NT m], t = the thread.  w1, w2, w4: the factors exp(-2 pi i (t + s)/L) and its powers (s = 0; s = 1/2 for
+// frequencies shifted by one half, x[8 p + c] then carries exp(-8 pi i p/L)).  The last reads of Z are of
+// columns Z[k PS + .] of the thread's own wavefront.
+template <int L, int TS = 1>
+__device__ __forceinline__ void pen_fft_placed(cd* v, cd* Z, const cd* __restrict__ tw, cd w1, cd w2, cd w4, int t)
 {
     constexpr int PS = Pen<L>::PS, NT = Pen<L>::NT;
-#pragma unroll
-    for (int c = 0; c < 8; c++) Z[c * PS + t] = v[c];
     __syncthreads();
-    pen_rows<L>(v, Z, tw, t);
+    pen_rows<L, TS>(v, Z, tw, t);
     wave_lds_order();
     // position p of a row is stored at p ^ (8/W (p/8) mod 8): both sides then spread over the banks
     constexpr int X = 8 / Pen<L>::W;
@@ -178,6 +167,15 @@ __device__ __forceinline__ void pen_fft_dit(cd* v, cd* Z, const cd* __restrict__
     for (int c = 0; c < 8; c++) v[c] = Z[c * PS + ts];
     twiddle8(v, w1, w2, w4);
     reg_dft<8>(v);
+}
+// the same for v[c] = x[8 t + c]; Z must be free on entry
+template <int L>
+__device__ __forceinline__ void pen_fft_dit(cd* v, cd* Z, const cd* __restrict__ tw, cd w1, cd w2, cd w4, int t)
+{
+    constexpr int PS = Pen<L>::PS;
+#pragma unroll
+    for (int c = 0; c < 8; c++) Z[c * PS + t] = v[c];
+    pen_fft_placed<L>(v, Z, tw, w1, w2, w4, t);
 }
 
 // x of the lane before (after) in the wavefront, 0 in lane 0 (63)
@@ -253,13 +251,16 @@ struct SplineTab {
 // intervals, and gets the moments M[k][c] = S''(C t + c), c = 0 .. C (M[k][C] is the next thread's first).
 // Both recursions start from zero in each chunk; the state S that enters a chunk adds z^(c+1) S, a
 // chunk's own carries come from the lanes before by D Horner steps, and those of the wavefront before
-// through sx (2 K W doubles) over the one barrier.  The next chunk's first moment needs no exchange:
-// A (z u_(C-1) + S_w).  The boundary modes come from lane 0 of the first and lane 63 of the last wavefront;
+// through sx (3 K W doubles) over the one barrier.  M[k][C] is the next thread's M[k][0] to the last bit (from
+// the next lane, or formed from the same numbers by the same operations at the wavefront's end): the Fourier sums
+// of (M_(j+1) - M_j)/h telescope, and two roundings of one moment would leave L/(2 pi n) times as much noise in them.
+// The second differences are formed from first differences, exact for neighbouring samples (6/h^2 multiplies their
+// rounding); yl (may be null) holds low-order parts of the samples.  The boundary modes come from lane 0 of the first and lane 63 of the last wavefront;
 // their mutual term z^(N-1) is below 1e-290 here.  trap[k] (may be null): the thread's part of the integral.
 template <int N, int NT, int K>
 __device__ __forceinline__ void pen_spline(const double (*y)[N / NT + 2], const PenStep& g, const double* d0, const double* dN,
                                            double (*M)[N / NT + 1], double* sx, const SplineTab<N / NT>& zt,
-                                           double* trap, int tid)
+                                           double* trap, int tid, const float (*yl)[N / NT + 2] = nullptr)
 {
     constexpr int C = N / NT, W = NT / 64;
     static_assert(N >= 512 && N % NT == 0, "long pencils");
@@ -273,7 +274,11 @@ __device__ __forceinline__ void pen_spline(const double (*y)[N / NT + 2], const 
         double* const T = M[k];
         double r[C];
 #pragma unroll
-        for (int c = 0; c < C; c++) r[c] = g.r2 * (y[k][c + 2] - 2.0 * y[k][c + 1] + y[k][c]);
+        for (int c = 0; c < C; c++) {
+            r[c] = (y[k][c + 2] - y[k][c + 1]) - (y[k][c + 1] - y[k][c]);
+            if (yl) r[c] += (double)((yl[k][c + 2] - yl[k][c + 1]) - (yl[k][c + 1] - yl[k][c]));
+            r[c] *= g.r2;
+        }
         r[0] = (tid == 0) ? 0.0 : r[0];
         double s = 0.0;
 #pragma unroll
@@ -297,28 +302,37 @@ __device__ __forceinline__ void pen_spline(const double (*y)[N / NT + 2], const 
         Su[k] = a;
         Sw[k] = b;
         if constexpr (W > 1) {
-            if (lane == 63) sx[(2 * k) * W + wave] = uE[k] + zc * a;
-            if (lane == 0) sx[(2 * k + 1) * W + wave] = s + zc * b;
+            if (lane == 63) sx[(3 * k) * W + wave] = fma(zc, a, uE[k]);
+            if (lane == 0) {
+                sx[(3 * k + 1) * W + wave] = s;
+                sx[(3 * k + 2) * W + wave] = b;
+            }
         }
         __builtin_amdgcn_sched_barrier(0);  // one sequence after the other: fewer registers
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; k++) {
+        double sn = 0.0, bn = 0.0;  // of the next wavefront's first lane
+        const double X = fma(zc, Su[k], uE[k]);
         if constexpr (W > 1) {
-            if (wave > 0) Su[k] += zt[lane] * sx[(2 * k) * W + wave - 1];
-            if (wave < W - 1) Sw[k] += zt[63 - lane] * sx[(2 * k + 1) * W + wave + 1];
+            if (wave > 0) Su[k] += zt[lane] * sx[(3 * k) * W + wave - 1];
+            if (wave < W - 1) {
+                sn = sx[(3 * k + 1) * W + wave + 1];
+                bn = sx[(3 * k + 2) * W + wave + 1];
+                Sw[k] += zt[63 - lane] * fma(zc, bn, sn);
+            }
         }
         double* const m = M[k];
 #pragma unroll
-        for (int c = 0; c < C; c++) m[c] = A * (m[c] + zp.v[c + 1] * Su[k] + zp.v[C - c] * Sw[k]);
-        m[C] = A * (z * (uE[k] + zc * Su[k]) + Sw[k]);
+        for (int c = 0; c < C; c++) m[c] = A * fma(zp.v[C - c], Sw[k], fma(zp.v[c + 1], Su[k], m[c]));
+        m[C] = A * fma(zp.v[C], bn, fma(zp.v[1], X, sn));  // lane 63; the others' follows
         constexpr double idg = 1.0 / (2.0 + z);
         if (wave == 0) {
             const double r0 = g.r1 * ((y[k][2] - y[k][1]) * g.ih - d0[k]);
             const double al = lane_get((r0 - 2.0 * m[0] - m[1]) * idg, 0) * zt[lane];
 #pragma unroll
-            for (int c = 0; c <= C; c++) m[c] += al * zp.v[c];
+            for (int c = 0; c < C; c++) m[c] += al * zp.v[c];
         }
         if (wave == W - 1) {
             const double rN = g.r1 * (dN[k] - (y[k][C + 1] - y[k][C]) * g.ih);
@@ -326,9 +340,10 @@ __device__ __forceinline__ void pen_spline(const double (*y)[N / NT + 2], const 
             const double bz = be * (z * zt[63 - lane]);
 #pragma unroll
             for (int c = 0; c < C; c++) m[c] += bz * zp.v[C - 1 - c];
-            // z^(N - j) one chunk on; 1 at j = N
-            m[C] += be * zt[63 - lane];
+            m[C] += be;  // lane 63: j = N
         }
+        const double mn = lane_shl1(m[0]);
+        m[C] = (lane == 63) ? m[C] : mn;
         if (trap) {
             double sy = 0.0, sm = 0.0;
 #pragma unroll
