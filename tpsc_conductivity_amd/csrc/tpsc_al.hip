@@ -8,18 +8,19 @@
 // Per boson frequency q_n of the sparse set (:5350-6400):
 //   k_al_HG_pencil   HG(q,iq_p) = Gamma(q,iq_p) [hG(p) - hG(p+n)] / [chi0(p) - chi0(p+n)] on the
 //                    window p in [-Nw/2 - n/2, Nw/2 - n/2), to tau with the two-pole tail
-//   k_al_prod_slab   HG(r,tau) G0(r,-tau) and HG(r,beta-tau) G0(r,-tau) back to k, slopes
-//   k_al_k_pencil    splines + shifted fermionic transforms of both products, then the sum
-//                    over k and w_m of v_k G(k,iw_m) G(k,iw_m+iq_n) [HG - HG2]
+//   k_al_prod_slab   HG(r,tau) G0(r,-tau) back to k, slopes
+//   k_al_k_pencil    spline + shifted fermionic transform of the product, then the sum over k and
+//                    w_m of v_k G(k,iw_m) G(k,iw_m+iq_n) [HG - HG2], HG2 the conjugate of HG
+//                    at -w_m
 // Layout: slab-major arrays [tau][q] feed the slab kernels, point-major rows [q][tau] feed the
 // pencils (k_transpose in between); complex tau arrays are two real planes (re, im).
 // Lambda grid q = m + l*nk: kx = (l+1) pi/(nk-1), ky = m pi/(nk-1), nq = nk (nk-2).
 #include "tpsc_launch.hpp"
+#include "tpsc_pencil.hpp"
 
 namespace tpsc {
 
 #define AL_PEN_THREADS 256
-#define AL_K_THREADS 512
 
 // Block j <= Nw: Grt[j*nk8 + w] = G0(r_w, -tau_j) (cond_opt.cpp:4396-4400).  Block Nw+1: dGrt[w] = d/dtau
 // G0(r,-tau) at tau = 0 (x G0(k,0-), :4417-4421) and dGrt[nk8 + w] = eps(r) - mu0 delta_r0 - dGrt[w] at
@@ -166,14 +167,73 @@ __global__ void __launch_bounds__(AL_PEN_THREADS)
 //   (4 D_{j-1} - D_{j-2})/3; Gamma = 3 Usp chi_sp + Uch chi_ch.
 //   HG(q,tau_t) = FORWARD DFT_t [T (HG_j - Hinf_j)] + hg2 tail(tau_t), Hinf the two-pole
 //   asymptote, tail its imaginary-time form; slopes at 0+ and beta-.
-// chiwP: chi0(q,iq_p) point-major [w][p], p <= H.  Writes HGp planes [c][q][t], t <= L, and
-// dHq[(c*2 + side)*nq + q].
+// HG_j is real and the tail real and even about beta/2 (spin poles +-i a: cos(a(beta/2 - tau))/(2a sin(a beta/2)),
+// charge poles +-c: (e^{-c tau} + e^{-c(beta - tau)})/(2c(e^{-c beta} - 1))), so HG(q,beta - tau) = conj HG(q,tau): only
+// t <= H is formed, and everything that the reference builds from HG(beta - tau) is a conjugate.
+// chiwP: chi0(q,iq_p) point-major [w][p], p <= H.  Writes HGp planes [c][q][t], t <= H, and the slope at 0+
+// dHq[c*nq + q] (at beta-: -re, +im).
+struct ALInput {  // one point's T (HG_j - Hinf_j)
+    const double *cw, *hv;
+    double ci, ci2, g2, Usp, Uch, T, tpT;
+    int nn, nc, L;
+    __device__ __forceinline__ double chi0(int p) const
+    {
+        p = abs(p);
+        if (p <= L / 2) return cw[p];
+        const double iw = rcp_nr(tpT * p), iw2 = iw * iw;
+        return (ci + ci2 * iw2) * iw2;
+    }
+    __device__ __forceinline__ double hG(int p) const
+    {
+        p = abs(p);
+        if (p == 0) return hv[0];
+        const double iw = rcp_nr(tpT * p), iw2 = iw * iw;
+        return (-g2 + hv[(p < L / 2) ? p : L / 2 - 1] * iw2) * iw2;
+    }
+    __device__ __forceinline__ int p1(int j) const { return (j < L / 2 - nc) ? j : j - L; }
+    __device__ __forceinline__ double D(int j) const
+    {
+        const int a = p1(j), b = a + nn;
+        return (hG(a) - hG(b)) * rcp_nr(chi0(a) - chi0(b));
+    }
+    // dr accumulates -w_j f_j
+    __device__ __forceinline__ double f(int j, double& dr) const
+    {
+        const int p = p1(j);
+        const double c1 = chi0(p);
+        const double G = 3 * Usp * c1 * rcp_nr(1.0 - Usp * c1 / 2) + Uch * c1 * rcp_nr(1.0 + Uch * c1 / 2);
+        const double Dj = (nn % 2 == 0 && p == -(nn / 2)) ? (4 * D(j - 1) - D(j - 2)) / 3.0 : D(j);
+        const double wn = tpT * p, w2 = wn * wn;
+        const double Hinf = g2 * (3.0 * Usp * rcp_nr(-w2 + 0.5 * Usp * ci) - Uch * rcp_nr(w2 + 0.5 * Uch * ci));
+        const double v = T * (G * Dj - Hinf);
+        dr -= wn * v;
+        return v;
+    }
+};
+// g2 x the tail at tau
+struct ALTail {
+    double a, c, hb, beta, ks, kc;
+    __device__ __forceinline__ ALTail(double Usp, double Uch, double ci, double g2, double T)
+    {
+        beta = 1.0 / T;
+        hb = 0.5 * beta;
+        a = sqrt(0.5 * Usp * ci);
+        c = sqrt(0.5 * Uch * ci);
+        ks = 3.0 * Usp * g2 / (2.0 * a * sin(a * hb));
+        kc = Uch * g2 / (2.0 * c * (exp(-c * beta) - 1.0));
+    }
+    __device__ __forceinline__ double at(double tau) const
+    {
+        return ks * cos(a * (hb - tau)) + kc * (exp(-c * tau) + exp(-c * (beta - tau)));
+    }
+};
+
 template <int L>
 __global__ void __launch_bounds__(AL_PEN_THREADS)
-    k_al_HG_pencil(const double* __restrict__ chiwP, const double* __restrict__ chi0inf,
-                   const double* __restrict__ chi0inf2, const double* __restrict__ hw,
-                   const double* __restrict__ hg2, int N, double T, double Usp, double Uch, long nn,
-                   const cd* __restrict__ tw, double* HGp, double* dHq)
+    k_al_HG_pencil_short(const double* __restrict__ chiwP, const double* __restrict__ chi0inf,
+                         const double* __restrict__ chi0inf2, const double* __restrict__ hw,
+                         const double* __restrict__ hg2, int N, double T, double Usp, double Uch, int nn,
+                         const cd* __restrict__ tw, double* HGp, double* dHq)
 {
     constexpr int NT = AL_PEN_THREADS;
     constexpr int H = L / 2;
@@ -188,96 +248,95 @@ __global__ void __launch_bounds__(AL_PEN_THREADS)
     const long r = fold_idx(l + 1, m, N);
     for (int p = tid; p <= H; p += NT) cw[p] = chiwP[r * (H + 1) + p];
     for (int p = tid; p < H; p += NT) hv[p] = hw[q * H + p];
-    const double ci = chi0inf[r], ci2 = chi0inf2[r], g2 = hg2[q];
-    const int nc = (int)(nn / 2);
-    const double tpT = 2.0 * kPi * T;
+    const ALInput in = {cw, hv, chi0inf[r], chi0inf2[r], hg2[q], Usp, Uch, T, 2.0 * kPi * T, nn, nn / 2, L};
     __syncthreads();
-    auto chi0 = [&](long p) -> double {
-        if (p < 0) p = -p;
-        if (p <= H) return cw[p];
-        const double iw = 1.0 / (tpT * p), iw2 = iw * iw;
-        return (ci + ci2 * iw2) * iw2;
-    };
-    auto hG = [&](long p) -> double {
-        if (p < 0) p = -p;
-        if (p == 0) return hv[0];
-        const double iw = 1.0 / (tpT * p), iw2 = iw * iw;
-        return (-g2 + hv[(p < H) ? p : H - 1] * iw2) * iw2;
-    };
-    auto Dq = [&](int j) -> double {
-        const long p1 = (j < H - nc) ? j : j - L, p2 = p1 + nn;
-        return (hG(p1) - hG(p2)) / (chi0(p1) - chi0(p2));
-    };
-    const double asp = 0.5 * Usp * ci, ach = 0.5 * Uch * ci;
     double dr = 0.0;
-    for (int j = tid; j < L; j += NT) {
-        const long p1 = (j < H - nc) ? j : j - L;
-        const double c1 = chi0(p1);
-        const double G = 3 * Usp * c1 / (1.0 - Usp * c1 / 2) + Uch * c1 / (1.0 + Uch * c1 / 2);
-        const double D = (nn % 2 == 0 && p1 == -(nn / 2)) ? (4 * Dq(j - 1) - Dq(j - 2)) / 3.0 : Dq(j);
-        const double wn = tpT * p1, w2 = wn * wn;
-        const double Hinf = g2 * (3.0 * Usp / (-w2 + asp) + Uch / (-w2 - ach));
-        const double f = T * (G * D - Hinf);
-        X[j] = cd{f, 0.0};
-        dr -= wn * f;
-    }
+    for (int j = tid; j < L; j += NT) X[j] = cd{in.f(j, dr), 0.0};
     const double dtauH0 = block_sum(dr, sc);
     block_fft<L, NT>(X, -1, tw);
-    // two-pole tail: spin poles +-i a, charge poles +-c (cond_opt.cpp:5556-5618)
-    const double beta = 1.0 / T;
-    const double a = sqrt(asp), c = sqrt(ach);
-    const cd zs0 = cd{0.0, a}, zs1 = cd{0.0, -a};
-    const cd es0 = cexpd(cd{0.0, -a * beta}), es1 = cexpd(cd{0.0, a * beta});  // e^{-zs0 beta}, e^{-zs1 beta}
-    const cd A0 = cd{1.0, 0.0} / ((es0 - cd{1.0, 0.0}) * (zs0 - zs1));
-    const cd A1 = cd{1.0, 0.0} / ((es1 - cd{1.0, 0.0}) * (zs1 - zs0));
-    const double ec = exp(-c * beta);
-    const double B0 = 1.0 / ((ec - 1.0) * (2.0 * c)), B1 = 1.0 / ((1.0 - ec) * (-2.0 * c));
-    double* Pr = HGp + q * (L + 1);
-    double* Pi = Pr + nq * (L + 1);
-    for (int t = tid; t < L; t += NT) {
-        const double tau = t / (L * T);
-        const cd tsp = cis(-a * tau) * A0 + cis(a * tau) * A1;
-        const double tch = exp(-c * tau) * B0 + exp(-c * (beta - tau)) * B1;
-        const cd v = X[t] + g2 * (3.0 * Usp * tsp + cd{Uch * tch, 0.0});
-        Pr[t] = v.x;
-        Pi[t] = v.y;
+    const ALTail tail(Usp, Uch, in.ci, in.g2, T);
+    double* Pr = HGp + q * (H + 1);
+    double* Pi = Pr + nq * (H + 1);
+    for (int t = tid; t <= H; t += NT) {
+        Pr[t] = X[t].x + tail.at(t / (L * T));
+        Pi[t] = X[t].y;
     }
     if (tid == 0) {
-        // tau = beta
-        const cd tspb = cd{1.0, 0.0} / ((cd{1.0, 0.0} - es1) * (zs0 - zs1)) +
-                        cd{1.0, 0.0} / ((cd{1.0, 0.0} - es0) * (zs1 - zs0));
-        const double tchb = ec / ((ec - 1.0) * (2.0 * c)) + 1.0 / ((1.0 - ec) * (-2.0 * c));
-        const cd vb = X[0] + g2 * (3.0 * Usp * tspb + cd{Uch * tchb, 0.0});
-        Pr[L] = vb.x;
-        Pi[L] = vb.y;
-        // slopes at 0+ and beta-
-        const cd s0 = -(zs0 * A0) - zs1 * A1;
-        const double c0 = -c * B0 + c * ec * B1;
-        const cd sb = -(zs0 * es0 * A0) - zs1 * es1 * A1;
-        const double cb = -c * ec * B0 + c * B1;
-        const cd d0 = cd{0.0, dtauH0} + g2 * (3.0 * Usp * s0 + cd{Uch * c0, 0.0});
-        const cd dN = cd{0.0, dtauH0} + g2 * (3.0 * Usp * sb + cd{Uch * cb, 0.0});
-        dHq[0 * nq + q] = d0.x;
-        dHq[1 * nq + q] = dN.x;
-        dHq[2 * nq + q] = d0.y;
-        dHq[3 * nq + q] = dN.y;
+        dHq[q] = 0.5 * in.g2 * (3.0 * Usp + Uch);
+        dHq[nq + q] = dtauH0;
     }
 }
 
-// Products of HG(r,tau) with G0(r,-tau), back to k (cond_opt.cpp:5622-5905, 6000-6170).
-// Blocks b < 2(L+1): t = b/2, part c = b%2 (re, im):
-//   S = DST x DCT [HG_c(q,tau_t)/N^2] (q -> r), then
-//   P1_c(k,tau_t)   = DST x DCT [S G0(r,-tau_t)]
-//   P2_c(k,tau_L-t) = DST x DCT [S G0(r,-tau_{L-t})]       (HG2(r,tau) = HG(r,beta-tau))
-// Blocks 2(L+1) + 4 which + 2 side + c: the slopes of P1 (which 0) and P2 (which 1) at
-// tau = 0 / beta from HG(r,tau_b') dG0(r,-tau_b) + dHG(r) G0(r,-tau_b), with
-// dHG2(r,0) = -dHG(r,beta), dHG2(r,beta) = -dHG(r,0).
-// Planes: HGs, P1s, P2s [c][t][q]; dHq [c][side][q]; dP [which][side][c][q].
+// The same for L >= 1024: the DFT of the real HG_j as one of length H = L/2 of z_i = f_2i + i f_2i+1, in registers
+// (tpsc_pencil.hpp): X_t = (Z_t + conj Z_{H-t})/2 - (i/2) e^{-2 pi i t/L} (Z_t - conj Z_{H-t}).
+// What bounds it: FP64 VALU (the ratios).  128^2 x 1024: 47 us a frequency (length-L LDS FFT, all tau: 82).
+template <int L>
+__global__ void __launch_bounds__(L / 16, 3)
+    k_al_HG_pencil(const double* __restrict__ chiwP, const double* __restrict__ chi0inf,
+                   const double* __restrict__ chi0inf2, const double* __restrict__ hw, const double* __restrict__ hg2,
+                   int N, double T, double Usp, double Uch, int nn, const cd* __restrict__ tw, double* HGp, double* dHq)
+{
+    constexpr int H = L / 2, NT = Pen<H>::NT, W = Pen<H>::W, PS = Pen<H>::PS;
+    __shared__ __align__(16) cd Z[Pen<H>::ZD / 2];
+    __shared__ double sc[W];
+    const int nk = N / 2 + 1;
+    const long nq = (long)nk * (nk - 2);
+    const int q = blockIdx.x, t = threadIdx.x;
+    const int l = q / nk, m0 = q - l * nk;
+    const long r = fold_idx(l + 1, m0, N);
+    const ALInput in = {chiwP + r * (H + 1), hw + (long)q * H, chi0inf[r], chi0inf2[r], hg2[q], Usp, Uch, T, 2.0 * kPi * T, nn, nn / 2, L};
+    double dr = 0.0;
+    cd v[8];
+#pragma unroll 1
+    for (int m = 0; m < 8; m++) {  // through the thread's own LDS cells: one copy of the code, few registers
+        const int j = 2 * (t + NT * m);
+        const double f0 = in.f(j, dr), f1 = in.f(j + 1, dr);
+        Z[m * PS + t] = cd{f0, f1};
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int m = 0; m < 8; m++) v[m] = Z[m * PS + t];
+    dr = wave_total63(dr);
+    if ((t & 63) == 63) sc[t >> 6] = dr;
+    pen_fft_dif<H, 2>(v, Z, tw, t);
+    wave_lds_order();
+    // element j at row j mod 8, place j/8: the thread's own cells
+#pragma unroll
+    for (int m = 0; m < 8; m++) Z[PS * pen_row<H>(t) + pen_o<H>(t) + (NT / 8) * m] = v[m];
+    __syncthreads();
+    const ALTail tail(Usp, Uch, in.ci, in.g2, T);
+    double* const Pr = HGp + (long)q * (H + 1);
+    double* const Pi = Pr + nq * (H + 1);
+    auto z = [&](int j) { return Z[(j & 7) * PS + (j >> 3)]; };
+#pragma unroll 1
+    for (int j = t; j <= H; j += NT) {
+        const cd A = z(j & (H - 1)), B = conjg(z((H - j) & (H - 1))), s = A + B, d = tw[j] * (A - B);
+        Pr[j] = 0.5 * (s.x + d.y) + tail.at(j / (L * T));
+        Pi[j] = 0.5 * (s.y - d.x);
+    }
+    if (t == 0) {
+        double d0 = 0.0;
+        for (int i = 0; i < W; i++) d0 += sc[i];
+        dHq[q] = 0.5 * in.g2 * (3.0 * Usp + Uch);
+        dHq[nq + q] = d0;
+    }
+}
+
+// Products of HG(r,tau) with G0(r,-tau), back to k (cond_opt.cpp:5622-5905, 6000-6170).  The reference's second
+// product, HG(r,beta-tau) G0(r,-tau), is the conjugate of the first and is not formed.
+// Blocks b < 2(H+1): t = b/2 <= H, part c = b%2 (re, im):
+//   S = DST x DCT [HG_c(q,tau_t)/N^2] (q -> r), then P_c(k,tau_t) = DST x DCT [S G0(r,-tau_t)] and, from the same
+//   S, P_c(k,tau_L-t) = +-DST x DCT [S G0(r,-tau_{L-t})] (+ re, - im).
+// Blocks 2(H+1) + 2 side + c: the slopes of P at tau = 0 / beta from HG(r,tau_b) dG0(r,-tau_b) + dHG(r) G0(r,-tau_b),
+// with HG(r,beta) = conj HG(r,0) and dHG(r,beta) = -conj dHG(r,0).
+// Planes: HGs [c][t][q], t <= H; Ps [c][t][q], t <= L; dHq [c][q]; dP [side][c][q].
+// What bounds it: latency at 3 to 4 workgroups per CU (128^2: 38 KB of LDS each), so up to 128^2 the registers are
+// capped for four waves per SIMD (108 us against 122 uncapped and 143 for five at 128^2 x 1024; both products and
+// all tau before: 228).
 template <int N>
-__global__ void __launch_bounds__(SlabShape<N>::NT)
+__global__ void __launch_bounds__(SlabShape<N>::NT, (N <= 128 ? 4 : 1))
     k_al_prod_slab(const unsigned* __restrict__ wt, const double* __restrict__ HGs, const double* __restrict__ dHq,
-                   const double* __restrict__ Grt, const double* __restrict__ dGrt, int L, double* P1s, double* P2s,
-                   double* dP)
+                   const double* __restrict__ Grt, const double* __restrict__ dGrt, int L, double* Ps, double* dP)
 {
     constexpr int nk = N / 2 + 1;
     constexpr long nq = (long)nk * (nk - 2);
@@ -288,22 +347,12 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     double* slab = smem;
     cd* tw = slab_tw<N>(slab);
     fill_twiddles<N>(tw);
-    const long plane = (long)(L + 1) * nq;
-    const int b = blockIdx.x;
-    int tA, c, which = 0, side = 0;
-    const bool main_blk = b < 2 * (L + 1);
-    if (main_blk) {
-        tA = b >> 1;
-        c = b & 1;
-    } else {
-        const int bb = b - 2 * (L + 1);
-        which = bb >> 2;
-        side = (bb >> 1) & 1;
-        c = bb & 1;
-        tA = which ? (side ? 0 : L) : (side ? L : 0);
-    }
-    const double* src = HGs + c * plane + (long)tA * nq;
-    each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = nf * src[s]; });
+    const int H = L / 2, b = blockIdx.x, c = b & 1;
+    const bool main_blk = b < 2 * (H + 1);
+    const int t = main_blk ? b >> 1 : 0, side = main_blk ? 0 : (b - 2 * (H + 1)) >> 1;
+    const double* src = HGs + ((long)c * (H + 1) + t) * nq;
+    const double f = (side && c) ? -nf : nf;
+    each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = f * src[s]; });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
     double sa[PER], sb[PER];  // HG(r,tau) at (l, m) and (m, l) of the thread's points
@@ -315,146 +364,221 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
     if (main_blk) {
 #pragma unroll 1
         for (int pass = 0; pass < 2; pass++) {
-            const int tg = pass ? L - tA : tA;
+            if (pass && t == H) break;
+            const int tg = pass ? L - t : t;
             const double* g = Grt + (long)tg * nk8;
+            const double sgn = (pass && c) ? -1.0 : 1.0;
             each_wedge_slot<N>(wt, [&](int o, int p, int w, int i) {
-                slab[o] = sa[i] * g[w];
-                slab[p] = sb[i] * g[w];
+                const double gw = sgn * g[w];
+                slab[o] = sa[i] * gw;
+                slab[p] = sb[i] * gw;
             });
             __syncthreads();
             slab_r2r_2d<double, N, 1>(slab, tw);
-            double* out = (pass ? P2s : P1s) + c * plane + (long)tg * nq;
+            double* out = Ps + ((long)c * (L + 1) + tg) * nq;
             each_lambda<N>([&](int l, int m, int s) { out[s] = slab[at<N>(l + 1, m)]; });
             __syncthreads();
         }
         return;
     }
     const double* dg = dGrt + side * nk8;
-    const int ds = which ? 1 - side : side;
-    const double sgn = which ? -1.0 : 1.0;
-    const double* dsrc = dHq + (long)(c * 2 + ds) * nq;
-    each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = nf * dsrc[s]; });
+    const double* dsrc = dHq + (long)c * nq;
+    const double fd = (side && !c) ? -nf : nf;
+    each_lambda<N>([&](int l, int m, int s) { slab[at<N>(l + 1, m)] = fd * dsrc[s]; });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
     const double* g = Grt + (long)(side ? L : 0) * nk8;
     each_wedge_slot<N>(wt, [&](int o, int p, int w, int i) {
-        const double ra = sgn * slab[o] * g[w] + sa[i] * dg[w], rb = sgn * slab[p] * g[w] + sb[i] * dg[w];
+        const double ra = slab[o] * g[w] + sa[i] * dg[w], rb = slab[p] * g[w] + sb[i] * dg[w];
         slab[o] = ra;
         slab[p] = rb;
     });
     __syncthreads();
     slab_r2r_2d<double, N, 1>(slab, tw);
-    double* out = dP + (long)((which * 2 + side) * 2 + c) * nq;
+    double* out = dP + (long)(side * 2 + c) * nq;
     each_lambda<N>([&](int l, int m, int s) { out[s] = slab[at<N>(l + 1, m)]; });
 }
 
 // Dyson G(k, i w_f) = 1/(i w_f + mu - e - Sigma(k,iw_f)), Sigma from the stored form for
 // |f + 1/2| < H, from its moments beyond, conjugated for f < 0 (cond_opt.cpp:6314-6377)
 template <typename SelfT>
-__device__ __forceinline__ cd al_G(const SelfT* __restrict__ Self, long ki, int H, long f, double C2, double C3,
-                                   double Sinf, double e, double mu, double T)
+__device__ __forceinline__ cd al_G(const SelfT* __restrict__ Self, long ki, int H, int f, double C2, double C3,
+                                   double Sinf, double e0, double piT)
 {
-    const double kn = (2.0 * f + 1) * kPi * T;
-    const long g = (f >= 0) ? f : -f - 1;
-    cd sg = (g < H) ? sigma_kw(Self, ki * H + g, Sinf, C2, C3, fabs(kn)) : sigma_mom(Sinf, C2, C3, cd{0.0, 0.0}, fabs(kn));
-    if (f < 0) sg = conjg(sg);
-    return cd{1.0, 0.0} / (cd{mu - e, kn} - sg);
+    const int g = (f >= 0) ? f : -f - 1;
+    const double kn = (2 * g + 1) * piT;
+    const cd sg = (g < H) ? sigma_kw(Self, ki * H + g, Sinf, C2, C3, kn) : sigma_mom(Sinf, C2, C3, cd{0.0, 0.0}, kn);
+    const cd G = sdiv_rcp(1.0, cd{e0 - sg.x, kn - sg.y});
+    return (f < 0) ? conjg(G) : G;
 }
 
-// Per Lambda point k (cond_opt.cpp:5907-6400): clamped splines of the four real pencils
-// (P1 re/im, P2 re/im) with the slopes dP; HG(k, i w_(f+nn)) from P1 and HG2(k, i w_f) from P2
-// by  -i (z_0 + z_L)/w - (z'_0 + z'_L)/w^2 + i (z''_0 + z''_L)/w^3 + (1 - e^{-i w beta/L}) F/w^4,
-// F = FORWARD DFT of e^{-i pi t/L} 6a_t (re + i im); f = j (j < H - nn/2) or j - L; then
-// contrib[k] = Re[-i U T wt v_k / (N^2 2 qn) sum_j G(f) G(f+nn) (HG_j - HG2_j)].
-template <int L, int NT, typename SelfT>
-__global__ void __launch_bounds__(NT)
-    k_al_k_pencil(const double* __restrict__ P1p, const double* __restrict__ P2p, const double* __restrict__ dP,
-                  const double* __restrict__ ek, const double* __restrict__ dek, const SelfT* __restrict__ Self,
-                  const double* __restrict__ Sinf2, const double* __restrict__ Sinf3, const double* __restrict__ Sinfp,
-                  int N, double T, double mu, double U, long nn, const cd* __restrict__ tw,
-                  const cd* __restrict__ twX, const cd* __restrict__ twS, double* contrib)
+// Per Lambda point k (cond_opt.cpp:5907-6400): clamped splines of P re, im with the slopes dP, and
+//   V(s) = HG(k, i w_s) = -i (z_0 + z_L)/w - (z'_0 + z'_L)/w^2 + i (z''_0 + z''_L)/w^3 + (1 - e^{-i w beta/L}) F_s/w^4,
+// F = FORWARD DFT of e^{-i pi t/L} 6a_t (re + i im).  The second function of the reference, HG2(k, i w_f) from the
+// conjugate of P, is conj V(-f-1), so its sum over the window f = j (j < H - nn/2) or j - L is
+//   sum over s = f + nn of G(s - nn) G(s) [V(s) - conj V(nn - 1 - s)],
+// and the term of nn - 1 - s is minus the conjugate of that of s: contrib[k] = Re[-i U T wt v_k / (N^2 2 qn) sum] takes
+// the upper half, s = nn/2 + i (nn/2 rounded down), twice; for odd nn, i = 0 (its own partner) and i = H (partner
+// outside the window) once.
+struct ALPoint {
+    cd cw, ds, dd;  // z_0 + z_L, slopes, second derivatives
+    double piT;
+    // V(s) from F_s; x = 1 - e^{i w beta/L}
+    __device__ __forceinline__ cd V(int s, cd F, cd x) const
+    {
+        const double iw = rcp_nr((2 * s + 1) * piT), iw2 = iw * iw;
+        return cd{(cw.y - ds.x * iw - dd.y * iw2) * iw, (-cw.x - ds.y * iw + dd.x * iw2) * iw} +
+               (conjg(x) * F) * (iw2 * iw2);
+    }
+};
+
+template <int L, typename SelfT>
+__global__ void __launch_bounds__(AL_PEN_THREADS)
+    k_al_k_pencil_short(const double* __restrict__ Pp, const double* __restrict__ dP, const double* __restrict__ ek,
+                        const double* __restrict__ dek, const SelfT* __restrict__ Self,
+                        const double* __restrict__ Sinf2, const double* __restrict__ Sinf3,
+                        const double* __restrict__ Sinfp, int N, double T, double mu, double U, int nn,
+                        const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS,
+                        double* contrib)
 {
-    constexpr int H = L / 2;
-    __shared__ __align__(16) double Yb[4 * (L + 1)];
+    constexpr int H = L / 2, NT = AL_PEN_THREADS;
+    __shared__ double Yb[2 * (L + 1)];
     __shared__ cd X[L];
-    __shared__ double ES[4 * (2 * NT + 8)];
-    __shared__ double sc[2 * (NT / 64)];
+    __shared__ double ES[2 * (2 * NT + 8)];
+    __shared__ double sc[NT / 64];
     const int nk = N / 2 + 1;
     const long nq = (long)nk * (nk - 2);
-    const long plane = nq * (L + 1);
     const long k = blockIdx.x;
     const int tid = threadIdx.x;
     const int l = (int)(k / nk), m = (int)(k % nk);
     const long ki = fold_idx(l + 1, m, N);
-    const double hstep = 1.0 / (L * T);
-    const int nc = (int)(nn / 2);
-    double* Y[4] = {Yb, Yb + (L + 1), Yb + 2 * (L + 1), Yb + 3 * (L + 1)};
-    const double* rows[4] = {P1p + k * (L + 1), P1p + plane + k * (L + 1), P2p + k * (L + 1),
-                             P2p + plane + k * (L + 1)};
+    const double hstep = 1.0 / (L * T), ih = L * T;
+    const int nc = nn / 2;
+    double* const Y0 = Yb;
+    double* const Y1 = Yb + (L + 1);
+    const double* const row = Pp + k * (L + 1);
     for (int j = tid; j <= L; j += NT) {
-        Y[0][j] = rows[0][j];
-        Y[1][j] = rows[1][j];
-        Y[2][j] = rows[2][j];
-        Y[3][j] = rows[3][j];
+        Y0[j] = row[j];
+        Y1[j] = row[nq * (L + 1) + j];
     }
-    // dP [which][side][c][q]
-    const double d0[4] = {dP[0 * nq + k], dP[1 * nq + k], dP[4 * nq + k], dP[5 * nq + k]};
-    const double dN[4] = {dP[2 * nq + k], dP[3 * nq + k], dP[6 * nq + k], dP[7 * nq + k]};
+    const double d0[2] = {dP[k], dP[nq + k]}, dN[2] = {dP[2 * nq + k], dP[3 * nq + k]};  // dP [side][c][q]
     __syncthreads();
-    const cd cw1 = cd{Y[0][0] + Y[0][L], Y[1][0] + Y[1][L]};
-    const cd cw2 = cd{Y[2][0] + Y[2][L], Y[3][0] + Y[3][L]};
-    block_spline_fixed<L, NT, 4>(Y, hstep, d0, dN, ES, nullptr);
-    const cd dd1 = cd{Y[0][0] + Y[0][L], Y[1][0] + Y[1][L]};  // z''(0) + z''(beta)
-    const cd dd2 = cd{Y[2][0] + Y[2][L], Y[3][0] + Y[3][L]};
-    const cd ds1 = cd{d0[0] + dN[0], d0[1] + dN[1]};
-    const cd ds2 = cd{d0[2] + dN[2], d0[3] + dN[3]};
-    const double ih = 1.0 / hstep;
-    // P1 -> HG(k, i w_(f+nn)), kept in the P1 half of Yb
+    ALPoint p;
+    p.piT = kPi * T;
+    p.cw = cd{Y0[0] + Y0[L], Y1[0] + Y1[L]};
+    p.ds = cd{d0[0] + dN[0], d0[1] + dN[1]};
+    __syncthreads();
+    {
+        double* const ys[2] = {Y0, Y1};
+        block_spline_fixed<L, NT, 2>(ys, hstep, d0, dN, ES, nullptr);
+    }
+    p.dd = cd{Y0[0] + Y0[L], Y1[0] + Y1[L]};
     for (int t = tid; t < L; t += NT)
-        X[t] = conjg(twX[t]) * cd{(Y[0][t + 1] - Y[0][t]) * ih, (Y[1][t + 1] - Y[1][t]) * ih};
+        X[t] = conjg(twX[t]) * cd{(Y0[t + 1] - Y0[t]) * ih, (Y1[t + 1] - Y1[t]) * ih};
     __syncthreads();
     block_fft<L, NT>(X, -1, tw);
-    cd* HGK = (cd*)Yb;
-    for (int j = tid; j < L; j += NT) {
-        const long f = (j < H - nc) ? j : j - L;
-        const long s = f + nn;
-        const double w = (2 * s + 1) * kPi * T;
-        const double iw = 1.0 / w, iw2 = iw * iw;
-        // -i cw/w - ds/w^2 + i dd/w^3
-        cd v = cd{(cw1.y - ds1.x * iw - dd1.y * iw2) * iw, (-cw1.x - ds1.y * iw + dd1.x * iw2) * iw};
-        if (s < L) {
-            const long fi = (s < 0) ? s + L : s;
-            v = v + (conjg(twS[fi]) * X[fi]) * (iw2 * iw2);
-        }
-        HGK[j] = v;
+    const double C2 = Sinf2[ki], C3 = Sinf3[ki], Sinf = Sinfp[0], e0 = mu - ek[m + (l + 1) * nk];
+    double acc = 0.0;
+    for (int i = tid; i <= H; i += NT) {
+        const bool odd = nn & 1;
+        const double w = (i == H) ? (odd ? 1.0 : 0.0) : (odd && i == 0) ? 1.0 : 2.0;
+        if (w == 0.0) continue;
+        const int s = nc + i, s2 = nn - 1 - s;
+        const int a = s & (L - 1), b = s2 & (L - 1);
+        const cd d = p.V(s, X[a], twS[a]) - conjg(p.V(s2, X[b], twS[b]));
+        const cd g = al_G(Self, ki, H, s - nn, C2, C3, Sinf, e0, p.piT) * al_G(Self, ki, H, s, C2, C3, Sinf, e0, p.piT);
+        acc += w * (g.x * d.y + g.y * d.x);
     }
-    __syncthreads();
-    for (int t = tid; t < L; t += NT)
-        X[t] = conjg(twX[t]) * cd{(Y[2][t + 1] - Y[2][t]) * ih, (Y[3][t + 1] - Y[3][t]) * ih};
-    __syncthreads();
-    block_fft<L, NT>(X, -1, tw);
-    const double C2 = Sinf2[ki], C3 = Sinf3[ki], Sinf = Sinfp[0];
-    const double e = ek[m + (l + 1) * nk];
-    double acc[2] = {0.0, 0.0};
-    for (int j = tid; j < L; j += NT) {
-        const long f = (j < H - nc) ? j : j - L;
-        const double w = (2 * f + 1) * kPi * T;
-        const double iw = 1.0 / w, iw2 = iw * iw;
-        const long fi = (f < 0) ? f + L : f;
-        const cd v2 = cd{(cw2.y - ds2.x * iw - dd2.y * iw2) * iw, (-cw2.x - ds2.y * iw + dd2.x * iw2) * iw} +
-                      (conjg(twS[fi]) * X[fi]) * (iw2 * iw2);
-        const cd G1 = al_G(Self, ki, H, f, C2, C3, Sinf, e, mu, T);
-        const cd G2 = al_G(Self, ki, H, f + nn, C2, C3, Sinf, e, mu, T);
-        const cd t = (G1 * G2) * (HGK[j] - v2);
-        acc[0] += t.x;
-        acc[1] += t.y;
-    }
-    block_sum_k<2>(acc, sc);
+    acc = block_sum(acc, sc);
     if (tid == 0) {
         const double wt = (m == 0 || m == nk - 1) ? 2.0 : 4.0;
         const double qn = 2.0 * nn * kPi * T;
-        const double fac = U * T * wt * dek[k] / ((double)N * N * 2.0 * qn);
-        contrib[k] = fac * acc[1];  // Re[-i fac acc]
+        contrib[k] = U * T * wt * dek[k] / ((double)N * N * 2.0 * qn) * acc;
+    }
+}
+
+// The same for L >= 512 in registers (tpsc_pencil.hpp).  128^2 x 1024: 37 us a frequency (four splines,
+// two LDS FFTs, the whole window: 395).
+template <int L, typename SelfT>
+__global__ void __launch_bounds__(Pen<L>::NT, 3)
+    k_al_k_pencil(const double* __restrict__ Pp, const double* __restrict__ dP, const double* __restrict__ ek,
+                  const double* __restrict__ dek, const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
+                  const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, PenStep g, double T,
+                  double mu, double U, int nn, const cd* __restrict__ tw, const cd* __restrict__ twX,
+                  const cd* __restrict__ twS, double* contrib)
+{
+    constexpr int H = L / 2, NT = Pen<L>::NT, W = Pen<L>::W, PS = Pen<L>::PS;
+    __shared__ __align__(16) cd Z[Pen<L>::ZD / 2];
+    __shared__ double sx[6 * W], sc[W], ends[8];
+    __shared__ SplineTab<8> zt;
+    const int nk = N / 2 + 1, nq = nk * (nk - 2);
+    const int k = blockIdx.x, t = threadIdx.x;
+    zt.fill(t);  // ordered by the barrier of the spline
+    const int l = k / nk, m0 = k - l * nk;
+    const long ki = fold_idx(l + 1, m0, N);
+    const int nc = nn / 2;
+    const double d0[2] = {dP[k], dP[nq + k]}, dN[2] = {dP[2 * nq + k], dP[3 * nq + k]};  // dP [side][c][q]
+    cd v[8];
+    {
+        double y[2][10], M[2][9];
+        const double* const r0 = Pp + (long)k * (L + 1) + 8 * t;
+        const double* const r1 = r0 + (long)nq * (L + 1);
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+            y[0][1 + i] = r0[i];
+            y[1][1 + i] = r1[i];
+        }
+        y[0][0] = r0[t > 0 ? -1 : 0];
+        y[1][0] = r1[t > 0 ? -1 : 0];
+        pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, nullptr, t);
+        if (t == 0) {
+            ends[0] = y[0][1];
+            ends[1] = y[1][1];
+            ends[2] = M[0][0];
+            ends[3] = M[1][0];
+        }
+        if (t == NT - 1) {
+            ends[4] = y[0][9];
+            ends[5] = y[1][9];
+            ends[6] = M[0][8];
+            ends[7] = M[1][8];
+        }
+        const cd h = tw[4 * t];  // exp(-8 pi i t / L)
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = h * cd{(M[0][i + 1] - M[0][i]) * g.ih, (M[1][i + 1] - M[1][i]) * g.ih};
+    }
+    pen_fft_dit<L>(v, Z, tw, conjg(twX[2 * t + 1]), tw[2 * t + 1], tw[4 * t + 2], t);
+    wave_lds_order();
+#pragma unroll
+    for (int m = 0; m < 8; m++) Z[m * PS + t] = v[m];  // F_s, s = t + NT m
+    __syncthreads();
+    ALPoint p;
+    p.piT = kPi * T;
+    p.cw = cd{ends[0] + ends[4], ends[1] + ends[5]};
+    p.dd = cd{ends[2] + ends[6], ends[3] + ends[7]};
+    p.ds = cd{d0[0] + dN[0], d0[1] + dN[1]};
+    const double C2 = Sinf2[ki], C3 = Sinf3[ki], Sinf = Sinfp[0], e0 = mu - ek[m0 + (l + 1) * nk];
+    double acc = 0.0;
+    const bool odd = nn & 1;
+    auto F = [&](int s) { return Z[(s / NT) * PS + (s & (NT - 1))]; };
+#pragma unroll 1
+    for (int i = t; i < H + (odd ? 1 : 0); i += NT) {
+        const double w = (odd && (i == 0 || i == H)) ? 1.0 : 2.0;
+        const int s = nc + i, s2 = nn - 1 - s;
+        const int a = s & (L - 1), b = s2 & (L - 1);
+        const cd d = p.V(s, F(a), twS[a]) - conjg(p.V(s2, F(b), twS[b]));
+        const cd gg = al_G(Self, ki, H, s - nn, C2, C3, Sinf, e0, p.piT) * al_G(Self, ki, H, s, C2, C3, Sinf, e0, p.piT);
+        acc += w * (gg.x * d.y + gg.y * d.x);
+    }
+    acc = wave_total63(acc);
+    if ((t & 63) == 63) sc[t >> 6] = acc;
+    __syncthreads();
+    if (t == 0) {
+        double s = 0.0;
+        for (int i = 0; i < W; i++) s += sc[i];
+        const double wt = (m0 == 0 || m0 == nk - 1) ? 2.0 : 4.0;
+        const double qn = 2.0 * nn * kPi * T;
+        contrib[k] = U * T * wt * dek[k] / ((double)N * N * 2.0 * qn) * s;
     }
 }
 
@@ -475,28 +599,15 @@ __global__ void __launch_bounds__(NT)
         case 256: { constexpr int NN = 256; __VA_ARGS__; } break;   \
         default: return hipErrorInvalidValue;                       \
     }
-#define AL_DISPATCH_L(Lv, ...)                                      \
-    switch (Lv) {                                                   \
-        case 16: { constexpr int LL = 16; __VA_ARGS__; } break;     \
-        case 32: { constexpr int LL = 32; __VA_ARGS__; } break;     \
-        case 64: { constexpr int LL = 64; __VA_ARGS__; } break;     \
-        case 128: { constexpr int LL = 128; __VA_ARGS__; } break;   \
-        case 256: { constexpr int LL = 256; __VA_ARGS__; } break;   \
-        case 512: { constexpr int LL = 512; __VA_ARGS__; } break;   \
-        case 1024: { constexpr int LL = 1024; __VA_ARGS__; } break; \
-        case 2048: { constexpr int LL = 2048; __VA_ARGS__; } break; \
-        default: return hipErrorInvalidValue;                       \
-    }
-
-// ST: stored form of Sigma(k,iwn) (FP64 remainder, or the assembled FP32 value in the mixed path)
-#define DISPATCH_AL_SELF(prec, ...) \
-    if (prec) {                     \
-        using ST = cf;              \
-        __VA_ARGS__;                \
-    } else {                        \
-        using ST = cd;              \
-        __VA_ARGS__;                \
-    }
+// Nw <= 2048 (the launchers refuse larger ones)
+#define AL_DISPATCH_HW(Lv, ...) \
+    switch (Lv) { TPSC_LS_256(__VA_ARGS__) TPSC_CASE_L(512, __VA_ARGS__) TPSC_CASE_L(1024, __VA_ARGS__) \
+                  TPSC_CASE_L(2048, __VA_ARGS__) default: return hipErrorInvalidValue; }
+#define AL_DISPATCH_FROM1024(Lv, ...) \
+    switch (Lv) { TPSC_CASE_L(1024, __VA_ARGS__) TPSC_CASE_L(2048, __VA_ARGS__) default: return hipErrorInvalidValue; }
+#define AL_DISPATCH_FROM512(Lv, ...) \
+    switch (Lv) { TPSC_CASE_L(512, __VA_ARGS__) TPSC_CASE_L(1024, __VA_ARGS__) TPSC_CASE_L(2048, __VA_ARGS__) \
+                  default: return hipErrorInvalidValue; }
 
 template <typename K>
 static void al_set_lds(K kern, size_t bytes)
@@ -514,12 +625,12 @@ hipError_t launch_al_setup(const Grid& g, const DevArrays& d, const ALArrays& a,
                            mu0, g.T, g.Nw, a.Grt, a.dGrt);
         al_set_lds(k_al_hg_slab<NN>, lds);
         hipLaunchKernelGGL(k_al_hg_slab<NN>, dim3(g.Nw + 3), dim3(SlabShape<NN>::NT), lds, s, d.wt, d.ekw, d.fw, d.vw,
-                           a.Grt, a.dGrt, mu0, g.T, g.Nw, a.P1s, a.dhG);
+                           a.Grt, a.dGrt, mu0, g.T, g.Nw, a.Ps, a.dhG);
     });
-    hipError_t e = launch_transpose_d(a.P1s, a.P1p, g.nq, g.Nw + 1, s);
+    hipError_t e = launch_transpose_d(a.Ps, a.Pp, g.nq, g.Nw + 1, s);
     if (e != hipSuccess) return e;
-    AL_DISPATCH_L(g.Nw, {
-        hipLaunchKernelGGL(k_al_hw_pencil<LL>, dim3((unsigned)g.nq), dim3(AL_PEN_THREADS), 0, s, a.P1p, a.dhG, g.nq,
+    AL_DISPATCH_HW(g.Nw, {
+        hipLaunchKernelGGL(k_al_hw_pencil<LL>, dim3((unsigned)g.nq), dim3(AL_PEN_THREADS), 0, s, a.Pp, a.dhG, g.nq,
                            g.T, d.twN, d.twM, a.hw, a.hg2);
     });
     // chi0(q,iq_p) point-major for the per-frequency pencils
@@ -527,32 +638,39 @@ hipError_t launch_al_setup(const Grid& g, const DevArrays& d, const ALArrays& a,
 }
 
 hipError_t launch_al_freq(const Grid& g, const DevArrays& d, const ALArrays& a, double Usp, double Uch, double mu,
-                          double U, long nn, double* contrib, hipStream_t s)
+                          double U, long n, double* contrib, hipStream_t s)
 {
-    const long plane = (long)(g.Nw + 1) * g.nq;
-    AL_DISPATCH_L(g.Nw, {
-        hipLaunchKernelGGL(k_al_HG_pencil<LL>, dim3((unsigned)g.nq), dim3(AL_PEN_THREADS), 0, s, a.chiwP, d.chi0inf,
-                           d.chi0inf2, a.hw, a.hg2, g.N, g.T, Usp, Uch, nn, d.twN, a.P1p, a.dHq);
-    });
-    hipError_t e;
-    for (int c = 0; c < 2; c++)
-        if ((e = launch_transpose_d(a.P1p + c * plane, a.HGs + c * plane, g.Nw + 1, (int)g.nq, s)) != hipSuccess)
-            return e;
+    const int nn = (int)n, H = g.Nw / 2;
+    const long plane = (long)(g.Nw + 1) * g.nq, half = (long)(H + 1) * g.nq;
+    const unsigned nq = (unsigned)g.nq;
+    if (g.Nw <= 512) {
+        DISPATCH_L_TO512(g.Nw, hipLaunchKernelGGL(k_al_HG_pencil_short<LL>, dim3(nq), dim3(AL_PEN_THREADS), 0, s, a.chiwP,
+                         d.chi0inf, d.chi0inf2, a.hw, a.hg2, g.N, g.T, Usp, Uch, nn, d.twN, a.Pp, a.dHq));
+    } else {
+        AL_DISPATCH_FROM1024(g.Nw, hipLaunchKernelGGL(k_al_HG_pencil<LL>, dim3(nq), dim3(LL / 16), 0, s, a.chiwP,
+                             d.chi0inf, d.chi0inf2, a.hw, a.hg2, g.N, g.T, Usp, Uch, nn, d.twN, a.Pp, a.dHq));
+    }
+    hipError_t e = launch_transpose_d2(a.Pp, a.HGs, a.Pp + half, a.HGs + half, H + 1, (int)g.nq, s);
+    if (e != hipSuccess) return e;
     AL_DISPATCH_N(g.N, {
         constexpr size_t lds = slab_bytes(NN, sizeof(double));
         al_set_lds(k_al_prod_slab<NN>, lds);
-        hipLaunchKernelGGL(k_al_prod_slab<NN>, dim3(2 * (g.Nw + 1) + 8), dim3(SlabShape<NN>::NT), lds, s, d.wt, a.HGs, a.dHq,
-                           a.Grt, a.dGrt, g.Nw, a.P1s, a.P2s, a.dP);
+        hipLaunchKernelGGL(k_al_prod_slab<NN>, dim3(2 * (H + 1) + 4), dim3(SlabShape<NN>::NT), lds, s, d.wt, a.HGs, a.dHq,
+                           a.Grt, a.dGrt, g.Nw, a.Ps, a.dP);
     });
-    for (int c = 0; c < 2; c++) {
-        if ((e = launch_transpose_d(a.P1s + c * plane, a.P1p + c * plane, g.nq, g.Nw + 1, s)) != hipSuccess) return e;
-        if ((e = launch_transpose_d(a.P2s + c * plane, a.P2p + c * plane, g.nq, g.Nw + 1, s)) != hipSuccess) return e;
-    }
-    DISPATCH_AL_SELF(g.prec, AL_DISPATCH_L(g.Nw, {
-        hipLaunchKernelGGL((k_al_k_pencil<LL, AL_K_THREADS, ST>), dim3((unsigned)g.nq), dim3(AL_K_THREADS), 0, s,
-                           a.P1p, a.P2p, a.dP, d.ek, d.dek, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, g.T, mu,
-                           U, nn, d.twN, d.twX, d.twS, contrib);
-    }));
+    if ((e = launch_transpose_d2(a.Ps, a.Pp, a.Ps + plane, a.Pp + plane, g.nq, g.Nw + 1, s)) != hipSuccess) return e;
+    const PenStep step = pen_step(1.0 / (g.Nw * g.T));
+    DISPATCH_S(g.prec, {
+        if (g.Nw <= 256) {
+            DISPATCH_L_SHORT(g.Nw, hipLaunchKernelGGL((k_al_k_pencil_short<LL, ST>), dim3(nq), dim3(AL_PEN_THREADS), 0, s,
+                             a.Pp, a.dP, d.ek, d.dek, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, g.T, mu, U, nn,
+                             d.twN, d.twX, d.twS, contrib));
+        } else {
+            AL_DISPATCH_FROM512(g.Nw, hipLaunchKernelGGL((k_al_k_pencil<LL, ST>), dim3(nq), dim3(Pen<LL>::NT), 0, s, a.Pp,
+                                a.dP, d.ek, d.dek, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, step, g.T, mu, U,
+                                nn, d.twN, d.twX, d.twS, contrib));
+        }
+    });
     return hipGetLastError();
 }
 

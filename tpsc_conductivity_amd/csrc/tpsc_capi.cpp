@@ -1008,13 +1008,11 @@ int al_alloc(tpsc_ctx* c)
     rc |= dalloc(c, &a.hw, (size_t)g.nq * (g.Nw / 2));
     rc |= dalloc(c, &a.hg2, (size_t)g.nq);
     rc |= dalloc(c, &a.chiwP, (size_t)g.nk8 * g.nwb);
-    rc |= dalloc(c, &a.P1p, 2 * plane);
-    rc |= dalloc(c, &a.P2p, 2 * plane);
-    rc |= dalloc(c, &a.HGs, 2 * plane);
-    rc |= dalloc(c, &a.P1s, 2 * plane);
-    rc |= dalloc(c, &a.P2s, 2 * plane);
-    rc |= dalloc(c, &a.dHq, 4 * (size_t)g.nq);
-    rc |= dalloc(c, &a.dP, 8 * (size_t)g.nq);
+    rc |= dalloc(c, &a.Pp, 2 * plane);
+    rc |= dalloc(c, &a.HGs, 2 * (size_t)g.nwb * g.nq);
+    rc |= dalloc(c, &a.Ps, 2 * plane);
+    rc |= dalloc(c, &a.dHq, 2 * (size_t)g.nq);
+    rc |= dalloc(c, &a.dP, 4 * (size_t)g.nq);
     rc |= dalloc(c, &a.contrib, (size_t)g.nwb * g.nq);
     rc |= dalloc(c, &a.red, (size_t)g.nwb);
     if (rc) return rc;
@@ -1641,7 +1639,7 @@ int tpsc_chijj(tpsc_ctx* c, int chi3, int mmin, int N_theta_k)
         return fail(c, TPSC_E_INVALID, "N_theta_k must be in 1.." + std::to_string(kMaxTheta));
     if (chi3 && (mmin < 0 || mmin > 30)) return fail(c, TPSC_E_INVALID, "mmin must be in 0..30");
     if (chi3 && c->p.Nw0 > 2048)
-        return fail(c, TPSC_E_INVALID, "the Aslamazov-Larkin term needs Nw <= 2048 (its pencils hold 4 tau rows in LDS)");
+        return fail(c, TPSC_E_INVALID, "the Aslamazov-Larkin term needs Nw <= 2048");
     int rc = stage_chijj(c, N_theta_k);
     if (rc || !chi3) return rc;
     return stage_al(c, mmin, N_theta_k);

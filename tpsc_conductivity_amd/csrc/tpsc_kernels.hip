@@ -1497,6 +1497,15 @@ hipError_t launch_transpose_d(const double* in, double* out, long ncols, int nro
     return hipGetLastError();
 }
 
+// the same for two arrays
+hipError_t launch_transpose_d2(const double* in0, double* out0, const double* in1, double* out1, long ncols, int nrows,
+                               hipStream_t s)
+{
+    const dim3 gr((unsigned)((ncols + kTT - 1) / kTT), (unsigned)((nrows + kTT - 1) / kTT), 2);
+    hipLaunchKernelGGL(k_transpose<double>, gr, dim3(256), 0, s, in0, out0, in1, out1, ncols, nrows);
+    return hipGetLastError();
+}
+
 // out[r] = sum of part[r*n .. r*n+n) in a fixed order, r < nrows
 hipError_t launch_sum_rows(const double* part, int nrows, int n, double* out, hipStream_t s)
 {

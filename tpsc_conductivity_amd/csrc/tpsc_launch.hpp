@@ -86,13 +86,11 @@ struct ALArrays {
     double* hw = nullptr;       // nq*(Nw/2)   hG(q,iq_p), point-major [q][p]
     double* hg2 = nullptr;      // nq          1/qn^2 coefficient of hG
     double* chiwP = nullptr;    // nk8*nwb     chi0(q,iq_p), point-major [w][p]
-    double* P1p = nullptr;      // 2 planes    point-major [c][q][t]: HG(q,tau), then P1(k,tau)
-    double* P2p = nullptr;      // 2 planes    point-major P2(k,tau)
-    double* HGs = nullptr;      // 2 planes    slab-major HG(q,tau) [c][t][q]
-    double* P1s = nullptr;      // 2 planes    slab-major P1 (and hG(q,tau) at set-up)
-    double* P2s = nullptr;      // 2 planes    slab-major P2
-    double* dHq = nullptr;      // 4*nq        HG slopes [c][side][q]
-    double* dP = nullptr;       // 8*nq        P1/P2 slopes [which][side][c][k]
+    double* Pp = nullptr;       // 2 planes    point-major [c][q][t]: HG(q,tau), t <= Nw/2, then P(k,tau)
+    double* HGs = nullptr;      // 2 x (Nw/2+1)*nq  slab-major HG(q,tau) [c][t][q]
+    double* Ps = nullptr;       // 2 planes    slab-major P (and hG(q,tau) at set-up)
+    double* dHq = nullptr;      // 2*nq        HG slope at 0+ [c][q]
+    double* dP = nullptr;       // 4*nq        P slopes [side][c][k]
     double* contrib = nullptr;  // nwb*nq      per-frequency, per-k contributions [n][k]
     double* red = nullptr;      // nwb         Lambda_jj3 on the sparse set
     int N = 0, Nw = 0;          // grid the arrays were sized for
@@ -271,6 +269,8 @@ hipError_t launch_hf0_bnd_tan(const Grid& g, const DevArrays& d, const TanArrays
 hipError_t launch_jj_pencil_tan(const Grid& g, const DevArrays& d, const TanArrays& t, double mu, double dmu,
                                 int nblk, hipStream_t s);
 hipError_t launch_transpose_d(const double* in, double* out, long ncols, int nrows, hipStream_t s);
+hipError_t launch_transpose_d2(const double* in0, double* out0, const double* in1, double* out1, long ncols, int nrows,
+                               hipStream_t s);
 hipError_t launch_sum_rows(const double* part, int nrows, int n, double* out, hipStream_t s);
 hipError_t launch_al_setup(const Grid& g, const DevArrays& d, const ALArrays& a, double mu0, hipStream_t s);
 hipError_t launch_al_freq(const Grid& g, const DevArrays& d, const ALArrays& a, double Usp, double Uch, double mu,

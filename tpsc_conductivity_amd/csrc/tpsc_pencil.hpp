@@ -131,17 +131,17 @@ __device__ __forceinline__ void pen_rows(cd* v, cd* Z, const cd* __restrict__ tw
 
 // Forward DFT, v[r] = x[t + NT r] on entry, v[m] = X[pen_beta + NT m] on exit.  Z must be free on entry; no
 // thread's rows are read by others afterwards.
-template <int L>
+template <int L, int TS = 1>
 __device__ __forceinline__ void pen_fft_dif(cd* v, cd* Z, const cd* __restrict__ tw, int t)
 {
     constexpr int PS = Pen<L>::PS;
-    const cd a1 = tw[t], a2 = tw[2 * t], a4 = tw[4 * t];
+    const cd a1 = tw[TS * t], a2 = tw[2 * TS * t], a4 = tw[4 * TS * t];
     reg_dft<8>(v);
     twiddle8(v, a1, a2, a4);
 #pragma unroll
     for (int k = 0; k < 8; k++) Z[k * PS + t] = v[k];
     __syncthreads();
-    pen_rows<L>(v, Z, tw, t);
+    pen_rows<L, TS>(v, Z, tw, t);
 }
 
 // Forward DFT of x, whose element 8 p + c lies at Z[c PS + p] (written before, no barrier yet); on exit v[m] = X[t +
