@@ -298,7 +298,9 @@ int root_chunk_graph(tpsc_ctx* c, int kind, const std::function<hipError_t()>& p
 
 int mu0_ready(tpsc_ctx* c);
 // chi0max (device) != nullptr: the bracket is (0, 2/chi0max - 2 eps), set on the device.
-int device_halley(tpsc_ctx* c, int kind, const std::function<hipError_t()>& pass, HalleyState s0, double* root,
+// A grid whose searches fit one workgroup (sum_in_one, mu_in_one) runs all passes in one launch instead: search().
+int device_halley(tpsc_ctx* c, int kind, const std::function<hipError_t()>& pass,
+                  const std::function<hipError_t(const RootInit&, int)>& search, HalleyState s0, double* root,
                   int* nevals, bool* ok, const double* chi0max = nullptr)
 {
     static const bool graphs = !(getenv("TPSC_NO_GRAPHS") && atoi(getenv("TPSC_NO_GRAPHS")) != 0);
@@ -306,10 +308,17 @@ int device_halley(tpsc_ctx* c, int kind, const std::function<hipError_t()>& pass
         if (int rc = mu0_ready(c)) return rc;
     s0.T = c->g.T;
     s0.mu0 = c->mu0;
-    HIPCHK(c, launch_halley_init(c->d.root, s0, chi0max, c->dev_scalar + 8, c->stream));
+    const RootInit in = {s0, chi0max, nullptr, nullptr, 0.0, 0.0, 0.0};
     volatile const double* m = c->host_scalar + 8;
-    int issued = 0;
-    for (;;) {
+    const bool one = (kind == kRootMu) ? mu_in_one(c->g) : sum_in_one(c->g);
+    int issued = one ? s0.itmax : 0;
+    if (one) {
+        HIPCHK(c, search(in, s0.itmax));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+    } else {
+        HIPCHK(c, launch_halley_init(c->d.root, in, c->dev_scalar + 8, c->stream));
+    }
+    while (!one) {
         const int n = std::min(kRootChunk, s0.itmax - issued);
         hipGraphExec_t exec = nullptr;
         if (graphs && n == kRootChunk) {
@@ -322,11 +331,11 @@ int device_halley(tpsc_ctx* c, int kind, const std::function<hipError_t()>& pass
             for (int k = 0; k < n; k++) HIPCHK(c, pass());
         issued += n;
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        if (trace_roots() && (int)m[0] != kRootRunning)
-            fprintf(stderr, "[tpsc root] settled after %d passes: x=%.17g f=%.6e f1=%.6e [%.17g, %.17g] status %d\n",
-                    (int)m[3], m[2], m[4], m[5], m[6], m[7], (int)m[0]);
         if ((int)m[0] != kRootRunning || issued >= s0.itmax) break;
     }
+    if (trace_roots() && (int)m[0] != kRootRunning)
+        fprintf(stderr, "[tpsc root] settled after %d passes: x=%.17g f=%.6e f1=%.6e [%.17g, %.17g] status %d\n",
+                (int)m[3], m[2], m[4], m[5], m[6], m[7], (int)m[0]);
     *ok = (int)m[0] == kRootConverged;
     *root = m[1];
     if (nevals) *nevals = (int)m[3];
@@ -578,6 +587,12 @@ int stage_UspUch_grid(tpsc_ctx* c, int nq0, int nw0, double Usc[2], bool* ok_out
     const double n = c->p.n, nsr = c->nsr;
     auto pass_sp = [&]() { return launch_sum_rule3_pass(c->g, c->d, -1.0, c->dev_scalar + 8, c->stream); };
     auto pass_ch = [&]() { return launch_sum_rule3_pass(c->g, c->d, 1.0, c->dev_scalar + 8, c->stream); };
+    auto one_sp = [&](const RootInit& in, int n) {
+        return launch_sum_rule_search(c->g, c->d, -1.0, in, c->dev_scalar + 8, n, c->stream);
+    };
+    auto one_ch = [&](const RootInit& in, int n) {
+        return launch_sum_rule_search(c->g, c->d, 1.0, in, c->dev_scalar + 8, n, c->stream);
+    };
     double root = 0.0;
     bool ok = true;
     int nh = 0;
@@ -586,7 +601,7 @@ int stage_UspUch_grid(tpsc_ctx* c, int nq0, int nw0, double Usc[2], bool* ok_out
     // the Stoner bound 2/chi0max, where the function has its pole: the derivative-based search
     // starts at the midpoint instead (same root).  The device sets both from its chi0max, so the
     // first passes follow the chi0 stage without a host round trip.
-    rc = device_halley(c, kRootUsp, pass_sp,
+    rc = device_halley(c, kRootUsp, pass_sp, one_sp,
                        halley_start(U / 2.0, 0.0, 0.0, 40, n - n * n / 2.0 - nsr, nsr * nsr / (2.0 * U)), &root,
                        &nh, &hok, c->d.red);
     if (!rc) rc = chi0_ready(c);
@@ -604,7 +619,7 @@ int stage_UspUch_grid(tpsc_ctx* c, int nq0, int nw0, double Usc[2], bool* ok_out
     root = 0.0;
     init[0] = 0;
     init[2] = 1000.0 * U;
-    rc = device_halley(c, kRootUch, pass_ch,
+    rc = device_halley(c, kRootUch, pass_ch, one_ch,
                        halley_start(init[0], init[1], init[2], 40,
                                     n - n * n / 2.0 - (nsr + c->Usp * nsr * nsr / (2.0 * U) - nsr * nsr), 0.0),
                        &root, &nh, &hok);
@@ -806,9 +821,12 @@ int stage_mu(tpsc_ctx* c)
     const double init[3] = {0.0, -10.0, 10.0}, lims[2] = {-20, 20};
     double root = 0.0;
     auto pass = [&]() { return launch_trace_diffG3_pass(c->g, c->d, c->dev_scalar + 8, c->stream); };
+    auto one = [&](const RootInit& in, int n) {
+        return launch_mu_search(c->g, c->d, in, c->dev_scalar + 8, n, c->stream);
+    };
     int nh = 0;
     bool ok = false;
-    rc = device_halley(c, kRootMu, pass, halley_start(init[0], lims[0], lims[1], 40, 0.0, 0.0), &root, &nh, &ok);
+    rc = device_halley(c, kRootMu, pass, one, halley_start(init[0], lims[0], lims[1], 40, 0.0, 0.0), &root, &nh, &ok);
     if (rc) return rc;
     c->roots_dev = (c->roots_dev & ~4) | (ok ? 4 : 0);
     if (ok)
@@ -2181,13 +2199,11 @@ int tpsc_queue_solve(tpsc_ctx* c, const tpsc_params* p, double* slot_dev, bool c
     // constant formed on the device from Usp; each search settles into its own mirror in psc
     HalleyState s0 = halley_start(U / 2.0, 0.0, 0.0, 40, n - n * n / 2.0 - nsr, nsr * nsr / (2.0 * U));
     s0.T = g.T;
-    HIPCHK(c, launch_halley_init(d.root, s0, d.red, psc + kPscUsp, s));
-    for (int k = 0; k < nsp; k++) HIPCHK(c, launch_sum_rule3_pass(g, d, -1.0, psc + kPscUsp, s));
+    HIPCHK(c, launch_sum_rule_search(g, d, -1.0, {s0, d.red, nullptr, nullptr, 0.0, 0.0, 0.0}, psc + kPscUsp, nsp, s));
     s0 = halley_start(0.0, 0.0, 1000.0 * U, 40, 0.0, 0.0);
     s0.T = g.T;
-    HIPCHK(c, launch_halley_init(d.root, s0, nullptr, psc + kPscUch, s, nullptr, psc + kPscUsp + 1, n - n * n / 2.0,
-                                 nsr, U));
-    for (int k = 0; k < nch; k++) HIPCHK(c, launch_sum_rule3_pass(g, d, 1.0, psc + kPscUch, s));
+    HIPCHK(c, launch_sum_rule_search(g, d, 1.0, {s0, nullptr, nullptr, psc + kPscUsp + 1, n - n * n / 2.0, nsr, U},
+                                     psc + kPscUch, nch, s));
     // vertex and self-energy (stage_vertex, stage_sigma)
     HIPCHK(c, launch_vertex_slab(g, d, U, 0.0, 0.0, s, psc));
     HIPCHK(c, launch_vertex_pencil(g, d, U, 0.0, 0.0, s, psc));
@@ -2197,8 +2213,7 @@ int tpsc_queue_solve(tpsc_ctx* c, const tpsc_params* p, double* slot_dev, bool c
     // mu (stage_mu): start 0 in the limits (-20, 20), mu0 from the device
     s0 = halley_start(0.0, -20.0, 20.0, 40, 0.0, 0.0);
     s0.T = g.T;
-    HIPCHK(c, launch_halley_init(d.root, s0, nullptr, psc + kPscMu, s, d.mu0v));
-    for (int k = 0; k < nmu; k++) HIPCHK(c, launch_trace_diffG3_pass(g, d, psc + kPscMu, s));
+    HIPCHK(c, launch_mu_search(g, d, {s0, nullptr, d.mu0v, nullptr, 0.0, 0.0, 0.0}, psc + kPscMu, nmu, s));
     // Lambda_jj bubble + Maki-Thompson and the diamagnetic rows (stage_chijj, N_theta_k = 1)
     HIPCHK(c, launch_hf0_bnd(g, d, 0.0, 0.0, s, d.mu0v, U, psc));
     for (int which = 0; which < 2; which++) HIPCHK(c, launch_hV_slab(g, d, which, s));

@@ -71,24 +71,76 @@ __global__ void k_finalize_k(const double* __restrict__ part, int n, double* out
 // that the host need not wait for chi0max before the first pass
 // a0src (device Usp, may be null): a0 = uch_a0(a0A, nsr, U, *a0src); mu0p (may be null): the
 // state's mu0 from the device
-__global__ void k_halley_init(HalleyState* st, HalleyState s0, const double* chi0max, double* mirror,
-                              const double* mu0p, const double* a0src, double a0A, double nsr, double U)
+__device__ __forceinline__ HalleyState halley_begin(const RootInit& in)
 {
-    HalleyState s = s0;
-    if (chi0max) {
-        const double lo = 0.0, hi = 2.0 / chi0max[0] - 2 * DBL_EPSILON;
-        const double x0 = (s0.x > lo && s0.x < hi) ? s0.x : 0.5 * (lo + hi);
-        s = halley_start(x0, lo, hi, s0.itmax, s0.a0, s0.a1);
-        s.T = s0.T;
-        s.mu0 = s0.mu0;
+    HalleyState s = in.s0;
+    if (in.chi0max) {
+        const double lo = 0.0, hi = 2.0 / in.chi0max[0] - 2 * DBL_EPSILON;
+        const double x0 = (in.s0.x > lo && in.s0.x < hi) ? in.s0.x : 0.5 * (lo + hi);
+        s = halley_start(x0, lo, hi, in.s0.itmax, in.s0.a0, in.s0.a1);
+        s.T = in.s0.T;
+        s.mu0 = in.s0.mu0;
     }
-    if (mu0p) s.mu0 = *mu0p;
-    if (a0src) s.a0 = uch_a0(a0A, nsr, U, *a0src);
+    if (in.mu0p) s.mu0 = *in.mu0p;
+    if (in.a0src) s.a0 = uch_a0(in.a0A, in.nsr, in.U, *in.a0src);
+    return s;
+}
+__device__ __forceinline__ void halley_mirror(const HalleyState& s, double* mirror)
+{
+    mirror[0] = s.status;
+    mirror[1] = s.root;
+    mirror[2] = s.x;
+    mirror[3] = s.ne;
+    mirror[4] = s.f;
+    mirror[5] = s.f1;
+    mirror[6] = s.lo;
+    mirror[7] = s.hi;
+}
+__global__ void k_halley_init(HalleyState* st, RootInit in, double* mirror)
+{
+    const HalleyState s = halley_begin(in);
     *st = s;
     mirror[0] = s.status;
     mirror[1] = s.root;
     mirror[2] = s.x;
     mirror[3] = s.ne;
+}
+
+// A whole search in one workgroup of 1024 threads, for grids whose passes would be launch-bound: at most npass
+// evaluations, pass(x, acc) adding this thread's part of {f, f', f''}, from values that the kernel keeps in registers.
+// What bounds it: the latency of a pass's reduction (two barriers) and update.  A search of five passes
+// over 5800 terms takes 16 us; five pass kernels take 33 us and their launches.
+constexpr int kSearchThreads = 1024;
+template <typename Pass>
+__device__ __forceinline__ void search_block(HalleyState* st, const HalleyState& s0, double* mirror, int npass,
+                                             const Pass& pass)
+{
+    constexpr int NWV = kSearchThreads / 64;  // 16: the wavefront sums of one value fill a DPP row
+    __shared__ HalleyState s;
+    __shared__ double sc[3 * NWV];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0) s = s0;
+    __syncthreads();
+    for (int k = 0; k < npass && s.status == kRootRunning; k++) {
+        double acc[3] = {0.0, 0.0, 0.0};
+        pass(s.x, acc);
+#pragma unroll
+        for (int i = 0; i < 3; i++) acc[i] = wave_total63(acc[i]);
+        if (lane == 63)
+#pragma unroll
+            for (int i = 0; i < 3; i++) sc[i * NWV + wave] = acc[i];
+        __syncthreads();
+        if (wave == 0) {
+            const double v = row_total15((lane < 3 * NWV) ? sc[lane] : 0.0);
+            const double f[3] = {lane_get(v, 15), lane_get(v, 31), lane_get(v, 47)};
+            if (lane == 0) halley_update(s, f);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        *st = s;
+        halley_mirror(s, mirror);
+    }
 }
 
 // One Halley step after a pass, by one workgroup of 256 threads: the three partial sums of
@@ -110,30 +162,25 @@ __device__ __forceinline__ void halley_step_block(const double* part, int n, Hal
         HalleyState s = s0;
         halley_update(s, v);
         *st = s;
-        if (s.status != kRootRunning) {
-            mirror[0] = s.status;
-            mirror[1] = s.root;
-            mirror[2] = s.x;
-            mirror[3] = s.ne;
-            mirror[4] = s.f;
-            mirror[5] = s.f1;
-            mirror[6] = s.lo;
-            mirror[7] = s.hi;
-        }
+        if (s.status != kRootRunning) halley_mirror(s, mirror);
     }
 }
 
-// True in the workgroup of a pass that finishes last, once every workgroup's partial sums
-// (stored by its thread 0) are visible to it; that workgroup resets the ticket for the next pass.
-// No workgroup waits for another: the others return at once.  Only thread 0 releases (its
-// part[] stores, written back from its XCD's L2 before the ticket) and only the last workgroup
-// acquires: a full fence in every workgroup would also invalidate each XCD's L2 while the
-// other workgroups still stream the pass's input from it.
-__device__ __forceinline__ bool last_workgroup(unsigned* ticket, unsigned nblk)
+// True in the workgroup of a pass that finishes last, once every workgroup's partial sums acc[k] -> part[k * nblk + b]
+// (stored here by its thread 0) are visible to it; that workgroup resets the ticket for the next pass.  No workgroup
+// waits for another: the others return at once.  The sums are stored at agent scope, past the XCD's L2, and have
+// arrived when the ticket is taken: no workgroup needs a release fence (a write-back of its whole L2), and only the
+// last one acquires.
+__device__ __forceinline__ bool last_workgroup(unsigned* ticket, unsigned nblk, unsigned b, const double acc[3],
+                                               double* part)
 {
     __shared__ unsigned last;
     if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        for (int k = 0; k < 3; k++)
+            __hip_atomic_store(part + (long)k * nblk + b, acc[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0);  // the stores have been acknowledged
+        asm volatile("" ::: "memory");
         last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nblk - 1;
     }
     __syncthreads();
@@ -406,9 +453,43 @@ __global__ void __launch_bounds__(256)
     }
     block_sum_k<3>(acc, sc);
     const int nblk = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 3; k++) part[k * nblk + b] = acc[k];
-    if (ticket && last_workgroup(ticket, nblk)) halley_step_block(part, nblk, st, mirror, sc);
+    if (ticket) {
+        if (last_workgroup(ticket, nblk, b, acc, part)) halley_step_block(part, nblk, st, mirror, sc);
+    } else if (threadIdx.x == 0) {
+        for (int k = 0; k < 3; k++) part[(long)k * nblk + b] = acc[k];
+    }
+}
+
+// The whole search in one workgroup: the nk8 (2 nwmax + 1) <= CN * 1024 values of chi0 and their weights are read
+// once, CN per thread (no series part on such grids)
+template <int CN>
+__global__ void __launch_bounds__(kSearchThreads)
+    k_sum_rule_search(const double* __restrict__ chi, const double* __restrict__ inf1, const double* __restrict__ inf2,
+                      const double* __restrict__ wq, int nk8, int nwmax, double Nq, double sgn, HalleyState* st,
+                      RootInit in, double* mirror, int npass)
+{
+    const HalleyState s0 = halley_begin(in);
+    const double wT = 2.0 * s0.T / Nq;
+    double c[CN], w[CN];
+#pragma unroll
+    for (int u = 0; u < CN; u++) {
+        const int i = threadIdx.x + u * kSearchThreads, j = i / nk8, q = i - j * nk8;
+        c[u] = w[u] = 0.0;
+        if (j <= 2 * nwmax) {
+            w[u] = (j == 0) ? 0.5 * wT * wq[q] : wT * wq[q];
+            if (j <= nwmax) {
+                c[u] = chi[i];
+            } else {
+                const double wn = 2 * j * kPi * s0.T;
+                const double i2 = rcp_nr(wn * wn);
+                c[u] = (inf1[q] + inf2[q] * i2) * i2;
+            }
+        }
+    }
+    search_block(st, s0, mirror, npass, [&](double Ux, double* acc) {
+#pragma unroll
+        for (int u = 0; u < CN; u++) sum_rule3_term(c[u], w[u], sgn * Ux, sgn, acc);
+    });
 }
 
 // Row moments of the sum-rule terms (one workgroup per row j <= 2 nwmax, stored rows from chi,
@@ -830,14 +911,54 @@ __global__ void __launch_bounds__(256)
         }
         for (; j <= Nw; j += 64) {
             const double wn = (2 * j + 1) * kPi * T;
-            const double iw = 1.0 / wn, iw2 = iw * iw;
+            const double iw = rcp_nr(wn), iw2 = iw * iw;
             trace_diffG3_term(wn, (-s2 + s4 * iw2) * iw2, (-Si + s3 * iw2) * iw, e, c, w, mu0, pmu, acc);
         }
     }
     block_sum_k<3>(acc, sc);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 3; k++) part[k * gridDim.x + blockIdx.x] = acc[k];
-    if (ticket && last_workgroup(ticket, gridDim.x)) halley_step_block(part, gridDim.x, st, mirror, sc);
+    if (ticket) {
+        if (last_workgroup(ticket, gridDim.x, blockIdx.x, acc, part))
+            halley_step_block(part, gridDim.x, st, mirror, sc);
+    } else if (threadIdx.x == 0) {
+        for (int k = 0; k < 3; k++) part[(long)k * gridDim.x + blockIdx.x] = acc[k];
+    }
+}
+// The whole search in one workgroup: Sigma and the weights of the nk8 (Nw + 1) <= CN * 1024 terms, CN per thread
+template <int CN, typename SelfT>
+__global__ void __launch_bounds__(kSearchThreads)
+    k_mu_search(const double* __restrict__ ekw, const double* __restrict__ wq, const SelfT* __restrict__ Self,
+                const double* __restrict__ Sinf2, const double* __restrict__ Sinf3, const double* __restrict__ Sinf4,
+                const double* __restrict__ Sinf, int nk8, int Nw, HalleyState* st, RootInit in, double* mirror,
+                int npass)
+{
+    const HalleyState s0 = halley_begin(in);
+    const double Si = Sinf[0];
+    const int H = Nw / 2;
+    double wn[CN], rS[CN], iS[CN], e[CN], w[CN];
+#pragma unroll
+    for (int u = 0; u < CN; u++) {
+        const int i = threadIdx.x + u * kSearchThreads, q = i / (Nw + 1), j = i - q * (Nw + 1);
+        wn[u] = (2 * j + 1) * kPi * s0.T;
+        rS[u] = iS[u] = e[u] = w[u] = 0.0;
+        if (q < nk8) {
+            e[u] = ekw[q];
+            w[u] = 2.0 * wq[q];
+            if (j < H) {
+                const cd s = sigma_kw(Self + (long)q * H, j, Si, Sinf2[q], Sinf3[q], wn[u]);
+                rS[u] = s.x;
+                iS[u] = s.y;
+            } else {
+                const double iw = rcp_nr(wn[u]), iw2 = iw * iw;
+                rS[u] = (-Sinf2[q] + Sinf4[q] * iw2) * iw2;
+                iS[u] = (-Si + Sinf3[q] * iw2) * iw;
+            }
+        }
+    }
+    search_block(st, s0, mirror, npass, [&](double pmu, double* acc) {
+#pragma unroll
+        for (int u = 0; u < CN; u++)
+            trace_diffG3_term(wn[u], rS[u], iS[u], e[u], e[u] - s0.mu0, w[u], s0.mu0, pmu, acc);
+    });
 }
 
 // which = 0: Tr Sigma G0 main sum (green.cpp:3018-3051); 1: its Sigma_inf correction
@@ -1266,11 +1387,9 @@ hipError_t launch_sum_rule_part(int N, int Nw, double T, const double* chiw, con
     return hipGetLastError();
 }
 
-hipError_t launch_halley_init(HalleyState* st, const HalleyState& s0, const double* chi0max, double* mirror,
-                              hipStream_t s, const double* mu0p, const double* a0src, double a0A, double nsr,
-                              double U)
+hipError_t launch_halley_init(HalleyState* st, const RootInit& in, double* mirror, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_halley_init, dim3(1), dim3(1), 0, s, st, s0, chi0max, mirror, mu0p, a0src, a0A, nsr, U);
+    hipLaunchKernelGGL(k_halley_init, dim3(1), dim3(1), 0, s, st, in, mirror);
     return hipGetLastError();
 }
 
@@ -1286,6 +1405,29 @@ hipError_t launch_sum_rule3_pass(const Grid& g, const DevArrays& d, double sgn, 
                        series ? d.srmax : nullptr);
     if (!fused) hipLaunchKernelGGL(k_halley_step, dim3(1), dim3(256), 0, s, d.part, nblk, d.root, mirror);
     return hipGetLastError();
+}
+
+hipError_t launch_sum_rule_search(const Grid& g, const DevArrays& d, double sgn, const RootInit& in, double* mirror,
+                                  int npass, hipStream_t s)
+{
+    if (sum_in_one(g)) {
+        const long n = g.nk8 * (g.Nw + 1);
+        const double Nq = 4.0 * (g.nk - 1) * (g.nk - 1);
+#define SUM_SEARCH(CN)                                                                                              \
+    hipLaunchKernelGGL(k_sum_rule_search<CN>, dim3(1), dim3(kSearchThreads), 0, s, d.chiw, d.chi0inf, d.chi0inf2,   \
+                       d.wq, (int)g.nk8, g.Nw / 2, Nq, sgn, d.root, in, mirror, npass)
+        if (n <= 4 * kSearchThreads)
+            SUM_SEARCH(4);
+        else if (n <= 8 * kSearchThreads)
+            SUM_SEARCH(8);
+        else
+            SUM_SEARCH(kSumOneMax / kSearchThreads);
+#undef SUM_SEARCH
+        return hipGetLastError();
+    }
+    hipError_t e = launch_halley_init(d.root, in, mirror, s);
+    for (int k = 0; k < npass && e == hipSuccess; k++) e = launch_sum_rule3_pass(g, d, sgn, mirror, s);
+    return e;
 }
 
 hipError_t launch_sr_moments(const Grid& g, const DevArrays& d, hipStream_t s)
@@ -1394,6 +1536,28 @@ hipError_t launch_trace_diffG3_pass(const Grid& g, const DevArrays& d, double* m
     });
     if (!fused) hipLaunchKernelGGL(k_halley_step, dim3(1), dim3(256), 0, s, d.part, nblk, d.root, mirror);
     return hipGetLastError();
+}
+
+hipError_t launch_mu_search(const Grid& g, const DevArrays& d, const RootInit& in, double* mirror, int npass,
+                            hipStream_t s)
+{
+    if (mu_in_one(g)) {
+        const long n = g.nk8 * (g.Nw + 1);
+#define MU_SEARCH(CN)                                                                                              \
+    hipLaunchKernelGGL((k_mu_search<CN, ST>), dim3(1), dim3(kSearchThreads), 0, s, d.ekw, d.wq, (const ST*)d.Self, \
+                       d.Sinf2, d.Sinf3, d.Sinf4, d.Sinf, (int)g.nk8, g.Nw, d.root, in, mirror, npass)
+        DISPATCH_S(g.prec, {
+            if (n <= 4 * kSearchThreads)
+                MU_SEARCH(4);
+            else
+                MU_SEARCH(kMuOneMax / kSearchThreads);
+        });
+#undef MU_SEARCH
+        return hipGetLastError();
+    }
+    hipError_t e = launch_halley_init(d.root, in, mirror, s);
+    for (int k = 0; k < npass && e == hipSuccess; k++) e = launch_trace_diffG3_pass(g, d, mirror, s);
+    return e;
 }
 
 hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu0, double mu, int which, double* out,

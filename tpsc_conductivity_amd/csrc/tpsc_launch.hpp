@@ -153,10 +153,23 @@ constexpr int kRowGroups = 32;       // frequency-row groups of the reduction gr
 constexpr int kPartCap = 8192;       // capacity of DevArrays::part
 // Root-search passes over at most this many workgroups take their Halley step in the workgroup
 // that finishes last (one launch per pass: small grids are launch-bound); larger passes launch
-// the step kernel after them, since each workgroup's release fence (a write-back of its XCD's
-// L2) costs more there than the launch it saves (256^2: sum-rule passes of 1056 workgroups,
-// trace passes of 2097).
+// the step kernel after them, since the tickets of all workgroups on one counter cost more
+// there than the launch they save (256^2 x 2048 with every pass fused: 2.17 against 2.10 ms).
 constexpr int kFusedStepMax = 640;
+// Grids of at most this many (wedge point, frequency) terms run a whole root search in one workgroup of 1024 threads with
+// the terms in registers (12 and 6 per thread): a search of five passes takes 11-20 us, against 33 (sum rule) and 45 us
+// (mu) in passes.  With 16 and 8 per thread the registers spill: 30 and 33 us.
+constexpr long kSumOneMax = 12 * 1024, kMuOneMax = 6 * 1024;
+inline bool sum_in_one(const Grid& g) { return g.nk8 * (g.Nw + 1) <= kSumOneMax; }
+inline bool mu_in_one(const Grid& g) { return g.nk8 * (g.Nw + 1) <= kMuOneMax; }
+// Start of a device-driven search.  chi0max (device, may be null): the bracket is (0, 2/chi0max - 2 eps); mu0p (device,
+// may be null): the state's mu0; a0src (device Usp, may be null): the charge sum rule's constant a0 = a0A - (nsr + Usp
+// nsr^2/(2U) - nsr^2), formed on the device
+struct RootInit {
+    HalleyState s0;
+    const double *chi0max, *mu0p, *a0src;
+    double a0A, nsr, U;
+};
 // series terms of the sum-rule passes' small-chi rows and the moments they take, M_2 .. M_{K+3}
 constexpr int kSRK = 18;
 constexpr int kSRM = kSRK + 2;
@@ -193,15 +206,15 @@ hipError_t launch_sum_rule_part(int N, int Nw, double T, const double* chiw, con
 // state, so a pass depends on the point only through d.root.  mirror (mapped host memory)
 // holds {status, root, x, passes, f, f', lo, hi}: "running" from the initialisation, the
 // outcome once the search has settled.
-// mu0p (device, may be null): the state's mu0; a0src (device Usp, may be null): the charge sum
-// rule's constant a0 = a0A - (nsr + Usp nsr^2/(2U) - nsr^2), formed on the device
-hipError_t launch_halley_init(HalleyState* st, const HalleyState& s0, const double* chi0max, double* mirror,
-                              hipStream_t s, const double* mu0p = nullptr, const double* a0src = nullptr,
-                              double a0A = 0.0, double nsr = 0.0, double U = 0.0);
-// psc[slot], psc[3 + slot], psc[6 + slot] = root, status, evaluations of the search in st
+hipError_t launch_halley_init(HalleyState* st, const RootInit& in, double* mirror, hipStream_t s);
 hipError_t launch_sum_rule3_pass(const Grid& g, const DevArrays& d, double sgn, double* mirror, hipStream_t s);
 hipError_t launch_sr_moments(const Grid& g, const DevArrays& d, hipStream_t s);
 hipError_t launch_trace_diffG3_pass(const Grid& g, const DevArrays& d, double* mirror, hipStream_t s);
+// The initialisation and npass passes of a search: one launch where sum_in_one(g) / mu_in_one(g), npass + 1 otherwise
+hipError_t launch_sum_rule_search(const Grid& g, const DevArrays& d, double sgn, const RootInit& in, double* mirror,
+                                  int npass, hipStream_t s);
+hipError_t launch_mu_search(const Grid& g, const DevArrays& d, const RootInit& in, double* mirror, int npass,
+                            hipStream_t s);
 // green0::find_mu on the device (one workgroup, the whole bracketing search): out = {found, mu0, evaluations}
 hipError_t launch_mu0_root(const Grid& g, const DevArrays& d, double n, double preset, double* out, hipStream_t s);
 hipError_t launch_model(const Grid& g, const DevArrays& d, double t, double tp, double tpp, double t3,

@@ -219,6 +219,14 @@ __device__ __forceinline__ double wave_total63(double x)
     x = dpp_add<0x142, 0xA>(x);
     return dpp_add<0x143, 0xC>(x);
 }
+// sums over the rows of 16 lanes, in lanes 15, 31, 47, 63
+__device__ __forceinline__ double row_total15(double x)
+{
+    x = dpp_add<0x111, 0xF>(x);
+    x = dpp_add<0x112, 0xF>(x);
+    x = dpp_add<0x114, 0xF>(x);
+    return dpp_add<0x118, 0xF>(x);
+}
 
 // Step of a pencil's spline: h, 1/h, 6/h, 6/h^2 (formed on the host: uniform values stay out of the vector registers)
 struct PenStep {
