@@ -40,6 +40,7 @@ __host__ __device__ inline cd conjg(cd a) { return cd{a.x, -a.y}; }
 __host__ __device__ inline double cabs2(cd a) { return sqrt(a.x * a.x + a.y * a.y); }
 __device__ inline cd cexpd(cd z)
 {
+    if (z.y == 0.0) return cd{exp(z.x), z.y};  // the two-pole asymptotes' poles are real as a rule
     double s, c;
     sincos(z.y, &s, &c);
     const double e = exp(z.x);

@@ -324,13 +324,44 @@ __device__ __forceinline__ PolesT poles_tan(dual e, dual mu, dual Sinf, dual CJ1
     return P;
 }
 
+// what the pencil needs of them: poles, residues over the denominators, the parts of the slopes at tau = 0+, beta- (those
+// of k_jj_poles) and of J at tau = beta
+struct PointPoles {
+    cdual r[2], ad[2], bd[2];
+    dual dGp, dGm, dJ0, dJb, Jbeta;
+};
+__device__ __forceinline__ PointPoles point_poles(dual e, dual mu, dual Sinf, dual CJ1, double T)
+{
+    const PolesT P = poles_tan(e, mu, Sinf, CJ1, T);
+    const double iT = 1.0 / T;
+    PointPoles o;
+    o.dGp = o.dGm = o.dJ0 = o.dJb = o.Jbeta = dual{0.0, 0.0};
+    for (int k = 0; k < 2; k++) {
+        const cdual r = P.r[k];
+        const bool pos = r.v.x > 0;
+        const cdual ex = pos ? cexpdual(-(r * iT)) : cexpdual(r * iT);
+        const cdual a = P.a[k] / P.den[k], b = P.b[k] / P.den[k], ra = r * a, rb = r * b;
+        o.r[k] = r;
+        o.ad[k] = a;
+        o.bd[k] = b;
+        o.dGp = o.dGp + rpart(pos ? ra : ra * ex);
+        o.dGm = o.dGm + rpart(pos ? ra * ex : ra);
+        o.dJ0 = o.dJ0 + rpart(pos ? rb * ex : rb);
+        o.dJb = o.dJb + rpart(pos ? rb : rb * ex);
+        o.Jbeta = o.Jbeta + rpart(pos ? b : b * ex);
+    }
+    return o;
+}
+
 // Per-k tangent of the Lambda_jj contributions (the steps of k_jj_pencil, cond_opt.cpp:
 // 3179-3822) of every Lambda-grid point q = blk, blk + nblk, ...: workgroup blk adds them into
 // its own tangent rows part[blk*2*nwb + n] (bubble) and part[blk*2*nwb + nwb + n] (MT).
 // Primal arrays as the forward left them (hT, f0T point-major, FP64 Sigma remainder R);
-// tangent arrays t* alike.  LDS: samples and transforms of value and tangent.
+// tangent arrays t* alike.  LDS: samples and transforms of value and tangent.  What bounds it: FP64 VALU and latency at
+// two workgroups per CU, the registers of the dual arithmetic (capped at 256; compiled like tpsc_jj.hip).  64^2 x 512:
+// 104 us a parameter (all slots, four splines and three pairs of transforms, each thread its own poles: 224).
 template <int L, int NT>
-__global__ void __launch_bounds__(NT)
+__global__ void __launch_bounds__(NT, 2)
     k_jj_pencil_tan(const double* __restrict__ ek, const double* __restrict__ tek, const double* __restrict__ vel,
                     const double* __restrict__ tvel, const double* __restrict__ hT, const double* __restrict__ thT,
                     const double* __restrict__ f0T, const double* __restrict__ tf0T, const double* __restrict__ dhV,
@@ -349,8 +380,9 @@ __global__ void __launch_bounds__(NT)
     __shared__ double Y[2 * (L + 1)], dY[2 * (L + 1)];
     __shared__ cd X[L], dX[L];
     __shared__ double ES[2 * (2 * NT + 8)];
-    __shared__ double sc[16 * nw];
+    __shared__ double sc[7 * nw];
     __shared__ double Jb[2];
+    __shared__ PointPoles pp;  // formed by one thread: every thread's own copy would take 120 registers
     double* Y1 = Y;
     double* Y2 = Y + (L + 1);
     double* dY1 = dY;
@@ -367,8 +399,6 @@ __global__ void __launch_bounds__(NT)
     double* const c1 = part + blk * 2 * NWB;
     double* const c2 = c1 + NWB;
     for (int n = tid; n < 2 * NWB; n += NT) c1[n] = 0.0;
-    auto slot_jx = [](int s) { return (s >= H) ? s - H : s + H; };
-    auto dyson_idx = [](int s) { return (s < H) ? H - s - 1 : s - H; };
     for (long q = blk; q < nq; q += nblk) {
         const int l = (int)(q / nk), m = (int)(q % nk);
         const long ki = fold_idx(l + 1, m, N);
@@ -388,6 +418,7 @@ __global__ void __launch_bounds__(NT)
         const dual cj01{-f0Vb[q] - f0Vb[nq + q], -tf0Vb[q] - tf0Vb[nq + q]};
         const dual cj02{df0V[q] + df0V[q + nq], tdf0V[q] + tdf0V[q + nq]};
         const dual cj2{dhV[q] + dhV[q + nq], tdhV[q] + tdhV[q + nq]};
+        if (tid == NT - 1) pp = point_poles(e, mud, Sinf, CJ1, T);
         __syncthreads();
         {
             double* const ys[2] = {Y1, Y2};
@@ -405,96 +436,73 @@ __global__ void __launch_bounds__(NT)
         __syncthreads();
         block_fft<L, NT>(X, +1, tw);
         block_fft<L, NT>(dX, +1, tw);
-        // (2) Matsubara slots: Dyson G, J0 (f0V), J (hV); sums r[0..5] and their tangents
-        double r6[12];
-        for (int k = 0; k < 12; k++) r6[k] = 0.0;
+        // (2) Matsubara slots n >= 0 (k_n = (2n+1) pi T; slot -n-1 holds the conjugates): Dyson G, J0 (f0V), J (hV);
+        // half of the sums T G G J0 / T, k Im Gn, -k Im Jn over all slots and their tangents
+        double r6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         const dual C2{Sinf2[ki], tSinf2[ki]}, C3{Sinf3[ki], tSinf3[ki]};
-        for (int s = tid; s < L; s += NT) {
-            const int jx = slot_jx(s);
-            const cd Fj = X[jx], Fc = conjg(X[L - 1 - jx]);
-            const cd tFj = dX[jx], tFc = conjg(dX[L - 1 - jx]);
-            const cd Af = cd{0.5 * (Fj.x + Fc.x), 0.5 * (Fj.y + Fc.y)};
-            const cd Bh = cd{0.5 * (Fj.y - Fc.y), -0.5 * (Fj.x - Fc.x)};
-            const cd tAf = cd{0.5 * (tFj.x + tFc.x), 0.5 * (tFj.y + tFc.y)};
-            const cd tBh = cd{0.5 * (tFj.y - tFc.y), -0.5 * (tFj.x - tFc.x)};
-            const double knj = (jx < H) ? (2 * jx + 1) * kPi * T : (2 * (jx - L) + 1) * kPi * T;
-            const double ik = 1.0 / knj, ik2 = ik * ik;
-            const cd ts = twS[jx];
+        for (int n = tid; n < H; n += NT) {
+            const cd Fj = X[n], Fq = X[L - 1 - n], tFj = dX[n], tFq = dX[L - 1 - n];
+            const cd Af = cd{0.5 * (Fj.x + Fq.x), 0.5 * (Fj.y - Fq.y)};
+            const cd Bh = cd{0.5 * (Fj.y + Fq.y), -0.5 * (Fj.x - Fq.x)};
+            const cd tAf = cd{0.5 * (tFj.x + tFq.x), 0.5 * (tFj.y - tFq.y)};
+            const cd tBh = cd{0.5 * (tFj.y + tFq.y), -0.5 * (tFj.x - tFq.x)};
+            const double kn = (2 * n + 1) * kPi * T;
+            const double ik = rcp_nr(kn), ik2 = ik * ik;
+            const cd ts = twS[n];
             const cd af = ts * Af, ah = ts * Bh, taf = ts * tAf, tah = ts * tBh;
             const cdual J0 = cdl((-cj02 + dual{af.x, taf.x} * ik2) * ik2,
                                  (-cj01 + (cj03 + dual{af.y, taf.y} * ik) * ik2) * ik);
             const cdual Jv = cdl((-cj2 + dual{ah.x, tah.x} * ik2) * ik2,
                                  (-CJ1 + (cj3 + dual{ah.y, tah.y} * ik) * ik2) * ik);
-            const double kn = (2.0 * (s - H) + 1) * kPi * T;
-            const long o = ki * H + dyson_idx(s);
-            cd sg = sigma_mom(Sinf.v, C2.v, C3.v, Self[o], fabs(kn));
-            cd tsg = sigma_mom(Sinf.d, C2.d, C3.d, tSelf[o], fabs(kn));
-            if (s < H) {
-                sg = conjg(sg);
-                tsg = conjg(tsg);
-            }
-            const cdual den{cd{-e.v + mu - sg.x, kn - sg.y}, cd{-e.d + dmu - tsg.x, -tsg.y}};
-            const cdual Tc{cd{T, 0.0}, cd{0.0, 0.0}};
-            const cdual Gv = Tc / den;
+            const cd sg = sigma_mom_i(Sinf.v, C2.v, C3.v, Self[ki * H + n], ik);
+            const cd tsg = sigma_mom_i(Sinf.d, C2.d, C3.d, tSelf[ki * H + n], ik);
+            // T/den and its tangent -T dden/den^2
+            const cd g = sdiv_rcp(T, cd{-e.v + mu - sg.x, kn - sg.y});
+            const cdual Gv{g, -(iT * (g * g * cd{-e.d + dmu - tsg.x, -tsg.y}))};
             const cdual t = (Gv * Gv * J0) * iT;
-            const double ikn = 1.0 / kn;
-            const cdual G2 = Tc / cdl(mud - e, dual{kn, 0.0} + Sinf * ikn);
-            const cdual Jn = Gv * Jv - G2 * cdl(dual{0.0, 0.0}, -(CJ1 * ikn));
+            const dual im2 = Sinf * ik;
+            const cd g2 = sdiv_rcp(T, cd{mu - e.v, kn + im2.v});
+            const cdual G2{g2, -(iT * (g2 * g2 * cd{dmu - e.d, im2.d}))};
+            const cdual Jn = Gv * Jv - G2 * cdl(dual{0.0, 0.0}, -(CJ1 * ik));
             const cdual Gn = Gv - G2;
             r6[0] += t.v.x;
-            r6[1] += t.v.y;
-            r6[2] += Gn.v.x;
-            r6[3] += Gn.v.y;
-            r6[4] += kn * Gn.v.y;
-            r6[5] -= kn * Jn.v.y;
-            r6[6] += t.d.x;
-            r6[7] += t.d.y;
-            r6[8] += Gn.d.x;
-            r6[9] += Gn.d.y;
-            r6[10] += kn * Gn.d.y;
-            r6[11] -= kn * Jn.d.y;
-            W[s] = cd{Gn.v.x + Jn.v.y, Gn.v.y + Jn.v.x};
-            dW[s] = cd{Gn.d.x + Jn.d.y, Gn.d.y + Jn.d.x};
+            r6[1] += t.d.x;
+            r6[2] += kn * Gn.v.y;
+            r6[3] += kn * Gn.d.y;
+            r6[4] -= kn * Jn.v.y;
+            r6[5] -= kn * Jn.d.y;
+            W[H + n] = cd{Gn.v.x + Jn.v.y, Gn.v.y + Jn.v.x};
+            W[H - 1 - n] = cd{Gn.v.x - Jn.v.y, Jn.v.x - Gn.v.y};
+            dW[H + n] = cd{Gn.d.x + Jn.d.y, Gn.d.y + Jn.d.x};
+            dW[H - 1 - n] = cd{Gn.d.x - Jn.d.y, Jn.d.x - Gn.d.y};
         }
-        // block sums of the twelve slot sums (fixed order: waves, then lanes by wave_sum)
-        for (int k = 0; k < 12; k++) r6[k] = wave_sum(r6[k]);
+        // block sums of the six (fixed order: waves, then lanes by wave_sum)
+        for (int k = 0; k < 6; k++) r6[k] = wave_sum(r6[k]);
         if (lane == 0)
-            for (int k = 0; k < 12; k++) sc[k * nw + wave] = r6[k];
+            for (int k = 0; k < 6; k++) sc[k * nw + wave] = r6[k];
         __syncthreads();
-        double S6[12];
-        for (int k = 0; k < 12; k++) {
+        double S6[6];
+        for (int k = 0; k < 6; k++) {
             double a = 0.0;
             for (int i = 0; i < nw; i++) a += sc[k * nw + i];
-            S6[k] = a;
+            S6[k] = 2.0 * a;
         }
-        // (3) two-pole asymptote
-        const PolesT P = poles_tan(e, mud, Sinf, CJ1, T);
-        cdual ad[2], bd[2];
-        for (int k = 0; k < 2; k++) {
-            ad[k] = P.a[k] / P.den[k];
-            bd[k] = P.b[k] / P.den[k];
-        }
-        // (4) to imaginary time
+        // (3) to imaginary time, with the two-pole asymptote
         block_fft<L, NT>(W, -1, tw);
         block_fft<L, NT>(dW, -1, tw);
         if (tid == 0) {
-            cdual Jinf{cd{0.0, 0.0}, cd{0.0, 0.0}};
-            for (int k = 0; k < 2; k++) {
-                const cdual ej = (P.r[k].v.x > 0) ? cdual{cd{1.0, 0.0}, cd{0.0, 0.0}} : cexpdual(P.r[k] * iT);
-                Jinf = Jinf + bd[k] * ej;
-            }
-            Jb[0] = (cd{W[0].y, 0.0} / phT[L]).x + Jinf.v.x;
-            Jb[1] = (cd{dW[0].y, 0.0} / phT[L]).x + Jinf.d.x;
+            Jb[0] = (cd{W[0].y, 0.0} / phT[L]).x + pp.Jbeta.v;
+            Jb[1] = (cd{dW[0].y, 0.0} / phT[L]).x + pp.Jbeta.d;
         }
         for (int j = tid; j < L; j += NT) {
             const double t = j / (L * T);
             cdual G0t{cd{0.0, 0.0}, cd{0.0, 0.0}}, Jt{cd{0.0, 0.0}, cd{0.0, 0.0}};
             for (int k = 0; k < 2; k++) {
-                const cdual r = P.r[k];
+                const cdual r = pp.r[k];
                 const cdual ep = (r.v.x > 0) ? cexpdual(r * (-t)) : cexpdual(r * (1.0 / T - t));
                 const cdual ej = (r.v.x > 0) ? cexpdual(r * (t - 1.0 / T)) : cexpdual(r * t);
-                G0t = G0t - ad[k] * ep;
-                Jt = Jt + bd[k] * ej;
+                G0t = G0t - pp.ad[k] * ep;
+                Jt = Jt + pp.bd[k] * ej;
             }
             const cd ph = phT[j];
             const cd R = ph * W[j], dR = ph * dW[j];
@@ -503,102 +511,60 @@ __global__ void __launch_bounds__(NT)
         }
         __syncthreads();
         const dual G0{X[0].x, dX[0].x}, J0t{X[0].y, dX[0].y}, Jbeta{Jb[0], Jb[1]};
-        // pole sums at tau = 0+, beta- (k_jj_poles)
-        cdual fp[2], fm[2], fj[2], fjb[2];
-        for (int k = 0; k < 2; k++) {
-            const cdual r = P.r[k], a = P.a[k], b = P.b[k], dn = P.den[k];
-            const bool pos = r.v.x > 0;
-            const cdual ex = pos ? cexpdual(-(r * iT)) : cexpdual(r * iT);
-            fp[k] = pos ? a / dn : a * ex / dn;
-            fm[k] = pos ? a * ex / dn : a / dn;
-            fj[k] = pos ? r * b * ex / dn : r * b / dn;
-            fjb[k] = pos ? r * b / dn : r * b * ex / dn;
-        }
-        const dual s4{S6[4], S6[10]}, s5{S6[5], S6[11]};
-        const dual dGp = s4 + rpart(P.r[0] * fp[0] + P.r[1] * fp[1]);
-        const dual dGm = -s4 + rpart(P.r[0] * fm[0] + P.r[1] * fm[1]);
-        const dual dJ0 = s5 + rpart(fj[0] + fj[1]);
-        const dual dJb = -s5 + rpart(fjb[0] + fjb[1]);
-        // (5) Maki-Thompson G(tau) J(-tau) -> Y1, bubble -G(tau) G(-tau) -> Y2 (and tangents)
+        const dual s4{S6[2], S6[3]}, s5{S6[4], S6[5]};
+        const dual dGp = s4 + pp.dGp, dGm = -s4 + pp.dGm, dJ0 = s5 + pp.dJ0, dJb = -s5 + pp.dJb;
+        // (5) Maki-Thompson G(tau) J(-tau) and bubble -G(tau) G(-tau).  What follows is linear in them, so that the
+        // tangents of the weighted products (weights wv, wb) go through one spline each and one transform.
+        const dual wv = (nf * wt) * v, wb = 2.0 * wv * v;
         for (int j = tid; j < L; j += NT) {
             const cd g = X[j], tg = dX[j];
-            Y1[j] = g.x * g.y;
-            dY1[j] = tg.x * g.y + g.x * tg.y;
-            if (j == 0) {
-                Y2[0] = G0.v * (G0.v + 1.0);
-                dY2[0] = G0.d * (2.0 * G0.v + 1.0);
-            } else {
-                Y2[j] = -(g.x * X[L - j].x);
-                dY2[j] = -(tg.x * X[L - j].x + g.x * dX[L - j].x);
-            }
+            Y1[j] = (wv * (dual{g.x, tg.x} * dual{g.y, tg.y})).d;
+            const dual gm = (j == 0) ? -(G0 + 1.0) : dual{X[(L - j) & (L - 1)].x, dX[(L - j) & (L - 1)].x};
+            Y2[j] = -(wb * (dual{g.x, tg.x} * gm)).d;
         }
         if (tid == 0) {
-            const dual y1L = (-G0 - 1.0) * Jbeta, y2L = G0 * (G0 + 1.0);
-            Y1[L] = y1L.v;
-            dY1[L] = y1L.d;
-            Y2[L] = y2L.v;
-            dY2[L] = y2L.d;
+            Y1[L] = (wv * ((-G0 - 1.0) * Jbeta)).d;
+            Y2[L] = (wb * (G0 * (G0 + 1.0))).d;
         }
         __syncthreads();
-        const dual gd0 = dGp * J0t + G0 * dJ0;
-        const dual gdN = dGm * Jbeta - (G0 + 1.0) * dJb;
-        const dual MJ1{Y1[0] - Y1[L], dY1[0] - dY1[L]};
-        const dual dchi = dGp * (G0 + 1.0) + G0 * dGm;
-        double integ[2] = {0.0, 0.0}, tinteg[2] = {0.0, 0.0};
+        const double gd0 = (wv * (dGp * J0t + G0 * dJ0)).d;
+        const double gdN = (wv * (dGm * Jbeta - (G0 + 1.0) * dJb)).d;
+        const double MJ1 = Y1[0] - Y1[L];
+        const double dchi = (wb * (dGp * (G0 + 1.0) + G0 * dGm)).d;
+        double integ[2] = {0.0, 0.0};
         {
             double* const ys[2] = {Y1, Y2};
-            const double d0s[2] = {gd0.v, dchi.v}, dNs[2] = {gdN.v, -dchi.v};
+            const double d0s[2] = {gd0, dchi}, dNs[2] = {gdN, -dchi};
             block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, integ);
-            double* const ts[2] = {dY1, dY2};
-            const double t0s[2] = {gd0.d, dchi.d}, tNs[2] = {gdN.d, -dchi.d};
-            block_spline_fixed<L, NT, 2>(ts, hstep, t0s, tNs, ES, tinteg);
         }
         {
-            const double a = wave_sum(integ[1]), b = wave_sum(tinteg[1]);
-            if (lane == 0) {
-                sc[12 * nw + wave] = a;
-                sc[13 * nw + wave] = b;
-            }
+            const double a = wave_sum(integ[1]);
+            if (lane == 0) sc[6 * nw + wave] = a;
         }
-        const dual MJ3{Y1[0] - Y1[L], dY1[0] - dY1[L]};
+        const double MJ3 = Y1[0] - Y1[L];
         // (6) packed transform of the two moment sequences
         for (int j = tid; j < L; j += NT) {
             const double a = (Y1[j + 1] - Y1[j]) / hstep;
             const double b = (j < H) ? (Y2[j + 1] - Y2[j]) / hstep : -(Y2[L - j] - Y2[L - 1 - j]) / hstep;
-            const double ta = (dY1[j + 1] - dY1[j]) / hstep;
-            const double tb = (j < H) ? (dY2[j + 1] - dY2[j]) / hstep : -(dY2[L - j] - dY2[L - 1 - j]) / hstep;
             X[j] = cd{a, b};
-            dX[j] = cd{ta, tb};
         }
         __syncthreads();
         block_fft<L, NT>(X, -1, tw);
-        block_fft<L, NT>(dX, -1, tw);
-        const dual wv = (nf * wt) * v;
         for (int n = tid; n <= H; n += NT) {
-            dual bub;
             if (n == 0) {
-                double a = 0.0, b = 0.0;
-                for (int i = 0; i < nw; i++) {
-                    a += sc[12 * nw + i];
-                    b += sc[13 * nw + i];
-                }
-                bub = dual{a, b};
-                const dual m0 = wv * dual{S6[0], S6[6]};
-                c2[0] -= m0.d;
+                double a = 0.0;
+                for (int i = 0; i < nw; i++) a += sc[6 * nw + i];
+                c1[0] -= a;
+                c2[0] -= (wv * dual{S6[0], S6[1]}).d;
             } else {
-                const cd Fn = X[n], Fc = conjg(X[(L - n) & (L - 1)]);
-                const cd tFn = dX[n], tFc = conjg(dX[(L - n) & (L - 1)]);
-                const double iw = 1.0 / (2 * n * kPi * T), iw2 = iw * iw;
+                const cd Fn = X[n], Fq = X[(L - n) & (L - 1)];
+                const double iw = rcp_nr(2 * n * kPi * T), iw2 = iw * iw;
                 const cd tm = twM[n];
-                const cd a = tm * cd{0.5 * (Fn.x + Fc.x), 0.5 * (Fn.y + Fc.y)};
-                const cd ta = tm * cd{0.5 * (tFn.x + tFc.x), 0.5 * (tFn.y + tFc.y)};
-                const dual imJ = (-2.0 * MJ1 + (2.0 * MJ3 + 2.0 * dual{a.y, ta.y} * iw) * iw2) * iw;
-                c2[n] -= (wv * imJ * iw).d;
-                const cd b = tm * cd{0.5 * (Fn.y - Fc.y), -0.5 * (Fn.x - Fc.x)};
-                const cd tb = tm * cd{0.5 * (tFn.y - tFc.y), -0.5 * (tFn.x - tFc.x)};
-                bub = (-2.0 * dchi + dual{b.x, tb.x} * iw2) * iw2;
+                const cd a = tm * cd{0.5 * (Fn.x + Fq.x), 0.5 * (Fn.y - Fq.y)};
+                const cd b = tm * cd{0.5 * (Fn.y + Fq.y), -0.5 * (Fn.x - Fq.x)};
+                c2[n] -= (-2.0 * MJ1 + (2.0 * MJ3 + 2.0 * a.y * iw) * iw2) * iw * iw;
+                c1[n] -= (-2.0 * dchi + b.x * iw2) * iw2;
             }
-            c1[n] -= (2.0 * wv * v * bub).d;
         }
         __syncthreads();
     }
