@@ -767,8 +767,7 @@ int stage_sigma(tpsc_ctx* c)
 int stage_trace_selfG(tpsc_ctx* c)
 {
     if (!c->have_sigma) return fail(c, TPSC_E_ORDER, "traceSelfG before the self-energy");
-    HIPCHK(c, launch_trace_selfG(c->g, c->d, c->mu0, c->mu, 0, c->dev_scalar + 21, c->stream));
-    HIPCHK(c, launch_trace_selfG(c->g, c->d, c->mu0, c->mu, 1, c->dev_scalar + 22, c->stream));
+    HIPCHK(c, launch_trace_selfG0(c->g, c->d, c->mu0, c->dev_scalar + 21, c->stream));
     c->trace_async |= 1;
     c->have_trSG = true;
     return 0;
@@ -777,7 +776,7 @@ int stage_trace_selfG(tpsc_ctx* c)
 // green::traceSelfG2, green.cpp:2929-2997: host_scalar[23]
 int stage_trace_selfG2(tpsc_ctx* c)
 {
-    HIPCHK(c, launch_trace_selfG(c->g, c->d, c->mu0, c->mu, 2, c->dev_scalar + 23, c->stream));
+    HIPCHK(c, launch_trace_selfG(c->g, c->d, c->mu, c->dev_scalar + 23, c->stream));
     c->trace_async |= 2;
     c->have_trSG2 = true;
     return 0;

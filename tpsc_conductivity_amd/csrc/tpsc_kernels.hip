@@ -190,8 +190,7 @@ __device__ __forceinline__ bool last_workgroup(unsigned* ticket, unsigned nblk, 
     return true;
 }
 
-// the Halley step as a kernel of its own, launched after a pass of more than kFusedStepMax
-// workgroups
+// the Halley step as a kernel of its own, launched after a trace pass of more than kFusedStepMax workgroups
 __global__ void __launch_bounds__(256) k_halley_step(const double* part, int n, HalleyState* st, double* mirror)
 {
     __shared__ double sc[3 * 4];
@@ -393,8 +392,8 @@ __device__ __forceinline__ void sum_rule3_term(double c, double w, double sU, do
 // its asymptotic continuation are positive, so the moments carry no cancellation.
 constexpr double kSRRho = 1.0 / 16.0;
 // Ux (and T) come from the root search st, so that a captured pass graph serves every point;
-// a settled search leaves nothing to do.  ticket != null: the workgroup that finishes last takes
-// the Halley step.  srm != null: rows j >= n0(Ux) (all rows whose elements satisfy
+// a settled search leaves nothing to do.  The workgroup that finishes last takes the Halley step;
+// large grids have fewer row groups (kSumRuleGrid).  srm != null: rows j >= n0(Ux) (all rows whose elements satisfy
 // |Ux c/2| <= rho, from the suffix maxima srmax) are not read; workgroup (0, 0) adds their
 // part from the suffix moments srm[n0].
 __global__ void __launch_bounds__(256)
@@ -453,11 +452,7 @@ __global__ void __launch_bounds__(256)
     }
     block_sum_k<3>(acc, sc);
     const int nblk = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
-    if (ticket) {
-        if (last_workgroup(ticket, nblk, b, acc, part)) halley_step_block(part, nblk, st, mirror, sc);
-    } else if (threadIdx.x == 0) {
-        for (int k = 0; k < 3; k++) part[(long)k * nblk + b] = acc[k];
-    }
+    if (last_workgroup(ticket, nblk, b, acc, part)) halley_step_block(part, nblk, st, mirror, sc);
 }
 
 // The whole search in one workgroup: the nk8 (2 nwmax + 1) <= CN * 1024 values of chi0 and their weights are read
@@ -872,6 +867,21 @@ __device__ __forceinline__ void trace_diffG3_term(double wn, double rS, double i
 // pmu (and T, mu0) come from the root search st, so that a captured pass graph serves every
 // point; a settled search leaves nothing to do.  ticket != null: the workgroup that finishes
 // last takes the Halley step.
+// f(j, Sq[j]) for the stored frequencies j = lane, lane + 64, ... < H of a wavefront, in batches of kTD loads issued
+// before any use
+template <typename SelfT, typename Fn>
+__device__ __forceinline__ void each_stored(const SelfT* __restrict__ Sq, int H, int lane, Fn&& f)
+{
+    int j = lane;
+    for (; j + (kTD - 1) * 64 < H; j += kTD * 64) {
+        SelfT v[kTD];
+#pragma unroll
+        for (int u = 0; u < kTD; u++) v[u] = Sq[j + u * 64];
+#pragma unroll
+        for (int u = 0; u < kTD; u++) f(j + u * 64, v[u]);
+    }
+    for (; j < H; j += 64) f(j, Sq[j]);
+}
 template <typename SelfT>
 __global__ void __launch_bounds__(256)
     k_trace_diffG3(const double* __restrict__ ekw, const double* __restrict__ wq, const SelfT* __restrict__ Self,
@@ -883,33 +893,20 @@ __global__ void __launch_bounds__(256)
     if (st->status != kRootRunning) return;
     const double pmu = st->x, T = st->T, mu0 = st->mu0;
     const int lane = threadIdx.x & 63;
-    const int q = blockIdx.x * kTraceK + (threadIdx.x >> 6);
     const int H = Nw / 2;
     double acc[3] = {0.0, 0.0, 0.0};
+    const int q = blockIdx.x * kTraceK + (threadIdx.x >> 6);
     if (q < nk8) {
         const double Si = Sinf[0];
         const double e = ekw[q], w = 2.0 * wq[q];
         const double s2 = Sinf2[q], s3 = Sinf3[q], s4 = Sinf4[q];
-        const SelfT* Sq = Self + (long)q * H;
         const double c = e - mu0;
-        int j = lane;
-        for (; j + (kTD - 1) * 64 < H; j += kTD * 64) {
-            SelfT v[kTD];
-#pragma unroll
-            for (int u = 0; u < kTD; u++) v[u] = Sq[j + u * 64];
-#pragma unroll
-            for (int u = 0; u < kTD; u++) {
-                const double wn = (2 * (j + u * 64) + 1) * kPi * T;
-                const cd s = sigma_kw(v + u, 0, Si, s2, s3, wn);
-                trace_diffG3_term(wn, s.x, s.y, e, c, w, mu0, pmu, acc);
-            }
-        }
-        for (; j < H; j += 64) {
+        each_stored(Self + (long)q * H, H, lane, [&](int j, SelfT raw) {
             const double wn = (2 * j + 1) * kPi * T;
-            const cd s = sigma_kw(Sq, j, Si, s2, s3, wn);
+            const cd s = sigma_kw(&raw, 0, Si, s2, s3, wn);
             trace_diffG3_term(wn, s.x, s.y, e, c, w, mu0, pmu, acc);
-        }
-        for (; j <= Nw; j += 64) {
+        });
+        for (int j = lane + ((H - lane + 63) / 64) * 64; j <= Nw; j += 64) {
             const double wn = (2 * j + 1) * kPi * T;
             const double iw = rcp_nr(wn), iw2 = iw * iw;
             trace_diffG3_term(wn, (-s2 + s4 * iw2) * iw2, (-Si + s3 * iw2) * iw, e, c, w, mu0, pmu, acc);
@@ -961,46 +958,66 @@ __global__ void __launch_bounds__(kSearchThreads)
     });
 }
 
-// which = 0: Tr Sigma G0 main sum (green.cpp:3018-3051); 1: its Sigma_inf correction
-// (:3053-3084, the n < Nw/2 terms plus one per k); 2: Tr Sigma G (green.cpp:2944-2976)
+// Tr Sigma G0 (green.cpp:3018-3084) in one pass over Sigma: part[b] its main sum, part[nblk + b] the Sigma_inf correction
+// (the n < Nw/2 terms plus one per k).  256^2 x 2048: 32 us mixed, 61 FP64 (a pass each: 2 x 27, 2 x 53)
+template <typename SelfT>
+__global__ void __launch_bounds__(256)
+    k_trace_selfG0(const double* __restrict__ ekw, const double* __restrict__ wq, const SelfT* __restrict__ Self,
+                   const double* __restrict__ Sinf2, const double* __restrict__ Sinf3, const double* __restrict__ Sinf,
+                   int nk8, int Nw, double T, double mu0, double nk02, double* part)
+{
+    __shared__ double sc[2 * 4];
+    const int lane = threadIdx.x & 63;
+    const int q = blockIdx.x * kTraceK + (threadIdx.x >> 6);
+    double acc[2] = {0.0, 0.0};
+    if (q < nk8) {
+        const double Si = Sinf[0], s2 = Sinf2[q], s3 = Sinf3[q];
+        const double x = ekw[q] - mu0, w = wq[q] / nk02;
+        each_stored(Self + (long)q * (Nw / 2), Nw / 2, lane, [&](int j, SelfT raw) {
+            const double wn = (2 * j + 1) * kPi * T;
+            const cd s = sigma_kw(&raw, 0, Si, s2, s3, wn);
+            const double r = rcp_nr(wn * wn + x * x);
+            acc[0] += r * (s.y * wn - s.x * x);
+            acc[1] += r;
+        });
+        acc[0] *= w * T * 2;
+        acc[1] *= w * Si * T * 2;
+        if (lane == 0) {
+            if (fabs(x) > 1.0e-12)
+                acc[1] += w * Si * (1.0 / (exp(x / T) + 1.0) - 0.5) / x;
+            else {
+                const double ex = x < 0 ? exp(x / T) : exp(-x / T);
+                acc[1] -= w * Si * ex / ((ex + 1.0) * (ex + 1.0) * T);
+            }
+        }
+    }
+    block_sum_k<2>(acc, sc);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = acc[0];
+        part[gridDim.x + blockIdx.x] = acc[1];
+    }
+}
+// Tr Sigma G (green.cpp:2944-2976)
 template <typename SelfT>
 __global__ void __launch_bounds__(256)
     k_trace_selfG(const double* __restrict__ ekw, const double* __restrict__ wq, const SelfT* __restrict__ Self,
                   const double* __restrict__ Sinf2, const double* __restrict__ Sinf3, const double* __restrict__ Sinf,
-                  int nk8, int Nw, double T, double mu0, double mu, double nk02, int which, double* part)
+                  int nk8, int Nw, double T, double mu, double nk02, double* part)
 {
     __shared__ double sc[16];
     const int lane = threadIdx.x & 63;
     const int q = blockIdx.x * kTraceK + (threadIdx.x >> 6);
-    const int H = Nw / 2;
     double acc = 0.0;
     if (q < nk8) {
-        const double Si = Sinf[0];
-        const double e = ekw[q], w = wq[q];
-        const SelfT* Sq = Self + (long)q * H;
-        for (int j = lane; j < H; j += 64) {
+        const double Si = Sinf[0], s2 = Sinf2[q], s3 = Sinf3[q];
+        const double x = ekw[q] - mu;
+        each_stored(Self + (long)q * (Nw / 2), Nw / 2, lane, [&](int j, SelfT raw) {
             const double wn = (2 * j + 1) * kPi * T;
-            if (which == 1) {
-                acc += w * Si * T * 2 / (nk02 * (wn * wn + (e - mu0) * (e - mu0)));
-                if (j == 0) {
-                    if (fabs(e - mu0) > 1.0e-12)
-                        acc += w * Si * (1.0 / (exp((e - mu0) / T) + 1.0) - 0.5) / (e - mu0) / nk02;
-                    else {
-                        const double ex = (e - mu0) < 0 ? exp((e - mu0) / T) : exp(-(e - mu0) / T);
-                        acc -= w * Si * ex / ((ex + 1.0) * (ex + 1.0) * nk02 * T);
-                    }
-                }
-                continue;
-            }
-            const cd s = sigma_kw(Sq, j, Si, Sinf2[q], Sinf3[q], wn);
-            if (which == 0) {
-                const double tmp = w * T * 2 / (nk02 * (wn * wn + (e - mu0) * (e - mu0)));
-                acc += tmp * (s.x * (mu0 - e) + s.y * wn);
-            } else {
-                const double tmp = w * T * 2 / (nk02 * ((wn - s.y) * (wn - s.y) + (e - mu + s.x) * (e - mu + s.x)));
-                acc += tmp * (s.y * wn - s.y * s.y - (e - mu) * s.x - s.x * s.x);
-            }
-        }
+            const cd s = sigma_kw(&raw, 0, Si, s2, s3, wn);
+            const double a = x + s.x, b = wn - s.y;
+            acc += rcp_nr(a * a + b * b) * (s.y * b - s.x * a);
+        });
+        acc *= wq[q] * T * 2 / nk02;
     }
     acc = block_sum(acc, sc);
     if (threadIdx.x == 0) part[blockIdx.x] = acc;
@@ -1396,14 +1413,12 @@ hipError_t launch_halley_init(HalleyState* st, const RootInit& in, double* mirro
 hipError_t launch_sum_rule3_pass(const Grid& g, const DevArrays& d, double sgn, double* mirror, hipStream_t s)
 {
     const double Nq = 4.0 * (g.nk - 1) * (g.nk - 1);
-    const dim3 gr = red_grid(g);
-    const int nblk = (int)(gr.x * gr.y);
-    const bool fused = nblk <= kFusedStepMax;
+    dim3 gr = red_grid(g);
+    while (gr.x * gr.y > (unsigned)kSumRuleGrid && gr.y > 1) gr.y /= 2;
     const bool series = d.srm && g.nk8 * g.nwb >= kSRMinElems;  // the moments exist (launch_sr_moments)
     hipLaunchKernelGGL(k_sum_rule3, gr, dim3(256), 0, s, d.chiw, d.chi0inf, d.chi0inf2, d.wq, (int)g.nk8, g.Nw / 2,
-                       Nq, sgn, d.root, d.part, fused ? d.ticket : nullptr, mirror, series ? d.srm : nullptr,
+                       Nq, sgn, d.root, d.part, d.ticket, mirror, series ? d.srm : nullptr,
                        series ? d.srmax : nullptr);
-    if (!fused) hipLaunchKernelGGL(k_halley_step, dim3(1), dim3(256), 0, s, d.part, nblk, d.root, mirror);
     return hipGetLastError();
 }
 
@@ -1528,13 +1543,12 @@ hipError_t launch_trace_diffG(const Grid& g, const DevArrays& d, double pmu, dou
 hipError_t launch_trace_diffG3_pass(const Grid& g, const DevArrays& d, double* mirror, hipStream_t s)
 {
     const dim3 gr = trace_grid(g);
-    const int nblk = (int)gr.x;
-    const bool fused = nblk <= kFusedStepMax;
+    const bool fused = gr.x <= (unsigned)kFusedStepMax;
     DISPATCH_S(g.prec, {
         hipLaunchKernelGGL(k_trace_diffG3<ST>, gr, dim3(256), 0, s, d.ekw, d.wq, (const ST*)d.Self, d.Sinf2, d.Sinf3,
                            d.Sinf4, d.Sinf, (int)g.nk8, g.Nw, d.root, d.part, fused ? d.ticket : nullptr, mirror);
     });
-    if (!fused) hipLaunchKernelGGL(k_halley_step, dim3(1), dim3(256), 0, s, d.part, nblk, d.root, mirror);
+    if (!fused) hipLaunchKernelGGL(k_halley_step, dim3(1), dim3(256), 0, s, d.part, (int)gr.x, d.root, mirror);
     return hipGetLastError();
 }
 
@@ -1560,16 +1574,27 @@ hipError_t launch_mu_search(const Grid& g, const DevArrays& d, const RootInit& i
     return e;
 }
 
-hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu0, double mu, int which, double* out,
-                              hipStream_t s)
+hipError_t launch_trace_selfG0(const Grid& g, const DevArrays& d, double mu0, double* out, hipStream_t s)
+{
+    const double nk02 = 4.0 * (g.nk - 1) * (g.nk - 1);
+    const dim3 gr = trace_grid(g);
+    DISPATCH_S(g.prec, {
+        hipLaunchKernelGGL(k_trace_selfG0<ST>, gr, dim3(256), 0, s, d.ekw, d.wq, (const ST*)d.Self, d.Sinf2, d.Sinf3,
+                           d.Sinf, (int)g.nk8, g.Nw, g.T, mu0, nk02, d.part);
+    });
+    hipLaunchKernelGGL(k_finalize_k, dim3(2), dim3(256), 0, s, d.part, (int)gr.x, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu, double* out, hipStream_t s)
 {
     const double nk02 = 4.0 * (g.nk - 1) * (g.nk - 1);
     const dim3 gr = trace_grid(g);
     DISPATCH_S(g.prec, {
         hipLaunchKernelGGL(k_trace_selfG<ST>, gr, dim3(256), 0, s, d.ekw, d.wq, (const ST*)d.Self, d.Sinf2, d.Sinf3,
-                           d.Sinf, (int)g.nk8, g.Nw, g.T, mu0, mu, nk02, which, d.part);
+                           d.Sinf, (int)g.nk8, g.Nw, g.T, mu, nk02, d.part);
     });
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, d.part, (int)(gr.x * gr.y), out);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, d.part, (int)gr.x, out);
     return hipGetLastError();
 }
 

@@ -151,11 +151,12 @@ struct Grid {
 constexpr int kRedBlocks = 1024;
 constexpr int kRowGroups = 32;       // frequency-row groups of the reduction grids
 constexpr int kPartCap = 8192;       // capacity of DevArrays::part
-// Root-search passes over at most this many workgroups take their Halley step in the workgroup
-// that finishes last (one launch per pass: small grids are launch-bound); larger passes launch
-// the step kernel after them, since the tickets of all workgroups on one counter cost more
-// there than the launch they save (256^2 x 2048 with every pass fused: 2.17 against 2.10 ms).
-constexpr int kFusedStepMax = 640;
+// A root-search pass ends with the Halley step of the workgroup that finishes last, through tickets on one counter at
+// 12 ns each.  A sum-rule pass has at most kSumRuleGrid workgroups (256^2 x 2048, moments for the small rows: 11.7 us
+// with 264 against 14.9 with 528, 20.9 with 1056, and 7.9 + 6.2 for a step kernel behind 1056).  Trace passes of more
+// than kFusedStepMax workgroups launch the step kernel after them (256^2 x 2048 mixed: 41 + 6 us with 2097 workgroups,
+// 53, 64 and 68 fused with 1049, 525 and 300, whose wavefronts take several points).
+constexpr int kFusedStepMax = 640, kSumRuleGrid = 300;
 // Grids of at most this many (wedge point, frequency) terms run a whole root search in one workgroup of 1024 threads with
 // the terms in registers (12 and 6 per thread): a search of five passes takes 11-20 us, against 33 (sum rule) and 45 us
 // (mu) in passes.  With 16 and 8 per thread the registers spill: 30 and 33 us.
@@ -237,8 +238,9 @@ hipError_t launch_sigma_slab(const Grid& g, const DevArrays& d, double mu0, hipS
 hipError_t launch_sigma_pencil(const Grid& g, const DevArrays& d, hipStream_t s);
 hipError_t launch_trace_diffG(const Grid& g, const DevArrays& d, double pmu, double mu0, double* out,
                               hipStream_t s);
-hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu0, double mu, int which, double* out,
-                              hipStream_t s);
+// out[0], out[1] = Tr Sigma G0's main sum and its Sigma_inf correction; out[0] = Tr Sigma G
+hipError_t launch_trace_selfG0(const Grid& g, const DevArrays& d, double mu0, double* out, hipStream_t s);
+hipError_t launch_trace_selfG(const Grid& g, const DevArrays& d, double mu, double* out, hipStream_t s);
 hipError_t launch_hf0_bnd(const Grid& g, const DevArrays& d, double mu0, double fact4, hipStream_t s,
                           const double* mu0p = nullptr, double U = 0.0, const double* dsc = nullptr);
 // hV (which 0, into d.h) or f0V (1, into d.f0) for tau_j, 0 < j < Nw
