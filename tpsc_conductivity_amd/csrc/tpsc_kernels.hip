@@ -112,13 +112,13 @@ __global__ void k_halley_init(HalleyState* st, RootInit in, double* mirror)
 // over 5800 terms takes 16 us; five pass kernels take 33 us and their launches.
 constexpr int kSearchThreads = 1024;
 template <typename Pass>
-__device__ __forceinline__ void search_block(HalleyState* st, const HalleyState& s0, double* mirror, int npass,
-                                             const Pass& pass)
+__device__ __forceinline__ HalleyState search_block(const HalleyState& s0, int npass, const Pass& pass)
 {
     constexpr int NWV = kSearchThreads / 64;  // 16: the wavefront sums of one value fill a DPP row
     __shared__ HalleyState s;
     __shared__ double sc[3 * NWV];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x < 3 * NWV) sc[threadIdx.x] = 0.0;  // a smaller workgroup leaves the other wavefronts' places zero
     if (threadIdx.x == 0) s = s0;
     __syncthreads();
     for (int k = 0; k < npass && s.status == kRootRunning; k++) {
@@ -137,10 +137,13 @@ __device__ __forceinline__ void search_block(HalleyState* st, const HalleyState&
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        *st = s;
-        halley_mirror(s, mirror);
-    }
+    return s;
+}
+__device__ __forceinline__ void search_end(const HalleyState& s, HalleyState* st, double* mirror)
+{
+    if (threadIdx.x != 0) return;
+    *st = s;
+    halley_mirror(s, mirror);
 }
 
 // One Halley step after a pass, by one workgroup of 256 threads: the three partial sums of
@@ -481,10 +484,11 @@ __global__ void __launch_bounds__(kSearchThreads)
             }
         }
     }
-    search_block(st, s0, mirror, npass, [&](double Ux, double* acc) {
+    const HalleyState r = search_block(s0, npass, [&](double Ux, double* acc) {
 #pragma unroll
         for (int u = 0; u < CN; u++) sum_rule3_term(c[u], w[u], sgn * Ux, sgn, acc);
     });
+    search_end(r, st, mirror);
 }
 
 // Row moments of the sum-rule terms (one workgroup per row j <= 2 nwmax, stored rows from chi,
@@ -574,9 +578,6 @@ __global__ void __launch_bounds__(1024) k_sr_suffix(double* R, double* rmax, int
     }
 }
 
-// wedge points per thread in k_mu0_root: 16 waves hold the 8385 points of N = 256
-constexpr int kMu0K = 9;
-
 // green0::find_mu (green0.cpp:240-262) in one workgroup, on block-wide sums of the
 // finite-lattice density n(mu) = (2/N^2) sum_wedge w f(eps - mu) (green0.cpp:182-203): every
 // thread sees the same sums, so the control flow stays uniform.  One evaluation gives n - dens
@@ -586,21 +587,23 @@ constexpr int kMu0K = 9;
 // when the root lies outside the bracket or the derivative underflows (no level within ~700 T
 // of the iterate); the derivative-free bracketed search (bracket_root, which widens the
 // interval) then takes over.  out = {found, mu0, evaluations}.
-// Each thread keeps its kMu0K strided wedge points (eps, weight) in registers for all the
+// Each thread keeps its K strided wedge points (eps, weight) in registers for all the
 // evaluations; a padded slot has weight 0 and adds +0.  The launcher sizes the workgroup so
-// that blockDim.x * kMu0K >= nk8.
+// that blockDim.x * K >= nk8: K = 1, 3, 9 for up to 1024, 3072, 9216 points (nine slots, division and LDS
+// reductions for every size: 11.5, 17.1, 29.2 us a search on 45, 2145, 8385 points; now 7.4, 14.0, 28.1).
 // The root goes to out (mapped host memory) and to the device slot mu0v, which the chi0 and
 // h/f0 kernels read, so that the host need not wait for it; a failed search leaves mu0v as it
 // was (the previous mu0).  A preset value (not NaN) is stored without a search.  fw (2 nk8): the
 // Fermi factors of the slabs at that mu0.
+template <int K>
 __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ekw, const double* __restrict__ wq,
                                                    long nk8, double Nk2, double T, double dens, double preset,
                                                    double* out, double* mu0v, double* fw)
 {
     __shared__ double sc[3 * 16];
-    double e[kMu0K], w[kMu0K];
+    double e[K], w[K];
 #pragma unroll
-    for (int k = 0; k < kMu0K; k++) {
+    for (int k = 0; k < K; k++) {
         const long i = threadIdx.x + (long)k * blockDim.x;
         e[k] = (i < nk8) ? ekw[i] : 0.0;
         w[k] = (i < nk8) ? 2.0 * wq[i] / Nk2 : 0.0;
@@ -610,7 +613,7 @@ __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ek
     // G0, h and f0 that do not depend on tau, once per mu0 for all the slabs
     auto weights = [&](double mu) {
 #pragma unroll
-        for (int k = 0; k < kMu0K; k++) {
+        for (int k = 0; k < K; k++) {
             const long i = threadIdx.x + (long)k * blockDim.x;
             if (i < nk8) {
                 const double x = e[k] - mu, ex = exp(-fabs(x) / T), f = 1.0 / (ex + 1.0);
@@ -629,34 +632,28 @@ __global__ void __launch_bounds__(1024) k_mu0_root(const double* __restrict__ ek
         weights(preset);
         return;
     }
-    // v = {n(mu) - dens, n'(mu), n''(mu)}
+    // this thread's part of n(mu), n'(mu), n''(mu); e^{-|x|/T} so that the reciprocal's argument stays within 1..2
     auto density3 = [&](double mup, double* v) {
-        v[0] = v[1] = v[2] = 0.0;
 #pragma unroll
-        for (int k = 0; k < kMu0K; k++) {
-            const double f = 1.0 / (exp((e[k] - mup) * iT) + 1.0), g = f * (1.0 - f) * iT;
+        for (int k = 0; k < K; k++) {
+            const double x = e[k] - mup, ex = exp(-fabs(x) * iT), r = rcp_nr(1.0 + ex);
+            const double f = (x > 0) ? ex * r : r, g = f * (1.0 - f) * iT;
             v[0] += w[k] * f;
             v[1] += w[k] * g;
             v[2] += w[k] * g * (1.0 - 2.0 * f) * iT;
         }
-        block_sum_k<3>(v, sc);
-        v[0] -= dens;
     };
-    HalleyState hs = halley_start(0.0, -8.0, 8.0, 60, 0.0, 0.0);
-    while (hs.status == kRootRunning) {
-        double v[3];
-        density3(hs.x, v);
-        halley_update(hs, v);
-    }
+    const HalleyState hs = search_block(halley_start(0.0, -8.0, 8.0, 60, -dens, 0.0), 60, density3);
     bool ok = hs.status == kRootConverged;
     double root = hs.root;
     int ne = hs.ne;
     if (!ok) {
         int nb = 0;
         auto density = [&](double mup) {
-            double v[3];
+            double v[3] = {0.0, 0.0, 0.0};
             density3(mup, v);
-            return v[0];
+            block_sum_k<3>(v, sc);
+            return v[0] - dens;
         };
         ok = bracket_root(density, 0.0, -8.0, 8.0, nullptr, 1.0e-16, &root, &nb);
         ne += nb;
@@ -951,11 +948,12 @@ __global__ void __launch_bounds__(kSearchThreads)
             }
         }
     }
-    search_block(st, s0, mirror, npass, [&](double pmu, double* acc) {
+    const HalleyState r = search_block(s0, npass, [&](double pmu, double* acc) {
 #pragma unroll
         for (int u = 0; u < CN; u++)
             trace_diffG3_term(wn[u], rS[u], iS[u], e[u], e[u] - s0.mu0, w[u], s0.mu0, pmu, acc);
     });
+    search_end(r, st, mirror);
 }
 
 // Tr Sigma G0 (green.cpp:3018-3084) in one pass over Sigma: part[b] its main sum, part[nblk + b] the Sigma_inf correction
@@ -1484,11 +1482,12 @@ hipError_t launch_reduce_cols2(const double* p1, int ncols1, double* o1, const d
 hipError_t launch_mu0_root(const Grid& g, const DevArrays& d, double n, double preset, double* out, hipStream_t s)
 {
     const double Nk2 = 4.0 * (g.nk - 1) * (g.nk - 1);
-    // fewest waves that hold the wedge at kMu0K points per thread (barriers get cheaper)
-    const long waves = (g.nk8 + 64L * kMu0K - 1) / (64L * kMu0K);
+    const int K = (g.nk8 <= 1024) ? 1 : (g.nk8 <= 3072) ? 3 : 9;
+    const long waves = (g.nk8 + 64L * K - 1) / (64L * K);
     if (waves > 16) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_mu0_root, dim3(1), dim3((unsigned)(64 * waves)), 0, s, d.ekw, d.wq, g.nk8, Nk2, g.T, n,
-                       preset, out, d.mu0v, d.fw);
+    auto* const kern = (K == 1) ? k_mu0_root<1> : (K == 3) ? k_mu0_root<3> : k_mu0_root<9>;
+    hipLaunchKernelGGL(kern, dim3(1), dim3((unsigned)(64 * waves)), 0, s, d.ekw, d.wq, g.nk8, Nk2, g.T, n, preset, out,
+                       d.mu0v, d.fw);
     return hipGetLastError();
 }
 
