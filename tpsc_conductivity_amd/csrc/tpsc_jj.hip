@@ -42,11 +42,44 @@ __device__ __forceinline__ void roots2(cd A, cd B, cd Cc, cd* roots)
     }
 }
 
+// the same for real roots (B^2 - 4 Cc >= 0, A = 1) in real arithmetic: a chain of dependent operations on few threads,
+// so its latency counts (complex roots for every point: k_jj_poles 10.4 us at 16 x 16, 19.2 at 256 x 256; now 7.6, 12.9)
+__device__ __forceinline__ void roots2_real(double B, double Cc, double* roots)
+{
+    const double Rr = sqrt(B * B - 4.0 * Cc);
+    roots[0] = 0.5 * (-B - Rr);
+    roots[1] = 0.5 * (-B + Rr);
+    for (int j = 0; j < 2; j++) {
+        double x = roots[j], yv = x * x + B * x + Cc, p = 2.0 * x + B;
+        const double y0 = yv;
+        for (int it = 0; p != 0.0 && it < 10 && fabs(yv) > 1.0e-16; it++) {
+            const double x2 = x, y2 = yv;
+            x = (p * x - yv) / p;
+            yv = x * x + B * x + Cc;
+            p = 2.0 * x + B;
+            if (fabs(y2) < fabs(yv)) {
+                x = 0.5 * (x + x2);
+                yv = x * x + B * x + Cc;
+                p = 2.0 * x + B;
+            }
+            if (x == x2) break;  // the remaining steps would repeat this one
+        }
+        if (fabs(yv) < fabs(y0)) roots[j] = x;
+    }
+}
+
 __device__ __forceinline__ Poles make_poles(double e, double mu, double Sinf, double CJ1, double T)
 {
     Poles P;
     cd roots[2] = {cd{0, 0}, cd{0, 0}};
-    roots2(cd{1.0, 0.0}, cd{-e + mu, 0.0}, cd{-Sinf, 0.0}, roots);
+    if ((mu - e) * (mu - e) + 4.0 * Sinf >= 0.0) {
+        double r[2];
+        roots2_real(mu - e, -Sinf, r);
+        roots[0].x = r[0];
+        roots[1].x = r[1];
+    } else {
+        roots2(cd{1.0, 0.0}, cd{-e + mu, 0.0}, cd{-Sinf, 0.0}, roots);
+    }
     P.r1 = roots[0];
     P.r2 = roots[1];
     P.a1 = P.r1 / (P.r1 - P.r2);
@@ -56,27 +89,6 @@ __device__ __forceinline__ Poles make_poles(double e, double mu, double Sinf, do
     P.den1 = (P.r1.x > 0 ? cexpd(-(P.r1 / T)) : cexpd(P.r1 / T)) + cd{1.0, 0.0};
     P.den2 = (P.r2.x > 0 ? cexpd(-(P.r2 / T)) : cexpd(P.r2 / T)) + cd{1.0, 0.0};
     return P;
-}
-
-// Dyson G at Matsubara slot s (n = s - Nw/2), with the conjugate Sigma for n < 0
-// (cond_opt.cpp:3354-3407).  dyson_n: the stored frequency index of slot s.
-__device__ __forceinline__ int dyson_n(int s, int H) { return (s < H) ? H - s - 1 : s - H; }
-// from the stored value raw = Self[ki * H + dyson_n(s, H)]
-template <typename SelfT>
-__device__ __forceinline__ cd dyson_G_raw(SelfT raw, int s, int H, double C2, double C3, double Sinf, double e,
-                                          double mu, double T, double& kn)
-{
-    kn = (2.0 * (s - H) + 1) * kPi * T;
-    cd sg = sigma_kw(&raw, 0, Sinf, C2, C3, fabs(kn));
-    if (s < H) sg = conjg(sg);
-    const cd den = cd{0.0 - e, kn} + cd{mu, 0.0} - sg;
-    return sdiv_rcp(T, den);
-}
-template <typename SelfT>
-__device__ __forceinline__ cd dyson_G(const SelfT* __restrict__ Self, long ki, long nk8, int s, int H, double C2,
-                                      double C3, double Sinf, double e, double mu, double T, double& kn)
-{
-    return dyson_G_raw(Self[ki * H + dyson_n(s, H)], s, H, C2, C3, Sinf, e, mu, T, kn);
 }
 
 // Two-pole asymptote data of every Lambda-grid point (cond_opt.cpp:3409-3467): the roots of
@@ -809,27 +821,25 @@ __global__ void k_kx0_rows(const double* __restrict__ ek, const double* __restri
     if (dsc) mu = dsc[kPscMu + 1];
     __shared__ double sc[16];
     const int nk = N / 2 + 1;
-    const long nk8 = (long)nk * (nk + 1) / 2;
     const int l = (blockIdx.x < nk) ? 0 : nk - 1, m = blockIdx.x % nk;
     const long ki = fold_idx(l, m, N);
     const double C2 = Sinf2[ki], C3 = Sinf3[ki], Sinf = Sinfp[0];
     const double e = ek[m + l * nk];
     const int H = L / 2;
-    cd k0 = cd{0, 0};
-    for (int s = threadIdx.x; s < L; s += blockDim.x) {
-        double kn;
-        const cd Gv = dyson_G(Self, ki, nk8, s, H, C2, C3, Sinf, e, mu, T, kn);
-        const cd G0v = T / cd{-e + mu, kn + Sinf / kn};
-        k0 = k0 + (Gv - G0v);
+    // Re of the sum over all slots: twice that of n >= 0, the slots -n-1 being the conjugates (both halves with
+    // divisions: 13.0 us at 16 x 128, 19.9 at 256 x 2048 mixed; now 6.9, 12.3)
+    double k0[1] = {0.0};
+    for (int n = threadIdx.x; n < H; n += blockDim.x) {
+        const double kn = (2 * n + 1) * kPi * T, ik = rcp_nr(kn);
+        const cd sg = sigma_ik(Self[ki * H + n], Sinf, C2, C3, ik);
+        k0[0] += 2.0 * (sdiv_rcp(T, cd{mu - e - sg.x, kn - sg.y}).x - sdiv_rcp(T, cd{mu - e, kn + Sinf * ik}).x);
     }
-    double kv[2] = {k0.x, k0.y};
-    block_sum_k<2>(kv, sc);
-    k0 = cd{kv[0], kv[1]};
+    block_sum_k<1>(k0, sc);
     if (threadIdx.x == 0) {
         const Poles P = make_poles(e, mu, Sinf, 0.0, T);
         const cd f1m = (P.r1.x > 0) ? P.a1 * cexpd(-(P.r1 / T)) / P.den1 : P.a1 / P.den1;
         const cd f2m = (P.r2.x > 0) ? P.a2 * cexpd(-(P.r2 / T)) / P.den2 : P.a2 / P.den2;
-        const double k0r = k0.x + (f1m + f2m).x;
+        const double k0r = k0[0] + (f1m + f2m).x;
         double wt = 2;
         if (m == 0 || m == nk - 1) wt = wt / 2;
         out[blockIdx.x] = -2.0 * wt / ((double)N * N) * d2ek[m + l * nk] * k0r;
