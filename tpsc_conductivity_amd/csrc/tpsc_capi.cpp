@@ -498,10 +498,10 @@ int stage_chi0(tpsc_ctx* c, int nq0, int nw0, bool defer = false)
         dx.chi = c->d.chiw;
         dx.chirt = c->chirt64;
     }
-    // Nothing waits for mu0 on the host.  The tau = 0 slice (one workgroup of 1024 threads)
+    // Nothing waits for mu0 on the host.  The tau = 0 slice (one workgroup)
     // follows the mu0 search in the main stream, so that it takes its CU before the slab kernel
-    // on the side stream fills the chip: alone it runs ~240 us at N = 256, behind the slab
-    // kernel's workgroups more than twice that, and the chi0 pencils wait for it.
+    // on the side stream fills the chip: alone it runs ~75 us at N = 256, behind the slab
+    // kernel's workgroups (185-250 us) their time more, and the chi0 pencils wait for it.
     if ((rc = fork_side(c))) return rc;
     prof_begin(c, "chi0_slab", c->side);
     HIPCHK(c, launch_chi0_slab(gx, dx, c->side));

@@ -1,20 +1,20 @@
 // tpsc_kernels.hip -- HIP kernels of the TPSC hot path for gfx950.
 //
-// Stage map (tpsc_jj.hip holds the Lambda pencils; reference = dbergeron1/TPSC_conductivity):
-//   k_chi0_tau0, k_chi0_slab     chi0.cpp:310-559   G0(k,+-tau) -> G(r,+-tau) -> chi0(r,tau) -> chi0(q,tau)
-
-//   k_sum_rule                   chi.cpp:738-830    sum-rule traces (one candidate U per launch)
+// Stage map (tpsc_tau.hip holds the chi0, V and Sigma pencils, tpsc_jj.hip the Lambda pencils; reference =
+// dbergeron1/TPSC_conductivity):
 //   k_mu0_root                   green0.cpp:182-203, 240-262 finite-lattice density and the mu0 root
-//   k_vertex_slab/_pencil        chi.cpp:85-170     V(r,tau)
-//   k_sigma_bnd/_slab/_pencil    green.cpp:1743-2018 Sigma(k,iwn) moments + remainder
-//   k_trace_diffG, k_trace_selfG green.cpp:2929-3182 traces for mu and consistency checks
+//   k_chi0_tau0, k_chi0_slab     chi0.cpp:310-559   G0(k,+-tau) -> G(r,+-tau) -> chi0(r,tau) -> chi0(q,tau)
+//   k_sum_rule*, k_sr_*          chi.cpp:738-830    sum-rule traces and the searches for Usp, Uch
+//   k_vertex_slab                chi.cpp:85-170     V(r,iqn)
+//   k_sigma_bnd, k_sigma_slab    green.cpp:1743-1892 Sigma(k,tau), end values and slopes
+//   k_trace_*, k_mu_search       green.cpp:2929-3282 traces for mu and consistency checks
 //   k_hf0_bnd, k_hV_slab         cond_opt.cpp:2584-3180 Lambda_jj: hV, f0V
 // Slab kernels hold one (nk x nk) slab in LDS (151 KB at N=256 in FP64) and transform it with
-// register FFTs of line pairs; pencil kernels hold one tau-pencil per workgroup.
+// register FFTs of line pairs.
 // Precision: S is the storage and slab-arithmetic type of the tau arrays (chi0(q,tau),
-// chi0(r,tau), V, Sigma(k,tau), h, f0); chi0(q,iqn) is stored in FP64 in both paths.  S = double is the FP64 path.  S = float is the mixed path: the
-// slab transforms and pointwise products run in FP32, while the tau = 0 / beta boundary data,
-// the spline moments, the tail moments, the pencil Fourier sums, the root-finder reductions
+// chi0(r,tau), V, Sigma(k,tau), h, f0); chi0(q,iqn) is stored in FP64 in both paths.  S = double
+// is the FP64 path.  S = float is the mixed path: the slab transforms and pointwise products run
+// in FP32, while the tau = 0 / beta boundary data, the spline moments, the tail moments, the pencil Fourier sums, the root-finder reductions
 // and the Lambda_jj Matsubara sums stay in FP64.  Self holds the remainder R(k,n) as FP64
 // complex (S = double) or the assembled Sigma(k,iwn) as FP32 complex (S = float).
 #include <algorithm>
@@ -1186,7 +1186,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
 // phases run over the wedge: one exponential serves (kx, ky) and (ky, kx), and V(r) is read in order.
 // Bound by the two transforms (VALU and LDS).  At 256^2 x 2048 the h and f0 slices took 976 + 844 us (FP64)
 // and 628 + 399 us (FP32) as two kernels with h, f0 in global memory between them, two exponentials and
-// two divisions per point and index; now 2 x 513 and 2 x 374 us beside the self-energy pencil.
+// two divisions per point and index; now 2 x 452 and 2 x 295 us beside the self-energy kernels (FP32 alone: 195).
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     k_hV_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,
