@@ -1077,23 +1077,26 @@ __global__ void __launch_bounds__(1024) k_reduce_cols2(const double* __restrict_
 
 // dispersion tables on the device (hamiltonien.cpp:49-68,125-155; green0 wedge weights).  wt[w]: the slab
 // offsets of wedge point (l, m) (low half) and of (m, l) (high half), line stride LD.  vw, vw + nk8:
-// v_x at (kx, ky) = (l, m) and (m, l), 0 at kx = 0 and pi, for the Lambda slabs.
+// v_x at (kx, ky) = (l, m) and (m, l), 0 at kx = 0 and pi, for the Lambda slabs.  Bound by the latency of the sines
+// and cosines: four pairs per point serve every table (3.5 - 5.0 us; evaluated per table 7.8 - 11.8).
 __global__ void k_model(int N, int LD, double t, double tp, double tpp, double t3, double* ek, double* ekw, double* wq,
                         double* er, double* d2ek, double* dek, unsigned* wt, double* vw)
 {
     const int nk = N / 2 + 1;
-    const long nk8 = (long)nk * (nk + 1) / 2, nq = (long)nk * (nk - 2);
+    const long nk8 = (long)nk * (nk + 1) / 2;
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
     const double dk = kPi / (nk - 1);
-    auto vx = [&](int l, int m) {
-        const double kx = l * dk, ky = m * dk;
-        return 2.0 * t * sin(kx) + 4.0 * tp * sin(kx) * cos(ky) + 4.0 * tpp * sin(2 * kx) +
-               4 * t3 * (2.0 * sin(2 * kx) * cos(ky) + cos(2 * ky) * sin(kx));
+    auto vx = [&](double sx, double s2x, double cy, double c2y) {
+        return 2.0 * t * sx + 4.0 * tp * sx * cy + 4.0 * tpp * s2x + 4 * t3 * (2.0 * s2x * cy + c2y * sx);
     };
     if (i < (long)nk * nk) {
         const int l = (int)(i / nk), m = (int)(i % nk);
         const double kx = l * dk, ky = m * dk;
-        const double cx = cos(kx), cy = cos(ky), c2x = cos(2 * kx), c2y = cos(2 * ky);
+        double sx, cx, sy, cy, s2x, c2x, s2y, c2y;
+        sincos(kx, &sx, &cx);
+        sincos(ky, &sy, &cy);
+        sincos(2 * kx, &s2x, &c2x);
+        sincos(2 * ky, &s2y, &c2y);
         ek[i] = -2.0 * t * (cx + cy) - 4.0 * tp * cx * cy - 2.0 * tpp * (c2x + c2y) - 4 * t3 * (c2x * cy + c2y * cx);
         d2ek[i] = 2.0 * t * cx + 4.0 * tp * cx * cy + 8.0 * tpp * c2x + 4 * t3 * (4.0 * c2x * cy + c2y * cx);
         if (m <= l) {
@@ -1102,11 +1105,11 @@ __global__ void k_model(int N, int LD, double t, double tp, double tpp, double t
             wq[w] = wedge_weight(l, m, nk);
             er[w] = (w == 1) ? -t : (w == 2) ? -tp : (w == 3) ? -tpp : (w == 4) ? -t3 : 0.0;
             wt[w] = (unsigned)(m + l * LD) | ((unsigned)(l + m * LD) << 16);
-            vw[w] = (l >= 1 && l <= nk - 2) ? vx(l, m) : 0.0;
-            vw[nk8 + w] = (m >= 1 && m <= nk - 2) ? vx(m, l) : 0.0;
+            vw[w] = (l >= 1 && l <= nk - 2) ? vx(sx, s2x, cy, c2y) : 0.0;
+            vw[nk8 + w] = (m >= 1 && m <= nk - 2) ? vx(sy, s2y, cx, c2x) : 0.0;
         }
+        if (l >= 1 && l <= nk - 2) dek[i - nk] = vx(sx, s2x, cy, c2y);
     }
-    if (i < nq) dek[i] = vx((int)(i / nk) + 1, (int)(i % nk));
 }
 
 // ================================================================== Lambda_jj slabs
@@ -1472,7 +1475,7 @@ hipError_t launch_sr_moments(const Grid& g, const DevArrays& d, hipStream_t s)
 hipError_t launch_model(const Grid& g, const DevArrays& d, double t, double tp, double tpp, double t3,
                         hipStream_t s)
 {
-    const long n = std::max<long>((long)g.nk * g.nk, g.nq);
+    const long n = (long)g.nk * g.nk;
     hipLaunchKernelGGL(k_model, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g.N, slab_dims(g.N).LD, t, tp,
                        tpp, t3, d.ek, d.ekw, d.wq, d.er, d.d2ek, d.dek, d.wt, d.vw);
     return hipGetLastError();
