@@ -22,7 +22,6 @@ constexpr double kPi = 3.14159265358979323846;
 struct cd {
     double x, y;
 };
-__host__ __device__ inline cd mk(double a, double b) { return cd{a, b}; }
 __host__ __device__ inline cd operator+(cd a, cd b) { return cd{a.x + b.x, a.y + b.y}; }
 __host__ __device__ inline cd operator-(cd a, cd b) { return cd{a.x - b.x, a.y - b.y}; }
 __host__ __device__ inline cd operator-(cd a) { return cd{-a.x, -a.y}; }
@@ -126,8 +125,6 @@ struct cplx_of<float> {
 // ---------------------------------------------------------------------------------
 template <typename C>
 __device__ inline C mul_mi(C a) { return C{a.y, -a.x}; }  // a * (-i)
-template <typename C>
-__device__ inline C mul_pi(C a) { return C{-a.y, a.x}; }  // a * (+i)
 
 template <int R, typename C>
 __device__ __forceinline__ void reg_dft(C* v)

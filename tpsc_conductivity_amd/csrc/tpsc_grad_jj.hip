@@ -72,7 +72,6 @@ __device__ __forceinline__ cdual cexpdual(cdual z)
 }
 __device__ __forceinline__ cdual cdl(dual re, dual im) { return cdual{cd{re.v, im.v}, cd{re.d, im.d}}; }
 __device__ __forceinline__ dual rpart(cdual z) { return dual{z.v.x, z.d.x}; }
-__device__ __forceinline__ dual ipart(cdual z) { return dual{z.v.y, z.d.y}; }
 
 // ------------------------------------------------------------------ pointwise integrands
 // h and f0 integrands at tau = t (cond_opt.cpp:2697-2735, 2795-2827), x = e - mu0, v = v_x(k)

@@ -1359,12 +1359,6 @@ hipError_t launch_fill_tw(const DevArrays& d, int L, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_finalize(const double* part, int n, double* out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, part, n, out);
-    return hipGetLastError();
-}
-
 hipError_t launch_chi0_tau0(const Grid& g, const DevArrays& d, hipStream_t s)
 {
     const size_t lds = slab_bytes(g.N, sizeof(double));

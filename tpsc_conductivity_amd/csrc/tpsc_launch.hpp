@@ -257,7 +257,6 @@ hipError_t launch_sum_rows_binned(const double* part, int nrows, int n, const in
                                   hipStream_t s);
 hipError_t launch_kx0_rows(const Grid& g, const DevArrays& d, double mu, hipStream_t s, const double* dsc = nullptr,
                            double* out = nullptr);
-hipError_t launch_finalize(const double* part, int n, double* out, hipStream_t s);
 
 constexpr int kGlocChunks = 64;  // k chunks of k_gloc (partials: kGlocChunks x Nw doubles)
 hipError_t launch_gloc(const Grid& g, const DevArrays& d, double mu, double* part, double* out, hipStream_t s);
