@@ -1,0 +1,24 @@
+"""Stages called on a sub-lattice between full solves: the buffers hold the sub-lattice too, and a full solve
+afterwards gives its first values bit for bit (the solve is deterministic)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+P = dict(n=0.9, T=0.2, params=(-0.15, 0.0, 0.0, 2.0), coarse_pass=False)
+
+
+def test_lambda_on_a_sub_lattice_with_more_workgroups():
+    """64^2 (1023 points) takes 1023 workgroups, the context's 96^2 (2303 points) 768"""
+    from tpsc_conductivity_amd.tpsc import CondOpt
+
+    print("[sub-lattice] 96 x 512, Lambda on 64 x 512", flush=True)
+    g = CondOpt(96, 512, P["n"], P["T"], params=P["params"], coarse_pass=False)
+    g.solve()
+    first = {f: g.get(f) for f in ("chijj1", "chijj2")}
+    g.calc_chiqw_FFT_spline(64, 512)
+    g.calc_chijj_vertex_corr_all_optim()
+    g.solve()
+    for f in first:
+        assert np.array_equal(g.get(f), first[f]), f
+    g.close()

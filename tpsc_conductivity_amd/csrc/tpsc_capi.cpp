@@ -942,7 +942,7 @@ int stage_chijj(tpsc_ctx* c, int ntheta)
         HIPCHK(c, launch_jj_transpose(g, c->d, s));
         prof_end(c);
     }
-    const int nblk = (int)((g.nq + jj_points(g.nq) - 1) / jj_points(g.nq));
+    const int nblk = (int)jj_blocks(g.nq);
     const int nwb = g.nwb;
     double* part = c->d.jjpart;
     double* redrows = c->d.jjred;
@@ -1493,9 +1493,9 @@ int tpsc_create(const tpsc_params* p, tpsc_ctx** out)
     rc |= dalloc(c, &d.hT, (size_t)(Nw + 1) * std::max<long>(nq, 1), es);
     rc |= dalloc(c, &d.f0T, (size_t)(Nw + 1) * std::max<long>(nq, 1), es);
     rc |= dalloc(c, &d.poles, 64 * (size_t)std::max<long>(nq, 1));
-    const long nblk = (nq + jj_points(nq) - 1) / jj_points(nq);
-    rc |= dalloc(c, &d.jjpart, (size_t)std::max<long>(nblk, 1) * 2 * nwb);
-    rc |= dalloc(c, &d.jjscal, (size_t)std::max<long>(nblk, 1) * 4);
+    const size_t nblk = (size_t)jj_blocks_max(nq);
+    rc |= dalloc(c, &d.jjpart, nblk * 2 * nwb);
+    rc |= dalloc(c, &d.jjscal, nblk * 4);
     rc |= dalloc(c, &d.kx0part, 2 * (size_t)nk);
     rc |= dalloc(c, &d.part, kPartCap);
     rc |= dalloc(c, &d.jjred, 2 * (size_t)nwb + 4);
@@ -2220,7 +2220,7 @@ int tpsc_queue_solve(tpsc_ctx* c, const tpsc_params* p, double* slot_dev, bool c
     double* const slot_rows = slot_dev + kPscDoubles;  // reduced Lambda rows, scalar sums, kx0 rows
     HIPCHK(c, launch_kx0_rows(g, d, 0.0, s, psc, slot_rows + 2 * g.nwb + 4));
     HIPCHK(c, launch_jj_poles(g, d, 0.0, s, psc));
-    const int nblk = (int)((g.nq + jj_points(g.nq) - 1) / jj_points(g.nq));
+    const int nblk = (int)jj_blocks(g.nq);
     HIPCHK(c, launch_jj_pencil(g, d, 0.0, d.jjpart, nullptr, 1, s, psc));
     // the column sums straight into the slot, and the point scalars with them (block 0)
     HIPCHK(c, launch_reduce_cols2(d.jjpart, 2 * g.nwb, slot_rows, d.jjscal, 4, slot_rows + 2 * g.nwb, nblk, s, psc,

@@ -859,7 +859,7 @@ hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double
                             hipStream_t s, const double* dsc)
 {
     const int kp = jj_points(g.nq);
-    const unsigned nblk = (unsigned)((g.nq + kp - 1) / kp);
+    const unsigned nblk = (unsigned)jj_blocks(g.nq);
     const PenStep step = pen_step(1.0 / (g.Nw * g.T));
     const JJScale sc = {g.T, kPi * g.T, 1.0 / g.T, 1.0 / ((double)g.N * g.N), 1.0 / (jj_samples(g.Nw) * g.T)};
     DISPATCH_S(g.prec, {

@@ -186,6 +186,10 @@ constexpr int jj_points(long nq)
     const long kp = (nq + 1023) / 1024;
     return kp > 16 ? 16 : kp < 1 ? 1 : (int)kp;
 }
+// Workgroups on nq points, and the most on any lattice of at most nq points: a smaller lattice can have more (1023 points:
+// 1023, 2303 points: 768), and the stages run on sub-lattices of the context's
+constexpr long jj_blocks(long nq) { return (nq + jj_points(nq) - 1) / jj_points(nq); }
+constexpr long jj_blocks_max(long nq) { return nq > 1024 ? 1024 : nq < 1 ? 1 : nq; }
 constexpr int jj_samples(int Nw) { return Nw > 256 ? 8 : Nw > 64 ? Nw / 64 : 1; }
 
 // ---- launchers; each returns hipGetLastError() of its launch
