@@ -22,3 +22,23 @@ def test_lambda_on_a_sub_lattice_with_more_workgroups():
     for f in first:
         assert np.array_equal(g.get(f), first[f]), f
     g.close()
+
+
+def test_angle_bins_of_two_lattices():
+    """the same number of bins on a sub-lattice first: the full lattice's bins are its own"""
+    from tpsc_conductivity_amd.tpsc import CondOpt
+
+    print("[sub-lattice] 32 x 64, 3 bins on 16 x 64 first", flush=True)
+    ref = CondOpt(32, 64, P["n"], P["T"], params=P["params"], coarse_pass=False)
+    ref.solve()
+    ref.calc_chijj_vertex_corr_all_optim(N_theta_k=3)
+    g = CondOpt(32, 64, P["n"], P["T"], params=P["params"], coarse_pass=False)
+    g.solve()
+    g.calc_chiqw_FFT_spline(16, 64)
+    g.calc_chijj_vertex_corr_all_optim(N_theta_k=3)
+    g.solve()
+    g.calc_chijj_vertex_corr_all_optim(N_theta_k=3)
+    for f in ("chijj1_k", "chijj2_k"):
+        assert np.array_equal(g.get(f), ref.get(f)), f
+    ref.close()
+    g.close()

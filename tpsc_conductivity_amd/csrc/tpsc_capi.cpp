@@ -66,7 +66,7 @@ struct tpsc_ctx {
     std::vector<double> chijj1_k, chijj2_k;    // angle-binned Lambda_jj1, Lambda_jj2, [b + n*ntheta]
     std::vector<double> chijj3_k;              // angle-binned Lambda_jj3 on the sparse set
     int* jjbins = nullptr;                     // angle bin of each Lambda point (ntheta > 1)
-    int jjbins_ntheta = 0;
+    int jjbins_ntheta = 0, jjbins_N = 0;       // bins and lattice that it holds
     double* jjpart_t = nullptr;                // binned partial rows and their reduction (ntheta > 1)
     double* jjred_t = nullptr;
     size_t jjpart_t_cap = 0, jjred_t_cap = 0;
@@ -869,14 +869,17 @@ int grow(tpsc_ctx* c, double** buf, size_t* cap, size_t n)
 // with theta = atan((N/2 - m)/(N/2 - l - 1)) (cond_opt.cpp:3174, 3792-3793), on the host
 int angle_bins(tpsc_ctx* c, int ntheta)
 {
-    if (c->jjbins && c->jjbins_ntheta == ntheta) return 0;
     const Grid& g = c->g;
+    if (c->jjbins && c->jjbins_ntheta == ntheta && c->jjbins_N == g.N) return 0;
+    c->jjbins_ntheta = 0;  // of no table until the copy below has ended
     if (!c->jjbins) {
-        if (hipMalloc((void**)&c->jjbins, sizeof(int) * (size_t)std::max<long>(g.nq, 1)) != hipSuccess) {
+        const int nk = c->p.nk0 / 2 + 1;  // room for the context's own lattice, whichever comes first
+        const size_t bytes = sizeof(int) * (size_t)std::max(nk * (nk - 2), 1);
+        if (hipMalloc((void**)&c->jjbins, bytes) != hipSuccess) {
             c->jjbins = nullptr;
             return fail(c, TPSC_E_NOMEM, "device allocation failed");
         }
-        c->dev_bytes += sizeof(int) * (size_t)std::max<long>(g.nq, 1);
+        c->dev_bytes += bytes;
     }
     const int nk0 = g.N;
     const double Dtheta = kPi / (2.0 * ntheta);
@@ -889,6 +892,7 @@ int angle_bins(tpsc_ctx* c, int ntheta)
     }
     HIPCHK(c, hipMemcpy(c->jjbins, b.data(), sizeof(int) * g.nq, hipMemcpyHostToDevice));
     c->jjbins_ntheta = ntheta;
+    c->jjbins_N = g.N;
     return 0;
 }
 
