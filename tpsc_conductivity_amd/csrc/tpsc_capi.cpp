@@ -2010,7 +2010,8 @@ int tpsc_gwn_local(tpsc_ctx* c, double* out)
     const Grid& g = c->g;
     const int H = g.Nw / 2;
     if (!c->gloc_buf) {
-        int rc = dalloc(c, &c->gloc_buf, (size_t)(kGlocChunks + 1) * 2 * H);
+        // for the context's own grid, whichever comes first
+        int rc = dalloc(c, &c->gloc_buf, (size_t)(kGlocChunks + 1) * c->p.Nw0);
         if (rc) return rc;
     }
     double* res = c->gloc_buf + (size_t)kGlocChunks * 2 * H;
