@@ -2138,7 +2138,8 @@ int tpsc_keep_chi_tau(tpsc_ctx* c, int on)
     c->keep_chi_tau = on != 0;
     if (on && !c->chi_tau) {
         const size_t n = (size_t)(c->p.Nw0 / 2 + 1) * ((long)(c->p.nk0 / 2 + 1) * (c->p.nk0 / 2 + 2) / 2);
-        HIPCHK(c, hipMalloc((void**)&c->chi_tau, n * elem_bytes(c)));
+        // FP64 also in the mixed path, whose strongly enhanced points run the chi0 stage in FP64
+        HIPCHK(c, hipMalloc((void**)&c->chi_tau, n * sizeof(double)));
     }
     return 0;
 }
