@@ -65,7 +65,9 @@ struct tpsc_ctx {
     int ntheta = 1;                            // angle bins of the last Lambda_jj call
     std::vector<double> chijj1_k, chijj2_k;    // angle-binned Lambda_jj1, Lambda_jj2, [b + n*ntheta]
     std::vector<double> chijj3_k;              // angle-binned Lambda_jj3 on the sparse set
-    int* jjbins = nullptr;                     // angle bin of each Lambda point (ntheta > 1)
+    int* jjbins = nullptr;                     // angle bin of each Lambda point (ntheta > 1), and behind it
+    JJGroups jjgroups;                         // the points grouped by bin and
+    const int* jjrow0 = nullptr;               // each bin's first group
     int jjbins_ntheta = 0, jjbins_N = 0;       // bins and lattice that it holds
     double* jjpart_t = nullptr;                // binned partial rows and their reduction (ntheta > 1)
     double* jjred_t = nullptr;
@@ -866,31 +868,54 @@ int grow(tpsc_ctx* c, double** buf, size_t* cap, size_t n)
 }
 
 // the angle bin of every Lambda point (kx index l + 1, ky index m): floor(theta / (pi/(2 ntheta)))
-// with theta = atan((N/2 - m)/(N/2 - l - 1)) (cond_opt.cpp:3174, 3792-3793), on the host
+// with theta = atan((N/2 - m)/(N/2 - l - 1)) (cond_opt.cpp:3174, 3792-3793), on the host; and the points in
+// the order of their bins, in groups of at most jj_points of one bin for the Lambda pencils: group g holds
+// order[first[g]] .. order[first[g+1] - 1], bin b the groups row0[b] .. row0[b+1] - 1
 int angle_bins(tpsc_ctx* c, int ntheta)
 {
     const Grid& g = c->g;
     if (c->jjbins && c->jjbins_ntheta == ntheta && c->jjbins_N == g.N) return 0;
     c->jjbins_ntheta = 0;  // of no table until the copy below has ended
+    // one table of four parts, with room for the context's own lattice, whichever comes first
+    const int nk = c->p.nk0 / 2 + 1, nq0 = std::max(nk * (nk - 2), 1);
+    const int oorder = nq0, ofirst = 2 * nq0, orow = ofirst + (int)jj_blocks_max(nq0) + kMaxTheta + 1;
+    const size_t count = (size_t)orow + kMaxTheta + 1;
     if (!c->jjbins) {
-        const int nk = c->p.nk0 / 2 + 1;  // room for the context's own lattice, whichever comes first
-        const size_t bytes = sizeof(int) * (size_t)std::max(nk * (nk - 2), 1);
-        if (hipMalloc((void**)&c->jjbins, bytes) != hipSuccess) {
+        if (hipMalloc((void**)&c->jjbins, sizeof(int) * count) != hipSuccess) {
             c->jjbins = nullptr;
             return fail(c, TPSC_E_NOMEM, "device allocation failed");
         }
-        c->dev_bytes += bytes;
+        c->dev_bytes += sizeof(int) * count;
     }
-    const int nk0 = g.N;
+    const int nk0 = g.N, kp = jj_points(g.nq);
     const double Dtheta = kPi / (2.0 * ntheta);
-    std::vector<int> b(g.nq);
+    std::vector<int> tab(count, 0);
+    std::vector<std::vector<int>> of(ntheta);
     for (long q = 0; q < g.nq; q++) {
         const int l = (int)(q / g.nk), m = (int)(q % g.nk);
         const double th = atan((1.0 * (nk0 / 2 - m)) / (nk0 / 2 - l - 1));
-        int it = (int)floor(th / Dtheta);
-        b[q] = std::min(std::max(it, 0), ntheta - 1);
+        const int it = std::min(std::max((int)floor(th / Dtheta), 0), ntheta - 1);
+        tab[q] = it;
+        of[it].push_back((int)q);
     }
-    HIPCHK(c, hipMemcpy(c->jjbins, b.data(), sizeof(int) * g.nq, hipMemcpyHostToDevice));
+    int* const order = tab.data() + oorder;
+    int* const first = tab.data() + ofirst;
+    int* const row0 = tab.data() + orow;
+    int n = 0, i = 0;
+    for (int b = 0; b < ntheta; b++) {
+        // neighbouring groups take neighbouring points at the same time, as the workgroups do without bins
+        const int nb = (int)of[b].size(), ng = (nb + kp - 1) / kp;
+        row0[b] = n;
+        for (int k = 0; k < ng; k++) {
+            first[n++] = i;
+            for (int p = k; p < nb; p += ng) order[i++] = of[b][p];
+        }
+    }
+    row0[ntheta] = n;
+    first[n] = i;
+    HIPCHK(c, hipMemcpy(c->jjbins, tab.data(), sizeof(int) * count, hipMemcpyHostToDevice));
+    c->jjgroups = JJGroups{c->jjbins + oorder, c->jjbins + ofirst, n};
+    c->jjrow0 = c->jjbins + orow;
     c->jjbins_ntheta = ntheta;
     c->jjbins_N = g.N;
     return 0;
@@ -946,25 +971,26 @@ int stage_chijj(tpsc_ctx* c, int ntheta)
         HIPCHK(c, launch_jj_transpose(g, c->d, s));
         prof_end(c);
     }
-    const int nblk = (int)jj_blocks(g.nq);
     const int nwb = g.nwb;
-    double* part = c->d.jjpart;
-    double* redrows = c->d.jjred;
-    const int* bins = nullptr;
+    double *part = c->d.jjpart, *scal = c->d.jjscal, *redrows = c->d.jjred;
+    JJGroups gr;
     if (ntheta > 1) {
         if ((rc = angle_bins(c, ntheta))) return rc;
-        if ((rc = grow(c, &c->jjpart_t, &c->jjpart_t_cap, (size_t)nblk * 2 * nwb * ntheta))) return rc;
+        gr = c->jjgroups;
+        if ((rc = grow(c, &c->jjpart_t, &c->jjpart_t_cap, (size_t)gr.n * (2 * nwb + 4)))) return rc;
         if ((rc = grow(c, &c->jjred_t, &c->jjred_t_cap, (size_t)2 * nwb * ntheta))) return rc;
         part = c->jjpart_t;
+        scal = part + (size_t)gr.n * 2 * nwb;
         redrows = c->jjred_t;
-        bins = c->jjbins;
     }
     if ((rc = join_side(c))) return rc;
     prof_begin(c, "jj_pencil");
-    HIPCHK(c, launch_jj_pencil(g, c->d, c->mu, part, bins, ntheta, s));
+    HIPCHK(c, launch_jj_pencil(g, c->d, c->mu, part, scal, gr, s));
     prof_end(c);
-    HIPCHK(c, launch_reduce_cols2(part, 2 * nwb * ntheta, redrows, c->d.jjscal, 4, c->d.jjred + 2 * nwb, nblk,
-                                  c->stream));
+    if (ntheta > 1)
+        HIPCHK(c, launch_reduce_bins(part, 2 * nwb, c->jjrow0, ntheta, redrows, scal, gr.n, c->d.jjred + 2 * nwb, s));
+    else
+        HIPCHK(c, launch_reduce_cols2(part, 2 * nwb, redrows, scal, 4, c->d.jjred + 2 * nwb, (int)jj_blocks(g.nq), s));
     std::vector<double> red(2 * nwb * ntheta), sc4(4), rows(2 * g.nk);
     HIPCHK(c, hipMemcpyAsync(red.data(), redrows, sizeof(double) * red.size(), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(sc4.data(), c->d.jjred + 2 * nwb, sizeof(double) * 4, hipMemcpyDeviceToHost, c->stream));
@@ -2227,7 +2253,7 @@ int tpsc_queue_solve(tpsc_ctx* c, const tpsc_params* p, double* slot_dev, bool c
     HIPCHK(c, launch_kx0_rows(g, d, 0.0, s, psc, slot_rows + 2 * g.nwb + 4));
     HIPCHK(c, launch_jj_poles(g, d, 0.0, s, psc));
     const int nblk = (int)jj_blocks(g.nq);
-    HIPCHK(c, launch_jj_pencil(g, d, 0.0, d.jjpart, nullptr, 1, s, psc));
+    HIPCHK(c, launch_jj_pencil(g, d, 0.0, d.jjpart, d.jjscal, JJGroups{}, s, psc));
     // the column sums straight into the slot, and the point scalars with them (block 0)
     HIPCHK(c, launch_reduce_cols2(d.jjpart, 2 * g.nwb, slot_rows, d.jjscal, 4, slot_rows + 2 * g.nwb, nblk, s, psc,
                                   kPscDoubles, slot_dev));

@@ -142,10 +142,9 @@ __global__ void k_jj_poles(const double* __restrict__ ek, const double* __restri
 }
 
 // Per-k Lambda_jj contributions (cond_opt.cpp:3179-3822).  Workgroup blk handles the points
-// q = blk + kk*nblk, kk < kp, one at a time, and writes one pair of rows per angle bin b
-// (bins[q], cond_opt.cpp:3792-3793; bin 0 when bins is null):
-// part[(blk*ntheta + b)*2*nwb + n] (bubble) and part[(blk*ntheta + b)*2*nwb + nwb + n]
-// (Maki-Thompson).
+// q = blk + kk*nblk, kk < kp, one at a time, or, by angle of k (cond_opt.cpp:3792-3793), the points
+// order[i], first[blk] <= i < first[blk+1], all of one bin (JJGroups), and writes one pair of rows:
+// part[blk*2*nwb + n] (bubble) and part[blk*2*nwb + nwb + n] (Maki-Thompson).
 //
 // Per point, two complex FFTs of pairs of sequences whose transforms have a known symmetry:
 //   (1) the f0V and hV spline moments 6a_j (real) at half-integer frequencies: for real a,
@@ -156,8 +155,8 @@ __global__ void k_jj_poles(const double* __restrict__ ek, const double* __restri
 //       Gn + i conj Jn at tau_j is real for each, G(tau_j) + i J(tau_j) before the two-pole terms.
 // Everything after the products -G(tau) G(-tau) and G(tau) J(-tau) is linear in them: the spline
 // over [0, beta], its integral and the third transform.  The weighted products and end slopes
-// are therefore summed over the points of a bin, and the spline and the transform follow once per
-// bin and workgroup instead of once per point.  The sums of up to 16 points carry their
+// are therefore summed over the points of a workgroup, and the spline and the transform follow once
+// per workgroup instead of once per point.  The sums of up to 16 points carry their
 // rounding along (add_lo), since the spline divides second differences by h^2; up to L = 256 that
 // factor is small and plain sums do.
 // The bubble samples are symmetric about beta/2 (the product is the same in both orders), so
@@ -305,7 +304,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
                 const double* __restrict__ df0V, const double* __restrict__ hVb, const double* __restrict__ f0Vb,
                 const JJPoles* __restrict__ poles, const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
                 const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, PenStep g, JJScale u, double mu,
-                const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS, double* part, double* scal, const int* __restrict__ bins, int ntheta,
+                const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS, double* part, double* scal, JJGroups gr,
                 int kp, const double* __restrict__ dsc)
 {
     if (dsc) mu = dsc[kPscMu + 1];
@@ -329,292 +328,283 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
     JJPoint c;
     c.Sinf = Sinfp[0];
     double k0acc = 0.0, inf1 = 0.0, inf2 = 0.0, inf4 = 0.0;
-    for (int b = 0; b < ntheta; b++) {
-        // sums of the products at j = beta + NT m: bubble (j <= L/2) in registers, Maki-Thompson in the thread's
-        // own LDS cells
-        double aB[4], aH = 0.0, aq = 0.0;
-        float lM[8], lB[4];
+    const int i0 = gr.order ? gr.first[blk] : 0, ni = gr.order ? gr.first[blk + 1] - i0 : kp;
+    // sums of the products at j = beta + NT m: bubble (j <= L/2) in registers, Maki-Thompson in the thread's
+    // own LDS cells
+    double aB[4], aH = 0.0, aq = 0.0;
+    float lM[8], lB[4];
 #pragma unroll
-        for (int m = 0; m < 8; m++) {
-            aM[m * NT + tid] = 0.0;
-            lM[m] = 0.0f;
-        }
+    for (int m = 0; m < 8; m++) {
+        aM[m * NT + tid] = 0.0;
+        lM[m] = 0.0f;
+    }
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
-            aB[m] = 0.0;
-            lB[m] = 0.0f;
-        }
-        if (tid == 0) tot[0] = tot[1] = tot[2] = tot[3] = 0.0;
-        bool any = false;
-        // the workgroups resident on one XCD (consecutive blk) work on consecutive q at the same time and
-        // share the cache lines of Sigma and of the pole data
+    for (int m = 0; m < 4; m++) {
+        aB[m] = 0.0;
+        lB[m] = 0.0f;
+    }
+    if (tid == 0) tot[0] = tot[1] = tot[2] = tot[3] = 0.0;
+    // the workgroups resident on one XCD (consecutive blk) work on consecutive q at the same time and
+    // share the cache lines of Sigma and of the pole data
 #pragma unroll 1
-        for (int kk = 0; kk < kp; kk++) {
-            const int q = blk + kk * nblk;
-            if (q >= nq) break;
-            if (bins && bins[q] != b) continue;
-            any = true;
-            int t = tid;
-            asm volatile("" : "+v"(t));
-            const int l = q / nk, m0 = q - l * nk;
-            const int kl = max(l + 1, m0), km = min(l + 1, m0), ki = kl * (kl + 1) / 2 + km;
-            const double e = ek[m0 + (l + 1) * nk], vq = dek[q];
-            const double wt = (m0 == 0 || m0 == nk - 1) ? 2.0 : 4.0;
-            const double wv = u.nf * wt * vq, wb = 2.0 * wv * vq;
-            const double fb0 = f0Vb[q], fbL = f0Vb[nq + q], hb0 = hVb[q], hbL = hVb[nq + q];
-            const double df0 = df0V[q], dfL = df0V[nq + q], dh0 = dhV[q], dhL = dhV[nq + q];
-            cd v[8];
-            // (1) f0V and hV samples 8 t - 1 .. 8 t + 8, their splines, one packed transform
-            {
-                double y[2][10], M[2][9];
-                const S* const pf = f0T + (long)q * (L + 1) + 8 * t;
-                const S* const ph = hT + (long)q * (L + 1) + 8 * t;
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    y[0][1 + i] = (double)pf[i];
-                    y[1][1 + i] = (double)ph[i];
-                }
-                const int im = (t == 0) ? 0 : -1;
-                const double f_m = (double)pf[im], h_m = (double)ph[im], f_p = (double)pf[8], h_p = (double)ph[8];
-                if (t == 0) {
-                    y[0][1] = fb0;
-                    y[1][1] = hb0;
-                }
-                y[0][0] = f_m;
-                y[1][0] = h_m;
-                // sample 0 of the chunk's left neighbour is the FP64 boundary value (thread 0 alone holds it)
-                y[0][9] = (t == NT - 1) ? fbL : f_p;
-                y[1][9] = (t == NT - 1) ? hbL : h_p;
-                const double d0[2] = {df0, dh0}, dN[2] = {dfL, dhL};
-                pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, nullptr, t);
-                if (t == 0) {
-                    ends[0] = M[0][0];
-                    ends[1] = M[1][0];
-                }
-                if (t == NT - 1) {
-                    ends[2] = M[0][8];
-                    ends[3] = M[1][8];
-                }
-                const cd p = tw[4 * t];  // exp(-8 pi i t / L)
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    v[i] = p * cd{(M[0][i + 1] - M[0][i]) * g.ih, (M[1][i + 1] - M[1][i]) * g.ih};
-            }
-            // exp(-2 pi i (t + 1/2) s / L), s = 1, 2, 4: odd multiples of pi/L come from the half-step table
-            pen_fft_dit<L>(v, Z, tw, conjg(twX[2 * t + 1]), tw[2 * t + 1], tw[4 * t + 2], t);
-            // (2) slots n = t + NT m, m < 4, with D_{L-1-n} from thread NT - 1 - t (row 7 - m)
-            wave_lds_order();
-#pragma unroll
-            for (int m = 0; m < 4; m++) Z[m * PS + t] = v[4 + m];
-            SelfT raw[4];
-            cd ts[4];
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                raw[m] = Self[(long)ki * H + t + NT * m];
-                ts[m] = twS[t + NT * m];
-            }
-            c.e0 = mu - e;
-            c.C2 = Sinf2[ki];
-            c.C3 = Sinf3[ki];
-            c.cj01 = -fb0 - fbL;
-            c.cj1 = -hb0 - hbL;
-            c.cj02 = df0 + dfL;
-            c.cj2 = dh0 + dhL;
-            __syncthreads();
-            c.cj03 = -(ends[0] + ends[2]);
-            c.cj3 = -(ends[1] + ends[3]);
-            double sg = 0.0, s4 = 0.0, s5 = 0.0, sq = 0.0;
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const cd D = v[m], E = Z[(3 - m) * PS + NT - 1 - t];
-                const cd A = cd{0.5 * (D.x + E.x), -0.5 * (D.y - E.y)};
-                const cd B = cd{0.5 * (D.y + E.y), 0.5 * (D.x - E.x)};
-                const double kn = (2 * (t + NT * m) + 1) * u.piT;
-                cd Gn, Jn;
-                double qn0;
-                jj_slot(c, A, B, ts[m], raw[m], kn, u.T, Gn, Jn, qn0);
-                sq += qn0;
-                sg += Gn.x;
-                s4 += kn * Gn.y;
-                s5 -= kn * Jn.y;
-                v[m] = cd{Gn.x + Jn.y, Gn.y + Jn.x};                        // Gn + i conj(Jn)
-                Z[(7 - m) * PS + t] = cd{Gn.x - Jn.y, Jn.x - Gn.y};  // the same of slot -n-1
-                __builtin_amdgcn_sched_barrier(0);  // one slot after the other: fewer registers
-            }
-            aq += wv * sq;
-            k0acc -= 4.0 * wt * u.nf * d2ek[m0 + (l + 1) * nk] * sg;
-            // summed here: the compiler would otherwise hold all their operands up to the end of the point
-            asm volatile("" : "+v"(aq), "+v"(k0acc));
-            // the two sums over the slots that the end slopes need, one value per wavefront
-            s4 = wave_total63(s4);
-            s5 = wave_total63(s5);
-            if (lane == 63) {
-                sc[wave] = s4;
-                sc[W + wave] = s5;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int m = 4; m < 8; m++) v[m] = Z[m * PS + NT - 1 - t];
-            __syncthreads();
-            // (3) to imaginary time: v[m] = G(tau_j) + i J(tau_j), j = beta + NT m
-            pen_fft_dif<L>(v, Z, tw, t);
-            const int beta = pen_beta<L>(t);
-            {
-                // half a slot: exp(-i pi j / L)
-                constexpr double c1 = 0.92387953251128675613, s1 = 0.38268343236508977173, r2 = 0.70710678118654752440;
-                cd w[4];
-                w[0] = conjg(twX[beta]);
-                w[1] = w[0] * cd{c1, -s1};
-                w[2] = w[0] * cd{r2, -r2};
-                w[3] = w[0] * cd{s1, -c1};
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    v[m] = w[m] * v[m];
-                    v[m + 4] = mul_mi(w[m] * v[m + 4]);
-                }
-            }
-            const JJPoles& pp = poles[q];
-            const double Jbeta = pp.Jinf_beta - v[0].y;  // thread 0: J at beta from the slot sum at tau = 0
-            const double t0 = beta * g.h;
-            wave_lds_order();
-            jj_poles_add<8>(v, pp, t0, u.dt, u.beta, Z + PS * pen_row<L>(t) + pen_o<L>(t), NT / 8);
-            // (4) the products; G(tau_{L-j}) of j < L/2 through LDS (own rows: value j at row j mod 8, place j/8)
-            double* const gz = (double*)Z;
-            wave_lds_order();
-#pragma unroll
-            for (int m = 4; m < 8; m++) gz[2 * PS * pen_row<L>(t) + pen_o<L>(t) + (NT / 8) * m] = v[m].x;
-            __syncthreads();
-#pragma unroll
-            for (int m = 0; m < 8; m++) add_lo(aM[m * NT + t], lM[m], wv * (v[m].x * v[m].y));
-            const int rb = NT - beta;  // L - j = rb + NT (7 - m); for beta = 0 the next row up
-            const double* const gr = gz + 2 * PS * (rb & 7) + (rb >> 3);
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const bool z0 = (m == 0) && t == 0;
-                const double gm = z0 ? 0.0 : gr[(NT / 8) * (7 - m)];
-                // at tau = 0: G(0-) = G(0+) + 1
-                const double x = z0 ? -(v[m].x + 1.0) : gm;
-                add_lo(aB[m], lB[m], -wb * (v[m].x * x));
-            }
-            if (t == 0) {
-                aH -= wb * (v[4].x * v[4].x);
-                const double G0 = v[0].x, J0 = v[0].y;
-                double S4 = 0.0, S5 = 0.0;
-#pragma unroll
-                for (int i = 0; i < W; i++) {
-                    S4 += sc[i];
-                    S5 += sc[W + i];
-                }
-                S4 *= 2.0;
-                S5 *= 2.0;
-                const double dGp = S4 + pp.dGp, dGm = -S4 + pp.dGm, dJ0 = S5 + pp.dJ0, dJb = -S5 + pp.dJb;
-                tot[0] += wv * (dGp * J0 + G0 * dJ0);
-                tot[1] += wv * (dGm * Jbeta - (G0 + 1.0) * dJb);
-                tot[2] -= wv * ((G0 + 1.0) * Jbeta);
-                tot[3] += wb * (dGp * (G0 + 1.0) + G0 * dGm);
-                k0acc -= 2.0 * wt * u.nf * d2ek[m0 + (l + 1) * nk] * pp.k0r;
-            }
-        }
-        double* const c1 = part + ((long)blk * ntheta + b) * 2 * NWB;
-        double* const c2 = c1 + NWB;
-        if (!any) {
-            for (int n = tid; n < 2 * NWB; n += NT) c1[n] = 0.0;
-            continue;
-        }
-        // (5) the splines of the summed samples and (6) the packed transform of their moments
+    for (int kk = 0; kk < ni; kk++) {
+        const int q = gr.order ? gr.order[i0 + kk] : blk + kk * nblk;
+        if (q >= nq) break;
         int t = tid;
         asm volatile("" : "+v"(t));
-        const int beta = pen_beta<L>(t);
-        double* const Y1 = (double*)Z;
-        double* const Y2 = Y1 + P8::YS;
-        __syncthreads();
-        float* const l1 = (float*)aM;  // the low-order parts, once the sums are read
-        float* const l2 = l1 + L;
-        double am[8];
-#pragma unroll
-        for (int m = 0; m < 8; m++) am[m] = aM[m * NT + t];
-        __syncthreads();
-#pragma unroll
-        for (int m = 0; m < 8; m++) {
-            const int j = beta + NT * m;
-            Y1[j + (j >> 3)] = am[m];
-            l1[j] = lM[m];
-            if (m < 4) {
-                Y2[j + (j >> 3)] = aB[m];
-                Y2[(L - j) + ((L - j) >> 3)] = aB[m];
-                l2[j] = lB[m];
-                if (j > 0) l2[L - j] = lB[m];
-            }
-        }
-        if (t == 0) {
-            Y1[9 * NT] = tot[2];
-            Y2[H + H / 8] = aH;
-            l2[H] = 0.0f;
-        }
-        __syncthreads();
-        const double MJ1 = Y1[0] - Y1[9 * NT], dchi = tot[3];
+        const int l = q / nk, m0 = q - l * nk;
+        const int kl = max(l + 1, m0), km = min(l + 1, m0), ki = kl * (kl + 1) / 2 + km;
+        const double e = ek[m0 + (l + 1) * nk], vq = dek[q];
+        const double wt = (m0 == 0 || m0 == nk - 1) ? 2.0 : 4.0;
+        const double wv = u.nf * wt * vq, wb = 2.0 * wv * vq;
+        const double fb0 = f0Vb[q], fbL = f0Vb[nq + q], hb0 = hVb[q], hbL = hVb[nq + q];
+        const double df0 = df0V[q], dfL = df0V[nq + q], dh0 = dhV[q], dhL = dhV[nq + q];
         cd v[8];
-        double bsum;
+        // (1) f0V and hV samples 8 t - 1 .. 8 t + 8, their splines, one packed transform
         {
-            double y[2][10], M[2][9], integ[2];
-            float yl[2][10];
+            double y[2][10], M[2][9];
+            const S* const pf = f0T + (long)q * (L + 1) + 8 * t;
+            const S* const ph = hT + (long)q * (L + 1) + 8 * t;
 #pragma unroll
-            for (int k = 0; k < 2; k++) {
-                const double* const Y = (k == 0 ? Y1 : Y2) + 9 * t;
-                const float* const l = (k == 0 ? l1 : l2) + 8 * t;
-                yl[k][0] = (t > 0) ? l[-1] : 0.0f;
-#pragma unroll
-                for (int i = 0; i < 8; i++) yl[k][1 + i] = l[i];
-                yl[k][9] = (t < NT - 1) ? l[8] : (k == 0) ? 0.0f : l2[0];
-                y[k][0] = (t > 0) ? Y[-2] : 0.0;
-#pragma unroll
-                for (int i = 0; i < 8; i++) y[k][1 + i] = Y[i];
-                y[k][9] = Y[9];
+            for (int i = 0; i < 8; i++) {
+                y[0][1 + i] = (double)pf[i];
+                y[1][1 + i] = (double)ph[i];
             }
-            const double d0[2] = {tot[0], dchi}, dN[2] = {tot[1], -dchi};
-            pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, integ, t, yl);
-            bsum = integ[1];
-            if (t == 0) ends[0] = M[0][0];
-            if (t == NT - 1) ends[1] = M[0][8];
+            const int im = (t == 0) ? 0 : -1;
+            const double f_m = (double)pf[im], h_m = (double)ph[im], f_p = (double)pf[8], h_p = (double)ph[8];
+            if (t == 0) {
+                y[0][1] = fb0;
+                y[1][1] = hb0;
+            }
+            y[0][0] = f_m;
+            y[1][0] = h_m;
+            // sample 0 of the chunk's left neighbour is the FP64 boundary value (thread 0 alone holds it)
+            y[0][9] = (t == NT - 1) ? fbL : f_p;
+            y[1][9] = (t == NT - 1) ? hbL : h_p;
+            const double d0[2] = {df0, dh0}, dN[2] = {dfL, dhL};
+            pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, nullptr, t);
+            if (t == 0) {
+                ends[0] = M[0][0];
+                ends[1] = M[1][0];
+            }
+            if (t == NT - 1) {
+                ends[2] = M[0][8];
+                ends[3] = M[1][8];
+            }
+            const cd p = tw[4 * t];  // exp(-8 pi i t / L)
 #pragma unroll
             for (int i = 0; i < 8; i++)
-                v[i] = cd{M[0][i], M[1][i]};
+                v[i] = p * cd{(M[0][i + 1] - M[0][i]) * g.ih, (M[1][i + 1] - M[1][i]) * g.ih};
         }
-        bsum = wave_total63(bsum);
-        aq = wave_total63(aq);
-        if (lane == 63) {
-            sc[2 * W + wave] = bsum;
-            sc[3 * W + wave] = aq;
-        }
-        pen_fft_dit<L>(v, Z, tw, tw[t], tw[2 * t], tw[4 * t], t);
+        // exp(-2 pi i (t + 1/2) s / L), s = 1, 2, 4: odd multiples of pi/L come from the half-step table
+        pen_fft_dit<L>(v, Z, tw, conjg(twX[2 * t + 1]), tw[2 * t + 1], tw[4 * t + 2], t);
+        // (2) slots n = t + NT m, m < 4, with D_{L-1-n} from thread NT - 1 - t (row 7 - m)
         wave_lds_order();
 #pragma unroll
         for (int m = 0; m < 4; m++) Z[m * PS + t] = v[4 + m];
-        __syncthreads();
-        const double MJ3 = ends[0] - ends[1];
-        auto row_n = [&](int n, cd Fn, cd Fq) { jj_rows(c1, c2, n, Fn, Fq, twX[n], MJ1, MJ3, dchi, 2.0 * u.piT, g.ih); };
-        // L - n = NT - t + NT (7 - m); for t = 0 the next row's first column
-        const cd* const zq = Z + NT - t + (t == 0 ? 1 : 0);
+        SelfT raw[4];
+        cd ts[4];
 #pragma unroll
-        for (int m = 0; m < 4; m++)
-            if (t + NT * m > 0) row_n(t + NT * m, v[m], zq[(3 - m) * PS]);
+        for (int m = 0; m < 4; m++) {
+            raw[m] = Self[(long)ki * H + t + NT * m];
+            ts[m] = twS[t + NT * m];
+        }
+        c.e0 = mu - e;
+        c.C2 = Sinf2[ki];
+        c.C3 = Sinf3[ki];
+        c.cj01 = -fb0 - fbL;
+        c.cj1 = -hb0 - hbL;
+        c.cj02 = df0 + dfL;
+        c.cj2 = dh0 + dhL;
+        __syncthreads();
+        c.cj03 = -(ends[0] + ends[2]);
+        c.cj3 = -(ends[1] + ends[3]);
+        double sg = 0.0, s4 = 0.0, s5 = 0.0, sq = 0.0;
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const cd D = v[m], E = Z[(3 - m) * PS + NT - 1 - t];
+            const cd A = cd{0.5 * (D.x + E.x), -0.5 * (D.y - E.y)};
+            const cd B = cd{0.5 * (D.y + E.y), 0.5 * (D.x - E.x)};
+            const double kn = (2 * (t + NT * m) + 1) * u.piT;
+            cd Gn, Jn;
+            double qn0;
+            jj_slot(c, A, B, ts[m], raw[m], kn, u.T, Gn, Jn, qn0);
+            sq += qn0;
+            sg += Gn.x;
+            s4 += kn * Gn.y;
+            s5 -= kn * Jn.y;
+            v[m] = cd{Gn.x + Jn.y, Gn.y + Jn.x};                        // Gn + i conj(Jn)
+            Z[(7 - m) * PS + t] = cd{Gn.x - Jn.y, Jn.x - Gn.y};  // the same of slot -n-1
+            __builtin_amdgcn_sched_barrier(0);  // one slot after the other: fewer registers
+        }
+        aq += wv * sq;
+        k0acc -= 4.0 * wt * u.nf * d2ek[m0 + (l + 1) * nk] * sg;
+        // summed here: the compiler would otherwise hold all their operands up to the end of the point
+        asm volatile("" : "+v"(aq), "+v"(k0acc));
+        // the two sums over the slots that the end slopes need, one value per wavefront
+        s4 = wave_total63(s4);
+        s5 = wave_total63(s5);
+        if (lane == 63) {
+            sc[wave] = s4;
+            sc[W + wave] = s5;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 4; m < 8; m++) v[m] = Z[m * PS + NT - 1 - t];
+        __syncthreads();
+        // (3) to imaginary time: v[m] = G(tau_j) + i J(tau_j), j = beta + NT m
+        pen_fft_dif<L>(v, Z, tw, t);
+        const int beta = pen_beta<L>(t);
+        {
+            // half a slot: exp(-i pi j / L)
+            constexpr double c1 = 0.92387953251128675613, s1 = 0.38268343236508977173, r2 = 0.70710678118654752440;
+            cd w[4];
+            w[0] = conjg(twX[beta]);
+            w[1] = w[0] * cd{c1, -s1};
+            w[2] = w[0] * cd{r2, -r2};
+            w[3] = w[0] * cd{s1, -c1};
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                v[m] = w[m] * v[m];
+                v[m + 4] = mul_mi(w[m] * v[m + 4]);
+            }
+        }
+        const JJPoles& pp = poles[q];
+        const double Jbeta = pp.Jinf_beta - v[0].y;  // thread 0: J at beta from the slot sum at tau = 0
+        const double t0 = beta * g.h;
+        wave_lds_order();
+        jj_poles_add<8>(v, pp, t0, u.dt, u.beta, Z + PS * pen_row<L>(t) + pen_o<L>(t), NT / 8);
+        // (4) the products; G(tau_{L-j}) of j < L/2 through LDS (own rows: value j at row j mod 8, place j/8)
+        double* const gz = (double*)Z;
+        wave_lds_order();
+#pragma unroll
+        for (int m = 4; m < 8; m++) gz[2 * PS * pen_row<L>(t) + pen_o<L>(t) + (NT / 8) * m] = v[m].x;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 8; m++) add_lo(aM[m * NT + t], lM[m], wv * (v[m].x * v[m].y));
+        const int rb = NT - beta;  // L - j = rb + NT (7 - m); for beta = 0 the next row up
+        const double* const gr = gz + 2 * PS * (rb & 7) + (rb >> 3);
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const bool z0 = (m == 0) && t == 0;
+            const double gm = z0 ? 0.0 : gr[(NT / 8) * (7 - m)];
+            // at tau = 0: G(0-) = G(0+) + 1
+            const double x = z0 ? -(v[m].x + 1.0) : gm;
+            add_lo(aB[m], lB[m], -wb * (v[m].x * x));
+        }
         if (t == 0) {
-            double s0 = 0.0, s1 = 0.0;
+            aH -= wb * (v[4].x * v[4].x);
+            const double G0 = v[0].x, J0 = v[0].y;
+            double S4 = 0.0, S5 = 0.0;
 #pragma unroll
             for (int i = 0; i < W; i++) {
-                s0 += sc[2 * W + i];
-                s1 += sc[3 * W + i];
+                S4 += sc[i];
+                S5 += sc[W + i];
             }
-            c1[0] = -s0;
-            c2[0] = -2.0 * s1 * u.beta;
-            int nh = H + t;
-            asm volatile("" : "+v"(nh));
-            row_n(nh, v[4], v[4]);
-            inf1 += 2.0 * dchi;
-            inf2 += 2.0 * MJ1;
-            inf4 -= 2.0 * MJ3;
+            S4 *= 2.0;
+            S5 *= 2.0;
+            const double dGp = S4 + pp.dGp, dGm = -S4 + pp.dGm, dJ0 = S5 + pp.dJ0, dJb = -S5 + pp.dJb;
+            tot[0] += wv * (dGp * J0 + G0 * dJ0);
+            tot[1] += wv * (dGm * Jbeta - (G0 + 1.0) * dJb);
+            tot[2] -= wv * ((G0 + 1.0) * Jbeta);
+            tot[3] += wb * (dGp * (G0 + 1.0) + G0 * dGm);
+            k0acc -= 2.0 * wt * u.nf * d2ek[m0 + (l + 1) * nk] * pp.k0r;
         }
-        __syncthreads();  // Z, sc, ends and tot are free again
+    }
+    double* const c1 = part + (long)blk * 2 * NWB;
+    double* const c2 = c1 + NWB;
+    // (5) the splines of the summed samples and (6) the packed transform of their moments
+    int t = tid;
+    asm volatile("" : "+v"(t));
+    const int beta = pen_beta<L>(t);
+    double* const Y1 = (double*)Z;
+    double* const Y2 = Y1 + P8::YS;
+    __syncthreads();
+    float* const l1 = (float*)aM;  // the low-order parts, once the sums are read
+    float* const l2 = l1 + L;
+    double am[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) am[m] = aM[m * NT + t];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+        const int j = beta + NT * m;
+        Y1[j + (j >> 3)] = am[m];
+        l1[j] = lM[m];
+        if (m < 4) {
+            Y2[j + (j >> 3)] = aB[m];
+            Y2[(L - j) + ((L - j) >> 3)] = aB[m];
+            l2[j] = lB[m];
+            if (j > 0) l2[L - j] = lB[m];
+        }
+    }
+    if (t == 0) {
+        Y1[9 * NT] = tot[2];
+        Y2[H + H / 8] = aH;
+        l2[H] = 0.0f;
+    }
+    __syncthreads();
+    const double MJ1 = Y1[0] - Y1[9 * NT], dchi = tot[3];
+    cd v[8];
+    double bsum;
+    {
+        double y[2][10], M[2][9], integ[2];
+        float yl[2][10];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const double* const Y = (k == 0 ? Y1 : Y2) + 9 * t;
+            const float* const l = (k == 0 ? l1 : l2) + 8 * t;
+            yl[k][0] = (t > 0) ? l[-1] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) yl[k][1 + i] = l[i];
+            yl[k][9] = (t < NT - 1) ? l[8] : (k == 0) ? 0.0f : l2[0];
+            y[k][0] = (t > 0) ? Y[-2] : 0.0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[k][1 + i] = Y[i];
+            y[k][9] = Y[9];
+        }
+        const double d0[2] = {tot[0], dchi}, dN[2] = {tot[1], -dchi};
+        pen_spline<L, NT, 2>(y, g, d0, dN, M, sx, zt, integ, t, yl);
+        bsum = integ[1];
+        if (t == 0) ends[0] = M[0][0];
+        if (t == NT - 1) ends[1] = M[0][8];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            v[i] = cd{M[0][i], M[1][i]};
+    }
+    bsum = wave_total63(bsum);
+    aq = wave_total63(aq);
+    if (lane == 63) {
+        sc[2 * W + wave] = bsum;
+        sc[3 * W + wave] = aq;
+    }
+    pen_fft_dit<L>(v, Z, tw, tw[t], tw[2 * t], tw[4 * t], t);
+    wave_lds_order();
+#pragma unroll
+    for (int m = 0; m < 4; m++) Z[m * PS + t] = v[4 + m];
+    __syncthreads();
+    const double MJ3 = ends[0] - ends[1];
+    auto row_n = [&](int n, cd Fn, cd Fq) { jj_rows(c1, c2, n, Fn, Fq, twX[n], MJ1, MJ3, dchi, 2.0 * u.piT, g.ih); };
+    // L - n = NT - t + NT (7 - m); for t = 0 the next row's first column
+    const cd* const zq = Z + NT - t + (t == 0 ? 1 : 0);
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+        if (t + NT * m > 0) row_n(t + NT * m, v[m], zq[(3 - m) * PS]);
+    if (t == 0) {
+        double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+        for (int i = 0; i < W; i++) {
+            s0 += sc[2 * W + i];
+            s1 += sc[3 * W + i];
+        }
+        c1[0] = -s0;
+        c2[0] = -2.0 * s1 * u.beta;
+        int nh = H + t;
+        asm volatile("" : "+v"(nh));
+        row_n(nh, v[4], v[4]);
+        inf1 += 2.0 * dchi;
+        inf2 += 2.0 * MJ1;
+        inf4 -= 2.0 * MJ3;
     }
     k0acc = wave_total63(k0acc);
     if (lane == 63) sc[wave] = k0acc;
@@ -629,9 +619,10 @@ __global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
     }
 }
 
-// The same for L <= 256 on one wavefront per workgroup (its barriers are free), thread t holding j = t + 64 i
+// The same for L <= 256 on one wavefront per workgroup (its barriers are free), thread t holding j = t + 64 i.  Two waves
+// per SIMD: uncapped, L = 16 and 32 take 276 registers and leave room for one.
 template <int L, typename S, typename SelfT>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64, 2)
     k_jj_pencil_short(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ d2ek,
                       const S* __restrict__ hT, const S* __restrict__ f0T, const double* __restrict__ dhV,
                       const double* __restrict__ df0V, const double* __restrict__ hVb,
@@ -640,7 +631,7 @@ __global__ void __launch_bounds__(64)
                       const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, double T, double mu,
                       const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS,
                       const cd* __restrict__ phT, double* part, double* scal,
-                      const int* __restrict__ bins, int ntheta, int kp, const double* __restrict__ dsc)
+                      JJGroups gr, int kp, const double* __restrict__ dsc)
 {
     if (dsc) mu = dsc[kPscMu + 1];
     constexpr int NT = 64, H = L / 2, NWB = H + 1, PER = (L + NT - 1) / NT;
@@ -660,147 +651,138 @@ __global__ void __launch_bounds__(64)
     JJPoint c;
     c.Sinf = Sinfp[0];
     double k0acc = 0.0, inf1 = 0.0, inf2 = 0.0, inf4 = 0.0;
-    for (int b = 0; b < ntheta; b++) {
-        // every lane holds the sums over the points: end slopes, sample L of the Maki-Thompson spline
-        double aM[PER], aB[PER], aq = 0.0, gd0 = 0.0, gdN = 0.0, YL = 0.0, dchi = 0.0;
+    const int i0 = gr.order ? gr.first[blk] : 0, ni = gr.order ? gr.first[blk + 1] - i0 : kp;
+    // every lane holds the sums over the points: end slopes, sample L of the Maki-Thompson spline
+    double aM[PER], aB[PER], aq = 0.0, gd0 = 0.0, gdN = 0.0, YL = 0.0, dchi = 0.0;
 #pragma unroll
-        for (int i = 0; i < PER; i++) aM[i] = aB[i] = 0.0;
-        bool any = false;
+    for (int i = 0; i < PER; i++) aM[i] = aB[i] = 0.0;
 #pragma unroll 1
-        for (int kk = 0; kk < kp; kk++) {
-            const long q = (long)blk + kk * nblk;
-            if (q >= nq) break;
-            if (bins && bins[q] != b) continue;
-            any = true;
-            const int l = (int)(q / nk), m0 = (int)(q % nk);
-            const long ki = fold_idx(l + 1, m0, N);
-            const double vq = dek[q];
-            const double wt = (m0 == 0 || m0 == nk - 1) ? 2.0 : 4.0;
-            const double wv = nf * wt * vq, wb = 2.0 * wv * vq;
-            const double fb0 = f0Vb[q], fbL = f0Vb[nq + q], hb0 = hVb[q], hbL = hVb[nq + q];
-            const double df0 = df0V[q], dfL = df0V[nq + q], dh0 = dhV[q], dhL = dhV[nq + q];
-            for (int j = tid; j <= L; j += NT) {
-                Y1[j] = (j == 0) ? fb0 : (j == L) ? fbL : (double)f0T[q * (L + 1) + j];
-                Y2[j] = (j == 0) ? hb0 : (j == L) ? hbL : (double)hT[q * (L + 1) + j];
-            }
-            __syncthreads();
-            {
-                double* const ys[2] = {Y1, Y2};
-                const double d0s[2] = {df0, dh0}, dNs[2] = {dfL, dhL};
-                block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, nullptr);
-            }
-            for (int j = tid; j < L; j += NT)
-                X[j] = twX[j] * cd{(Y1[j + 1] - Y1[j]) * ihstep, (Y2[j + 1] - Y2[j]) * ihstep};
-            c.cj03 = -(Y1[0] + Y1[L]);
-            c.cj3 = -(Y2[0] + Y2[L]);
-            c.e0 = mu - ek[m0 + (l + 1) * nk];
-            c.C2 = Sinf2[ki];
-            c.C3 = Sinf3[ki];
-            c.cj01 = -fb0 - fbL;
-            c.cj1 = -hb0 - hbL;
-            c.cj02 = df0 + dfL;
-            c.cj2 = dh0 + dhL;
-            __syncthreads();
-            block_fft_pp<L, NT>(X, Wk, +1, tw);
-            double sg = 0.0, s4 = 0.0, s5 = 0.0, sq = 0.0;
-            for (int n = tid; n < H; n += NT) {
-                const cd F = X[n], E = X[L - 1 - n];
-                const cd A = cd{0.5 * (F.x + E.x), 0.5 * (F.y - E.y)};
-                const cd B = cd{0.5 * (F.y + E.y), -0.5 * (F.x - E.x)};
-                const double kn = (2 * n + 1) * kPi * T;
-                cd Gn, Jn;
-                double qn0;
-                jj_slot(c, A, B, twS[n], Self[ki * H + n], kn, T, Gn, Jn, qn0);
-                sq += qn0;
-                sg += Gn.x;
-                s4 += kn * Gn.y;
-                s5 -= kn * Jn.y;
-                Wk[H + n] = cd{Gn.x + Jn.y, Gn.y + Jn.x};  // Gn + i conj(Jn), and of slot -n-1
-                Wk[H - 1 - n] = cd{Gn.x - Jn.y, Jn.x - Gn.y};
-            }
-            aq += wv * sq;
-            k0acc -= 4.0 * wt * nf * d2ek[m0 + (l + 1) * nk] * sg;
-            s4 = 2.0 * wave_sum(s4);
-            s5 = 2.0 * wave_sum(s5);
-            __syncthreads();
-            block_fft_pp<L, NT>(Wk, X, -1, tw);
-            const JJPoles& pp = poles[q];
-            const double Jbeta = pp.Jinf_beta - Wk[0].y;
-            const double t0 = tid * hstep;
-            cd v[PER];
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                const int j = tid + NT * i;
-                v[i] = (j < L) ? phT[j] * Wk[j] : cd{0.0, 0.0};
-            }
-            if (tid < L) jj_poles_add<PER>(v, pp, t0, dt, iT, X + tid, NT);
-#pragma unroll
-            for (int i = 0; i < PER; i++)
-                if (tid + NT * i < L) X[tid + NT * i] = v[i];
-            __syncthreads();
-            const double G0 = X[0].x, J0 = X[0].y;
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                const int j = tid + NT * i;
-                if (j < L) {
-                    // at tau = 0: G(0-) = G(0+) + 1
-                    const double x = (j == 0) ? -(G0 + 1.0) : X[L - j].x;
-                    aM[i] += wv * (v[i].x * v[i].y);
-                    aB[i] -= wb * (v[i].x * x);
-                }
-            }
-            const double dGp = s4 + pp.dGp, dGm = -s4 + pp.dGm, dJ0 = s5 + pp.dJ0, dJb = -s5 + pp.dJb;
-            gd0 += wv * (dGp * J0 + G0 * dJ0);
-            gdN += wv * (dGm * Jbeta - (G0 + 1.0) * dJb);
-            YL -= wv * ((G0 + 1.0) * Jbeta);
-            dchi += wb * (dGp * (G0 + 1.0) + G0 * dGm);
-            if (tid == 0) k0acc -= 2.0 * wt * nf * d2ek[m0 + (l + 1) * nk] * pp.k0r;
-            __syncthreads();
+    for (int kk = 0; kk < ni; kk++) {
+        const long q = gr.order ? (long)gr.order[i0 + kk] : (long)blk + kk * nblk;
+        if (q >= nq) break;
+        const int l = (int)(q / nk), m0 = (int)(q % nk);
+        const long ki = fold_idx(l + 1, m0, N);
+        const double vq = dek[q];
+        const double wt = (m0 == 0 || m0 == nk - 1) ? 2.0 : 4.0;
+        const double wv = nf * wt * vq, wb = 2.0 * wv * vq;
+        const double fb0 = f0Vb[q], fbL = f0Vb[nq + q], hb0 = hVb[q], hbL = hVb[nq + q];
+        const double df0 = df0V[q], dfL = df0V[nq + q], dh0 = dhV[q], dhL = dhV[nq + q];
+        for (int j = tid; j <= L; j += NT) {
+            Y1[j] = (j == 0) ? fb0 : (j == L) ? fbL : (double)f0T[q * (L + 1) + j];
+            Y2[j] = (j == 0) ? hb0 : (j == L) ? hbL : (double)hT[q * (L + 1) + j];
         }
-        double* const c1 = part + ((long)blk * ntheta + b) * 2 * NWB;
-        double* const c2 = c1 + NWB;
-        if (!any) {
-            for (int n = tid; n < 2 * NWB; n += NT) c1[n] = 0.0;
-            continue;
+        __syncthreads();
+        {
+            double* const ys[2] = {Y1, Y2};
+            const double d0s[2] = {df0, dh0}, dNs[2] = {dfL, dhL};
+            block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, nullptr);
         }
+        for (int j = tid; j < L; j += NT)
+            X[j] = twX[j] * cd{(Y1[j + 1] - Y1[j]) * ihstep, (Y2[j + 1] - Y2[j]) * ihstep};
+        c.cj03 = -(Y1[0] + Y1[L]);
+        c.cj3 = -(Y2[0] + Y2[L]);
+        c.e0 = mu - ek[m0 + (l + 1) * nk];
+        c.C2 = Sinf2[ki];
+        c.C3 = Sinf3[ki];
+        c.cj01 = -fb0 - fbL;
+        c.cj1 = -hb0 - hbL;
+        c.cj02 = df0 + dfL;
+        c.cj2 = dh0 + dhL;
+        __syncthreads();
+        block_fft_pp<L, NT>(X, Wk, +1, tw);
+        double sg = 0.0, s4 = 0.0, s5 = 0.0, sq = 0.0;
+        for (int n = tid; n < H; n += NT) {
+            const cd F = X[n], E = X[L - 1 - n];
+            const cd A = cd{0.5 * (F.x + E.x), 0.5 * (F.y - E.y)};
+            const cd B = cd{0.5 * (F.y + E.y), -0.5 * (F.x - E.x)};
+            const double kn = (2 * n + 1) * kPi * T;
+            cd Gn, Jn;
+            double qn0;
+            jj_slot(c, A, B, twS[n], Self[ki * H + n], kn, T, Gn, Jn, qn0);
+            sq += qn0;
+            sg += Gn.x;
+            s4 += kn * Gn.y;
+            s5 -= kn * Jn.y;
+            Wk[H + n] = cd{Gn.x + Jn.y, Gn.y + Jn.x};  // Gn + i conj(Jn), and of slot -n-1
+            Wk[H - 1 - n] = cd{Gn.x - Jn.y, Jn.x - Gn.y};
+        }
+        aq += wv * sq;
+        k0acc -= 4.0 * wt * nf * d2ek[m0 + (l + 1) * nk] * sg;
+        s4 = 2.0 * wave_sum(s4);
+        s5 = 2.0 * wave_sum(s5);
+        __syncthreads();
+        block_fft_pp<L, NT>(Wk, X, -1, tw);
+        const JJPoles& pp = poles[q];
+        const double Jbeta = pp.Jinf_beta - Wk[0].y;
+        const double t0 = tid * hstep;
+        cd v[PER];
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int j = tid + NT * i;
+            v[i] = (j < L) ? phT[j] * Wk[j] : cd{0.0, 0.0};
+        }
+        if (tid < L) jj_poles_add<PER>(v, pp, t0, dt, iT, X + tid, NT);
+#pragma unroll
+        for (int i = 0; i < PER; i++)
+            if (tid + NT * i < L) X[tid + NT * i] = v[i];
+        __syncthreads();
+        const double G0 = X[0].x, J0 = X[0].y;
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int j = tid + NT * i;
             if (j < L) {
-                Y1[j] = aM[i];
-                Y2[j] = aB[i];
-                if (j == 0) {
-                    Y1[L] = YL;
-                    Y2[L] = aB[0];
-                }
+                // at tau = 0: G(0-) = G(0+) + 1
+                const double x = (j == 0) ? -(G0 + 1.0) : X[L - j].x;
+                aM[i] += wv * (v[i].x * v[i].y);
+                aB[i] -= wb * (v[i].x * x);
             }
         }
-        __syncthreads();
-        const double MJ1 = Y1[0] - Y1[L];
-        double integ[2];
-        {
-            double* const ys[2] = {Y1, Y2};
-            const double d0s[2] = {gd0, dchi}, dNs[2] = {gdN, -dchi};
-            block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, integ);
-        }
-        const double MJ3 = Y1[0] - Y1[L];
-        const double bub0 = wave_sum(integ[1]), q0 = 2.0 * iT * wave_sum(aq);
-        for (int j = tid; j < L; j += NT) X[j] = cd{Y1[j], Y2[j]};
-        __syncthreads();
-        block_fft_pp<L, NT>(X, Wk, -1, tw);
-        for (int n = tid; n <= H; n += NT) {
-            if (n == 0) {
-                c1[0] = -bub0;
-                c2[0] = -q0;
-            } else {
-                jj_rows(c1, c2, n, X[n], X[L - n], twX[n], MJ1, MJ3, dchi, 2.0 * kPi * T, ihstep);
-            }
-        }
-        inf1 += 2.0 * dchi;
-        inf2 += 2.0 * MJ1;
-        inf4 -= 2.0 * MJ3;
+        const double dGp = s4 + pp.dGp, dGm = -s4 + pp.dGm, dJ0 = s5 + pp.dJ0, dJb = -s5 + pp.dJb;
+        gd0 += wv * (dGp * J0 + G0 * dJ0);
+        gdN += wv * (dGm * Jbeta - (G0 + 1.0) * dJb);
+        YL -= wv * ((G0 + 1.0) * Jbeta);
+        dchi += wb * (dGp * (G0 + 1.0) + G0 * dGm);
+        if (tid == 0) k0acc -= 2.0 * wt * nf * d2ek[m0 + (l + 1) * nk] * pp.k0r;
         __syncthreads();
     }
+    double* const c1 = part + (long)blk * 2 * NWB;
+    double* const c2 = c1 + NWB;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const int j = tid + NT * i;
+        if (j < L) {
+            Y1[j] = aM[i];
+            Y2[j] = aB[i];
+            if (j == 0) {
+                Y1[L] = YL;
+                Y2[L] = aB[0];
+            }
+        }
+    }
+    __syncthreads();
+    const double MJ1 = Y1[0] - Y1[L];
+    double integ[2];
+    {
+        double* const ys[2] = {Y1, Y2};
+        const double d0s[2] = {gd0, dchi}, dNs[2] = {gdN, -dchi};
+        block_spline_fixed<L, NT, 2>(ys, hstep, d0s, dNs, ES, integ);
+    }
+    const double MJ3 = Y1[0] - Y1[L];
+    const double bub0 = wave_sum(integ[1]), q0 = 2.0 * iT * wave_sum(aq);
+    for (int j = tid; j < L; j += NT) X[j] = cd{Y1[j], Y2[j]};
+    __syncthreads();
+    block_fft_pp<L, NT>(X, Wk, -1, tw);
+    for (int n = tid; n <= H; n += NT) {
+        if (n == 0) {
+            c1[0] = -bub0;
+            c2[0] = -q0;
+        } else {
+            jj_rows(c1, c2, n, X[n], X[L - n], twX[n], MJ1, MJ3, dchi, 2.0 * kPi * T, ihstep);
+        }
+    }
+    inf1 += 2.0 * dchi;
+    inf2 += 2.0 * MJ1;
+    inf4 -= 2.0 * MJ3;
     k0acc = wave_sum(k0acc);
     if (tid == 0) {
         scal[blk * 4 + 0] = k0acc;
@@ -855,11 +837,11 @@ hipError_t launch_jj_poles(const Grid& g, const DevArrays& d, double mu, hipStre
     return hipGetLastError();
 }
 
-hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double* part, const int* bins, int ntheta,
-                            hipStream_t s, const double* dsc)
+hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double* part, double* scal,
+                            const JJGroups& gr, hipStream_t s, const double* dsc)
 {
     const int kp = jj_points(g.nq);
-    const unsigned nblk = (unsigned)jj_blocks(g.nq);
+    const unsigned nblk = gr.order ? (unsigned)gr.n : (unsigned)jj_blocks(g.nq);
     const PenStep step = pen_step(1.0 / (g.Nw * g.T));
     const JJScale sc = {g.T, kPi * g.T, 1.0 / g.T, 1.0 / ((double)g.N * g.N), 1.0 / (jj_samples(g.Nw) * g.T)};
     DISPATCH_S(g.prec, {
@@ -867,12 +849,12 @@ hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double
             DISPATCH_L_SHORT(g.Nw, hipLaunchKernelGGL((k_jj_pencil_short<LL, SS, ST>), dim3(nblk), dim3(64), 0, s,
                              d.ek, d.dek, d.d2ek, (const SS*)d.hT, (const SS*)d.f0T, d.dhV, d.df0V, d.hVb, d.f0Vb,
                              (const JJPoles*)d.poles, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, g.T, mu,
-                             d.twN, d.twX, d.twS, d.ph, part, d.jjscal, bins, ntheta, kp, dsc));
+                             d.twN, d.twX, d.twS, d.ph, part, scal, gr, kp, dsc));
         } else {
             DISPATCH_L_LONG(g.Nw, hipLaunchKernelGGL((k_jj_pencil<LL, SS, ST>), dim3(nblk), dim3(Pen<LL>::NT), 0, s,
                             d.ek, d.dek, d.d2ek, (const SS*)d.hT, (const SS*)d.f0T, d.dhV, d.df0V, d.hVb, d.f0Vb,
                             (const JJPoles*)d.poles, (const ST*)d.Self, d.Sinf2, d.Sinf3, d.Sinf, g.N, step, sc, mu,
-                            d.twN, d.twX, d.twS, part, d.jjscal, bins, ntheta, kp, dsc));
+                            d.twN, d.twX, d.twS, part, scal, gr, kp, dsc));
         }
     });
     return hipGetLastError();

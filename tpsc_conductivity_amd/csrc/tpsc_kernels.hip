@@ -1059,6 +1059,18 @@ __global__ void __launch_bounds__(1024) k_reduce_cols(const double* __restrict__
 {
     reduce_cols_block(part, nrows, ncols, out, blockIdx.x);
 }
+// row ranges of one table (blockIdx.y < nbins), then all rows of another of four columns
+__global__ void __launch_bounds__(1024) k_reduce_bins(const double* __restrict__ part, int ncols,
+                                                      const int* __restrict__ row0, int nbins, double* out,
+                                                      const double* __restrict__ scal, int nrows, double* oscal)
+{
+    const int b = blockIdx.y;
+    if (b < nbins)
+        reduce_cols_block(part + (long)row0[b] * ncols, row0[b + 1] - row0[b], ncols, out + (long)b * ncols,
+                          blockIdx.x);
+    else if (blockIdx.x == 0)
+        reduce_cols_block(scal, nrows, 4, oscal, 0);
+}
 // two tables of the same row count in one launch (blocks of the first, then of the second);
 // block 0 also copies ncopy doubles from csrc to cdst (null: nothing)
 __global__ void __launch_bounds__(1024) k_reduce_cols2(const double* __restrict__ p1, int ncols1, double* o1,
@@ -1478,6 +1490,14 @@ hipError_t launch_model(const Grid& g, const DevArrays& d, double t, double tp, 
 hipError_t launch_reduce_cols(const double* part, int nrows, int ncols, double* out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_reduce_cols, dim3((ncols + kRedCols - 1) / kRedCols), dim3(1024), 0, s, part, nrows, ncols, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_reduce_bins(const double* part, int ncols, const int* row0, int nbins, double* out, const double* scal,
+                              int nrows, double* oscal, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_reduce_bins, dim3((ncols + kRedCols - 1) / kRedCols, nbins + 1), dim3(1024), 0, s, part, ncols,
+                       row0, nbins, out, scal, nrows, oscal);
     return hipGetLastError();
 }
 

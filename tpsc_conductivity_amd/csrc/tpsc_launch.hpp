@@ -190,6 +190,13 @@ constexpr int jj_points(long nq)
 // 1023, 2303 points: 768), and the stages run on sub-lattices of the context's
 constexpr long jj_blocks(long nq) { return (nq + jj_points(nq) - 1) / jj_points(nq); }
 constexpr long jj_blocks_max(long nq) { return nq > 1024 ? 1024 : nq < 1 ? 1 : nq; }
+// The points of the workgroups of a pencil launch by angle of k: workgroup g < n takes order[first[g]] .. order[first[g+1]
+// - 1], all of one bin, so that it writes one pair of rows (a pair for every bin, mostly zeros: 64 bins at 64^2 x 2048 took
+// 1.07 GB and 1380 us a call, now 18 MB and 815 us).  order null: workgroup g takes every jj_blocks-th point from g.
+struct JJGroups {
+    const int *order = nullptr, *first = nullptr;
+    int n = 0;
+};
 constexpr int jj_samples(int Nw) { return Nw > 256 ? 8 : Nw > 64 ? Nw / 64 : 1; }
 
 // ---- launchers; each returns hipGetLastError() of its launch
@@ -225,6 +232,10 @@ hipError_t launch_mu0_root(const Grid& g, const DevArrays& d, double n, double p
 hipError_t launch_model(const Grid& g, const DevArrays& d, double t, double tp, double tpp, double t3,
                         hipStream_t s);
 hipError_t launch_reduce_cols(const double* part, int nrows, int ncols, double* out, hipStream_t s);
+// out[b*ncols + c]: the sum of column c of part over the rows row0[b] .. row0[b+1] - 1, b < nbins; oscal[c]: of scal
+// (nrows x 4) over all rows
+hipError_t launch_reduce_bins(const double* part, int ncols, const int* row0, int nbins, double* out, const double* scal,
+                              int nrows, double* oscal, hipStream_t s);
 hipError_t launch_reduce_cols2(const double* p1, int ncols1, double* o1, const double* p2, int ncols2, double* o2,
                                int nrows, hipStream_t s, const double* csrc = nullptr, int ncopy = 0,
                                double* cdst = nullptr);
@@ -251,9 +262,9 @@ hipError_t launch_hf0_bnd(const Grid& g, const DevArrays& d, double mu0, double 
 hipError_t launch_hV_slab(const Grid& g, const DevArrays& d, int which, hipStream_t s);
 hipError_t launch_jj_poles(const Grid& g, const DevArrays& d, double mu, hipStream_t s, const double* dsc = nullptr);
 hipError_t launch_jj_transpose(const Grid& g, const DevArrays& d, hipStream_t s);
-// partial rows to part (nblk x ntheta x 2*nwb); bins: the angle bin of each Lambda point, or null
-hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double* part, const int* bins, int ntheta,
-                            hipStream_t s, const double* dsc = nullptr);
+// partial rows to part (workgroups x 2*nwb), k0 and inf sums to scal (workgroups x 4)
+hipError_t launch_jj_pencil(const Grid& g, const DevArrays& d, double mu, double* part, double* scal,
+                            const JJGroups& gr, hipStream_t s, const double* dsc = nullptr);
 // out[i] = (float)in[i], i < n
 hipError_t launch_narrow(const double* in, float* out, long n, hipStream_t s);
 // out[r*ntheta + b]: the sum of row r of part (nrows x n) over the columns k with bins[k] == b
