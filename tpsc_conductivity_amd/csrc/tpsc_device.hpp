@@ -262,10 +262,10 @@ __device__ __forceinline__ void reg_dft(C* v)
 // an immediate, with one select where the rotation wraps (1024 slabs of N = 256 alone on the chip:
 // 41.5 us per 2D transform in FP64, 25.2 in FP32; 48.5 and 27.1 with slots permuted by an exclusive or
 // and offsets computed per access).
-// Against cross-lane radix-2 stages (one FFT per wavefront, shuffles between lanes, a full-period FFT
-// for a line pair), kernel times at 256^2 x 2048 before -> after: FP64 chi0 1004 -> 461 us, vertex 298
-// -> 104, Sigma 1092 -> 362, h/f0 1636 -> 976, hV/f0V 1375 -> 844; FP32 384 -> 264, 115 -> 61, 440 ->
-// 222, 659 -> 628, 758 -> 399 (they overlap on three streams).
+// Kernel times at 256^2 x 2048 (kernel trace; three streams overlap), against cross-lane radix-2 stages (one
+// FFT per wavefront, shuffles between lanes, a full-period FFT for a line pair): FP64 chi0 1004 -> 248 us,
+// vertex 298 -> 94, Sigma 1092 -> 281, h and f0 with hV and f0V 3011 -> 2 x 445; FP32 384 -> 184,
+// 115 -> 57, 440 -> 197, 1417 -> 2 x 290.
 // ---------------------------------------------------------------------------------
 constexpr int slab_A(int N)
 {

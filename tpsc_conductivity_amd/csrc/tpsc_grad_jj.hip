@@ -13,7 +13,6 @@
 //    splines and transforms are linear and run unchanged on the tangent samples; the Dyson G,
 //    the two-pole asymptote (roots of z^2 + (mu - e) z - Sigma_inf, differentiated implicitly),
 //    the products G(tau) J(-tau), G(tau) G(-tau) and the end slopes take the product rule.
-// Straightforward code: this path serves gradient checks and fitting, not the timed solve.
 #include "tpsc_launch.hpp"
 
 namespace tpsc {

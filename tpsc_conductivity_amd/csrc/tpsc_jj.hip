@@ -167,10 +167,10 @@ __global__ void k_jj_poles(const double* __restrict__ ek, const double* __restri
 // from k_jj_poles.
 //
 // L = 512 .. 4096: L/8 threads per point, the transforms of tpsc_pencil.hpp, eight barriers a point.  LDS holds
-// one exchange buffer and the Maki-Thompson sums, 53 KB at L = 2048: three workgroups per CU at 168 registers.
+// one exchange buffer and the Maki-Thompson sums, 53 KB at L = 2048: three workgroups per CU at 160 registers.
 // What bounds it: FP64 VALU issue, then LDS.  With the last spline and transform once per workgroup, half
-// the slots (n >= 0), real poles by two exponentials and no LDS-resident passes, 256^2 x 2048 takes 0.43 ms in FP64
-// and 0.41 mixed (before: 1.55 and 1.48), 256^2 x 4096 mixed 0.90 (3.50), 128^2 x 1024 0.087 (0.40).
+// the slots (n >= 0), real poles by two exponentials and no LDS-resident passes, 256^2 x 2048 takes 0.44 ms in FP64
+// and 0.42 mixed (before: 1.55 and 1.48), 256^2 x 4096 mixed 0.94 (3.50), 128^2 x 1024 0.070 (0.40).
 
 // Scales of the Lambda pencils, formed on the host: T, pi T, beta, 1/N^2 and the threads' stride in tau
 struct JJScale {
@@ -294,18 +294,15 @@ __device__ __forceinline__ void add_lo(double& hi, float& lo, double p)
     hi = s;
 }
 
-#ifndef JJ_OCC
-#define JJ_OCC (L > 2048 ? 2 : 3)
-#endif
 template <int L, typename S, typename SelfT>
-__global__ void __launch_bounds__(Pen<L>::NT, JJ_OCC)
+__global__ void __launch_bounds__(Pen<L>::NT, (L > 2048 ? 2 : 3))
     k_jj_pencil(const double* __restrict__ ek, const double* __restrict__ dek, const double* __restrict__ d2ek,
                 const S* __restrict__ hT, const S* __restrict__ f0T, const double* __restrict__ dhV,
                 const double* __restrict__ df0V, const double* __restrict__ hVb, const double* __restrict__ f0Vb,
                 const JJPoles* __restrict__ poles, const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
                 const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, PenStep g, JJScale u, double mu,
-                const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS, double* part, double* scal, JJGroups gr,
-                int kp, const double* __restrict__ dsc)
+                const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS, double* part, double* scal,
+                JJGroups gr, int kp, const double* __restrict__ dsc)
 {
     if (dsc) mu = dsc[kPscMu + 1];
     using P8 = Pen<L>;
@@ -630,8 +627,8 @@ __global__ void __launch_bounds__(64, 2)
                       const SelfT* __restrict__ Self, const double* __restrict__ Sinf2,
                       const double* __restrict__ Sinf3, const double* __restrict__ Sinfp, int N, double T, double mu,
                       const cd* __restrict__ tw, const cd* __restrict__ twX, const cd* __restrict__ twS,
-                      const cd* __restrict__ phT, double* part, double* scal,
-                      JJGroups gr, int kp, const double* __restrict__ dsc)
+                      const cd* __restrict__ phT, double* part, double* scal, JJGroups gr, int kp,
+                      const double* __restrict__ dsc)
 {
     if (dsc) mu = dsc[kPscMu + 1];
     constexpr int NT = 64, H = L / 2, NWB = H + 1, PER = (L + NT - 1) / NT;

@@ -173,7 +173,8 @@ __device__ __forceinline__ void halley_step_block(const double* part, int n, Hal
 // (stored here by its thread 0) are visible to it; that workgroup resets the ticket for the next pass.  No workgroup
 // waits for another: the others return at once.  The sums are stored at agent scope, past the XCD's L2, and have
 // arrived when the ticket is taken: no workgroup needs a release fence (a write-back of its whole L2), and only the
-// last one acquires.
+// last one acquires.  That order is gfx950's (an agent-scope store is acknowledged past the L2, and s_waitcnt waits for
+// it), not the language's: only such stores may carry a pass's results to the last workgroup.
 __device__ __forceinline__ bool last_workgroup(unsigned* ticket, unsigned nblk, unsigned b, const double acc[3],
                                                double* part)
 {
@@ -861,9 +862,6 @@ __device__ __forceinline__ void trace_diffG3_term(double wn, double rS, double i
     acc[1] += w * (b2 - a2) * r * r;
     acc[2] += w * (6.0 * a * b2 - 2.0 * a * a2) * r * r * r;
 }
-// pmu (and T, mu0) come from the root search st, so that a captured pass graph serves every
-// point; a settled search leaves nothing to do.  ticket != null: the workgroup that finishes
-// last takes the Halley step.
 // f(j, Sq[j]) for the stored frequencies j = lane, lane + 64, ... < H of a wavefront, in batches of kTD loads issued
 // before any use
 template <typename SelfT, typename Fn>
@@ -879,6 +877,9 @@ __device__ __forceinline__ void each_stored(const SelfT* __restrict__ Sq, int H,
     }
     for (; j < H; j += 64) f(j, Sq[j]);
 }
+// pmu (and T, mu0) come from the root search st, so that a captured pass graph serves every
+// point; a settled search leaves nothing to do.  ticket != null: the workgroup that finishes
+// last takes the Halley step.
 template <typename SelfT>
 __global__ void __launch_bounds__(256)
     k_trace_diffG3(const double* __restrict__ ekw, const double* __restrict__ wq, const SelfT* __restrict__ Self,
@@ -957,7 +958,7 @@ __global__ void __launch_bounds__(kSearchThreads)
 }
 
 // Tr Sigma G0 (green.cpp:3018-3084) in one pass over Sigma: part[b] its main sum, part[nblk + b] the Sigma_inf correction
-// (the n < Nw/2 terms plus one per k).  256^2 x 2048: 32 us mixed, 61 FP64 (a pass each: 2 x 27, 2 x 53)
+// (the n < Nw/2 terms plus one per k).  256^2 x 2048: 24 us mixed, 50 FP64 (a pass each: 2 x 27, 2 x 53)
 template <typename SelfT>
 __global__ void __launch_bounds__(256)
     k_trace_selfG0(const double* __restrict__ ekw, const double* __restrict__ wq, const SelfT* __restrict__ Self,
@@ -1215,7 +1216,7 @@ __global__ void __launch_bounds__(SlabShape<N>::NT)
 // phases run over the wedge: one exponential serves (kx, ky) and (ky, kx), and V(r) is read in order.
 // Bound by the two transforms (VALU and LDS).  At 256^2 x 2048 the h and f0 slices took 976 + 844 us (FP64)
 // and 628 + 399 us (FP32) as two kernels with h, f0 in global memory between them, two exponentials and
-// two divisions per point and index; now 2 x 452 and 2 x 295 us beside the self-energy kernels (FP32 alone: 195).
+// two divisions per point and index; now 2 x 445 and 2 x 290 us beside the self-energy kernels (FP32 alone: 195).
 template <int N, typename S>
 __global__ void __launch_bounds__(SlabShape<N>::NT, slab_occ<S>())
     k_hV_slab(const unsigned* __restrict__ wt, const double* __restrict__ ekw, const double* __restrict__ fw,

@@ -148,7 +148,6 @@ struct Grid {
     int prec;  // 0: FP64; 1: mixed (FP32 slab arrays, FP32-complex Sigma(k,iwn))
 };
 
-constexpr int kRedBlocks = 1024;
 constexpr int kRowGroups = 32;       // frequency-row groups of the reduction grids
 constexpr int kPartCap = 8192;       // capacity of DevArrays::part
 // A root-search pass ends with the Halley step of the workgroup that finishes last, through tickets on one counter at
@@ -186,6 +185,7 @@ constexpr int jj_points(long nq)
     const long kp = (nq + 1023) / 1024;
     return kp > 16 ? 16 : kp < 1 ? 1 : (int)kp;
 }
+constexpr int jj_samples(int Nw) { return Nw > 256 ? 8 : Nw > 64 ? Nw / 64 : 1; }
 // Workgroups on nq points, and the most on any lattice of at most nq points: a smaller lattice can have more (1023 points:
 // 1023, 2303 points: 768), and the stages run on sub-lattices of the context's
 constexpr long jj_blocks(long nq) { return (nq + jj_points(nq) - 1) / jj_points(nq); }
@@ -197,7 +197,6 @@ struct JJGroups {
     const int *order = nullptr, *first = nullptr;
     int n = 0;
 };
-constexpr int jj_samples(int Nw) { return Nw > 256 ? 8 : Nw > 64 ? Nw / 64 : 1; }
 
 // ---- launchers; each returns hipGetLastError() of its launch
 hipError_t launch_fill_tw(const DevArrays& d, int L, hipStream_t s);

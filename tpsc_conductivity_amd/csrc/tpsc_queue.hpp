@@ -1,8 +1,9 @@
 // tpsc_queue.hpp -- a whole solve queued without host waits (tpsc_capi.cpp), for the batch driver.
 //
 // tpsc_queue_solve re-targets a context to a point of its grid and precision and queues mu0,
-// chi0, the Usp / Uch / mu root searches (a fixed number of Halley passes each, one launch per
-// pass, settling into device memory that the stages after them read), the vertex, the
+// chi0, the Usp / Uch / mu root searches (a fixed number of Halley passes each, in one launch on
+// small grids and one launch per pass beyond, settling into device memory that the stages after
+// them read), the vertex, the
 // self-energy and the Lambda_jj bubble + MT on the context's main stream, then one kernel that
 // writes the results into `slot_dev` (the device address of tpsc_queue_slot_doubles doubles of
 // pinned, mapped host memory).  Nothing waits: points of several contexts run on the GPU back to
@@ -24,6 +25,7 @@
 // Halley passes queued per search {Usp, Uch, mu}.  Usp settles in 3-5 passes, up to 15 next to
 // the antiferromagnetic instability; Uch in 4-6; mu in 3-4.  A pass queued after its search has
 // settled returns at once, but its launch still costs the host ~10 us, the batch's bottleneck.
+// (Grids whose search is one launch, sum_in_one and mu_in_one, take the same numbers.)
 constexpr int kQueuedPasses[3] = {7, 6, 5};
 constexpr int kQueuedPassesLong[3] = {20, 10, 8};
 constexpr int kQueuePromote = 1;

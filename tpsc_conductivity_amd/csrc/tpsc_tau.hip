@@ -11,7 +11,8 @@ namespace tpsc {
 // is one access of both values (their only alignment is the element's).  Of an odd count's last pair the missing
 // pencil is read as zero; the read itself may pass the array's end by one element, for which every device array has
 // room (dalloc).  Four pencils (two pairs in turn, one access a row) measured 0-30% slower: more registers, fewer
-// workgroups.
+// workgroups.  The split of a pair is exact to the rounding of the larger of the two, and a NaN in one pencil
+// spreads to its partner.
 template <typename S, int Q>
 struct __attribute__((packed, aligned(sizeof(S)))) Row {
     S v[Q];
@@ -461,7 +462,7 @@ __global__ void __launch_bounds__(Pen<L>::NT, 4)
     for (int m = 0; m < 4; m++) Z[m * PS + t] = v[4 + m];
     __syncthreads();
     const int ka = k0;
-    const bool wa = nq > 0, wb = nq > 1;
+    const bool two = nq > 1;
     const double s20 = d0[0] + dN[0], s21 = d0[1] + dN[1];
     const double s30 = -(ends[0] + ends[2]), s31 = -(ends[1] + ends[3]);
 #pragma unroll
@@ -472,18 +473,18 @@ __global__ void __launch_bounds__(Pen<L>::NT, 4)
         const cd A = sigma_tail(cd{0.5 * (D.x + E.x), -0.5 * (D.y - E.y)}, x, u, ends[0], ends[2], g.ih);
         const cd B = sigma_tail(cd{0.5 * (D.y + E.y), 0.5 * (D.x - E.x)}, x, u, ends[1], ends[3], g.ih);
         const double wn = (2 * n + 1) * piT;
-        if (wa) store_self(Self, (long)ka * H + n, A, Si, s20, s30, wn);
-        if (wb) store_self(Self, (long)(ka + 1) * H + n, B, Si, s21, s31, wn);
+        store_self(Self, (long)ka * H + n, A, Si, s20, s30, wn);
+        if (two) store_self(Self, (long)(ka + 1) * H + n, B, Si, s21, s31, wn);
         if (n == H - 1) {
-            if (wa) Sinf4[ka] = A.x;
-            if (wb) Sinf4[ka + 1] = B.x;
+            Sinf4[ka] = A.x;
+            if (two) Sinf4[ka + 1] = B.x;
         }
     }
-    if (t == 0 && wa) {
+    if (t == 0) {
         Sinf2[ka] = s20;
         Sinf3[ka] = s30;
     }
-    if (t == 0 && wb) {
+    if (t == 0 && two) {
         Sinf2[ka + 1] = s21;
         Sinf3[ka + 1] = s31;
     }
